@@ -17,6 +17,7 @@
 #include <string>
 #include <vector>
 
+#include "dense_args.h"
 #include "internal.h"
 
 using namespace s2m;
@@ -118,7 +119,7 @@ struct s2m_program {
     bool owns_device_copy = true;  // false: d_ops points into a caller-owned arena
     // compiled programs (hiprtc code object): dense-path kernels instead of a tape
     hipModule_t module = nullptr;
-    hipFunction_t k_eval = nullptr, k_normals = nullptr;
+    hipFunction_t k_lattice = nullptr, k_signs = nullptr, k_contour = nullptr, k_emit = nullptr;
 };
 
 struct s2m_ctx {
@@ -126,9 +127,8 @@ struct s2m_ctx {
     hipStream_t stream = nullptr;
     int profiling = 0;  // 0 off, 1 total + evaluation kernels, 2 every stage
     s2m_timing timing{};
-    DevBuf lattice, vidx, bcount, boffset, actbits, counters, tables, check;
-    DevBuf lattice2, actbits2, bcount2;  // the dense path's second slab buffers (evaluation and
-                                         // count pass one slab ahead)
+    DevBuf lattice, bcount, counters, tables, check;
+    DevBuf dense;  // the dense path's working buffers (DenseLayout)
     // s2m_mesh_batch_device: the meshes of its dense-path jobs (vertices, keys, signs,
     // triangles: four buffers per job), kept beside the shared pass's output buffers
     std::vector<DevBuf> batch_dense;
@@ -164,7 +164,7 @@ struct s2m_ctx {
     // streamed readback (s2m_mesh): device-to-host copies of finished passes run on
     // copy_stream while later passes compute on `stream`
     hipStream_t copy_stream = nullptr;
-    // dense slabs: the lattice of slab k + 1 is evaluated on eval_stream while slab k is
+    // dense slabs: the signs of slab k + 1 are evaluated on eval_stream while slab k is
     // contoured on `stream`
     hipStream_t eval_stream = nullptr;
     PinnedBuf host_snap;                 // per pass: k_snapshot's totals and capacity use
@@ -343,14 +343,21 @@ int prepare_job(const s2m_params* p, Job& j)
     return S2M_OK;
 }
 
-uint32_t pick_slab(const s2m_params* p, const Job& j)
+uint32_t pick_slab(const s2m_params* p, const Job& j, bool streamed)
 {
     const uint64_t plane = (uint64_t)j.res[0] * j.res[1];
     if (plane == 0) return 1;
     uint64_t t = p->slab;
-    // ~32M cells per slab: at 1024^2 cells per plane, 32 planes (fewer, fuller launches;
-    // measured 66 ms per Mandelbulb job against 75 ms at 8 planes, no gain beyond 32)
-    if (t == 0) t = std::max<uint64_t>(1, (32ull << 20) / plane);
+    // A slab costs about 65 us of launches and latency beside its cells, so as few as the
+    // tables allow (64M cells; Mandelbulb 1024^3 left on the device: 8.0 ms at 16 planes per
+    // slab, 6.1 at 32, 5.3 at 63).  Streamed to host memory, a slab's copy runs beside the next
+    // slab's work: 16 slabs of at least 8M cells (Mandelbulb 512^3: 3.28 ms in 2 slabs, 2.63
+    // in 16; 256^3: 1.02 ms in 1 slab, 0.98 in 2, but a compiled CSG program with a third of
+    // the vertices 0.385 in 1, 0.389 in 2, 0.454 in 4).
+    const uint64_t cells = plane * j.nz_cells;
+    const uint64_t slab_cells = streamed ? std::min<uint64_t>(std::max<uint64_t>(cells / 16, 8ull << 20), 64ull << 20)
+                                         : 64ull << 20;
+    if (t == 0) t = std::max<uint64_t>(1, (slab_cells + plane - 1) / plane);
     // keep the per-slab block count within one scan block
     const uint64_t max_t = std::max<uint64_t>(1, ((uint64_t)kMaxScanBlocks * kCellsPerBlock) / plane);
     t = std::min<uint64_t>(t, max_t);
@@ -366,45 +373,62 @@ size_t tables_bytes(const Job& j)
         nf += j.ax[a].coord.size();
         nu += 2 * j.ax[a].lo.size();
     }
-    return nf * 4 + nu * 4 + 64;
+    return (2 * nf * 4 + nu * 4 + 15) & ~size_t(15);
 }
 
-// Upload the three axis tables: [cx cy cz | lox hix loy hiy loz hiz] as one buffer, into
-// `dst` (tables_bytes(j) bytes of device memory) or, when dst is NULL, the context's
-// table buffer.
-int upload_tables(s2m_ctx* ctx, const Job& j, const float* (&c)[3], const uint32_t* (&lo)[3],
-                  const uint32_t* (&hi)[3], void* dst = nullptr)
+// The axis tables of a dense job on the device.
+struct DeviceTables {
+    const float* c[3];         // coordinates
+    const uint32_t* lo[3];     // per cell: index of its min / max corner's coordinate
+    const uint32_t* hi[3];
+    const uint32_t* cell[3];   // per coordinate: the cell whose min corner it is, kNoCell
+};
+
+// The three axis tables as one buffer, [cx cy cz | lox hix loy hiy loz hiz | cells], at `dst`
+// (tables_bytes(j) bytes of device memory).  staged != NULL: written to page-locked memory
+// mapped for the device, *staged, from which the job's first kernel copies them (unchanged
+// until the job's last synchronisation); else the copy is made here and waited for.
+int upload_tables(s2m_ctx* ctx, const Job& j, DeviceTables& t, void* dst, void** staged)
 {
+    const bool pinned = staged != nullptr;
     size_t nf = 0;
     for (int a = 0; a < 3; ++a) nf += j.ax[a].coord.size();
-    std::vector<uint8_t> host(tables_bytes(j));
-    float* fp = reinterpret_cast<float*>(host.data());
-    uint32_t* up = reinterpret_cast<uint32_t*>(host.data() + nf * 4);
-    size_t fo[3], lo_o[3], hi_o[3], f = 0, u = 0;
+    const size_t bytes = tables_bytes(j);
+    std::vector<uint8_t> own(pinned ? 0 : bytes);
+    if (pinned) HIP_TRY(ctx->host_img.ensure(bytes));
+    uint8_t* host = pinned ? ctx->host_img.as<uint8_t>() : own.data();
+    float* fp = reinterpret_cast<float*>(host);
+    uint32_t* up = reinterpret_cast<uint32_t*>(host + nf * 4);
+    size_t fo[3], lo_o[3], hi_o[3], ce_o[3], f = 0, u = 0;
     for (int a = 0; a < 3; ++a) {
+        const AxisTable& ax = j.ax[a];
         fo[a] = f;
-        std::copy(j.ax[a].coord.begin(), j.ax[a].coord.end(), fp + f);
-        f += j.ax[a].coord.size();
+        std::copy(ax.coord.begin(), ax.coord.end(), fp + f);
+        f += ax.coord.size();
         lo_o[a] = u;
-        std::copy(j.ax[a].lo.begin(), j.ax[a].lo.end(), up + u);
-        u += j.ax[a].lo.size();
+        std::copy(ax.lo.begin(), ax.lo.end(), up + u);
+        u += ax.lo.size();
         hi_o[a] = u;
-        std::copy(j.ax[a].hi.begin(), j.ax[a].hi.end(), up + u);
-        u += j.ax[a].hi.size();
+        std::copy(ax.hi.begin(), ax.hi.end(), up + u);
+        u += ax.hi.size();
+        ce_o[a] = u;
+        std::fill(up + u, up + u + ax.coord.size(), kNoCell);
+        for (uint32_t i = 0; i < ax.lo.size(); ++i) up[u + ax.lo[i]] = i;
+        u += ax.coord.size();
     }
-    if (!dst) {
-        HIP_TRY(ctx->tables.ensure(host.size()));
-        dst = ctx->tables.p;
+    if (pinned) {
+        HIP_TRY(hipHostGetDevicePointer(staged, host, 0));
+    } else {
+        HIP_TRY(hipMemcpyAsync(dst, host, bytes, hipMemcpyHostToDevice, ctx->stream));
+        HIP_TRY(hipStreamSynchronize(ctx->stream));  // `own` must outlive the copy
     }
-    HIP_TRY(hipMemcpyAsync(dst, host.data(), host.size(), hipMemcpyHostToDevice, ctx->stream));
-    // the host vector must outlive the async copy
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
     const float* dfp = static_cast<const float*>(dst);
     const uint32_t* dup = reinterpret_cast<const uint32_t*>(static_cast<const uint8_t*>(dst) + nf * 4);
     for (int a = 0; a < 3; ++a) {
-        c[a] = dfp + fo[a];
-        lo[a] = dup + lo_o[a];
-        hi[a] = dup + hi_o[a];
+        t.c[a] = dfp + fo[a];
+        t.lo[a] = dup + lo_o[a];
+        t.hi[a] = dup + hi_o[a];
+        t.cell[a] = dup + ce_o[a];
     }
     return S2M_OK;
 }
@@ -550,12 +574,15 @@ int readback_begin(s2m_ctx* ctx, Readback& rb, uint64_t vcap, uint64_t tcap)
     return S2M_OK;
 }
 
-// After pass (or slab) k's kernels: its snapshot and event.
+// After pass (or slab) k's kernels: its event, and its snapshot (counters NULL: the slab's
+// last kernel wrote it).
 int readback_mark(s2m_ctx* ctx, const uint64_t* counters, uint32_t k)
 {
-    void* dev = nullptr;
-    HIP_TRY(hipHostGetDevicePointer(&dev, ctx->host_snap.p, 0));
-    HIP_TRY(launch_snapshot(ctx->stream, counters, static_cast<uint64_t*>(dev) + 4 * (size_t)k));
+    if (counters) {
+        void* dev = nullptr;
+        HIP_TRY(hipHostGetDevicePointer(&dev, ctx->host_snap.p, 0));
+        HIP_TRY(launch_snapshot(ctx->stream, counters, static_cast<uint64_t*>(dev) + 4 * (size_t)k));
+    }
     hipEvent_t e = ctx->pass_event(k);
     if (!e) return fail(S2M_E_HIP, "event creation failed");
     HIP_TRY(hipEventRecord(e, ctx->stream));
@@ -1237,31 +1264,39 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
     return fail(S2M_E_OOM, "output buffers kept overflowing");
 }
 
-// Lattice evaluation and vertex normals of a program: the tape interpreter's kernels,
-// or the kernels of a compiled program (same bodies, device_dense.h).
-hipError_t eval_lattice_prog(hipStream_t s, const s2m_program* prog, const float* cx, const float* cy,
-                             const float* cz, uint32_t nx, uint32_t ny, uint32_t lz0, uint32_t nzl,
-                             uint32_t pitch, float* lat)
+// The evaluating kernels of a program: the tape interpreter's, or those of a compiled
+// program (same bodies, device_dense.h).
+hipError_t lattice_prog(hipStream_t s, const s2m_program* prog, const float* cx, const float* cy, const float* cz,
+                        uint32_t nx, uint32_t ny, uint32_t lz0, uint32_t nzl, uint32_t pitch, float* lat)
 {
-    if (!prog->module && prog->n == 1 && prog->ops[0].code == S2M_OP_MANDELBULB)
-        return launch_eval_mandelbulb(s, prog->d_ops, cx, cy, cz, nx, ny, lz0, nzl, pitch, lat);
     if (!prog->module)
         return launch_eval_lattice(s, prog->d_ops, prog->n, cx, cy, cz, nx, ny, lz0, nzl, pitch, lat);
     if (nx == 0 || ny == 0 || nzl == 0) return hipSuccess;
     void* args[] = {&cx, &cy, &cz, &nx, &ny, &lz0, &nzl, &pitch, &lat};
-    return hipModuleLaunchKernel(prog->k_eval, (nx + 15) / 16, (ny + 3) / 4, (nzl + 3) / 4, 256, 1, 1, 0, s,
+    return hipModuleLaunchKernel(prog->k_lattice, (nx + 15) / 16, (ny + 3) / 4, (nzl + 3) / 4, 256, 1, 1, 0, s,
                                  args, nullptr);
 }
 
-hipError_t normals_prog(hipStream_t s, const s2m_program* prog, float eps, const MeshBufs& b)
+hipError_t signs_prog(hipStream_t s, const s2m_program* prog, BrickArgs a)
 {
-    if (!prog->module)
-        return launch_normals(s, prog->d_ops, prog->n, eps, b, prog->n == 1 && prog->ops[0].code == S2M_OP_MANDELBULB);
-    float* vtx = b.vtx;
-    const uint64_t* counters = b.counters;
-    uint64_t vcap = b.vcap;
-    void* args[] = {&eps, &vtx, &counters, &vcap};
-    return hipModuleLaunchKernel(prog->k_normals, 1024, 1, 1, 256, 1, 1, 0, s, args, nullptr);
+    if (!prog->module) return launch_signs(s, a, prog->ops.data(), prog->d_ops, prog->n);
+    void* args[] = {&a};
+    const dim3 g = sign_grid(a);
+    return hipModuleLaunchKernel(prog->k_signs, g.x, g.y, g.z, 256, 1, 1, 0, s, args, nullptr);
+}
+
+hipError_t contour_prog(hipStream_t s, const s2m_program* prog, BrickArgs a)
+{
+    if (!prog->module) return launch_contour(s, a, prog->ops.data(), prog->d_ops, prog->n);
+    void* args[] = {&a};
+    return hipModuleLaunchKernel(prog->k_contour, kBrickBlocks, 1, 1, 256, 1, 1, 0, s, args, nullptr);
+}
+
+hipError_t emit_prog(hipStream_t s, const s2m_program* prog, BrickArgs a)
+{
+    if (!prog->module) return launch_emit(s, a, prog->ops.data(), prog->d_ops, prog->n);
+    void* args[] = {&a};
+    return hipModuleLaunchKernel(prog->k_emit, kBrickBlocks, 1, 1, 256, 1, 1, 0, s, args, nullptr);
 }
 
 // Buffers of a dense job that must not allocate (s2m_mesh_device_noalloc): every working
@@ -1277,37 +1312,56 @@ struct FixedBufs {
     uint64_t vcap, tcap;
 };
 
-// Working-buffer sizes of a dense job streamed in slabs of T cell planes.
+// Working buffers of a dense job streamed in slabs of T cell planes, carved from one
+// region, each part 256-byte aligned.  Two sets of sign words when the signs are evaluated
+// a slab ahead; always two of the activity bits and their prefix tables (the quads of a
+// slab read the slab before).
 struct DenseLayout {
-    uint32_t T, nx, ny, pitch, max_nzl, max_blocks;
-    size_t tables, lattice, vidx, blocks, actbits, counters;
-    size_t carved() const  // bytes when carved from one region, each part 256-byte aligned
+    uint32_t T, nx, ny, nbx, nby, max_nzl, max_blocks;
+    size_t stage_cap;
+    size_t tables, words, vals, recs, stage, stage_sign, actbits, wpre, blocks, chunks, tblocks, counters;
+    bool piped;   // two sets of words and values
+    size_t carved() const
     {
         size_t b = 0;
-        for (size_t n : {tables, lattice, vidx, blocks, blocks, actbits, counters}) b += (n + 255) & ~size_t(255);
+        for (size_t n : {tables, words, piped ? words : 0, vals, piped ? vals : 0, recs, stage, stage_sign, actbits, actbits, wpre, wpre,
+                         blocks, blocks, chunks, chunks, tblocks, tblocks, counters})
+            b += (n + 255) & ~size_t(255);
         return b;
     }
 };
 
-DenseLayout dense_layout(const Job& j, uint32_t T, bool lattice)
+// stage_cap: vertices staged per slab, 0 for one per cell.  vals: the values of bricks with
+// both signs are kept.
+DenseLayout dense_layout(const Job& j, uint32_t T, bool bricks, bool piped, uint64_t stage_cap, bool vals)
 {
     DenseLayout L{};
     const uint64_t plane = (uint64_t)j.res[0] * j.res[1];
     L.T = T;
     L.nx = (uint32_t)j.ax[0].coord.size();
     L.ny = (uint32_t)j.ax[1].coord.size();
-    L.pitch = (L.nx + 63u) & ~63u;
-    for (uint32_t z0 = 0; z0 < j.nz_cells; z0 += T) {  // largest lattice z extent of any slab
+    L.nbx = (L.nx + 3u) / 4u;
+    L.nby = (L.ny + 3u) / 4u;
+    for (uint32_t z0 = 0; bricks && z0 < j.nz_cells; z0 += T) {  // largest lattice z extent of any slab
         const uint32_t z1 = std::min(z0 + T, j.nz_cells);
         L.max_nzl = std::max(L.max_nzl, j.ax[2].hi[z1 - 1] - j.ax[2].lo[z0] + 1);
     }
+    const size_t nbricks = bricks ? (size_t)L.nbx * L.nby * ((L.max_nzl + 3u) / 4u) : 0;
     L.max_blocks = (uint32_t)((plane * T + kCellsPerBlock - 1) / kCellsPerBlock);
+    L.stage_cap = bricks ? (size_t)(stage_cap ? std::min<uint64_t>(stage_cap, plane * T) : plane * T) : 0;
+    L.piped = piped;
     L.tables = tables_bytes(j);
-    L.lattice = lattice ? (size_t)L.pitch * L.ny * L.max_nzl * sizeof(float) : 0;
-    L.vidx = (size_t)(T + 1) * plane * sizeof(uint32_t);
+    L.words = nbricks * sizeof(uint64_t);
+    L.vals = vals ? nbricks * 64 * sizeof(float) : 0;
+    L.recs = nbricks * sizeof(BrickRec);
+    L.stage = L.stage_cap * 3 * sizeof(float);
+    L.stage_sign = L.stage_cap;
     L.blocks = (size_t)L.max_blocks * sizeof(uint32_t);
     L.actbits = (size_t)L.max_blocks * (kCellsPerBlock / 64) * sizeof(uint64_t);
-    L.counters = (kNumCounters + kDenseScanParts) * sizeof(uint64_t);  // the scan's chunk sums after them
+    L.wpre = (size_t)L.max_blocks * (kCellsPerBlock / 64) * sizeof(uint16_t);
+    L.tblocks = (size_t)((plane * T + kBlock - 1) / kBlock) * sizeof(uint32_t);
+    L.chunks = kRankChunks * sizeof(uint32_t);
+    L.counters = kNumCounters * sizeof(uint64_t);
     return L;
 }
 
@@ -1331,69 +1385,15 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
     if (fx && h_corners) return fail(S2M_E_ARG, "corner dumps are not contoured without allocation");
     const bool prof = ctx->profiling && !fx;  // events are created on first use
 
-    uint32_t slab = pick_slab(p, j);
+    uint32_t slab = pick_slab(p, j, rb != nullptr);
     if (prog && !fx && p->slab == 0) {  // the autotuner's slab for this job, if it chose one
         TuneChoice tc;
         if (tune_lookup(tune_key(ctx, prog, p, j), &tc) && tc.dense_slab) {
             s2m_params q = *p;
             q.slab = tc.dense_slab;
-            slab = pick_slab(&q, j);
+            slab = pick_slab(&q, j, false);
         }
     }
-    DenseLayout L = dense_layout(j, slab, !h_corners);
-    if (fx) {  // the largest slab (at most the usual one) whose buffers fit the scratch
-        while (L.T > 1 && L.carved() > fx->scratch_bytes) L = dense_layout(j, L.T - 1, true);
-        if (L.carved() > fx->scratch_bytes)
-            return fail(S2M_E_ARG, "a %u x %u grid needs %llu bytes of working memory per cell plane; "
-                                   "the no-allocation scratch holds %llu",
-                        j.res[0], j.res[1], (unsigned long long)L.carved(),
-                        (unsigned long long)fx->scratch_bytes);
-    }
-    const uint32_t T = L.T, nx = L.nx, ny = L.ny, pitch = L.pitch, max_blocks = L.max_blocks;
-
-    float* lat = nullptr;
-    uint32_t *vidx = nullptr, *bcount = nullptr, *boffset = nullptr;
-    uint64_t *actbits = nullptr, *counters = nullptr;
-    void* tables_at = nullptr;
-    if (fx) {
-        uint8_t* at = fx->scratch;
-        auto take = [&at](size_t n) {
-            uint8_t* q = at;
-            at += (n + 255) & ~size_t(255);
-            return q;
-        };
-        tables_at = take(L.tables);
-        lat = reinterpret_cast<float*>(take(L.lattice));
-        vidx = reinterpret_cast<uint32_t*>(take(L.vidx));
-        bcount = reinterpret_cast<uint32_t*>(take(L.blocks));
-        boffset = reinterpret_cast<uint32_t*>(take(L.blocks));
-        actbits = reinterpret_cast<uint64_t*>(take(L.actbits));
-        counters = reinterpret_cast<uint64_t*>(take(L.counters));
-    } else {
-        if (!h_corners) HIP_TRY(ctx->lattice.ensure(L.lattice));
-        HIP_TRY(ctx->vidx.ensure(L.vidx));
-        HIP_TRY(ctx->bcount.ensure(L.blocks));
-        HIP_TRY(ctx->boffset.ensure(L.blocks));
-        HIP_TRY(ctx->actbits.ensure(L.actbits));
-        HIP_TRY(ctx->counters.ensure(L.counters));
-        lat = ctx->lattice.as<float>();
-        vidx = ctx->vidx.as<uint32_t>();
-        bcount = ctx->bcount.as<uint32_t>();
-        boffset = ctx->boffset.as<uint32_t>();
-        actbits = ctx->actbits.as<uint64_t>();
-        counters = ctx->counters.as<uint64_t>();
-    }
-    const float* dc[3];
-    const uint32_t* dlo[3];
-    const uint32_t* dhi[3];
-    rc = upload_tables(ctx, j, dc, dlo, dhi, tables_at);
-    if (rc) return rc;
-    if (h_corners) {
-        HIP_TRY(ctx->corners.ensure((size_t)total_cells * 8 * sizeof(float)));
-        HIP_TRY(hipMemcpyAsync(ctx->corners.p, h_corners, (size_t)total_cells * 8 * sizeof(float),
-                               hipMemcpyHostToDevice, ctx->stream));
-    }
-
     // Output capacity: a closed surface crosses O(res^2) cells; start from 12 per
     // row-plane cell and grow once if the counters report more.
     const uint64_t est_v = std::min<uint64_t>(total_cells, std::max<uint64_t>(65536, 12 * plane));
@@ -1403,33 +1403,84 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
         want_v = fx->vcap;
         want_t = fx->tcap;
     }
+    uint64_t want_s = fx ? 0 : est_v + est_v / 4;  // staged vertices of a slab (cells with a sign change)
+    // Several slabs: slab k + 1's signs are evaluated (VALU-bound) on eval_stream, into the
+    // other of two sets of sign words (and kept values), while slab k is contoured on the context's stream.
+    // Events order it: a slab's bricks are listed after its evaluation, an evaluation waits
+    // until the slab two before has contoured its bricks (the last reader of its words and
+    // kept values), and the first evaluation waits for the tables queued before it.
+    const bool piped = !fx && !h_corners && slab < j.nz_cells;
+    const bool keep_vals = prog && !fx && !h_corners && !sign_early(prog->ops.data(), prog->n);
+    DenseLayout L = dense_layout(j, slab, !h_corners, piped, want_s, keep_vals);
+    if (fx) {  // the largest slab (at most the usual one) whose buffers fit the scratch
+        while (L.T > 1 && L.carved() > fx->scratch_bytes) L = dense_layout(j, L.T - 1, true, false, 0, false);
+        if (L.carved() > fx->scratch_bytes)
+            return fail(S2M_E_ARG, "a %u x %u grid needs %llu bytes of working memory per cell plane; "
+                                   "the no-allocation scratch holds %llu",
+                        j.res[0], j.res[1], (unsigned long long)L.carved(),
+                        (unsigned long long)fx->scratch_bytes);
+    }
+    const uint32_t T = L.T;
+    if (h_corners) {
+        HIP_TRY(ctx->corners.ensure((size_t)total_cells * 8 * sizeof(float)));
+        HIP_TRY(hipMemcpyAsync(ctx->corners.p, h_corners, (size_t)total_cells * 8 * sizeof(float),
+                               hipMemcpyHostToDevice, ctx->stream));
+    }
     const bool normals = prog && !(p->flags & S2M_NO_NORMALS);
     const uint32_t nslabs = (j.nz_cells + T - 1) / T;
     if (nslabs == 1) rb = nullptr;  // nothing to overlap: the caller copies the finished mesh
-    if (rb) HIP_TRY(ctx->host_snap.ensure((size_t)nslabs * 4 * sizeof(uint64_t)));
-    // Several slabs: slab k + 1's lattice is evaluated (VALU-bound) on eval_stream, into
-    // the other of two sets of slab buffers, while slab k is counted (the activity bits and
-    // block counts: latency-bound gathers) and gets its map, vertices, normals and
-    // triangles on the context's stream; the two streams then carry about equal work per
-    // slab.  Events order it: a slab's count waits for its evaluation, an evaluation waits
-    // until the slab two before has finished with its buffers (its last kernel), and the
-    // first evaluation waits for the tables and clears queued before it.
-    const bool piped = !fx && !h_corners && nslabs > 1;
+    void* snap_dev = nullptr;
+    if (rb) {
+        HIP_TRY(ctx->host_snap.ensure((size_t)nslabs * 4 * sizeof(uint64_t)));
+        HIP_TRY(hipHostGetDevicePointer(&snap_dev, ctx->host_snap.p, 0));
+    }
     hipStream_t es = piped ? ctx->eval_stream : ctx->stream;
-    float* lat_buf[2] = {lat, lat};
-    uint64_t* act_buf[2] = {actbits, actbits};
-    uint32_t* cnt_buf[2] = {bcount, bcount};
-    if (piped) {
-        HIP_TRY(ctx->lattice2.ensure(L.lattice));
-        HIP_TRY(ctx->actbits2.ensure(L.actbits));
-        HIP_TRY(ctx->bcount2.ensure(L.blocks));
-        lat_buf[1] = ctx->lattice2.as<float>();
-        act_buf[1] = ctx->actbits2.as<uint64_t>();
-        cnt_buf[1] = ctx->bcount2.as<uint32_t>();
+    void* back_dev = nullptr;  // mapped host memory for the counters
+    if (!fx) {
+        HIP_TRY(ctx->host_back.ensure(kNumCounters * sizeof(uint64_t)));
+        HIP_TRY(hipHostGetDevicePointer(&back_dev, ctx->host_back.p, 0));
     }
 
     for (int attempt = 0; attempt < (fx ? 1 : 3); ++attempt) {
+        // the working buffers
+        if (!fx) {
+            if (attempt) L = dense_layout(j, T, !h_corners, piped, want_s, keep_vals);
+            HIP_TRY(ctx->dense.ensure(L.carved()));
+        }
+        uint8_t* at = fx ? fx->scratch : ctx->dense.as<uint8_t>();
+        auto take = [&at](size_t n) {
+            uint8_t* q = at;
+            at += (n + 255) & ~size_t(255);
+            return q;
+        };
+        DeviceTables dt;
+        void* const tables_at = take(L.tables);
+        void* tables_from = nullptr;
+        rc = upload_tables(ctx, j, dt, tables_at, fx ? nullptr : &tables_from);
+        if (rc) return rc;
+        uint64_t* words[2];
+        words[0] = words[1] = reinterpret_cast<uint64_t*>(take(L.words));
+        if (piped) words[1] = reinterpret_cast<uint64_t*>(take(L.words));
+        float* vals[2];
+        vals[0] = vals[1] = L.vals ? reinterpret_cast<float*>(take(L.vals)) : nullptr;
+        if (piped && L.vals) vals[1] = reinterpret_cast<float*>(take(L.vals));
+        BrickRec* recs = reinterpret_cast<BrickRec*>(take(L.recs));
+        float* stage = reinterpret_cast<float*>(take(L.stage));
+        uint8_t* stage_sign = take(L.stage_sign);
+        uint64_t* act_buf[2];
+        uint16_t* pre_buf[2];
+        uint32_t* off_buf[2];
+        uint32_t* base_buf[2];
+        for (int k = 0; k < 2; ++k) {
+            act_buf[k] = reinterpret_cast<uint64_t*>(take(L.actbits));
+            pre_buf[k] = reinterpret_cast<uint16_t*>(take(L.wpre));
+            off_buf[k] = reinterpret_cast<uint32_t*>(take(L.blocks));
+            base_buf[k] = reinterpret_cast<uint32_t*>(take(L.chunks));
+        }
         MeshBufs b{};
+        b.tcount = reinterpret_cast<uint32_t*>(take(L.tblocks));
+        b.toffset = reinterpret_cast<uint32_t*>(take(L.tblocks));
+        b.counters = reinterpret_cast<uint64_t*>(take(L.counters));
         if (fx) {
             b.vtx = fx->vtx;
             b.keys = fx->keys;
@@ -1449,21 +1500,14 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
         }
         b.vcap = want_v;
         b.tcap = want_t;
-        b.counters = counters;
-        b.bcount = bcount;
-        b.boffset = boffset;
-        b.actbits = actbits;
         if (rb) {  // host arrays for this job's own estimate, not the context's largest job
             const int rrc = readback_begin(ctx, *rb, std::min(want_v, est_v), std::min(want_t, 3 * est_v));
             if (rrc) return rrc;
         }
 
-        HIP_TRY(hipMemsetAsync(b.counters, 0, kNumCounters * sizeof(uint64_t), ctx->stream));
-        HIP_TRY(hipMemsetAsync(vidx, 0xff, (size_t)plane * sizeof(uint32_t), ctx->stream));
-        // the count pass ORs into zeroed words; each slab's words are cleared after its quad pass
-        for (uint64_t* words : {act_buf[0], act_buf[1]})
-            HIP_TRY(hipMemsetAsync(words, 0, (size_t)max_blocks * (kCellsPerBlock / 64) * sizeof(uint64_t),
-                                   ctx->stream));
+        HIP_TRY(launch_dense_begin(ctx->stream, b.counters, act_buf[0],
+                                   (uint32_t)(plane * std::min(T, j.nz_cells)), tables_from, tables_at,
+                                   tables_from ? L.tables : 0, base_buf[0]));
 
         ctx->events_used = 0;
         // per slab 6 marks: evaluation start and end (on the evaluation's stream), then on
@@ -1479,7 +1523,7 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
             if (e && hipEventRecord(e, st) != hipSuccess) e = nullptr;
             return e;
         };
-        hipEvent_t lat_free[2] = {nullptr, nullptr};  // per buffer set: its slab's last kernel done
+        hipEvent_t words_free[2] = {nullptr, nullptr};  // per set of sign words: read by its slab
         if (piped) {
             hipEvent_t ready = mark(ctx->stream);
             if (!ready) return fail(S2M_E_HIP, "event record failed");
@@ -1492,81 +1536,113 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
             const uint32_t lz0 = j.ax[2].lo[z0];
             const uint32_t nzl = j.ax[2].hi[z1 - 1] - lz0 + 1;
 
-            float* const lat_s = lat_buf[slabs & 1];
+            const int cur = (int)(slabs & 1);
             SlabArgs a{};
-            a.lat = lat_s;
-            a.pitch = pitch;
-            a.lat_ny = ny;
-            a.lz0 = lz0;
-            a.cx = dc[0];
-            a.cy = dc[1];
-            a.cz = dc[2];
-            a.lox = dlo[0];
-            a.hix = dhi[0];
-            a.loy = dlo[1];
-            a.hiy = dhi[1];
-            a.loz = dlo[2];
-            a.hiz = dhi[2];
+            a.cx = dt.c[0];
+            a.cy = dt.c[1];
+            a.cz = dt.c[2];
+            a.lox = dt.lo[0];
+            a.hix = dt.hi[0];
+            a.loy = dt.lo[1];
+            a.hiy = dt.hi[1];
+            a.loz = dt.lo[2];
+            a.hiz = dt.hi[2];
             a.rx = j.res[0];
             a.ry = j.res[1];
             a.z0 = z0;
             a.ncells = (uint32_t)(plane * nzc);
             a.div_rx = make_fastdiv(j.res[0]);
             a.div_rxy = make_fastdiv((uint32_t)plane);
-            a.vidx = vidx;
             a.flags = p->flags;
-            const uint32_t nb = (uint32_t)(((uint64_t)a.ncells + kCellsPerBlock - 1) / kCellsPerBlock);
+
+            MeshBufs bs = b;  // this slab's activity bits and their prefix tables
+            bs.actbits = act_buf[cur];
+            bs.bits = SlabBits{reinterpret_cast<unsigned long long*>(act_buf[cur]), pre_buf[cur], off_buf[cur],
+                               base_buf[cur], 0};
+            const SlabBits prev{reinterpret_cast<unsigned long long*>(act_buf[cur ^ 1]), pre_buf[cur ^ 1],
+                                off_buf[cur ^ 1], base_buf[cur ^ 1],
+                                (uint64_t)(T - 1) * plane};  // every earlier slab has T planes
+            BrickArgs A{};
+            A.cx = dt.c[0];
+            A.cy = dt.c[1];
+            A.cz = dt.c[2];
+            A.cox = dt.cell[0];
+            A.coy = dt.cell[1];
+            A.coz = dt.cell[2];
+            A.nx = L.nx;
+            A.ny = L.ny;
+            A.nzl = nzl;
+            A.lz0 = lz0;
+            A.nbx = L.nbx;
+            A.nby = L.nby;
+            A.nbz = (nzl + 3u) / 4u;
+            A.run = sign_run((uint64_t)A.nbx * A.nby * A.nbz);
+            A.rx = a.rx;
+            A.ry = a.ry;
+            A.z0 = z0;
+            A.z1 = z1;
+            A.words = words[piped ? cur : 0];
+            A.vals = vals[piped ? cur : 0];
+            A.recs = recs;
+            A.alloc = b.counters + kBrickAlloc;
+            A.stage = stage;
+            A.stage_sign = stage_sign;
+            A.stage_cap = (uint32_t)L.stage_cap;
+            A.actbits = reinterpret_cast<unsigned long long*>(act_buf[cur]);
+            A.wpre = pre_buf[cur];
+            A.boffset = off_buf[cur];
+            A.cbase = base_buf[cur];
+            A.vtx = b.vtx;
+            A.keys = b.keys;
+            A.signs = b.signs;
+            A.vcap = b.vcap;
+            A.eps = p->eps;
+            A.normals = normals ? 1u : 0u;
 
             hipEvent_t m[6] = {};
             if (prof)
                 for (auto& e : m) e = ctx->next_event();
-            if (piped && lat_free[slabs & 1]) HIP_TRY(hipStreamWaitEvent(es, lat_free[slabs & 1], 0));
+            if (piped && words_free[cur]) HIP_TRY(hipStreamWaitEvent(es, words_free[cur], 0));
             if (m[0]) HIP_TRY(hipEventRecord(m[0], es));
             if (!h_corners) {
-                HIP_TRY(eval_lattice_prog(es, prog, dc[0], dc[1], dc[2], nx, ny, lz0, nzl, pitch, lat_s));
-                lattice_points += (uint64_t)nx * ny * nzl;
+                HIP_TRY(signs_prog(es, prog, A));
+                lattice_points += (uint64_t)L.nx * L.ny * nzl;
             }
             if (m[1]) HIP_TRY(hipEventRecord(m[1], es));
-            if (m[5]) HIP_TRY(hipEventRecord(m[5], es));
-            MeshBufs bs = b;  // this slab's activity bits and block counts
-            bs.actbits = act_buf[slabs & 1];
-            bs.bcount = cnt_buf[slabs & 1];
             if (piped) {
                 hipEvent_t evaluated = mark(es);
                 if (!evaluated) return fail(S2M_E_HIP, "event record failed");
                 HIP_TRY(hipStreamWaitEvent(ctx->stream, evaluated, 0));
             }
-            if (!h_corners) HIP_TRY(launch_cells(ctx->stream, a, bs, 0, 0));  // the count pass
+            if (m[5]) HIP_TRY(hipEventRecord(m[5], ctx->stream));
+            const float* src = h_corners ? ctx->corners.as<float>() + (size_t)z0 * plane * 8 : nullptr;
             if (h_corners) {
-                const float* src = ctx->corners.as<float>() + (size_t)z0 * plane * 8;
-                HIP_TRY(launch_cells_from_corners(ctx->stream, a, src, b, 0));
-                HIP_TRY(launch_scan(ctx->stream, b, nb, 0));
-                HIP_TRY(launch_cells_from_corners(ctx->stream, a, src, b, 1));
+                HIP_TRY(launch_cells_from_corners(ctx->stream, a, src, bs, 0));
             } else {
-                HIP_TRY(launch_scan(ctx->stream, bs, nb, 0));
-                HIP_TRY(launch_cells(ctx->stream, a, bs, 1, normals ? 0 : 1));
+                HIP_TRY(launch_find_bricks(ctx->stream, A));
+                HIP_TRY(contour_prog(ctx->stream, prog, A));
+                if (piped) {
+                    words_free[cur] = mark(ctx->stream);
+                    if (!words_free[cur]) return fail(S2M_E_HIP, "event record failed");
+                }
             }
+            HIP_TRY(launch_ranks(ctx->stream, bs, a.ncells));
             if (m[2]) HIP_TRY(hipEventRecord(m[2], ctx->stream));
-            if (normals) HIP_TRY(normals_prog(ctx->stream, prog, p->eps, bs));
+            if (h_corners) HIP_TRY(launch_cells_from_corners(ctx->stream, a, src, bs, 1));
+            else HIP_TRY(emit_prog(ctx->stream, prog, A));
             if (m[3]) HIP_TRY(hipEventRecord(m[3], ctx->stream));
-            HIP_TRY(launch_quads(ctx->stream, a, bs, 0));
-            HIP_TRY(launch_scan(ctx->stream, bs, nb, 1));
-            HIP_TRY(launch_quads(ctx->stream, a, bs, 1));
-            HIP_TRY(launch_clear_bits(ctx->stream, bs.actbits, a.ncells));  // for the count two slabs on
+            HIP_TRY(launch_quads(ctx->stream, a, bs, prev));
+            // the other activity words cleared for the next slab; the totals for the host
+            HIP_TRY(launch_slab_end(ctx->stream, b.counters, act_buf[cur ^ 1],
+                                    (uint32_t)(plane * std::min(T, j.nz_cells - z1)), base_buf[cur ^ 1],
+                                    rb ? static_cast<uint64_t*>(snap_dev) + 4 * slabs : nullptr,
+                                    z1 == j.nz_cells ? static_cast<uint64_t*>(back_dev) : nullptr));
             if (m[4]) HIP_TRY(hipEventRecord(m[4], ctx->stream));
-            if (piped) {  // the slab's lattice, bits and counts are free for the slab two later
-                lat_free[slabs & 1] = mark(ctx->stream);
-                if (!lat_free[slabs & 1]) return fail(S2M_E_HIP, "event record failed");
-            }
             if (rb) {  // the slab's vertices and triangles are final; the copies of the slab two
                        // before (waiting for it leaves this slab and the next evaluation queued)
-                int rrc = readback_mark(ctx, b.counters, (uint32_t)slabs);
+                int rrc = readback_mark(ctx, nullptr, (uint32_t)slabs);
                 if (!rrc && slabs > 1) rrc = readback_pass(ctx, *rb, want_v, want_t, ~0ull, ~0ull);
                 if (rrc) return rrc;
-            }
-            if (z1 < j.nz_cells) {  // last map plane becomes the previous plane
-                HIP_TRY(hipMemcpyAsync(vidx, vidx + (size_t)nzc * plane, plane * sizeof(uint32_t),
-                                       hipMemcpyDeviceToDevice, ctx->stream));
             }
             if (prof) ev.insert(ev.end(), m, m + 6);
             ++slabs;
@@ -1580,8 +1656,9 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
             if (rrc) return rrc;
         }
         uint64_t cnt[kNumCounters];
-        HIP_TRY(hipMemcpyAsync(cnt, b.counters, sizeof cnt, hipMemcpyDeviceToHost, ctx->stream));
+        if (fx) HIP_TRY(hipMemcpyAsync(cnt, b.counters, sizeof cnt, hipMemcpyDeviceToHost, ctx->stream));
         HIP_TRY(hipStreamSynchronize(ctx->stream));
+        if (!fx) std::memcpy(cnt, ctx->host_back.p, sizeof cnt);
         if (prof) {
             float ms = 0;
             HIP_TRY(hipEventElapsedTime(&ms, ev_start, ev_end));
@@ -1609,7 +1686,8 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
         if (cnt[kVtxTotal] >= 0xffffffffull)
             return fail(S2M_E_ARG, "mesh has %llu vertices; indices are u32",
                         (unsigned long long)cnt[kVtxTotal]);
-        if (cnt[kVtxTotal] <= want_v && cnt[kTriTotal] <= want_t) {
+        const bool staged = cnt[kStageMax] <= L.stage_cap;
+        if (cnt[kVtxTotal] <= want_v && cnt[kTriTotal] <= want_t && staged) {
             ctx->last_nvtx = cnt[kVtxTotal];
             ctx->last_ntri = cnt[kTriTotal];
             ctx->last_invalid = cnt[kInvalid];
@@ -1627,8 +1705,9 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
         // vertices past the capacity form no quads, so after a vertex overflow the triangle
         // count is low: size triangles from the vertices as at the start
         if (cnt[kVtxTotal] > want_v) want_t = std::max<uint64_t>(want_t, 3 * (cnt[kVtxTotal] + cnt[kVtxTotal] / 8));
-        want_v = std::max<uint64_t>(want_v, cnt[kVtxTotal] + cnt[kVtxTotal] / 8 + 1024);
-        want_t = std::max<uint64_t>(want_t, cnt[kTriTotal] + cnt[kTriTotal] / 8 + 2048);
+        if (cnt[kVtxTotal] > want_v) want_v = cnt[kVtxTotal] + cnt[kVtxTotal] / 8 + 1024;
+        if (cnt[kTriTotal] > want_t) want_t = cnt[kTriTotal] + cnt[kTriTotal] / 8 + 2048;
+        if (!staged) want_s = cnt[kStageMax] + cnt[kStageMax] / 8 + 1024;
     }
     return fail(S2M_E_OOM, "output buffers kept overflowing");
 }
@@ -1751,7 +1830,7 @@ void s2m_destroy(s2m_ctx* ctx)
     (void)hipStreamSynchronize(ctx->stream);
     (void)hipStreamSynchronize(ctx->copy_stream);
     (void)hipStreamSynchronize(ctx->eval_stream);
-    for (DevBuf* b : {&ctx->lattice, &ctx->lattice2, &ctx->actbits2, &ctx->bcount2, &ctx->vidx, &ctx->bcount, &ctx->boffset, &ctx->actbits, &ctx->check, &ctx->counters,
+    for (DevBuf* b : {&ctx->lattice, &ctx->dense, &ctx->bcount, &ctx->check, &ctx->counters,
                       &ctx->tables, &ctx->vtx, &ctx->keys, &ctx->signs, &ctx->tri, &ctx->corners,
                       &ctx->tile_tab, &ctx->tile_lists, &ctx->tile_lens,
                       &ctx->tile_flops, &ctx->sp_slot_of_tile, &ctx->sp_tile_of_slot,
@@ -2506,14 +2585,13 @@ int s2m_eval_lattice_range(s2m_ctx* ctx, const s2m_program* prog, const s2m_para
     const uint64_t n = (uint64_t)dims[0] * dims[1] * dims[2];
     if (!out || cap < n) return fail(S2M_E_ARG, "output holds %llu floats, lattice has %llu",
                                      (unsigned long long)cap, (unsigned long long)n);
-    const float* dc[3];
-    const uint32_t* dlo[3];
-    const uint32_t* dhi[3];
-    rc = upload_tables(ctx, j, dc, dlo, dhi);
+    DeviceTables t;
+    HIP_TRY(ctx->tables.ensure(tables_bytes(j)));
+    rc = upload_tables(ctx, j, t, ctx->tables.p, nullptr);
     if (rc) return rc;
     HIP_TRY(ctx->lattice.ensure((size_t)n * sizeof(float)));
-    HIP_TRY(eval_lattice_prog(ctx->stream, prog, dc[0], dc[1], dc[2], dims[0], dims[1], *lz0, dims[2], dims[0],
-                              ctx->lattice.as<float>()));
+    HIP_TRY(lattice_prog(ctx->stream, prog, t.c[0], t.c[1], t.c[2], dims[0], dims[1], *lz0, dims[2], dims[0],
+                         ctx->lattice.as<float>()));
     HIP_TRY(hipMemcpyAsync(out, ctx->lattice.p, (size_t)n * sizeof(float), hipMemcpyDeviceToHost,
                            ctx->stream));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
@@ -2584,8 +2662,10 @@ int program_from_code_object(s2m_ctx* ctx, const void* code, size_t size, s2m_pr
     s2m_program* p = new s2m_program();
     p->device = ctx->device;
     hipError_t e = hipModuleLoadData(&p->module, code);
-    if (e == hipSuccess) e = hipModuleGetFunction(&p->k_eval, p->module, "s2m_c_eval_lattice");
-    if (e == hipSuccess) e = hipModuleGetFunction(&p->k_normals, p->module, "s2m_c_normals");
+    if (e == hipSuccess) e = hipModuleGetFunction(&p->k_lattice, p->module, "s2m_c_eval_lattice");
+    if (e == hipSuccess) e = hipModuleGetFunction(&p->k_signs, p->module, "s2m_c_signs");
+    if (e == hipSuccess) e = hipModuleGetFunction(&p->k_contour, p->module, "s2m_c_contour");
+    if (e == hipSuccess) e = hipModuleGetFunction(&p->k_emit, p->module, "s2m_c_emit");
     if (e != hipSuccess) {
         if (p->module) (void)hipModuleUnload(p->module);
         delete p;
@@ -2638,7 +2718,8 @@ uint64_t dense_request_bytes(const s2m_params* p)
     if (!p || prepare_job(p, j) != S2M_OK) return 0;
     const uint64_t plane = (uint64_t)j.res[0] * j.res[1];
     const uint64_t est_v = std::min<uint64_t>(plane * j.nz_cells, std::max<uint64_t>(65536, 12 * plane));
-    const DenseLayout L = dense_layout(j, pick_slab(p, j), true);
+    const uint32_t slab = pick_slab(p, j, true);
+    const DenseLayout L = dense_layout(j, slab, true, slab < j.nz_cells, est_v + est_v / 4, true);
     return L.carved() + est_v * (24 + 8 + 1) + 3 * est_v * 12;
 }
 

@@ -121,6 +121,100 @@ __device__ __forceinline__ float bailout_threshold(float b)
     return t;
 }
 
+// The power-8 Mandelbulb step without transcendentals or divisions, p already swizzled.
+// theta = atan(zy / zx) differs from the direction angle of (zx, zy) by 0 or pi, which
+// 8 * theta turns into a multiple of 8 pi: cos / sin of 8 theta are the components of
+// ((zx, zy) / rho)^8 as complex numbers (rho = |(zx, zy)|), three complex squarings of the
+// unit vector (1 / rho from a reciprocal square root).  phi = asin(zz / r) lies in
+// [-pi/2, pi/2], so r (cos phi, sin phi) = (rho, zz), and r^8 (cos 8 phi, sin 8 phi) =
+// (rho + i zz)^8: its first square is (rho^2 - zz^2, 2 rho zz) with rho^2 taken as
+// zx^2 + zy^2, then two more squarings.  So z' = (r^8 cos 8 phi (cos 8 theta, sin 8 theta),
+// r^8 sin 8 phi) + p without 1 / r; r^7 for dr is r^6 sqrt(r^2).  Fused multiply-adds where
+// a product meets a sum.  The same function as the written form, with its own roundings
+// (its error against the fp64 estimator is bounded as for the written form).  The bailout
+// test compares r^2 with the threshold whose correctly rounded square root first exceeds
+// the bailout, so every point leaves the loop where the written form does, with r = |z|
+// (hardware square root); a point that never bails out leaves with r = |z|^8 of the last
+// step, as the written form's r = pow(r, 8) (its z after that step is read by nothing and
+// not computed).  rho = 0 gives NaN, as atan(0 / 0) does.
+//
+// kSign: only the result's sign matters (the return is > 0 exactly where the value is).
+// The orbit is the same, ended as soon as the sign is certain; needs 1.5 <= bailout <= 16,
+// 0 <= offset <= 1000, iters >= 1 and gain <= 0.999 * 0.5 ln(bailout) bailout (mandel_gain):
+//   |p|^2 <= kMandelInner: |z| stays below 0.74 (0.74^8 + 0.648 < 0.74), so the last r < 1,
+//     ln r < 0 and the value is negative (or NaN);
+//   r >= bailout with dr * offset <= gain: 0.5 ln(r) r / dr exceeds the offset;
+//   r^8 > 1.01 (bailout + |p|): the next |z| >= r^8 - |p| is past the bailout (or, in the
+//     last step, r^8 itself is), with the dr of this step.  The percent covers the
+//     roundings of z' (about 2e-5) where xy2 is not tiny;
+//   a last r < 1: as for the inner ball.
+// On the cube of edge 2.5 this ends 58 % of the points in their first step.
+constexpr float kMandelInner = 0.42f;
+constexpr float kMandelAxis = 1e-27f;  // least xy2 the prediction of z' is used for
+
+__device__ __forceinline__ float mandel_gain(float bailout)
+{
+    return 0.4995f * 0.693147182f * __builtin_amdgcn_logf(bailout) * bailout;
+}
+
+template <bool kSign>
+__device__ __forceinline__ float mandelbulb8(float px, float py, float pz, float offset, uint32_t iters, float t2,
+                                             float bailout, float gain)
+{
+    float zx = px, zy = py, zz = pz;
+    float r = 0.0f, dr = 1.0f, far = 0.0f;
+    bool out = false;
+    if (kSign) {
+        const float c2 = (px * px + py * py) + pz * pz;
+        if (c2 <= kMandelInner) return -1.0f;
+        far = 1.01f * (bailout + __builtin_amdgcn_sqrtf(c2));
+    }
+    for (uint32_t i = 0; i < iters; ++i) {
+        const float xy2 = zx * zx + zy * zy;
+        const float r2 = xy2 + zz * zz;
+        if (r2 > t2) {  // z no longer changes past the bailout
+            r = __builtin_amdgcn_sqrtf(r2);
+            out = true;
+            break;
+        }
+        const float r4 = r2 * r2;
+        const float r7 = (r4 * r2) * __builtin_amdgcn_sqrtf(r2);
+        dr = __builtin_fmaf(r7 * dr, 8.0f, 1.0f);
+        r = r4 * r4;
+        if (kSign && r > far && xy2 >= kMandelAxis && dr * offset <= gain) return 1.0f;
+        if (i + 1u == iters) break;
+        const float irho = rsqrt_full(xy2);
+        const float rho = xy2 * irho;
+        float ct = zx * irho, st = zy * irho;
+        float cp = __builtin_fmaf(-zz, zz, xy2), sp = (rho + rho) * zz;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {  // (c + i s)^2 = (c^2 - s^2) + i 2cs, one rounding for the real part
+            const float c2 = __builtin_fmaf(ct, ct, -(st * st)), s2 = (ct + ct) * st;
+            ct = c2;
+            st = s2;
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const float p2 = __builtin_fmaf(cp, cp, -(sp * sp)), q2 = (cp + cp) * sp;
+            cp = p2;
+            sp = q2;
+        }
+        zx = __builtin_fmaf(cp, ct, px);
+        zy = __builtin_fmaf(cp, st, py);
+        zz = sp + pz;
+    }
+    if (kSign) {
+        if (!(r >= 1.0f)) return -1.0f;
+        if (out && dr * offset <= gain) return 1.0f;
+    }
+    // 0.5 ln(r) r / dr from the hardware log2 (times ln 2; a denormal r scaled by 2^24
+    // first) and reciprocal, each within about an ulp: dr >= 1, and r = 0 gives NaN as
+    // log(0) * 0 does
+    const bool tiny = r < 0x1p-126f;
+    const float lr = (__builtin_amdgcn_logf(tiny ? r * 0x1p24f : r) - (tiny ? 24.0f : 0.0f)) * 0.693147182f;
+    return ((0.5f * lr) * r) * __builtin_amdgcn_rcpf(dr) - offset;
+}
+
 // examples/mandelmesh.frag:3-28 with power, bailout, offset and the iteration count as
 // operands.  A bailed-out point keeps r = length(z): the loop `continue`s, so r is
 // recomputed from the unchanged z in every remaining iteration.  t2 =
@@ -135,71 +229,10 @@ __device__ __forceinline__ float sd_mandelbulb(float px, float py, float pz, flo
         pz = t;
     }
     const uint32_t iters = iarg & 0xffffu;
+    if (power == 8.0f && !(iarg & S2M_MANDEL_TRIG))
+        return mandelbulb8<false>(px, py, pz, offset, iters, t2, bailout, 0.0f);
     float zx = px, zy = py, zz = pz;
     float r = 0.0f, dr = 1.0f;
-    if (power == 8.0f && !(iarg & S2M_MANDEL_TRIG)) {
-        // The power-8 step without transcendentals or divisions.  theta = atan(zy / zx)
-        // differs from the direction angle of (zx, zy) by 0 or pi, which 8 * theta turns
-        // into a multiple of 8 pi: cos / sin of 8 theta are the components of
-        // ((zx, zy) / rho)^8 as complex numbers (rho = |(zx, zy)|), three complex squarings
-        // of the unit vector (1 / rho from a reciprocal square root).  phi = asin(zz / r)
-        // lies in [-pi/2, pi/2], so r (cos phi, sin phi) = (rho, zz), and
-        // r^8 (cos 8 phi, sin 8 phi) = (rho + i zz)^8: its first square is
-        // (rho^2 - zz^2, 2 rho zz) with rho^2 taken as zx^2 + zy^2, then two more squarings.
-        // So z' = (r^8 cos 8 phi (cos 8 theta, sin 8 theta), r^8 sin 8 phi) + p without 1 / r;
-        // r^7 for dr is r^6 sqrt(r^2).  Fused multiply-adds where a product meets a sum.
-        // The same function as the written form, with its own roundings (its error against
-        // the fp64 estimator is bounded as for the written form).  The bailout test
-        // compares r^2 with the threshold whose correctly rounded square root first exceeds
-        // the bailout, so every point leaves the loop where the written form does, with
-        // r = |z| (hardware square root); a point that never bails out leaves with
-        // r = |z|^8 of the last step, as the written form's r = pow(r, 8).  rho = 0 gives
-        // NaN, as atan(0 / 0) does.
-        float r2_out = -1.0f;  // r^2 where the point bailed out (the root is taken once, below)
-        float r2_last = 0.0f;  // r^2 of the last step taken
-        for (uint32_t i = 0; i < iters; ++i) {
-            const float xy2 = zx * zx + zy * zy;
-            const float r2 = xy2 + zz * zz;
-            if (r2 > t2) {  // as below: z no longer changes past the bailout
-                r2_out = r2;
-                break;
-            }
-            r2_last = r2;
-            const float irho = rsqrt_full(xy2);
-            const float rho = xy2 * irho;
-            float ct = zx * irho, st = zy * irho;
-            float cp = __builtin_fmaf(-zz, zz, xy2), sp = (rho + rho) * zz;
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {  // (c + i s)^2 = (c^2 - s^2) + i 2cs, one rounding for the real part
-                const float c2 = __builtin_fmaf(ct, ct, -(st * st)), s2 = (ct + ct) * st;
-                ct = c2;
-                st = s2;
-            }
-#pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                const float p2 = __builtin_fmaf(cp, cp, -(sp * sp)), q2 = (cp + cp) * sp;
-                cp = p2;
-                sp = q2;
-            }
-            const float r7 = ((r2 * r2) * r2) * __builtin_amdgcn_sqrtf(r2);
-            dr = __builtin_fmaf(r7 * dr, 8.0f, 1.0f);
-            zx = __builtin_fmaf(cp, ct, px);
-            zy = __builtin_fmaf(cp, st, py);
-            zz = sp + pz;
-        }
-        if (r2_out >= 0.0f) {
-            r = __builtin_amdgcn_sqrtf(r2_out);
-        } else {
-            const float r4 = r2_last * r2_last;
-            r = r4 * r4;
-        }
-        // 0.5 ln(r) r / dr from the hardware log2 (times ln 2; a denormal r scaled by 2^24
-        // first) and reciprocal, each within about an ulp: dr >= 1, and r = 0 gives NaN as
-        // log(0) * 0 does
-        const bool tiny = r < 0x1p-126f;
-        const float lr = (__builtin_amdgcn_logf(tiny ? r * 0x1p24f : r) - (tiny ? 24.0f : 0.0f)) * 0.693147182f;
-        return ((0.5f * lr) * r) * __builtin_amdgcn_rcpf(dr) - offset;
-    }
     for (uint32_t i = 0; i < iters; ++i) {
         r = len3(zx, zy, zz);
         // past the bailout z no longer changes, so every later step would recompute this

@@ -13,9 +13,11 @@ namespace s2m {
 constexpr uint32_t kBlock = 256;             // threads per block of the cell kernels
 constexpr uint32_t kRounds = 4;              // cells per thread (strided by kBlock)
 constexpr uint32_t kCellsPerBlock = kBlock * kRounds;
-constexpr uint32_t kMaxScanBlocks = 65536;   // most block counts one dense slab scans
-constexpr uint32_t kDenseScanChunk = 1024;        // block counts per workgroup of the dense scan
-constexpr uint32_t kDenseScanParts = kMaxScanBlocks / kDenseScanChunk;  // its chunk sums, after the counters
+constexpr uint32_t kMaxScanBlocks = 65536;   // most block counts one dense slab (sparse pass) scans
+constexpr uint32_t kRankChunks = kMaxScanBlocks / 1024;  // chunks of 1024 blocks of a dense slab
+static_assert(kRankChunks <= 256, "one block's threads set up the chunk bases");
+constexpr uint32_t kBrickBlocks = 2048;      // blocks of 4 waves of the per-brick kernels: 8 waves per
+                                             // SIMD of 256 CUs
 constexpr uint32_t kNone = 0xffffffffu;      // "no vertex" (u32::MAX, mesh.rs:330)
 
 // Unsigned division by a runtime constant d >= 1 (round-up multiplier method):
@@ -38,16 +40,13 @@ enum Counter : uint32_t {
     kSlotsUsed = 8,    // active tiles of the current slab (sparse path)
     kSlotsMax = 9,     // largest kSlotsUsed of the job so far
     kStageUsed = 10,   // staged active cells of the current pass (sparse path)
+    kBrickAlloc = 11,  // dense slab: listed bricks (low word), staged vertices (high word)
     kStageMax = 12,    // largest kStageUsed of the job so far
     kNumCounters = 16
 };
 
 // Everything the cell kernels need to address one slab of cells [z0, z0+nz).
 struct SlabArgs {
-    const float* lat;      // corner lattice of the slab, x fastest
-    uint32_t pitch;        // floats per lattice row
-    uint32_t lat_ny;       // lattice rows per lattice plane
-    uint32_t lz0;          // lattice z index of the slab's first lattice plane
     const float* cx;       // per-axis coordinate tables
     const float* cy;
     const float* cz;
@@ -62,8 +61,17 @@ struct SlabArgs {
     uint32_t ncells;       // rx * ry * nz
     FastDiv div_rx;
     FastDiv div_rxy;
-    uint32_t* vidx;        // (nz + 1) planes of rx*ry; plane 0 holds cell plane z0-1
     uint32_t flags;        // S2M_* flags
+};
+
+// A slab's cells with a vertex and their vertices' indices: cell c's is cbase[c / 2^20] +
+// boffset[c / 1024] + wpre[c / 64] + the bits before c in its word.
+struct SlabBits {
+    const unsigned long long* words;
+    const uint16_t* wpre;
+    const uint32_t* boffset;
+    const uint32_t* cbase;
+    uint64_t last_plane;   // first cell of the slab's last plane
 };
 
 constexpr uint32_t kTile = 8;  // cells per tile edge (sparse pipeline)
@@ -173,23 +181,35 @@ struct MeshBufs {
     uint32_t* tri;         // 3 per triangle
     uint64_t vcap, tcap;   // capacities (vertices, triangles)
     uint64_t* counters;    // Counter
-    uint32_t* bcount;      // per-block counts
-    uint32_t* boffset;     // per-block exclusive offsets
-    uint64_t* actbits;     // dense slab: bit c % 64 of word c / 64 = cell c has a vertex (zero between slabs)
+    uint32_t* bcount;      // sparse pass: the offset scan's chunk sums
+    // dense slab
+    uint64_t* actbits;     // bit c % 64 of word c / 64 = cell c has a vertex
+    SlabBits bits;         // the same words with their prefix tables
+    uint32_t* tcount;      // triangles per kBlock vertices, and their offsets
+    uint32_t* toffset;
 };
 
 // ---- launchers (kernels.hip) ----
 hipError_t launch_eval_lattice(hipStream_t s, const s2m_op* ops, uint32_t nops, const float* cx,
                                const float* cy, const float* cz, uint32_t nx, uint32_t ny,
                                uint32_t lz0, uint32_t nzl, uint32_t pitch, float* lat);
-// The lattice of a tape that is one Mandelbulb op (k_eval_mandelbulb: equal to
-// launch_eval_lattice's values).
-hipError_t launch_eval_mandelbulb(hipStream_t s, const s2m_op* op, const float* cx, const float* cy,
-                                  const float* cz, uint32_t nx, uint32_t ny, uint32_t lz0, uint32_t nzl,
-                                  uint32_t pitch, float* lat);
-hipError_t launch_cells(hipStream_t s, const SlabArgs& a, const MeshBufs& b, int emit,
-                        int write_zero_normals);
-hipError_t launch_scan(hipStream_t s, const MeshBufs& b, uint32_t nblocks, uint32_t which);
+// The dense slab's kernels (kernels.hip, bodies in device_dense.h).  host_ops: the host copy
+// of the tape (it selects the kernel).
+struct BrickArgs;
+bool mandel_power8(const s2m_op* ops, uint32_t n);  // the tape is one power-8 Mandelbulb op
+bool sign_early(const s2m_op* ops, uint32_t n);     // its signs are decided early (no values to keep)
+dim3 sign_grid(const BrickArgs& a);                 // blocks of 256
+uint32_t sign_run(uint64_t bricks);                 // BrickArgs::run for a slab of so many bricks
+hipError_t launch_signs(hipStream_t s, const BrickArgs& a, const s2m_op* host_ops, const s2m_op* ops, uint32_t nops);
+hipError_t launch_find_bricks(hipStream_t s, const BrickArgs& a);
+hipError_t launch_contour(hipStream_t s, const BrickArgs& a, const s2m_op* host_ops, const s2m_op* ops, uint32_t nops);
+hipError_t launch_emit(hipStream_t s, const BrickArgs& a, const s2m_op* host_ops, const s2m_op* ops, uint32_t nops);
+hipError_t launch_ranks(hipStream_t s, const MeshBufs& b, uint32_t ncells);
+hipError_t launch_dense_begin(hipStream_t s, uint64_t* counters, uint64_t* words, uint32_t ncells,
+                              const void* host_tables, void* tables, size_t bytes, uint32_t* cbase);
+hipError_t launch_slab_end(hipStream_t s, uint64_t* counters, uint64_t* words, uint32_t ncells, uint32_t* cbase,
+                           uint64_t* snap, uint64_t* back);
+hipError_t launch_quads(hipStream_t s, const SlabArgs& a, const MeshBufs& b, const SlabBits& prev);
 // cnt[0..4) (zeroed by the caller): k_sincos_check's mismatch counts.
 hipError_t launch_sincos_check(hipStream_t s, uint64_t* cnt);
 // cnt[0..2) (zeroed by the caller): k_bailout_check's comparisons and disagreements.
@@ -197,11 +217,6 @@ hipError_t launch_bailout_check(hipStream_t s, uint64_t* cnt);
 // A tape just copied to the device: every Mandelbulb op's f[3] set to the bailout
 // threshold of its f[1] (sd_mandelbulb reads it there instead of computing it per point).
 hipError_t launch_tape_prepare(hipStream_t s, s2m_op* ops, uint32_t n);
-hipError_t launch_normals(hipStream_t s, const s2m_op* ops, uint32_t nops, float eps,
-                          const MeshBufs& b, bool mandel = false);  // mandel: ops is one Mandelbulb op
-// After a slab's quad pass: its activity bits zeroed (the words of `ncells` cells).
-hipError_t launch_clear_bits(hipStream_t s, uint64_t* bits, uint32_t ncells);
-hipError_t launch_quads(hipStream_t s, const SlabArgs& a, const MeshBufs& b, int emit);
 // Between passes of a job: slot and staging counters folded into their maxima, the
 // previous pass's totals made the next pass's first indices, work queues and the
 // offset scan's nbsum chunk sums (bsum, kChunkSumStride words apart) cleared.
@@ -270,7 +285,7 @@ void tune_override(const TuneChoice* c);  // NULL: back to the table
 uint32_t tune_pick(const double* ms, uint32_t n);
 
 // ---- host helpers (api.cpp) for the server ----
-// A program from a gfx950 code object holding s2m_c_eval_lattice and s2m_c_normals.
+// A program from a gfx950 code object holding the s2m_c_* kernels (frontend_emit.cpp).
 int program_from_code_object(s2m_ctx* ctx, const void* code, size_t size, s2m_program** out);
 s2m_program* program_view(int device, const s2m_op* host_ops, uint32_t n, const s2m_op* d_ops);
 hipStream_t context_stream(s2m_ctx* ctx);

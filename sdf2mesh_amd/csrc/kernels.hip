@@ -1,18 +1,23 @@
 // kernels.hip - HIP kernels of the meshing path for gfx950 (wave64).
 //
-// Per z-slab of cells the host launches, in stream order:
-//   k_eval_lattice     SDF at every corner-lattice point of the slab       (VALU bound)
-//   k_count_cols + k_popc   activity bits and active-cell count per block of 1024 cells
-//                      (k_cells<0> for per-cell corner dumps)
-//   k_scan_sums + k_scan_offsets   exclusive scan of block counts + running vertex total
-//   k_cells_map + k_cell_vertices  cell->vertex map, vertex position/signs in order
-//                      (k_cells<1> for corner dumps)
-//   k_normals          4-tap normal of the slab's new vertices
-//   k_quads<0> / scan / k_quads<1>  the same count/scan/emit scheme for triangles
-// (with several slabs the evaluation runs one slab ahead on a second stream)
-// Cells are numbered in (z, y, x) order inside the slab and every block owns 1024
-// consecutive cells, so block offsets from the scan give each vertex and triangle its
-// place in the reference's output order (VertexList order, mesh.rs:280-321).
+// The dense path meshes programs that interval bounds cannot prune (the Mandelbulb,
+// compiled programs, S2M_DENSE_EVAL).  Per z-slab of cells the host launches, in stream
+// order (bodies of the evaluating kernels: device_dense.h):
+//   k_signs            sign of the SDF at every corner-lattice point, one bit each  (VALU bound)
+//   k_find_bricks      the 4x4x4 bricks whose cells change sign
+//   k_contour          their corner values again, the vertex rule, staged vertices, one
+//                      activity bit per cell
+//   k_ranks            vertices before each word of 64 cells, block of 1024 cells and chunk
+//   k_emit             staged vertices at their ordered index, with 4-tap normals
+//   k_quads<0>, k_tri_offsets, k_quads<1>   triangles per 256 vertices, their offsets, triangles
+//   k_slab_end         the other slab's bits cleared, staging counters folded, the totals
+//                      for the host
+// (with several slabs the signs are evaluated one slab ahead on a second stream; per-cell
+// corner dumps have k_cells<0/1> in place of the brick kernels).  A cell's vertex index is
+// never stored: it is its chunk's first vertex plus the vertices before it in the chunk.  Cells are
+// numbered in (z, y, x) order inside the slab, the reference's output order (VertexList
+// order, mesh.rs:280-321).
+#include <algorithm>
 #include <mutex>
 
 #include "device_dense.h"
@@ -55,148 +60,204 @@ __device__ __forceinline__ uint32_t block_exclusive_256(uint32_t v, uint32_t* ld
 }
 
 // ---------------------------------------------------------------------------------
-// Lattice evaluation: one thread per lattice point.  Each wave covers a 4 x 4 x 4 block
-// of points (a block: 16 x 4 x 4), so the lanes of a wave lie close together and a
-// program with data-dependent loops (the Mandelbulb's escape iteration) runs fewer
-// iterations with idle lanes than along a row of 64 points.  Held to 64 VGPRs (8 waves
-// per SIMD; a 12-byte spill): 3 % faster on a 64-primitive CSG program, neutral on the
-// Mandelbulb.
+// SDFs of the tape programs, for the dense bodies (device_dense.h).
 // ---------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_eval_lattice(
-    const s2m_op* __restrict__ ops, uint32_t nops,
-                                                      const float* __restrict__ cx,
-                                                      const float* __restrict__ cy,
-                                                      const float* __restrict__ cz, uint32_t nx,
-                                                      uint32_t ny, uint32_t lz0, uint32_t nzl,
-                                                      uint32_t pitch, float* __restrict__ lat)
-{
-    const uint32_t l = threadIdx.x & 63u, w = threadIdx.x >> 6;
-    const uint32_t ix = blockIdx.x * 16u + w * 4u + (l & 3u);
-    const uint32_t iy = blockIdx.y * 4u + ((l >> 2) & 3u);
-    const uint32_t iz = blockIdx.z * 4u + (l >> 4);
-    if (ix >= nx || iy >= ny || iz >= nzl) return;
-    lat[((size_t)iz * ny + iy) * pitch + ix] = tape_eval(ops, nops, cx[ix], cy[iy], cz[lz0 + iz]);
-}
+struct TapeSdf {
+    const s2m_op* ops;
+    uint32_t n;
+    __device__ float operator()(float x, float y, float z) const { return tape_eval(ops, n, x, y, z); }
+};
 
-// The same lattice for a tape that is one Mandelbulb op: the estimator called directly
-// with its operands (wave-uniform loads), as tape_eval calls it, so the values are the
-// interpreter's bit for bit without its per-point dispatch.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_eval_mandelbulb(
-    const s2m_op* __restrict__ op, const float* __restrict__ cx, const float* __restrict__ cy,
+// A tape that is one power-8 Mandelbulb op: the estimator called directly with its operands
+// (wave-uniform loads), as tape_eval calls it, so the values are the interpreter's bit for
+// bit without its dispatch and the other forms' registers.
+struct MandelSdf {
+    float offset, bailout, t2;
+    uint32_t iters;
+    bool swap;
+    __device__ explicit MandelSdf(const s2m_op* op)
+        : offset(op->f[2]), bailout(op->f[1]), t2(op->f[3]), iters(op->iarg & 0xffffu),
+          swap((op->iarg & S2M_MANDEL_SWAP_YZ) != 0)
+    {
+    }
+    __device__ float operator()(float x, float y, float z) const
+    {
+        return mandelbulb8<false>(x, swap ? z : y, swap ? y : z, offset, iters, t2, bailout, 0.0f);
+    }
+};
+
+// Its sign, with the early decisions of mandelbulb8<true> (their preconditions hold:
+// mandel_sign_ok), and of whole bricks by the two decisions of the first step on the box:
+// inside the inner ball everywhere, or past the bailout (or predicted past it) everywhere.
+struct MandelSign : MandelSdf {
+    float gain;
+    static constexpr bool kBricks = true;
+    static constexpr bool kValue = false;
+    __device__ explicit MandelSign(const s2m_op* op) : MandelSdf(op), gain(mandel_gain(op->f[1])) {}
+    __device__ float operator()(float x, float y, float z) const
+    {
+        return mandelbulb8<true>(x, swap ? z : y, swap ? y : z, offset, iters, t2, bailout, gain);
+    }
+    __device__ int brick(float x0, float x1, float y0, float y1, float z0, float z1) const
+    {
+        const float xn = fmaxf(fmaxf(x0, -x1), 0.0f), xf = fmaxf(fabsf(x0), fabsf(x1));
+        const float yn = fmaxf(fmaxf(y0, -y1), 0.0f), yf = fmaxf(fabsf(y0), fabsf(y1));
+        const float zn = fmaxf(fmaxf(z0, -z1), 0.0f), zf = fmaxf(fabsf(z0), fabsf(z1));
+        const float far2 = 1.0001f * (xf * xf + yf * yf + zf * zf);
+        if (!(far2 < 1e30f)) return -1;
+        if (far2 <= kMandelInner) return 0;
+        const float near2 = 0.9999f * (xn * xn + yn * yn + zn * zn), n4 = near2 * near2;
+        const float xy2 = xn * xn + (swap ? zn * zn : yn * yn);  // of the swizzled point
+        const float far = 1.0001f * __builtin_amdgcn_sqrtf(far2), r = fminf(far, 1.0001f * bailout);
+        const float r2 = r * r, r7 = r2 * r2 * r2 * r;
+        if (n4 * n4 > 1.02f * (bailout + far) && xy2 >= 2.0f * kMandelAxis &&
+            1.001f * (8.0f * r7 + 1.0f) * offset <= gain)
+            return 1;
+        return -1;
+    }
+};
+
+// Lattice evaluation (s2m_eval_lattice): one thread per lattice point, each wave a
+// 4 x 4 x 4 block.  Held to 64 VGPRs (8 waves per SIMD; a 12-byte spill): 3 % faster on
+// a 64-primitive CSG program.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_eval_lattice(
+    const s2m_op* __restrict__ ops, uint32_t nops, const float* __restrict__ cx, const float* __restrict__ cy,
     const float* __restrict__ cz, uint32_t nx, uint32_t ny, uint32_t lz0, uint32_t nzl, uint32_t pitch,
     float* __restrict__ lat)
 {
-    const uint32_t l = threadIdx.x & 63u, w = threadIdx.x >> 6;
-    const uint32_t ix = blockIdx.x * 16u + w * 4u + (l & 3u);
-    const uint32_t iy = blockIdx.y * 4u + ((l >> 2) & 3u);
-    const uint32_t iz = blockIdx.z * 4u + (l >> 4);
-    if (ix >= nx || iy >= ny || iz >= nzl) return;
-    const float* f = op->f;
-    lat[((size_t)iz * ny + iy) * pitch + ix] =
-        sd_mandelbulb(cx[ix], cy[iy], cz[lz0 + iz], f[0], f[1], f[2], op->iarg, f[3]);
+    eval_lattice_point(TapeSdf{ops, nops}, cx, cy, cz, nx, ny, lz0, nzl, pitch, lat);
+}
+
+// MANDEL = 1: the tape is one power-8 Mandelbulb op (k_signs<2>: its sign may be decided
+// early as well).
+template <int MANDEL>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_signs(BrickArgs a, const s2m_op* ops,
+                                                                                         uint32_t nops)
+{
+    if constexpr (MANDEL == 2) sign_words(MandelSign(ops), a);
+    else if constexpr (MANDEL == 1) sign_words(PointSign<MandelSdf>{MandelSdf(ops)}, a);
+    else sign_words(PointSign<TapeSdf>{TapeSdf{ops, nops}}, a);
+}
+
+template <int MANDEL>
+__global__ __launch_bounds__(256) void k_contour(BrickArgs a, const s2m_op* ops, uint32_t nops)
+{
+    if constexpr (MANDEL) contour_bricks(MandelSdf(ops), a);
+    else contour_bricks(TapeSdf{ops, nops}, a);
+}
+
+template <int MANDEL>
+__global__ __launch_bounds__(256) void k_emit(BrickArgs a, const s2m_op* ops, uint32_t nops)
+{
+    if constexpr (MANDEL) emit_bricks(MandelSdf(ops), LibraryNormal{}, a);
+    else emit_bricks(TapeSdf{ops, nops}, LibraryNormal{}, a);
 }
 
 // ---------------------------------------------------------------------------------
-// One cell: dualcontour.wgsl:72-131 (crossings, centroid) and :57-69 (sign bits).
-// c[] in corner order 000,100,010,110,001,101,011,111.
+// k_find_bricks: kFindBricks bricks per thread, kBlock apart.  A brick's 64 cells' corner
+// signs differ where the OR of the 8 shifted words (the brick's and its 7 neighbours'
+// towards +x, +y, +z) is set and the AND is not: axis by axis, OR and AND of the word and
+// its shift.  Cells between two coordinates a rounding apart, past the grid or in another
+// slab are masked off by the axes' cell tables.  Bricks with a cell left are appended to
+// the list, their cells reserving staging space: one 64-bit counter (records low, staged
+// vertices high), one update per block of 1024 bricks (a returning update of the one
+// address takes about 25 ns, one after the other: one per wave took 69 us for 157 K
+// bricks of which 2 500 waves listed some).  Reads 8 words per brick, mostly from cache.
 // ---------------------------------------------------------------------------------
-struct Edge {
-    uint8_t a, b;       // corner indices
-    uint8_t axis;       // component that carries t
-    uint8_t fx, fy, fz; // fixed components (0 or 1), the t component entry is unused
-};
-// z-edges 0-3, y-edges 4-7, x-edges 8-11 (dualcontour.wgsl:98-114)
-__constant__ Edge kEdges[12] = {
-    {0, 4, 2, 0, 0, 0}, {2, 6, 2, 0, 1, 0}, {1, 5, 2, 1, 0, 0}, {3, 7, 2, 1, 1, 0},
-    {0, 2, 1, 0, 0, 0}, {4, 6, 1, 0, 0, 1}, {1, 3, 1, 1, 0, 0}, {5, 7, 1, 1, 0, 1},
-    {0, 1, 0, 0, 0, 0}, {4, 5, 0, 0, 0, 1}, {2, 3, 0, 0, 1, 0}, {6, 7, 0, 0, 1, 1},
-};
+constexpr uint32_t kFindBricks = 4;
 
-__device__ __forceinline__ bool contour_cell(const float c[8], const float lo[3], const float hi[3],
-                                             float pos[3])
+__device__ __forceinline__ uint64_t mixed_cells(const BrickArgs& a, uint32_t i, uint32_t& bx, uint32_t& by, uint32_t& bz)
 {
-    // no edge changes sign when all eight corners fall on one side of `> 0`
-    uint32_t pos_mask = 0;
+    const uint32_t row = i / a.nbx;
+    bx = i - row * a.nbx;
+    bz = row / a.nby;
+    by = row - bz * a.nby;
+    const uint32_t dx = bx + 1 < a.nbx ? 1u : 0u;  // past the end: cells that are masked off
+    const size_t dy = by + 1 < a.nby ? a.nbx : 0u, dz = bz + 1 < a.nbz ? (size_t)a.nbx * a.nby : 0u;
+    const uint64_t* w = a.words + i;
+    uint64_t o[4], n4[4];  // OR / AND along x of the rows (y, z), (y + 1, z), (y, z + 1), (y + 1, z + 1)
 #pragma unroll
-    for (int k = 0; k < 8; ++k) pos_mask |= (uint32_t)(c[k] > 0.0f) << k;
-    if (pos_mask == 0u || pos_mask == 0xffu) return false;
-    float ax = 0.0f, ay = 0.0f, az = 0.0f, cnt = 0.0f;
+    for (int k = 0; k < 4; ++k) {
+        const uint64_t* r = w + (k & 1 ? dy : 0) + (k & 2 ? dz : 0);
+        const uint64_t u = r[0], v = r[dx];
+        const uint64_t s = ((u >> 1) & 0x7777777777777777ull) | ((v & 0x1111111111111111ull) << 3);
+        o[k] = u | s;
+        n4[k] = u & s;
+    }
+    auto shy = [](uint64_t u, uint64_t v) {
+        return ((u >> 4) & 0x0fff0fff0fff0fffull) | ((v & 0x000f000f000f000full) << 12);
+    };
+    const uint64_t o0 = o[0] | shy(o[0], o[1]), o1 = o[2] | shy(o[2], o[3]);
+    const uint64_t n0 = n4[0] & shy(n4[0], n4[1]), n1 = n4[2] & shy(n4[2], n4[3]);
+    const uint64_t mask = (o0 | (o0 >> 16) | (o1 << 48)) & ~(n0 & ((n0 >> 16) | (n1 << 48)));
+    if (!mask) return 0ull;
+    uint32_t vx = 0, vy = 0, vz = 0;  // the axes' cells
 #pragma unroll
-    for (int e = 0; e < 12; ++e) {
-        const float v0 = c[kEdges[e].a], v1 = c[kEdges[e].b];
-        const float t = (0.0f - v0) / (v1 - v0);  // _cell_adapt
-        float x = kEdges[e].fx, y = kEdges[e].fy, z = kEdges[e].fz;
-        if (kEdges[e].axis == 0) x = t;
-        else if (kEdges[e].axis == 1) y = t;
-        else z = t;
-        if ((v0 > 0.0f) == (v1 > 0.0f)) x = y = z = 0.0f;  // _cell_change
-        if (x > 0.0f || y > 0.0f || z > 0.0f) {
-            ax = ax + x;
-            ay = ay + y;
-            az = az + z;
-            cnt = cnt + 1.0f;
+    for (uint32_t k = 0; k < 4; ++k) {
+        const uint32_t ix = bx * 4u + k, iy = by * 4u + k, iz = bz * 4u + k;
+        if (ix < a.nx && a.cox[ix] != kNoCell) vx |= 1u << k;
+        if (iy < a.ny && a.coy[iy] != kNoCell) vy |= 1u << (4u * k);
+        if (iz + 1u < a.nzl) {
+            const uint32_t z = a.coz[a.lz0 + iz];
+            if (z >= a.z0 && z < a.z1) vz |= 1u << k;
         }
     }
-    if (cnt <= 1.0f) return false;
-    pos[0] = canonical_nan(lo[0] + ((hi[0] - lo[0]) * ax) / cnt);
-    pos[1] = canonical_nan(lo[1] + ((hi[1] - lo[1]) * ay) / cnt);
-    pos[2] = canonical_nan(lo[2] + ((hi[2] - lo[2]) * az) / cnt);
-    return true;
+    const uint64_t rows = vx * vy;
+    return mask & ((vz & 1u ? rows : 0ull) | (vz & 2u ? rows << 16 : 0ull) | (vz & 4u ? rows << 32 : 0ull) |
+                   (vz & 8u ? rows << 48 : 0ull));
 }
 
-// contour_cell's verdict alone (whether the cell gets a vertex), without the position.
-// An edge counts when its corners straddle `> 0` and its point has a component > 0.  Nine
-// of the twelve edges have a fixed component 1, so they count whenever their corners
-// straddle; the three edges from corner 000 (z: 0-4, y: 0-2, x: 0-1) have only the edge
-// parameter t = (0 - v0) / (v1 - v0), which must be > 0 as the IEEE quotient (it is 0
-// when the difference overflows or the quotient underflows).  The cell gets a vertex
-// when at least two edges count.
-__device__ __forceinline__ bool cell_active(const float c[8])
+__global__ __launch_bounds__(256) void k_find_bricks(BrickArgs a)
 {
-    uint32_t m = 0;
+    __shared__ uint32_t wrecs[kBlock / 64], wcells[kBlock / 64];
+    __shared__ uint64_t base;
+    const uint32_t n = a.nbx * a.nby * a.nbz;
+    uint64_t mask[kFindBricks];
+    BrickRec rec[kFindBricks];
+    uint32_t recs = 0, cells = 0;  // of this thread
 #pragma unroll
-    for (int k = 0; k < 8; ++k) m |= (uint32_t)(c[k] > 0.0f) << k;
-    if (m == 0u || m == 0xffu) return false;
-    const uint32_t ch = (m ^ (m >> 4)) | ((m ^ (m >> 2)) << 8) | ((m ^ (m >> 1)) << 16);
-    // bits of `ch`: z-edges a-(a+4) at a = 0..3, y-edges a-(a+2) at 8 + {0, 1, 4, 5},
-    // x-edges a-(a+1) at 16 + {0, 2, 4, 6}
-    const uint32_t fixed1 = ch & ((0xeu) | (0x32u << 8) | (0x54u << 16));
-    uint32_t cnt = (uint32_t)__builtin_popcount(fixed1);
-    auto from0 = [&](uint32_t bit, int b) -> uint32_t {
-        if (!((ch >> bit) & 1u)) return 0u;
-        const float t = (0.0f - c[0]) / (c[b] - c[0]);
-        return t > 0.0f ? 1u : 0u;
-    };
-    cnt += from0(0, 4) + from0(8, 2) + from0(16, 1);
-    return cnt >= 2u;
-}
-
-__device__ __forceinline__ uint32_t sign_bits(const float c[8])
-{
-    return (uint32_t)(c[1] > 0.0f) | ((uint32_t)(c[2] > 0.0f) << 1) |
-           ((uint32_t)(c[4] > 0.0f) << 2) | ((uint32_t)(c[0] > 0.0f) << 3);
-}
-
-// Corners of cell (x, y, zl) from the slab lattice, and the cell's bounds.
-__device__ __forceinline__ void gather_lattice(const SlabArgs& a, uint32_t x, uint32_t y, uint32_t zl,
-                                               float c[8], float lo[3], float hi[3])
-{
-    const uint32_t zg = a.z0 + zl;
-    const uint32_t xi[2] = {a.lox[x], a.hix[x]};
-    const uint32_t yi[2] = {a.loy[y], a.hiy[y]};
-    const uint32_t zi[2] = {a.loz[zg], a.hiz[zg]};
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        const size_t off = ((size_t)(zi[(k >> 2) & 1] - a.lz0) * a.lat_ny + yi[(k >> 1) & 1]) * a.pitch +
-                           xi[k & 1];
-        c[k] = a.lat[off];
+    for (uint32_t k = 0; k < kFindBricks; ++k) {
+        const uint32_t i = (blockIdx.x * kFindBricks + k) * kBlock + threadIdx.x;
+        uint32_t bx = 0, by = 0, bz = 0;
+        mask[k] = i < n ? mixed_cells(a, i, bx, by, bz) : 0ull;
+        rec[k] = BrickRec{mask[k], 0u, (uint16_t)bx, (uint16_t)by, (uint16_t)bz, 0};
+        recs += mask[k] != 0ull ? 1u : 0u;
+        cells += (uint32_t)__popcll(mask[k]);
     }
-    lo[0] = a.cx[xi[0]];
-    hi[0] = a.cx[xi[1]];
-    lo[1] = a.cy[yi[0]];
-    hi[1] = a.cy[yi[1]];
-    lo[2] = a.cz[zi[0]];
-    hi[2] = a.cz[zi[1]];
+    uint32_t ir = recs, ic = cells;  // inclusive prefixes over the wave
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t t = __shfl_up(ir, d, 64), u = __shfl_up(ic, d, 64);
+        if (lane_id() >= (uint32_t)d) {
+            ir += t;
+            ic += u;
+        }
+    }
+    const uint32_t w = threadIdx.x >> 6;
+    if (lane_id() == 63u) {
+        wrecs[w] = ir;
+        wcells[w] = ic;
+    }
+    __syncthreads();
+    uint32_t br = 0, bc = 0, tr = 0, tc = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kBlock / 64; ++k) {
+        br += k < w ? wrecs[k] : 0u;
+        bc += k < w ? wcells[k] : 0u;
+        tr += wrecs[k];
+        tc += wcells[k];
+    }
+    if (tr == 0) return;  // block-uniform
+    if (threadIdx.x == 0) base = atomicAdd((unsigned long long*)a.alloc, (unsigned long long)tr | ((unsigned long long)tc << 32));
+    __syncthreads();
+    uint32_t at = (uint32_t)base + br + ir - recs, to = (uint32_t)(base >> 32) + bc + ic - cells;
+#pragma unroll
+    for (uint32_t k = 0; k < kFindBricks; ++k) {
+        if (!mask[k]) continue;
+        rec[k].base = to;
+        a.recs[at++] = rec[k];
+        to += (uint32_t)__popcll(mask[k]);
+    }
 }
 
 __device__ __forceinline__ void cell_coords(const SlabArgs& a, uint32_t i, uint32_t& x, uint32_t& y,
@@ -209,71 +270,43 @@ __device__ __forceinline__ void cell_coords(const SlabArgs& a, uint32_t i, uint3
 }
 
 // ---------------------------------------------------------------------------------
-// Cell passes over per-cell corner dumps (FROM_CORNERS; the slab lattice has k_count_cols,
-// k_cells_map and k_cell_vertices).  EMIT = 0: every cell's vertex rule; block active
-// counts and each cell's activity bit (b.actbits, one ballot word per 64 cells).  EMIT = 1: the cell -> vertex
-// index map for every cell (kNone where no vertex), its ranks from the activity bits, then the block's active
-// cells, listed in LDS in vertex order, are gathered and contoured again on full waves
+// Cell passes over per-cell corner dumps (s2m_contour_cells).  EMIT = 0: every cell's
+// vertex rule, each cell's activity bit (one ballot word per 64 cells).  EMIT = 1: the
+// block's cells with a vertex, listed in LDS in order, are contoured again on full waves
 // (the same rule on the same corners gives the same vertex) and their vertices written.
-// FROM_CORNERS selects the per-cell corner dump source.
 // ---------------------------------------------------------------------------------
-template <int FROM_CORNERS>
 __device__ __forceinline__ bool cell_vertex(const SlabArgs& a, const float* __restrict__ corners, uint32_t i,
                                             uint32_t x, uint32_t y, uint32_t zl, float (&c)[8], float (&pos)[3])
 {
-    float lo[3], hi[3];
-    if (FROM_CORNERS) {
-        const float* src = corners + 8 * (size_t)i;
+    const float* src = corners + 8 * (size_t)i;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) c[k] = src[k];
-        const uint32_t zg = a.z0 + zl;
-        lo[0] = a.cx[a.lox[x]];
-        hi[0] = a.cx[a.hix[x]];
-        lo[1] = a.cy[a.loy[y]];
-        hi[1] = a.cy[a.hiy[y]];
-        lo[2] = a.cz[a.loz[zg]];
-        hi[2] = a.cz[a.hiz[zg]];
-    } else {
-        gather_lattice(a, x, y, zl, c, lo, hi);
-    }
+    for (int k = 0; k < 8; ++k) c[k] = src[k];
+    const uint32_t zg = a.z0 + zl;
+    const float lo[3] = {a.cx[a.lox[x]], a.cy[a.loy[y]], a.cz[a.loz[zg]]};
+    const float hi[3] = {a.cx[a.hix[x]], a.cy[a.hiy[y]], a.cz[a.hiz[zg]]};
     return contour_cell(c, lo, hi, pos);
 }
 
-template <int EMIT, int FROM_CORNERS>
-__global__ __launch_bounds__(256) void k_cells(SlabArgs a, MeshBufs b, const float* __restrict__ corners,
-                                               int zero_normals)
+template <int EMIT>
+__global__ __launch_bounds__(256) void k_cells(SlabArgs a, MeshBufs b, const float* __restrict__ corners)
 {
     const uint32_t base = blockIdx.x * kCellsPerBlock;
     if constexpr (!EMIT) {
-        __shared__ uint32_t lds[kBlock / 64];
-        uint32_t count = 0;
         for (uint32_t j = 0; j < kRounds; ++j) {
             const uint32_t i = base + j * kBlock + threadIdx.x;
             bool act = false;
             if (i < a.ncells) {
                 uint32_t x, y, zl;
-                float c[8];
+                float c[8], pos[3];
                 cell_coords(a, i, x, y, zl);
-                if (FROM_CORNERS) {
-                    const float* src = corners + 8 * (size_t)i;
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) c[k] = src[k];
-                } else {
-                    float lo[3], hi[3];
-                    gather_lattice(a, x, y, zl, c, lo, hi);
-                }
-                act = cell_active(c);
+                act = cell_vertex(a, corners, i, x, y, zl, c, pos);
             }
             const uint64_t w = __ballot(act);
             if (lane_id() == 0 && i < a.ncells) b.actbits[i >> 6] = w;
-            uint32_t total;
-            block_exclusive_256(act ? 1u : 0u, lds, &total);
-            count += total;
         }
-        if (threadIdx.x == 0) b.bcount[blockIdx.x] = count;
     } else {
         __shared__ uint32_t list[kCellsPerBlock];  // the block's active cells, in vertex order
-        const uint32_t first = b.boffset[blockIdx.x];
+        const uint32_t first = b.bits.cbase[blockIdx.x >> 10] + b.bits.boffset[blockIdx.x];
         uint32_t before = 0;  // active cells of earlier rounds
         for (uint32_t j = 0; j < kRounds; ++j) {
             const uint32_t i0 = base + j * kBlock, i = i0 + threadIdx.x;
@@ -289,15 +322,8 @@ __global__ __launch_bounds__(256) void k_cells(SlabArgs a, MeshBufs b, const flo
                 if (k < wv) rank += pc;
             }
             const uint64_t mine = wd[wv];
-            const bool act = (mine >> ln) & 1ull;
             rank += (uint32_t)__builtin_popcountll(mine & ((1ull << ln) - 1ull));
-            if (i < a.ncells) {
-                uint32_t x, y, zl;
-                cell_coords(a, i, x, y, zl);
-                const size_t m = ((size_t)(zl + 1) * a.ry + y) * a.rx + x;
-                a.vidx[m] = act ? first + rank : kNone;
-                if (act) list[rank] = i;
-            }
+            if (i < a.ncells && ((mine >> ln) & 1ull)) list[rank] = i;
             before += total;
         }
         __syncthreads();  // the block's list is complete
@@ -307,17 +333,15 @@ __global__ __launch_bounds__(256) void k_cells(SlabArgs a, MeshBufs b, const flo
             uint32_t x, y, zl;
             float c[8], pos[3];
             cell_coords(a, i, x, y, zl);
-            cell_vertex<FROM_CORNERS>(a, corners, i, x, y, zl, c, pos);
+            cell_vertex(a, corners, i, x, y, zl, c, pos);
             if (v < b.vcap) {
                 float* o = b.vtx + 6 * v;
                 o[0] = pos[0];
                 o[1] = pos[1];
                 o[2] = pos[2];
-                if (zero_normals) {
-                    o[3] = 0.0f;
-                    o[4] = 0.0f;
-                    o[5] = 0.0f;
-                }
+                o[3] = 0.0f;
+                o[4] = 0.0f;
+                o[5] = 0.0f;
                 b.keys[v] = (uint64_t)x | ((uint64_t)y << 16) | ((uint64_t)(a.z0 + zl) << 32);
                 b.signs[v] = (uint8_t)sign_bits(c);
             }
@@ -326,354 +350,162 @@ __global__ __launch_bounds__(256) void k_cells(SlabArgs a, MeshBufs b, const flo
 }
 
 // ---------------------------------------------------------------------------------
-// Emit pass over the slab lattice, in two kernels.  k_cells_map: the cell -> vertex map
-// for the cells with a vertex (and every cell of the slab's last plane), the ranks from
-// the activity bits (as k_cells<1>), and each vertex's cell key; the bits stay for the
-// quad pass (cleared after it).  k_cell_vertices: a grid-stride walk over
-// the slab's vertices [kVtxPrev, min(kVtxTotal, vcap)) that gathers each vertex's cell
-// from its key and writes the vertex (contour_cell, as the count pass decided) and its
-// sign bits.
+// k_ranks: from the slab's activity bits, the vertices before each word in its block of 16
+// words, before each block in its chunk of 1024 blocks, and each chunk's first vertex.
+// One workgroup of 1024 per chunk (a thread's 16 words, 1024 apart, in flight at once; 16
+// lanes per block), so a slab of 32 M cells is 32 workgroups of 128 KB each.  A chunk adds
+// its sum to the bases of the chunks after it and to the running total (set to the
+// slab's first vertex by the kernel that begins the slab): one launch, with no workgroup
+// waiting for others.  A count kernel and a two-launch scan took 14 us at any small size; a
+// last workgroup scanning behind device-scope fences more than that.
 // ---------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_cells_map(SlabArgs a, MeshBufs b)
+__global__ __launch_bounds__(1024) void k_ranks(const uint64_t* __restrict__ bits, uint32_t nwords,
+                                                uint16_t* __restrict__ wpre, uint32_t* __restrict__ boffset,
+                                                uint32_t* __restrict__ cbase, uint64_t* __restrict__ counters)
 {
-    // thread t: cells base + 4t .. base + 4t + 3, bits 4t % 64 .. of word t / 16; the map
-    // entry of slab cell i is vidx[plane + i] (plane 0 holds the previous slab's last plane)
-    constexpr uint32_t kWords = kCellsPerBlock / 64;
-    const uint32_t base = blockIdx.x * kCellsPerBlock, t = threadIdx.x;
-    const uint32_t first = b.boffset[blockIdx.x];
-    uint64_t wd[kWords];
+    __shared__ uint32_t count[1024], wsum[16];
+    const uint32_t t = threadIdx.x, l = t & 15u, w0 = blockIdx.x * 16384u;
+    uint64_t word[16];
 #pragma unroll
-    for (uint32_t k = 0; k < kWords; ++k) wd[k] = base + 64u * k < a.ncells ? b.actbits[(base >> 6) + k] : 0ull;
-    const uint32_t w = t >> 4, sh = (4u * t) & 63u;
-    uint32_t rank = first;
-    uint64_t mine = 0;
-#pragma unroll
-    for (uint32_t k = 0; k < kWords; ++k) {
-        if (k < w) rank += (uint32_t)__builtin_popcountll(wd[k]);
-        if (k == w) mine = wd[k];
+    for (uint32_t k = 0; k < 16u; ++k) {
+        const uint32_t i = w0 + k * 1024u + t;
+        word[k] = i < nwords ? bits[i] : 0ull;
     }
-    rank += (uint32_t)__builtin_popcountll(mine & ((1ull << sh) - 1ull));
-    const uint32_t i0 = base + 4u * t;
-    const size_t plane = (size_t)a.rx * a.ry;
-    uint32_t v[4];
 #pragma unroll
-    for (uint32_t u = 0; u < 4u; ++u) {
-        const bool act = (mine >> (sh + u)) & 1ull;
-        v[u] = act ? rank : kNone;
-        if (act && i0 + u < a.ncells && rank < b.vcap) {
-            uint32_t x, y, zl;
-            cell_coords(a, i0 + u, x, y, zl);
-            b.keys[rank] = (uint64_t)x | ((uint64_t)y << 16) | ((uint64_t)(a.z0 + zl) << 32);
+    for (uint32_t k = 0; k < 16u; ++k) {
+        const uint32_t i = w0 + k * 1024u + t, n = (uint32_t)__popcll(word[k]);
+        uint32_t upto = n;
+#pragma unroll
+        for (int d = 1; d < 16; d <<= 1) {
+            const uint32_t v = __shfl_up(upto, d, 16);
+            if (l >= (uint32_t)d) upto += v;
         }
-        rank += act ? 1u : 0u;
+        if (i < nwords) wpre[i] = (uint16_t)(upto - n);
+        if (l == 15u) count[k * 64u + (t >> 4)] = upto;
     }
-    // entries for the cells with a vertex only (k_quads tests a cell's activity bit before
-    // reading its entry), except in the slab's last cell plane, which the next slab reads
-    // as its previous plane without the bits: written in full, kNone where no vertex
-    uint32_t* m = a.vidx + plane + i0;
-    const uint32_t last = a.ncells - (uint32_t)plane;  // first cell of the last plane
-    if (i0 >= last && i0 + 3u < a.ncells && (plane & 3u) == 0u) {
-        *reinterpret_cast<uint4*>(m) = make_uint4(v[0], v[1], v[2], v[3]);
-    } else {
-#pragma unroll
-        for (uint32_t u = 0; u < 4u; ++u)
-            if (i0 + u < a.ncells && (v[u] != kNone || i0 + u >= last)) m[u] = v[u];
-    }
-}
-
-__global__ __launch_bounds__(256) void k_cell_vertices(SlabArgs a, MeshBufs b, int zero_normals)
-{
-    const uint64_t beg = b.counters[kVtxPrev];
-    const uint64_t end = b.counters[kVtxTotal] < b.vcap ? b.counters[kVtxTotal] : b.vcap;
-    for (uint64_t v = beg + (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v < end;
-         v += (uint64_t)gridDim.x * blockDim.x) {
-        const uint64_t key = b.keys[v];
-        const uint32_t x = (uint32_t)(key & 0xffffu), y = (uint32_t)((key >> 16) & 0xffffu);
-        const uint32_t zl = (uint32_t)(key >> 32) - a.z0;
-        float c[8], pos[3];
-        cell_vertex<0>(a, nullptr, 0, x, y, zl, c, pos);
-        float* o = b.vtx + 6 * v;
-        o[0] = pos[0];
-        o[1] = pos[1];
-        o[2] = pos[2];
-        if (zero_normals) {
-            o[3] = 0.0f;
-            o[4] = 0.0f;
-            o[5] = 0.0f;
-        }
-        b.signs[v] = (uint8_t)sign_bits(c);
-    }
-}
-
-// ---------------------------------------------------------------------------------
-// Count pass over the slab lattice, one z-column of cells per thread: block (bx, y),
-// thread x = 256 bx + t walks zl = 0 .. nzl - 1.  The walk is latency-bound (a handful
-// of gathers per cell, then the rule), so the corners of kCountDepth cells are loaded
-// before any of them is tested: one memory round trip per kCountDepth cells.  A cell's
-// faces shared with its z-neighbour are loaded twice; the second load hits the cache.
-// The vertex rule's verdict (cell_active) sets bit i % 64 of word i / 64 of `bits` (i = the cell's slab index); a wave's 64
-// cells of a row span at most two words, ORed in with atomics only where a bit is set.
-// `bits` is zero on entry (cleared after the slab's quad pass, launch_clear_bits).
-// ---------------------------------------------------------------------------------
-constexpr uint32_t kCountDepth = 8;
-
-__global__ __launch_bounds__(256) void k_count_cols(SlabArgs a, uint32_t nzl, uint64_t* __restrict__ bits)
-{
-    // Workgroups go to the device's 8 XCDs in turn (block b to XCD b % 8), and each XCD
-    // has its own L2.  Cell rows y and y + 1 share a lattice row (the upper face of one,
-    // the lower face of the other), so each XCD walks one contiguous band of rows: block b
-    // takes row-chunk (b % 8) * per + b / 8.  Neighbouring rows then run on one XCD and
-    // the shared lattice row is fetched from HBM once instead of once per XCD.
-    const uint32_t nxc = (a.rx + kBlock - 1) / kBlock, nblk = nxc * a.ry;
-    const uint32_t per = (nblk + 7u) / 8u;
-    const uint32_t lin = (blockIdx.x % 8u) * per + blockIdx.x / 8u;
-    if (lin >= nblk) return;  // the launch rounds up to a multiple of 8 blocks
-    const uint32_t xc = lin % nxc, y = lin / nxc;
-    const uint32_t x = xc * kBlock + threadIdx.x;
-    const uint32_t x0 = xc * kBlock + (threadIdx.x & ~63u);  // the wave's first cell
-    if (x0 >= a.rx) return;  // whole wave past the row (wave-uniform)
-    const bool in = x < a.rx;
-    const uint32_t xi0 = in ? a.lox[x] : 0u, xi1 = in ? a.hix[x] : 0u;
-    const size_t pl = (size_t)a.lat_ny * a.pitch;
-    const float* r0 = a.lat + (size_t)a.loy[y] * a.pitch;  // lattice rows of the cell's y lo / hi
-    const float* r1 = a.lat + (size_t)a.hiy[y] * a.pitch;
-    auto face = [&](uint32_t zi, float* f) {  // the 4 corners of lattice plane zi
-        const size_t o = (size_t)zi * pl;
-        f[0] = r0[o + xi0];
-        f[1] = r0[o + xi1];
-        f[2] = r1[o + xi0];
-        f[3] = r1[o + xi1];
-    };
-    for (uint32_t zb = 0; zb < nzl; zb += kCountDepth) {
-        float c[kCountDepth][8];
-#pragma unroll
-        for (uint32_t j = 0; j < kCountDepth; ++j) {
-            if (zb + j < nzl) {  // wave-uniform
-                face(a.loz[a.z0 + zb + j] - a.lz0, c[j]);
-                face(a.hiz[a.z0 + zb + j] - a.lz0, c[j] + 4);
-            }
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < kCountDepth; ++j) {
-            if (zb + j >= nzl) break;
-            const bool act = in && cell_active(c[j]);
-            const uint64_t w = __ballot(act);
-            if (w != 0ull && lane_id() == 0) {
-                const uint64_t i0 = x0 + (uint64_t)a.rx * (y + (uint64_t)a.ry * (zb + j));
-                const uint32_t sh = (uint32_t)(i0 & 63u);
-                unsigned long long* wp = reinterpret_cast<unsigned long long*>(bits + (i0 >> 6));
-                atomicOr(wp, (unsigned long long)(w << sh));
-                if (sh != 0u && (w >> (64u - sh)) != 0ull) atomicOr(wp + 1, (unsigned long long)(w >> (64u - sh)));
-            }
-        }
-    }
-}
-
-// Active cells per 1024-cell block: the popcount of its 16 bit words (words past the
-// slab's last cell are zero).
-__global__ __launch_bounds__(256) void k_popc(const uint64_t* __restrict__ bits, uint32_t nb,
-                                              uint32_t* __restrict__ bcount)
-{
-    const uint32_t blk = blockIdx.x * blockDim.x + threadIdx.x;
-    if (blk >= nb) return;
-    const uint4* w = reinterpret_cast<const uint4*>(bits + (size_t)blk * (kCellsPerBlock / 64));
-    uint32_t n = 0;
-#pragma unroll
-    for (uint32_t k = 0; k < kCellsPerBlock / 128; ++k) {
-        const uint4 q = w[k];
-        n += __builtin_popcount(q.x) + __builtin_popcount(q.y) + __builtin_popcount(q.z) + __builtin_popcount(q.w);
-    }
-    bcount[blk] = n;
-}
-
-// ---------------------------------------------------------------------------------
-// Exclusive scan of the per-block counts (which = 0: vertices, 1: triangles), in two
-// launches of one workgroup per kDenseScanChunk counts, so that no single workgroup's latency
-// is on the slab's critical path (the dense path evaluates the next slab on another stream
-// at the same time).  k_scan_sums: each chunk's sum into part[g] (the words after the
-// counters); workgroup 0 saves the running total of earlier slabs as the *_PREV counter.
-// k_scan_offsets: each chunk's offsets from that total, the chunk sums before it and a
-// scan within the workgroup; the last workgroup advances the running total.
-// ---------------------------------------------------------------------------------
-__device__ __forceinline__ uint4 load_counts4(const uint32_t* __restrict__ bcount, uint32_t nb, uint32_t i)
-{
-    uint4 q = make_uint4(0u, 0u, 0u, 0u);
-    if (i + 3 < nb) {
-        q = *reinterpret_cast<const uint4*>(bcount + i);
-    } else if (i < nb) {
-        q.x = bcount[i];
-        q.y = i + 1 < nb ? bcount[i + 1] : 0u;
-        q.z = i + 2 < nb ? bcount[i + 2] : 0u;
-    }
-    return q;
-}
-
-// Inclusive prefix sum over a 256-thread workgroup (wsum: 4 words of LDS); *total gets
-// the workgroup's sum.  Contains barriers.
-__device__ __forceinline__ uint64_t block_inclusive_256(uint64_t v, uint64_t* wsum, uint64_t* total)
-{
-    const uint32_t lane = lane_id(), w = threadIdx.x >> 6;
+    __syncthreads();
+    const uint32_t mine = count[t];
+    uint32_t upto = mine;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
-        const uint64_t t = __shfl_up(v, d, 64);
-        if (lane >= (uint32_t)d) v += t;
+        const uint32_t v = __shfl_up(upto, d, 64);
+        if (lane_id() >= (uint32_t)d) upto += v;
     }
-    if (lane == 63) wsum[w] = v;
+    if (lane_id() == 63u) wsum[t >> 6] = upto;
     __syncthreads();
-    uint64_t before = 0, all = 0;
+    uint32_t before = 0, all = 0;
 #pragma unroll
-    for (uint32_t k = 0; k < kBlock / 64; ++k) {
-        before += k < w ? wsum[k] : 0ull;
+    for (uint32_t k = 0; k < 16u; ++k) {
+        before += k < (t >> 6) ? wsum[k] : 0u;
         all += wsum[k];
     }
-    __syncthreads();  // wsum may be reused
-    *total = all;
-    return before + v;
+    if (blockIdx.x * 1024u + t < (nwords + 15u) / 16u) boffset[blockIdx.x * 1024u + t] = before + upto - mine;
+    if (all == 0u) return;
+    if (t < gridDim.x && t > blockIdx.x) atomicAdd(&cbase[t], all);
+    if (t == 0) atomicAdd((unsigned long long*)&counters[kVtxTotal], (unsigned long long)all);
 }
 
-static_assert(kDenseScanChunk == 4 * kBlock, "one 16-byte vector of counts per thread");
-
-__global__ __launch_bounds__(256) void k_scan_sums(const uint32_t* __restrict__ bcount, uint32_t nb,
-                                                   uint64_t* __restrict__ counters, uint32_t which)
+// The slab's vertices that have been written, [kVtxPrev, kVtxTotal) below the capacity, in
+// groups of kBlock.
+__device__ __forceinline__ uint32_t vertex_groups(const uint64_t* counters, uint64_t vcap)
 {
-    __shared__ uint64_t wsum[kBlock / 64];
-    const uint4 q = load_counts4(bcount, nb, blockIdx.x * kDenseScanChunk + 4u * threadIdx.x);
-    uint64_t total;
-    (void)block_inclusive_256((uint64_t)q.x + q.y + q.z + q.w, wsum, &total);
-    if (threadIdx.x == 0) {
-        counters[kNumCounters + blockIdx.x] = total;
-        if (blockIdx.x == 0) counters[which ? kTriPrev : kVtxPrev] = counters[which ? kTriTotal : kVtxTotal];
-    }
+    const uint64_t beg = counters[kVtxPrev], end = min(counters[kVtxTotal], vcap);
+    return end > beg ? (uint32_t)((end - beg + kBlock - 1u) / kBlock) : 0u;
 }
 
-__global__ __launch_bounds__(256) void k_scan_offsets(const uint32_t* __restrict__ bcount, uint32_t nb,
-                                                      uint32_t* __restrict__ boffset,
-                                                      uint64_t* __restrict__ counters, uint32_t which)
+// The groups' triangle counts (k_quads<0>) into their offsets, and the running total, by one
+// workgroup: a slab's 600 K vertices are 2 400 groups, one round.
+__global__ __launch_bounds__(1024) void k_tri_offsets(const uint32_t* __restrict__ tcount, uint32_t* __restrict__ toffset,
+                                                      uint64_t* __restrict__ counters, uint64_t vcap)
 {
-    __shared__ uint64_t wsum[kBlock / 64];
-    const uint32_t g = blockIdx.x;
-    uint64_t parts;  // the chunk sums before this chunk (at most kDenseScanParts of them)
-    (void)block_inclusive_256(threadIdx.x < g ? counters[kNumCounters + threadIdx.x] : 0ull, wsum, &parts);
-    const uint32_t i = g * kDenseScanChunk + 4u * threadIdx.x;
-    const uint4 q = load_counts4(bcount, nb, i);
-    const uint64_t s = (uint64_t)q.x + q.y + q.z + q.w;
-    uint64_t total;
-    const uint64_t inc = block_inclusive_256(s, wsum, &total);
-    const uint64_t base = counters[which ? kTriPrev : kVtxPrev] + parts;
-    uint64_t run = base + inc - s;
-    if (i < nb) {
-        uint4 o;
-        o.x = (uint32_t)run;
-        run += q.x;
-        o.y = (uint32_t)run;
-        run += q.y;
-        o.z = (uint32_t)run;
-        run += q.z;
-        o.w = (uint32_t)run;
-        if (i + 3 < nb) {
-            *reinterpret_cast<uint4*>(boffset + i) = o;
-        } else {
-            boffset[i] = o.x;
-            if (i + 1 < nb) boffset[i + 1] = o.y;
-            if (i + 2 < nb) boffset[i + 2] = o.z;
+    __shared__ uint32_t wsum[16];
+    const uint32_t groups = vertex_groups(counters, vcap), t = threadIdx.x;
+    const uint64_t prev = counters[kTriTotal];
+    uint64_t run = prev;
+    for (uint32_t g0 = 0; g0 < groups; g0 += 4096u) {
+        uint32_t n[4], sum = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            const uint32_t g = g0 + 4u * t + k;
+            n[k] = g < groups ? tcount[g] : 0u;
+            sum += n[k];
         }
-    }
-    if (g + 1 == gridDim.x && threadIdx.x == 0) counters[which ? kTriTotal : kVtxTotal] = base + total;
-}
-
-// ---------------------------------------------------------------------------------
-// Normals of the vertices emitted by the current slab: sdf3d_normal + normalize
-// (sdf3d_normal.wgsl:4-9, dualcontour.wgsl:170-171).  Grid-stride over the range
-// [prev, total) read from the device counters, so no host round trip is needed.
-// ---------------------------------------------------------------------------------
-static_assert(kDenseVtxTotal == kVtxTotal && kDenseVtxPrev == kVtxPrev, "counter layout");
-
-// library_normal over the vertices [counters[prev], min(counters[total], vcap)) with one
-// lane per tap: lanes 4j .. 4j + 3 of a wave evaluate taps d1 .. d4 of one vertex (the
-// same points as library_normal), lane 4j gathers them and writes the unit gradient.
-// MANDEL = 1: the tape is one Mandelbulb op, called directly as tape_eval calls it (the
-// same values without the interpreter's per-point dispatch).
-template <int MANDEL>
-__global__ __launch_bounds__(256) void k_normals(const s2m_op* __restrict__ ops, uint32_t nops,
-                                                 float eps, float* __restrict__ vtx,
-                                                 const uint64_t* __restrict__ counters, uint64_t vcap)
-{
-    const uint64_t beg = counters[kVtxPrev];
-    const uint64_t end = counters[kVtxTotal] < vcap ? counters[kVtxTotal] : vcap;
-    const uint32_t tap = threadIdx.x & 3u, l0 = lane_id() & ~3u;
-    // taps v1 = (1,-1,-1), v2 = (-1,-1,1), v3 = (-1,1,-1), v4 = (1,1,1) times eps
-    const float ex = (tap == 0u || tap == 3u) ? eps : -eps;
-    const float ey = tap >= 2u ? eps : -eps;
-    const float ez = (tap == 1u || tap == 3u) ? eps : -eps;
-    // the 4 lanes of a vertex share the loop condition
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; beg + (i >> 2) < end;
-         i += (uint64_t)gridDim.x * blockDim.x) {
-        float* o = vtx + 6 * (beg + (i >> 2));
-        const float px = o[0] + ex, py = o[1] + ey, pz = o[2] + ez;
-        const float d = MANDEL ? sd_mandelbulb(px, py, pz, ops->f[0], ops->f[1], ops->f[2], ops->iarg, ops->f[3])
-                               : tape_eval(ops, nops, px, py, pz);
-        const float d1 = __shfl(d, (int)l0, 64), d2 = __shfl(d, (int)l0 + 1, 64);
-        const float d3 = __shfl(d, (int)l0 + 2, 64), d4 = __shfl(d, (int)l0 + 3, 64);
-        if (tap == 0u) {
-            const float gx = ((d1 + (-d2)) + (-d3)) + d4;
-            const float gy = (((-d1) + (-d2)) + d3) + d4;
-            const float gz = (((-d1) + d2) + (-d3)) + d4;
-            write_unit(o, gx, gy, gz);
+        uint32_t upto = sum;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t v = __shfl_up(upto, d, 64);
+            if (lane_id() >= (uint32_t)d) upto += v;
         }
+        __syncthreads();  // the previous round's readers of wsum
+        if (lane_id() == 63u) wsum[t >> 6] = upto;
+        __syncthreads();
+        uint32_t before = 0, all = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < 16u; ++k) {
+            before += k < (t >> 6) ? wsum[k] : 0u;
+            all += wsum[k];
+        }
+        uint64_t at = run + before + upto - sum;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            const uint32_t g = g0 + 4u * t + k;
+            if (g < groups) toffset[g] = (uint32_t)at;
+            at += n[k];
+        }
+        run += all;
+    }
+    if (t == 0) {
+        counters[kTriPrev] = prev;
+        counters[kTriTotal] = run;
     }
 }
 
 // ---------------------------------------------------------------------------------
-// Quad pass (mesh.rs:267-324).  Per cell with a vertex: the x-, y- and z-edge quads,
-// neighbour vertices from the map planes of this and the previous cell plane.  A quad
-// with a missing vertex is skipped and counted (mesh.rs:270-278).  The cells with a
-// vertex are the slab's vertices [kVtxPrev, kVtxTotal), in cell order, each with its
-// cell key and sign bits, so block b walks vertices kVtxPrev + 1024 b ... (a grid sized
-// for a vertex in every cell; blocks past the slab's vertices count zero).  EMIT = 0
-// counts triangles per block, EMIT = 1 writes them in order.  A vertex beyond the
-// output capacity has no key: it forms no quads (the job repeats with a larger capacity).
+// Quad pass (mesh.rs:267-324).  Per vertex of the slab, [kVtxPrev, kVtxTotal) in cell
+// order: the x-, y- and z-edge quads of its cell from its key and sign bits, neighbour
+// vertices from the activity bits of this slab and, for plane z0 - 1, of the one before.
+// A quad with a missing vertex is skipped and counted (mesh.rs:270-278).  Blocks walk
+// groups of kBlock vertices (their number is only known on the device).  EMIT = 0 counts
+// the groups' triangles, EMIT = 1 writes them in order.  A vertex beyond the output
+// capacity has no key: it forms no quads (the job repeats with a larger capacity).
 // ---------------------------------------------------------------------------------
 template <int EMIT>
-__global__ __launch_bounds__(256) void k_quads(SlabArgs a, MeshBufs b)
+__global__ __launch_bounds__(256) void k_quads(SlabArgs a, MeshBufs b, SlabBits prev)
 {
     __shared__ uint32_t lds[kBlock / 64];
-    const uint64_t vbeg = b.counters[kVtxPrev] + (uint64_t)blockIdx.x * kCellsPerBlock;
-    const uint64_t vend = min(b.counters[kVtxTotal], b.vcap);
-    if (vbeg >= vend) {  // block-uniform
-        if (!EMIT && threadIdx.x == 0) b.bcount[blockIdx.x] = 0;
-        return;
-    }
-    uint64_t running = EMIT ? (uint64_t)b.boffset[blockIdx.x] : 0;
-    uint32_t count = 0, invalid = 0;
-    const size_t plane = (size_t)a.rx * a.ry;
+    const uint64_t vbeg = b.counters[kVtxPrev], vend = min(b.counters[kVtxTotal], b.vcap);
+    const uint32_t groups = vertex_groups(b.counters, b.vcap);
+    const uint64_t plane = (uint64_t)a.rx * a.ry;
     const bool lag = (a.flags & S2M_COMPAT_DROP_LAST_SLICE) != 0;
-    for (uint32_t j = 0; j < kRounds; ++j) {
-        const uint64_t vv = vbeg + j * kBlock + threadIdx.x;
+    uint32_t invalid = 0;
+    for (uint32_t g = blockIdx.x; g < groups; g += gridDim.x) {  // block-uniform
+        const uint64_t vv = vbeg + (uint64_t)g * kBlock + threadIdx.x;
         uint32_t q[3][4];
         uint32_t nq = 0;  // bit e set: quad e is valid
         if (vv < vend) {
             const uint32_t v = (uint32_t)vv;
             const uint64_t key = b.keys[v];
             const uint32_t x = (uint32_t)(key & 0xffffu), y = (uint32_t)((key >> 16) & 0xffffu);
-            const uint32_t zl = (uint32_t)(key >> 32) - a.z0;
-            // the vertex of the cell at offset `off` of map plane P (P = zl: the plane below,
-            // P = zl + 1: this plane): plane 0 (the previous slab's last plane) is written in
-            // full; in the slab's own planes only cells with a vertex have entries, so the
-            // cell's activity bit is tested first
-            auto at = [&](uint32_t P, size_t off) -> uint32_t {
-                if (P == 0) return a.vidx[off];
-                const size_t i = (size_t)(P - 1) * plane + off;  // the cell's slab index
-                return ((b.actbits[i >> 6] >> (i & 63u)) & 1ull) ? a.vidx[(size_t)P * plane + off] : kNone;
+            const uint32_t zg = (uint32_t)(key >> 32), zl = zg - a.z0;
+            // the vertex of the cell at offset `off` of the cell plane (EMIT = 0: whether it
+            // has one), in this plane or the one below
+            auto at = [&](bool below, uint64_t off) -> uint32_t {
+                const bool old = below && zl == 0;
+                const SlabBits& t = old ? prev : b.bits;
+                const uint64_t cell = old ? prev.last_plane + off : (uint64_t)(zl - (below ? 1u : 0u)) * plane + off;
+                const unsigned long long word = t.words[cell >> 6];
+                const uint32_t bit = (uint32_t)(cell & 63u);
+                if (!((word >> bit) & 1ull)) return kNone;
+                if (!EMIT) return 0u;
+                return t.cbase[cell >> 20] + t.boffset[cell >> 10] + t.wpre[cell >> 6] + (uint32_t)__popcll(word & ((1ull << bit) - 1ull));
             };
-            const uint32_t pc = zl + 1, pp = zl;  // map planes of this and the previous cell plane
             const uint32_t s = b.signs[v];
             const bool c0 = s & 1, c1 = (s >> 1) & 1, c2 = (s >> 2) & 1, c3 = (s >> 3) & 1;
-            const uint32_t zg = a.z0 + zl;
-            const size_t r0 = (size_t)y * a.rx, rm = (size_t)(y - 1) * a.rx;
+            const uint64_t r0 = (uint64_t)y * a.rx, rm = r0 - a.rx;
             // x-edge: Quad(v(x,y-1,z-1), v(x,y,z-1), v(x,y,z), v(x,y-1,z)).swap(c.0)
             if (c0 != c3 && y > 0) {
                 if (zg > 0) {
-                    uint32_t t[4] = {at(pp, rm + x), at(pp, r0 + x), v, at(pc, rm + x)};
+                    uint32_t t[4] = {at(true, rm + x), at(true, r0 + x), v, at(false, rm + x)};
                     if (c0) { q[0][0] = t[3]; q[0][1] = t[2]; q[0][2] = t[1]; q[0][3] = t[0]; }
                     else { q[0][0] = t[0]; q[0][1] = t[1]; q[0][2] = t[2]; q[0][3] = t[3]; }
                     if (t[0] != kNone && t[1] != kNone && t[3] != kNone) nq |= 1;
@@ -685,7 +517,7 @@ __global__ __launch_bounds__(256) void k_quads(SlabArgs a, MeshBufs b)
             // y-edge: Quad(v(x-1,y,z-1), v(x,y,z-1), v(x,y,z), v(x-1,y,z)).swap(!c.1)
             if (c1 != c3 && x > 0) {
                 if (zg > 0) {
-                    uint32_t t[4] = {at(pp, r0 + x - 1), at(pp, r0 + x), v, at(pc, r0 + x - 1)};
+                    uint32_t t[4] = {at(true, r0 + x - 1), at(true, r0 + x), v, at(false, r0 + x - 1)};
                     if (!c1) { q[1][0] = t[3]; q[1][1] = t[2]; q[1][2] = t[1]; q[1][3] = t[0]; }
                     else { q[1][0] = t[0]; q[1][1] = t[1]; q[1][2] = t[2]; q[1][3] = t[3]; }
                     if (t[0] != kNone && t[1] != kNone && t[3] != kNone) nq |= 2;
@@ -696,7 +528,7 @@ __global__ __launch_bounds__(256) void k_quads(SlabArgs a, MeshBufs b)
             }
             // z-edge: Quad(v(x-1,y-1,z), v(x,y-1,z), v(x,y,z), v(x-1,y,z)).swap(c.2)
             if (c2 != c3 && x > 0 && y > 0) {
-                uint32_t t[4] = {at(pc, rm + x - 1), at(pc, rm + x), v, at(pc, r0 + x - 1)};
+                uint32_t t[4] = {at(false, rm + x - 1), at(false, rm + x), v, at(false, r0 + x - 1)};
                 if (c2) { q[2][0] = t[3]; q[2][1] = t[2]; q[2][2] = t[1]; q[2][3] = t[0]; }
                 else { q[2][0] = t[0]; q[2][1] = t[1]; q[2][2] = t[2]; q[2][3] = t[3]; }
                 if (t[0] != kNone && t[1] != kNone && t[3] != kNone) nq |= 4;
@@ -706,8 +538,8 @@ __global__ __launch_bounds__(256) void k_quads(SlabArgs a, MeshBufs b)
         const uint32_t ntri = 2u * (uint32_t)__builtin_popcount(nq);
         uint32_t total;
         const uint32_t rank = block_exclusive_256(ntri, lds, &total);
-        if (EMIT && nq) {
-            uint64_t t = running + rank;
+        if (EMIT) {
+            uint64_t t = (uint64_t)b.toffset[g] + rank;
 #pragma unroll
             for (int e = 0; e < 3; ++e) {
                 if (!(nq & (1u << e))) continue;
@@ -723,14 +555,11 @@ __global__ __launch_bounds__(256) void k_quads(SlabArgs a, MeshBufs b)
                 }
                 t += 2;
             }
+        } else if (threadIdx.x == 0) {
+            b.tcount[g] = total;
         }
-        running += total;
-        count += total;
     }
-    if (!EMIT) {
-        if (invalid) atomicAdd((unsigned long long*)&b.counters[kInvalid], (unsigned long long)invalid);
-        if (threadIdx.x == 0) b.bcount[blockIdx.x] = count;
-    }
+    if (!EMIT && invalid) atomicAdd((unsigned long long*)&b.counters[kInvalid], (unsigned long long)invalid);
 }
 
 // ---------------------------------------------------------------------------------
@@ -805,32 +634,76 @@ hipError_t launch_eval_lattice(hipStream_t s, const s2m_op* ops, uint32_t nops, 
     return hipGetLastError();
 }
 
-hipError_t launch_eval_mandelbulb(hipStream_t s, const s2m_op* op, const float* cx, const float* cy,
-                                  const float* cz, uint32_t nx, uint32_t ny, uint32_t lz0, uint32_t nzl,
-                                  uint32_t pitch, float* lat)
+// Whether a tape is one power-8 Mandelbulb op, and whether mandelbulb8<true>'s
+// preconditions hold for it.
+bool mandel_power8(const s2m_op* ops, uint32_t n)
 {
-    if (nx == 0 || ny == 0 || nzl == 0) return hipSuccess;
-    dim3 grid((nx + 15) / 16, (ny + 3) / 4, (nzl + 3) / 4);
-    hipLaunchKernelGGL(k_eval_mandelbulb, grid, dim3(256), 0, s, op, cx, cy, cz, nx, ny, lz0, nzl, pitch, lat);
+    return n == 1 && ops[0].code == S2M_OP_MANDELBULB && ops[0].f[0] == 8.0f && !(ops[0].iarg & S2M_MANDEL_TRIG);
+}
+static bool mandel_sign_ok(const s2m_op& o)
+{
+    return o.f[1] >= 1.5f && o.f[1] <= 16.0f && o.f[2] >= 0.0f && o.f[2] <= 1000.0f && (o.iarg & 0xffffu) >= 1u;
+}
+
+bool sign_early(const s2m_op* ops, uint32_t n) { return mandel_power8(ops, n) && mandel_sign_ok(*ops); }
+
+dim3 sign_grid(const BrickArgs& a) { return dim3((a.nbx + a.run - 1u) / a.run, (a.nby + 3u) / 4u, a.nbz); }
+
+// Bricks per wave of the sign kernel: runs of 16 share their coordinate loads, brick tests
+// and store, but a slab gets at least four rounds of the device's 8192 waves, so that the
+// last round (and runs whose bricks iterate longest) leaves little of it idle.  Measured
+// over whole jobs, run 1 / 4 / 16: Mandelbulb 1024^3 in slabs of 680 K bricks 8.7 / 6.5 /
+// 6.1 ms, 128^3 (43 K bricks) 136 / 134 / 151 us, the compiled estimator at 200^3 (157 K
+// bricks) 1258 / 1249 / 1313 us.
+uint32_t sign_run(uint64_t bricks)
+{
+    uint32_t run = 16;
+    while (run > 1u && bricks / run < 4u * 8192u) run /= 2u;
+    return run;
+}
+
+hipError_t launch_signs(hipStream_t s, const BrickArgs& a, const s2m_op* host_ops, const s2m_op* ops, uint32_t nops)
+{
+    const dim3 grid = sign_grid(a);
+    if (!mandel_power8(host_ops, nops)) hipLaunchKernelGGL(k_signs<0>, grid, dim3(256), 0, s, a, ops, nops);
+    else if (!mandel_sign_ok(*host_ops)) hipLaunchKernelGGL(k_signs<1>, grid, dim3(256), 0, s, a, ops, nops);
+    else hipLaunchKernelGGL(k_signs<2>, grid, dim3(256), 0, s, a, ops, nops);
     return hipGetLastError();
 }
 
-hipError_t launch_cells(hipStream_t s, const SlabArgs& a, const MeshBufs& b, int emit,
-                        int write_zero_normals)
+hipError_t launch_contour(hipStream_t s, const BrickArgs& a, const s2m_op* host_ops, const s2m_op* ops, uint32_t nops)
 {
-    const uint32_t nb = (a.ncells + kCellsPerBlock - 1) / kCellsPerBlock;
-    if (nb == 0) return hipSuccess;
-    if (emit) {
-        hipLaunchKernelGGL(k_cells_map, dim3(nb), dim3(kBlock), 0, s, a, b);
-        // about one vertex per thread (a slab's vertex count is only known on the device):
-        // each vertex is a chain of dependent gathers, so many waves keep the loads in flight
-        hipLaunchKernelGGL(k_cell_vertices, dim3(4096), dim3(kBlock), 0, s, a, b, write_zero_normals);
-    } else {
-        const uint32_t nzl = a.ncells / (a.rx * a.ry);
-        const uint32_t nblk = (a.rx + kBlock - 1) / kBlock * a.ry;  // one block per 256 cells of a row
-        hipLaunchKernelGGL(k_count_cols, dim3((nblk + 7u) / 8u * 8u), dim3(kBlock), 0, s, a, nzl, b.actbits);
-        hipLaunchKernelGGL(k_popc, dim3((nb + kBlock - 1) / kBlock), dim3(kBlock), 0, s, b.actbits, nb, b.bcount);
-    }
+    if (mandel_power8(host_ops, nops))
+        hipLaunchKernelGGL(k_contour<1>, dim3(kBrickBlocks), dim3(256), 0, s, a, ops, nops);
+    else
+        hipLaunchKernelGGL(k_contour<0>, dim3(kBrickBlocks), dim3(256), 0, s, a, ops, nops);
+    return hipGetLastError();
+}
+
+hipError_t launch_emit(hipStream_t s, const BrickArgs& a, const s2m_op* host_ops, const s2m_op* ops, uint32_t nops)
+{
+    if (mandel_power8(host_ops, nops))
+        hipLaunchKernelGGL(k_emit<1>, dim3(kBrickBlocks), dim3(256), 0, s, a, ops, nops);
+    else
+        hipLaunchKernelGGL(k_emit<0>, dim3(kBrickBlocks), dim3(256), 0, s, a, ops, nops);
+    return hipGetLastError();
+}
+
+hipError_t launch_find_bricks(hipStream_t s, const BrickArgs& a)
+{
+    const uint64_t n = (uint64_t)a.nbx * a.nby * a.nbz;
+    if (n > 0x7fffffffull) return hipErrorInvalidValue;
+    const uint64_t per = kFindBricks * kBlock;
+    hipLaunchKernelGGL(k_find_bricks, dim3((uint32_t)((n + per - 1u) / per)), dim3(kBlock), 0, s, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_ranks(hipStream_t s, const MeshBufs& b, uint32_t ncells)
+{
+    const uint32_t nwords = (ncells + 63u) / 64u, chunks = (nwords + 16383u) / 16384u;
+    if (chunks > kRankChunks || chunks == 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_ranks, dim3(chunks), dim3(1024), 0, s, b.actbits, nwords, const_cast<uint16_t*>(b.bits.wpre),
+                       const_cast<uint32_t*>(b.bits.boffset), const_cast<uint32_t*>(b.bits.cbase), b.counters);
     return hipGetLastError();
 }
 
@@ -839,10 +712,8 @@ hipError_t launch_cells_from_corners(hipStream_t s, const SlabArgs& a, const flo
 {
     const uint32_t nb = (a.ncells + kCellsPerBlock - 1) / kCellsPerBlock;
     if (nb == 0) return hipSuccess;
-    if (emit)
-        hipLaunchKernelGGL((k_cells<1, 1>), dim3(nb), dim3(kBlock), 0, s, a, b, corners, 1);
-    else
-        hipLaunchKernelGGL((k_cells<0, 1>), dim3(nb), dim3(kBlock), 0, s, a, b, corners, 1);
+    if (emit) hipLaunchKernelGGL(k_cells<1>, dim3(nb), dim3(kBlock), 0, s, a, b, corners);
+    else hipLaunchKernelGGL(k_cells<0>, dim3(nb), dim3(kBlock), 0, s, a, b, corners);
     return hipGetLastError();
 }
 
@@ -874,47 +745,75 @@ hipError_t launch_bailout_check(hipStream_t s, uint64_t* cnt)
     return hipGetLastError();
 }
 
-hipError_t launch_scan(hipStream_t s, const MeshBufs& b, uint32_t nblocks, uint32_t which)
+// Before a job's first slab: its counters and the slab's activity bits cleared, and the
+// axis tables (n16 16-byte words) copied from mapped host memory, where given: one kernel
+// instead of a copy and memsets with gaps between them.
+__global__ __launch_bounds__(256) void k_dense_begin(uint64_t* __restrict__ counters, uint32_t n,
+                                                     uint64_t* __restrict__ words, uint32_t nwords,
+                                                     const uint4* __restrict__ host_tables, uint4* __restrict__ tables,
+                                                     uint32_t n16, uint32_t* __restrict__ cbase)
 {
-    if (nblocks > kMaxScanBlocks) return hipErrorInvalidValue;  // kDenseScanParts chunk sums at most
-    const uint32_t chunks = nblocks ? (nblocks + kDenseScanChunk - 1) / kDenseScanChunk : 1u;
-    hipLaunchKernelGGL(k_scan_sums, dim3(chunks), dim3(kBlock), 0, s, b.bcount, nblocks, b.counters, which);
-    hipLaunchKernelGGL(k_scan_offsets, dim3(chunks), dim3(kBlock), 0, s, b.bcount, nblocks, b.boffset, b.counters,
-                       which);
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
+    for (uint32_t i = t; i < n16; i += stride) tables[i] = host_tables[i];
+    if (t < n) counters[t] = 0ull;
+    if (t < kRankChunks) cbase[t] = 0u;
+    for (uint32_t i = t; i < nwords; i += stride) words[i] = 0ull;
+}
+
+// After a slab's quad pass: the staging use folded into its maximum, the allocation
+// counter reset, and the other activity words and chunk bases (the previous slab's, read
+// for the last time by this slab's quads) set up for the next slab.  snap: the totals so far, for the
+// host to copy the slab's finished mesh (as k_snapshot); back: after the last slab, all
+// counters (both in mapped host memory, NULL: not wanted).
+__global__ __launch_bounds__(256) void k_slab_end(uint64_t* __restrict__ counters, uint64_t* __restrict__ words,
+                                                  uint32_t nwords, uint32_t* __restrict__ cbase, uint64_t* snap,
+                                                  uint64_t* back)
+{
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < kRankChunks) cbase[t] = (uint32_t)counters[kVtxTotal];
+    if (t == 0) {
+        counters[kVtxPrev] = counters[kVtxTotal];
+        const uint64_t used = counters[kBrickAlloc] >> 32;
+        if (used > counters[kStageMax]) counters[kStageMax] = used;
+        counters[kBrickAlloc] = 0;
+        if (snap) {
+            snap[0] = counters[kVtxTotal];
+            snap[1] = counters[kTriTotal];
+            snap[2] = snap[3] = 0;
+        }
+        if (back)
+            for (uint32_t i = 0; i < kNumCounters; ++i) back[i] = counters[i];
+    }
+    for (uint32_t i = t; i < nwords; i += gridDim.x * blockDim.x) words[i] = 0ull;
+}
+
+hipError_t launch_dense_begin(hipStream_t s, uint64_t* counters, uint64_t* words, uint32_t ncells,
+                              const void* host_tables, void* tables, size_t bytes, uint32_t* cbase)
+{
+    const uint32_t n = (ncells + 63u) / 64u, n16 = (uint32_t)((bytes + 15u) / 16u);
+    hipLaunchKernelGGL(k_dense_begin, dim3(std::max(1u, std::min((std::max(n, n16) + 255u) / 256u, 2048u))), dim3(256), 0,
+                       s, counters, (uint32_t)kNumCounters, words, n, static_cast<const uint4*>(host_tables),
+                       static_cast<uint4*>(tables), n16, cbase);
     return hipGetLastError();
 }
 
-hipError_t launch_normals(hipStream_t s, const s2m_op* ops, uint32_t nops, float eps,
-                          const MeshBufs& b, bool mandel)
-{
-    if (mandel)
-        hipLaunchKernelGGL(k_normals<1>, dim3(4096), dim3(256), 0, s, ops, nops, eps, b.vtx, b.counters, b.vcap);
-    else
-        hipLaunchKernelGGL(k_normals<0>, dim3(4096), dim3(256), 0, s, ops, nops, eps, b.vtx, b.counters, b.vcap);
-    return hipGetLastError();
-}
-
-// Zero `n` words (a slab's activity bits once its quad pass has read them, for the count
-// pass that ORs into them two slabs later).
-__global__ __launch_bounds__(256) void k_clear_words(uint64_t* __restrict__ w, uint32_t n)
-{
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) w[i] = 0ull;
-}
-
-hipError_t launch_clear_bits(hipStream_t s, uint64_t* bits, uint32_t ncells)
+hipError_t launch_slab_end(hipStream_t s, uint64_t* counters, uint64_t* words, uint32_t ncells, uint32_t* cbase,
+                           uint64_t* snap, uint64_t* back)
 {
     const uint32_t n = (ncells + 63u) / 64u;
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_clear_words, dim3(std::min<uint32_t>((n + 255u) / 256u, 2048u)), dim3(256), 0, s, bits, n);
+    hipLaunchKernelGGL(k_slab_end, dim3(std::max(1u, std::min((n + 255u) / 256u, 2048u))), dim3(256), 0, s, counters,
+                       words, n, cbase, snap, back);
     return hipGetLastError();
 }
 
-hipError_t launch_quads(hipStream_t s, const SlabArgs& a, const MeshBufs& b, int emit)
+hipError_t launch_quads(hipStream_t s, const SlabArgs& a, const MeshBufs& b, const SlabBits& prev)
 {
-    const uint32_t nb = (a.ncells + kCellsPerBlock - 1) / kCellsPerBlock;
-    if (nb == 0) return hipSuccess;
-    if (emit) hipLaunchKernelGGL((k_quads<1>), dim3(nb), dim3(kBlock), 0, s, a, b);
-    else hipLaunchKernelGGL((k_quads<0>), dim3(nb), dim3(kBlock), 0, s, a, b);
+    if (a.ncells == 0) return hipSuccess;
+    const uint32_t groups = (a.ncells + kBlock - 1u) / kBlock;  // if every cell had a vertex
+    const dim3 grid(std::min(groups, 2048u));
+    hipLaunchKernelGGL((k_quads<0>), grid, dim3(kBlock), 0, s, a, b, prev);
+    hipLaunchKernelGGL(k_tri_offsets, dim3(1), dim3(1024), 0, s, b.tcount, b.toffset, b.counters, b.vcap);
+    hipLaunchKernelGGL((k_quads<1>), grid, dim3(kBlock), 0, s, a, b, prev);
     return hipGetLastError();
 }
 

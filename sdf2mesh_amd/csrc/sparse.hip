@@ -176,48 +176,6 @@ __device__ __forceinline__ uint32_t vertex_at(const SpPass& P, const SpJob& J, u
            (uint32_t)__builtin_popcount(b8 & ((1u << i) - 1u));
 }
 
-// dualcontour.wgsl:72-131: crossings on the 12 edges in the reference's order, counted
-// iff the sign changes and the crossing is not at the cell origin, centroid if >= 2.
-__device__ __forceinline__ bool contour_cell_sp(const float c[8], const float lo[3],
-                                                const float hi[3], float pos[3])
-{
-    uint32_t pm = 0;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) pm |= (uint32_t)(c[k] > 0.0f) << k;
-    if (pm == 0u || pm == 0xffu) return false;
-    // (corner a, corner b, axis of t, fixed x, fixed y, fixed z): z-, y-, then x-edges
-    constexpr uint8_t E[12][6] = {{0, 4, 2, 0, 0, 0}, {2, 6, 2, 0, 1, 0}, {1, 5, 2, 1, 0, 0},
-                                  {3, 7, 2, 1, 1, 0}, {0, 2, 1, 0, 0, 0}, {4, 6, 1, 0, 0, 1},
-                                  {1, 3, 1, 1, 0, 0}, {5, 7, 1, 1, 0, 1}, {0, 1, 0, 0, 0, 0},
-                                  {4, 5, 0, 0, 0, 1}, {2, 3, 0, 0, 1, 0}, {6, 7, 0, 0, 1, 1}};
-    float ax = 0.0f, ay = 0.0f, az = 0.0f, cnt = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 12; ++e) {
-        const float v0 = c[E[e][0]], v1 = c[E[e][1]];
-        const float t = (0.0f - v0) / (v1 - v0);
-        float x = E[e][3], y = E[e][4], z = E[e][5];
-        if (E[e][2] == 0) x = t;
-        else if (E[e][2] == 1) y = t;
-        else z = t;
-        if ((v0 > 0.0f) == (v1 > 0.0f)) x = y = z = 0.0f;
-        if (x > 0.0f || y > 0.0f || z > 0.0f) {
-            ax = ax + x;
-            ay = ay + y;
-            az = az + z;
-            cnt = cnt + 1.0f;
-        }
-    }
-    if (cnt <= 1.0f) return false;
-    pos[0] = canonical_nan(lo[0] + ((hi[0] - lo[0]) * ax) / cnt);
-    pos[1] = canonical_nan(lo[1] + ((hi[1] - lo[1]) * ay) / cnt);
-    pos[2] = canonical_nan(lo[2] + ((hi[2] - lo[2]) * az) / cnt);
-    return true;
-}
-
-}  // namespace
-
-namespace {
-
 // Exact pruning of postfix programs on boxes (device_interval.h).  The kept op indices
 // are written in order; the interval of the result is `top` when the walk ends.  The top
 // of the interval stack is kept in registers, deeper entries in LDS columns (entry d of
@@ -985,7 +943,7 @@ __device__ __forceinline__ void contour_tile(const SpPass& P, const TileGrid& G,
             tile_corners(box, A, G.bx, G.by, c, cv);
             const float lo[3] = {A.clo[0][cxl], A.clo[1][cyl], A.clo[2][czl]};
             const float hi[3] = {A.chi[0][cxl], A.chi[1][cyl], A.chi[2][czl]};
-            act[r] = contour_cell_sp(cv, lo, hi, pos[r]);
+            act[r] = contour_cell(cv, lo, hi, pos[r]);
             cell[r] = c;
             // cell_sign_changes (dualcontour.wgsl:57-69)
             sg[r] = (uint32_t)(cv[1] > 0.0f) | ((uint32_t)(cv[2] > 0.0f) << 1) |
