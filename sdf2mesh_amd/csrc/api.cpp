@@ -147,8 +147,9 @@ struct s2m_ctx {
     DevBuf vtx, keys, signs, tri, corners;
     DevBuf tile_tab, tile_lists, tile_lens, tile_flops;
     DevBuf sp_slot_of_tile, sp_tile_of_slot, sp_job_of_slot, sp_cellbits, sp_slot_rows, sp_boundary;
-    DevBuf sp_stage, sp_slot_nb, sp_slot_stage, sp_slot_live, sp_slot_hdr, sp_slot_rec, sp_block_stats;
-    DevBuf sp_queues, sp_super_iv, sp_super_lists, sp_super_lens, sp_super_act, sp_rows;
+    DevBuf sp_stage, sp_slot_nb, sp_slot_stage, sp_slot_live, sp_slot_hdr, sp_slot_rec;
+    DevBuf sp_queues, sp_super_iv, sp_super_lists, sp_super_act, sp_rows;
+    bool sp_dirty = false;  // a sparse pass was not queued to its end: `counters` may not be zero
     uint64_t slot_cap = 0;
     uint64_t stage_cap = 0;  // staged-cell entries of sp_stage
     int cus = 256;
@@ -574,15 +575,9 @@ int readback_begin(s2m_ctx* ctx, Readback& rb, uint64_t vcap, uint64_t tcap)
     return S2M_OK;
 }
 
-// After pass (or slab) k's kernels: its event, and its snapshot (counters NULL: the slab's
-// last kernel wrote it).
-int readback_mark(s2m_ctx* ctx, const uint64_t* counters, uint32_t k)
+// After pass (or slab) k's kernels (the last of which writes its snapshot): its event.
+int readback_mark(s2m_ctx* ctx, uint32_t k)
 {
-    if (counters) {
-        void* dev = nullptr;
-        HIP_TRY(hipHostGetDevicePointer(&dev, ctx->host_snap.p, 0));
-        HIP_TRY(launch_snapshot(ctx->stream, counters, static_cast<uint64_t*>(dev) + 4 * (size_t)k));
-    }
     hipEvent_t e = ctx->pass_event(k);
     if (!e) return fail(S2M_E_HIP, "event creation failed");
     HIP_TRY(hipEventRecord(e, ctx->stream));
@@ -876,7 +871,6 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
     size_t tab_bytes = 0;
     uint32_t list_stride = 1, box_stride = 1, prune_depth = 1;
     bool general_tiles = false;  // a tile's pruned program may not be a left fold
-    bool fold_jobs = false, other_jobs = false;  // programs that are / are not union folds
     uint64_t ntiles_all = 0, nrows_all = 0, plane_max = 0, cells_all = 0, planes_sum = 0;
     for (uint32_t i = 0; i < n; ++i) {
         build_sp_tables(jobs[i], progs[i], ps[i]->eps, tabs[i]);
@@ -884,7 +878,6 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
         tab_bytes += (tabs[i].bytes.size() + 255) & ~size_t(255);
         list_stride = std::max(list_stride, progs[i]->n);
         if (!left_fold_program(progs[i]->ops)) general_tiles = true;
-        (union_fold_program(progs[i]->ops) ? fold_jobs : other_jobs) = true;
         box_stride = std::max(box_stride, tabs[i].bmax[0] * tabs[i].bmax[1] * tabs[i].bmax[2]);
         uint32_t depth = 0;  // operand stack entries below the top (k_sp_prune's LDS stack)
         for (const s2m_op& o : progs[i]->ops) {
@@ -1034,13 +1027,21 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
     HIP_TRY(ctx->sp_rows.ensure(std::max<uint64_t>(nrows_pass, 1) * 4 * sizeof(uint32_t)));
     const uint32_t nsb_max = (uint32_t)((nrows_pass + kRowChunk - 1) / kRowChunk) + 1;  // vertex and triangle sums
     HIP_TRY(ctx->bcount.ensure((size_t)2 * nsb_max * kChunkSumStride * sizeof(uint32_t)));
-    // the counters, then per job kJobOut words (first vertex, first triangle, invalid quads)
+    // the counters, then per job kJobOut words (first vertex, first triangle, invalid quads);
+    // every pass leaves the counters it starts from at zero, so they are cleared here only
+    // when new or after a pass that was not queued to its end
+    const size_t counters_had = ctx->counters.bytes;
     HIP_TRY(ctx->counters.ensure((kNumCounters + (size_t)n * kJobOut) * sizeof(uint64_t)));
+    if (ctx->counters.bytes != counters_had || ctx->sp_dirty) {
+        HIP_TRY(hipMemsetAsync(ctx->counters.p, 0, ctx->counters.bytes, ctx->stream));
+        ctx->sp_dirty = false;
+    }
     HIP_TRY(ctx->sp_queues.ensure((size_t)kQueues * kQueueGroups * 32 * sizeof(uint32_t)));
     const uint64_t nsup_alloc = std::max<uint64_t>(nsuper_pass, 1);
-    HIP_TRY(ctx->sp_super_iv.ensure(nsup_alloc * list_stride * 2 * sizeof(double)));
-    HIP_TRY(ctx->sp_super_lists.ensure(nsup_alloc * list_stride * sizeof(uint16_t)));
-    HIP_TRY(ctx->sp_super_lens.ensure(nsup_alloc * sizeof(uint32_t)));
+    if (list_stride > kStageOps) {  // super-tile lists and intervals that do not fit LDS
+        HIP_TRY(ctx->sp_super_iv.ensure(nsup_alloc * list_stride * 2 * sizeof(double)));
+        HIP_TRY(ctx->sp_super_lists.ensure(nsup_alloc * list_stride * sizeof(uint16_t)));
+    }
     HIP_TRY(ctx->sp_super_act.ensure(nsup_alloc * sizeof(uint64_t)));
 
     // a closed surface crosses O(res^2) cells: start from 6 per row-plane cell
@@ -1050,7 +1051,11 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
     uint64_t want_s = std::min<uint64_t>(tiles_pass, std::max<uint64_t>({4096, tiles_pass / 4, ctx->slot_cap}));
     const uint64_t tile_blocks = (uint64_t)std::max(1, ctx->cus) * kTileBlocksPerCU;
     uint64_t stage_cap = ctx->stage_cap;
-    if (rb) HIP_TRY(ctx->host_snap.ensure((size_t)npass * 4 * sizeof(uint64_t)));
+    void* snap_dev = nullptr;
+    if (rb) {
+        HIP_TRY(ctx->host_snap.ensure((size_t)npass * 4 * sizeof(uint64_t)));
+        HIP_TRY(hipHostGetDevicePointer(&snap_dev, ctx->host_snap.p, 0));
+    }
 
     for (int attempt = 0; attempt < 4; ++attempt) {
         HIP_TRY(ctx->vtx.ensure(want_v * 6 * sizeof(float)));
@@ -1087,11 +1092,9 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
         b.vcap = want_v;
         b.tcap = want_t;
         b.counters = ctx->counters.as<uint64_t>();
-        b.bcount = ctx->bcount.as<uint32_t>();  // the offset scan's chunk sums
 
         uint64_t* job_out = b.counters + kNumCounters;
-        HIP_TRY(ctx->sp_block_stats.ensure(tile_blocks * 3 * sizeof(uint64_t)));
-        // the last pass folded and the counters and job rows written to mapped host memory
+        // the counters and job rows are written to mapped host memory by the last pass
         const uint32_t nback = kNumCounters + n * kJobOut;
         HIP_TRY(ctx->host_back.ensure(nback * sizeof(uint64_t)));
         void* back_dev = nullptr;
@@ -1102,11 +1105,7 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
         hipEvent_t ev_start = nullptr, ev_end = nullptr;
         uint64_t tiles_total = 0;
         auto enqueue = [&]() -> int {  // the job's kernels, in stream order
-        HIP_TRY(launch_sparse_job_begin(ctx->stream, b.counters, kNumCounters + n * kJobOut,
-                                        ctx->sp_queues.as<uint32_t>(), b.bcount, 2 * nsb_max,
-                                        ctx->sp_block_stats.as<uint64_t>(), (uint32_t)tile_blocks,
-                                        ctx->sp_boundary.as<uint32_t>(),
-                                        n == 1 && npass > 1 ? (uint32_t)plane_max : 0u));
+        ctx->sp_dirty = true;  // until every pass is queued
         if (ctx->profiling) {
             ev_start = ctx->next_event();
             HIP_TRY(hipEventRecord(ev_start, ctx->stream));
@@ -1150,7 +1149,6 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
             P.slot_hdr = ctx->sp_slot_hdr.as<SlotHdr>();
             P.slot_nb = ctx->sp_slot_nb.as<int32_t>();
             P.slot_rec = ctx->sp_slot_rec.as<uint4>();
-            P.block_stats = ctx->sp_block_stats.as<uint64_t>();
             P.slot_rows = ctx->sp_slot_rows.as<uint32_t>();
             P.row_sum = ctx->sp_rows.as<uint32_t>();
             P.row_off = P.row_sum + 2 * P.nrows;
@@ -1158,7 +1156,6 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
             P.queues = ctx->sp_queues.as<uint32_t>();
             P.super_iv = ctx->sp_super_iv.as<double2>();
             P.super_lists = ctx->sp_super_lists.as<uint16_t>();
-            P.super_lens = ctx->sp_super_lens.as<uint32_t>();
             P.super_act = ctx->sp_super_act.as<uint64_t>();
             P.job_out = job_out;
             hipEvent_t m[kSparseMarks] = {};
@@ -1166,23 +1163,25 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
                 for (auto& e : m) e = ctx->next_event();
             else if (ctx->profiling)  // the evaluation launches only: fewer markers between kernels
                 m[1] = ctx->next_event(), m[2] = ctx->next_event();
-            if (pass > 0)
-                HIP_TRY(launch_sparse_pass_begin(ctx->stream, b.counters, ctx->sp_queues.as<uint32_t>(), b.bcount,
-                                                 2 * nsb_max));
+            P.bsum = ctx->bcount.as<uint32_t>();
+            P.nbsum = 2 * nsb_max;
+            P.nclear = pass == 0 ? (uint32_t)(kNumCounters + n * kJobOut) : 0u;
+            P.nbnd = pass == 0 && n == 1 && npass > 1 ? (uint32_t)plane_max : 0u;
+            P.nback = nback;
+            P.back = pass + 1 == npass ? static_cast<uint64_t*>(back_dev) : nullptr;
+            P.snap = rb ? static_cast<uint64_t*>(snap_dev) + 4 * (size_t)pass : nullptr;
             const int boundary = (n == 1 && pass + 1 < npass) ? 1 : 0;
-            HIP_TRY(launch_sparse_pass(ctx->stream, P, b, ctx->cus, (uint32_t)tile_blocks, general_tiles, fold_jobs,
-                                       other_jobs, boundary,
-                                         ctx->profiling ? m : nullptr));
+            HIP_TRY(launch_sparse_pass(ctx->stream, P, b, ctx->cus, (uint32_t)tile_blocks, general_tiles, boundary,
+                                       ctx->profiling ? m : nullptr));
             if (ctx->profiling) ev.insert(ev.end(), m, m + kSparseMarks);
             tiles_total += P.ntiles;
             if (rb) {  // this pass's snapshot; the previous pass's copies once it ends
-                int rrc = readback_mark(ctx, b.counters, pass);
+                int rrc = readback_mark(ctx, pass);
                 if (!rrc && pass > 0) rrc = readback_pass(ctx, *rb, want_v, want_t, want_s, stage_cap);
                 if (rrc) return rrc;
             }
         }
-        HIP_TRY(launch_sparse_job_end(ctx->stream, b.counters, nback, static_cast<uint64_t*>(back_dev),
-                                      ctx->sp_block_stats.as<uint64_t>(), (uint32_t)tile_blocks));
+        ctx->sp_dirty = false;
         if (ctx->profiling) {
             ev_end = ctx->next_event();
             HIP_TRY(hipEventRecord(ev_end, ctx->stream));
@@ -1198,16 +1197,15 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
             std::string key(reinterpret_cast<const char*>(img), img_bytes);
             auto put = [&key](const void* q, size_t m) { key.append(static_cast<const char*>(q), m); };
             for (const DevBuf* d : {&ctx->vtx, &ctx->keys, &ctx->signs, &ctx->tri, &ctx->counters, &ctx->bcount,
-                                    &ctx->sp_queues, &ctx->sp_block_stats, &ctx->tile_tab, &ctx->tile_lists,
+                                    &ctx->sp_queues, &ctx->tile_tab, &ctx->tile_lists,
                                     &ctx->tile_lens, &ctx->tile_flops, &ctx->sp_slot_of_tile, &ctx->sp_tile_of_slot,
                                     &ctx->sp_job_of_slot, &ctx->sp_cellbits, &ctx->sp_stage, &ctx->sp_slot_stage,
                                     &ctx->sp_slot_live, &ctx->sp_slot_hdr, &ctx->sp_slot_nb, &ctx->sp_slot_rec,
                                     &ctx->sp_slot_rows, &ctx->sp_rows, &ctx->sp_super_iv, &ctx->sp_super_lists,
-                                    &ctx->sp_super_lens, &ctx->sp_super_act, &ctx->sp_boundary})
+                                    &ctx->sp_super_act, &ctx->sp_boundary})
                 put(&d->p, sizeof d->p);
             const uint64_t scal[] = {want_v, want_t, want_s, stage_cap, tile_blocks, nsb_max, list_stride,
-                                     prune_depth, box_stride, (uint64_t)general_tiles, (uint64_t)fold_jobs,
-                                     (uint64_t)other_jobs, n, (uint64_t)(uintptr_t)back_dev};
+                                     prune_depth, box_stride, (uint64_t)general_tiles, n, (uint64_t)(uintptr_t)back_dev};
             put(scal, sizeof scal);
             const int grc = run_graph(ctx, key, enqueue);
             if (grc) return grc;
@@ -1640,7 +1638,7 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
             if (m[4]) HIP_TRY(hipEventRecord(m[4], ctx->stream));
             if (rb) {  // the slab's vertices and triangles are final; the copies of the slab two
                        // before (waiting for it leaves this slab and the next evaluation queued)
-                int rrc = readback_mark(ctx, nullptr, (uint32_t)slabs);
+                int rrc = readback_mark(ctx, (uint32_t)slabs);
                 if (!rrc && slabs > 1) rrc = readback_pass(ctx, *rb, want_v, want_t, ~0ull, ~0ull);
                 if (rrc) return rrc;
             }
@@ -1836,8 +1834,8 @@ void s2m_destroy(s2m_ctx* ctx)
                       &ctx->tile_flops, &ctx->sp_slot_of_tile, &ctx->sp_tile_of_slot,
                       &ctx->sp_job_of_slot, &ctx->sp_cellbits, &ctx->sp_slot_rows,
                       &ctx->sp_boundary, &ctx->sp_queues, &ctx->sp_super_iv,
-                      &ctx->sp_super_lists, &ctx->sp_super_lens, &ctx->sp_super_act, &ctx->sp_rows,
-                      &ctx->sp_stage, &ctx->sp_slot_nb, &ctx->sp_slot_stage, &ctx->sp_slot_live, &ctx->sp_slot_hdr, &ctx->sp_slot_rec, &ctx->sp_block_stats})
+                      &ctx->sp_super_lists, &ctx->sp_super_act, &ctx->sp_rows,
+                      &ctx->sp_stage, &ctx->sp_slot_nb, &ctx->sp_slot_stage, &ctx->sp_slot_live, &ctx->sp_slot_hdr, &ctx->sp_slot_rec})
         b->release();
     for (DevBuf& b : ctx->batch_dense) b.release();
     for (s2m_ctx::PassSet& S : ctx->pset) {

@@ -9,10 +9,10 @@
 // bit-identical to tape_eval (device_sdf.h): the same functions in the same order.
 #pragma once
 #include "device_sdf.h"
+#include "internal.h"
 
 namespace s2m {
 
-constexpr uint32_t kStageOps = 128;            // longest program staged in LDS
 constexpr uint32_t kLinearFlag = 0x80000000u;  // SpPass::lens: the program is a left fold
 
 template <uint32_t CAP>

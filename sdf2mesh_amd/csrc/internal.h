@@ -41,6 +41,8 @@ enum Counter : uint32_t {
     kSlotsMax = 9,     // largest kSlotsUsed of the job so far
     kStageUsed = 10,   // staged active cells of the current pass (sparse path)
     kBrickAlloc = 11,  // dense slab: listed bricks (low word), staged vertices (high word)
+    kSlotsNow = 13,    // sparse pass: its slots and staged cells, once they are final
+    kStageNow = 14,
     kStageMax = 12,    // largest kStageUsed of the job so far
     kNumCounters = 16
 };
@@ -76,7 +78,8 @@ struct SlabBits {
 
 constexpr uint32_t kTile = 8;  // cells per tile edge (sparse pipeline)
 constexpr uint32_t kSuper = 4;  // tiles per super-tile edge (first pruning level)
-constexpr uint32_t kSingleSign = 0xffffffffu;  // super_lens: the SDF keeps one sign there
+constexpr uint32_t kStageOps = 128;  // longest program staged in LDS (device_staged.h)
+constexpr uint32_t kSingleSign = 0xffffffffu;  // a super-tile's list length: the SDF keeps one sign there
 constexpr uint32_t kStageChunkHost = 1024;  // staged-cell allocation chunk (sparse.hip)
 constexpr uint32_t kTileBlocksPerCU = 8;    // most k_sp_tiles blocks per compute unit
 constexpr uint32_t kTileRecBytes = 2720;    // per slot: k_sp_tiles' staged record (sparse.hip)
@@ -143,9 +146,8 @@ struct SpPass {
     uint64_t ntrows;           // tile rows (tile layer, ty) of the pass
     uint64_t boundary_cells;   // rx * ry of jobs[0] when a boundary plane is written
     uint64_t nsuper;           // super-tiles of the pass
-    double2* super_iv;         // [super-tile][list_stride] primitive intervals (lo, hi)
-    uint16_t* super_lists;     // [super-tile][list_stride] pruned op indices
-    uint32_t* super_lens;      // [super-tile] list length or kSingleSign
+    double2* super_iv;         // [super-tile][list_stride] primitive intervals (lo, hi), and pruned op
+    uint16_t* super_lists;     // indices, of programs too long for LDS (kStageOps; NULL if none is)
     uint64_t* super_act;       // [super-tile] bit (z * 4 + y) * 4 + x: that tile has a slot
     uint16_t* lists;           // [tile][list_stride] pruned op indices
     uint32_t* lens;            // [tile]
@@ -164,13 +166,21 @@ struct SpPass {
     SlotHdr* slot_hdr;         // [slot]
     int32_t* slot_nb;          // [slot][8] slots of the tile (tx - dx, ty - dy, tz - dz) at (dz * 2 + dy) * 2 + dx
     uint4* slot_rec;           // [slot] kTileRecBytes: k_sp_tiles<1>'s staged record
-    uint64_t* block_stats;     // [k_sp_tiles block][3]: tiles, points, flops of the job so far
     uint32_t* slot_rows;       // [4][slot_cap][64] per row of each slot's tile: vertices,
                                // triangles, first vertex / triangle within the row
     uint32_t* row_sum;         // [2][nrows] vertices, triangles per row
     uint32_t* row_off;         // [2][nrows] exclusive offsets: global vertex / triangle index
     uint64_t* counters;
-    uint32_t* queues;          // [kQueues][kQueueGroups][32] work queue counters (word 0)
+    uint32_t* queues;          // [kQueues][kQueueGroups][32] work queue counters (word 0); beside those of
+                               // queue 0, as u64 words 1..3: tiles, points, flops of the job so far
+    uint32_t* bsum;            // the offset scan's chunk sums, kChunkSumStride words apart
+    uint32_t nbsum;
+    uint32_t nclear;           // a job's first pass: counters and job rows to clear, else 0
+    uint32_t nbnd;             // before a multi-pass job: cells of the boundary plane to clear
+    uint32_t nback;            // words of `back`
+    uint64_t* back;            // mapped host memory for the counters and job rows after a job's last
+                               // pass, else NULL
+    uint64_t* snap;            // mapped host memory for the pass's totals, or NULL
     uint64_t* job_out;         // [job][kJobOut]
 };
 
@@ -181,7 +191,6 @@ struct MeshBufs {
     uint32_t* tri;         // 3 per triangle
     uint64_t vcap, tcap;   // capacities (vertices, triangles)
     uint64_t* counters;    // Counter
-    uint32_t* bcount;      // sparse pass: the offset scan's chunk sums
     // dense slab
     uint64_t* actbits;     // bit c % 64 of word c / 64 = cell c has a vertex
     SlabBits bits;         // the same words with their prefix tables
@@ -217,34 +226,11 @@ hipError_t launch_bailout_check(hipStream_t s, uint64_t* cnt);
 // A tape just copied to the device: every Mandelbulb op's f[3] set to the bailout
 // threshold of its f[1] (sd_mandelbulb reads it there instead of computing it per point).
 hipError_t launch_tape_prepare(hipStream_t s, s2m_op* ops, uint32_t n);
-// Between passes of a job: slot and staging counters folded into their maxima, the
-// previous pass's totals made the next pass's first indices, work queues and the
-// offset scan's nbsum chunk sums (bsum, kChunkSumStride words apart) cleared.
-hipError_t launch_sparse_pass_begin(hipStream_t s, uint64_t* counters, uint32_t* queues, uint32_t* bsum,
-                                    uint32_t nbsum);
-// After a job's last pass: slot and staging counters folded into their maxima, then
-// counters[0 .. n) copied to `out` (a device address of mapped host memory).
-// The tile blocks' statistics (nstats entries of tiles, points, flops) summed into
-// kTilesActive, kEvalPoints and kEvalFlops first.
-hipError_t launch_sparse_job_end(hipStream_t s, uint64_t* counters, uint32_t n, uint64_t* out,
-                                 const uint64_t* stats, uint32_t nstats);
-// A job's first pass: counters[0 .. n) (the counters and the job output rows), the work
-// queues and the nbsum chunk sums (bsum, kChunkSumStride words apart) cleared, and the
-// nbnd entries of a multi-pass job's boundary plane set to "no vertex".
-hipError_t launch_sparse_job_begin(hipStream_t s, uint64_t* counters, uint32_t n, uint32_t* queues,
-                                   uint32_t* bsum, uint32_t nbsum, uint64_t* stats, uint32_t nstats,
-                                   uint32_t* boundary, uint32_t nbnd);
 // cus: compute units of the device; tile_blocks: most blocks of a k_sp_tiles launch (each
 // holds a staging chunk); general_tiles: some tile's pruned program may not be a left fold
 // (false when every job's whole program is one: its pruned programs are then left folds).
-// fold_jobs / other_jobs: some job's program is / is not a left fold of unions (pruned at
-// the super-tile level without a sequential walk).
 hipError_t launch_sparse_pass(hipStream_t s, const SpPass& P, const MeshBufs& b, int cus,
-                              uint32_t tile_blocks, bool general_tiles, bool fold_jobs, bool other_jobs,
-                              int boundary_plane, hipEvent_t* marks);
-// out[0..4) (a device address of mapped host memory) = the vertex and triangle totals so
-// far and the current pass's slot and staging use, after the kernels queued before it.
-hipError_t launch_snapshot(hipStream_t s, const uint64_t* counters, uint64_t* out);
+                              uint32_t tile_blocks, bool general_tiles, int boundary_plane, hipEvent_t* marks);
 // Contour corner values given per cell (test hook): cells of the slab read their 8
 // corners from `corners` (8 floats per cell, cells in (z,y,x) order from plane z0).
 hipError_t launch_cells_from_corners(hipStream_t s, const SlabArgs& a, const float* corners,

@@ -6,12 +6,11 @@
 // are evaluated and contoured.  A pass covers the tiles of one slab of one job, or of
 // every job of a batch (each job whole); tiles, super-tiles and row segments of the pass
 // are numbered job after job.  In stream order:
-//   k_sp_prune_fold (left folds of unions / smooth unions) or k_sp_prune_prims +
-//   k_sp_prune_super (other programs), then k_sp_prune   exact interval pruning: the
-//                   job's program on each super-tile's padded box, then the super-tile's
-//                   list on each of its tiles (one lane per tile); single-signed tiles are
-//                   dropped, the others get a slot in a pool shared by all jobs (and a
-//                   flag when their list is a left fold)
+//   k_sp_prune      exact interval pruning, one wave per super-tile: the job's program on
+//                   the super-tile's padded box, then the super-tile's list on each of its
+//                   tiles (one lane per tile); single-signed tiles are dropped, the others
+//                   get a slot in a pool shared by all jobs (and a flag when their list is
+//                   a left fold).  Also clears what the pass's later kernels count into.
 //   k_sp_bricks     per slot, one lane per brick of 2x2x2 cells: interval bounds of a
 //                   left fold on the brick (bricks that keep one sign are not evaluated),
 //                   and the slot's record: header, live bricks, axis tables, box
@@ -32,6 +31,8 @@
 //                   4-tap normals (the tile's pruned program), then the triangles of
 //                   their quads, vertex indices relative to the job's first vertex
 //   k_sp_boundary   (multi-slab single job) cell -> vertex map of the slab's last plane
+// The totals go to mapped host memory from the last kernel, k_sp_emit<1>: a pass of folds is
+// seven launches (of about 4.5 us each at any small size).
 // The per-slot kernels are persistent (as many blocks as the device holds) and draw slots
 // from a work queue.  A cell's vertex index is never stored: it is the first index of its row segment plus
 // the number of cells with a vertex before it in the segment (the slot's cell bits).
@@ -62,9 +63,11 @@ namespace {
 
 __device__ __forceinline__ uint32_t lane() { return thread_id() & 63u; }
 
-__device__ __forceinline__ uint32_t active_slots(const SpPass& P)
+// Slots of the pass.  k_sp_rowdown moves the count from kSlotsUsed (zero when k_sp_prune
+// starts) to kSlotsNow, where k_sp_emit reads it.
+__device__ __forceinline__ uint32_t active_slots(const SpPass& P, uint32_t counter = kSlotsUsed)
 {
-    const uint64_t n = P.counters[kSlotsUsed];
+    const uint64_t n = P.counters[counter];
     return (uint32_t)(n < P.slot_cap ? n : P.slot_cap);
 }
 
@@ -366,38 +369,25 @@ __device__ __forceinline__ void super_tiles(const SpJob& J, uint64_t s, uint32_t
 }
 
 // ---------------------------------------------------------------------------------
-// Pruning, in three launches:
-//  k_sp_prune_prims  one lane per (super-tile, primitive): the primitive's interval on the
-//                    super-tile's padded box (super_iv)
-//  k_sp_prune_super  one lane per super-tile: the job's program combined in order from
-//                    those intervals, exactly pruned (super_lists), or kSingleSign when
-//                    the SDF keeps one sign on the super-tile (super_lens)
-//  k_sp_prune        one wave per super-tile, lane l = its tile (l % 4, l / 4 % 4, l / 16):
-//                    the super-tile's list pruned on the tile's padded box (every lane walks
-//                    the same list: wave-uniform op dispatch).  Tiles that keep one sign are
-//                    dropped, the others get a slot in the pool shared by all jobs (and a
-//                    flag when their list is a left fold).
-// Dynamic LDS of the last two: the prune stack (P.prune_depth entries per lane).
+// k_sp_prune, one wave per super-tile (one launch: three or four of these steps as kernels
+// of their own cost more in launches and list traffic than in work):
+//  1. the super-tile's list: the job's program exactly pruned on its padded box, or
+//     kSingleSign when the SDF keeps one sign there.  Left folds of unions: prune_fold, a
+//     lane per op.  Other programs: a lane per primitive for its interval on the box
+//     (prim_intervals), then every lane walks the program in order (walk_super; the walk is
+//     serial, so the lanes take the same steps).
+//  2. lane l = its tile (l % 4, l / 4 % 4, l / 16): the list pruned on the tile's padded box
+//     (every lane walks the same list: wave-uniform op dispatch).  Tiles that keep one sign
+//     are dropped, the others get a slot in the pool shared by all jobs (and a flag when
+//     their list is a left fold).
+// Dynamic LDS: the prune stack (P.prune_depth entries per lane).  Lists and intervals of
+// programs of at most kStageOps ops live in LDS, of longer ones in super_lists / super_iv.
 // ---------------------------------------------------------------------------------
-__global__ __launch_bounds__(64) void k_sp_prune_prims(SpPass P, uint32_t chunks)
-{
-    const uint64_t s = blockIdx.x / chunks;
-    const uint32_t k = (blockIdx.x % chunks) * 64u + (thread_id() & 63u);
-    const SpJob& J = P.jobs[__builtin_amdgcn_readfirstlane(job_of(P, s, true))];
-    if (J.union_fold || k >= J.nops || J.ops[k].code >= S2M_OP_UNION) return;  // folds: k_sp_prune_fold
-    uint32_t t0[3], t1[3];
-    super_tiles(J, s, t0, t1);
-    double bl[3], bh[3];
-    tiles_box(J, t0, t1, bl, bh);
-    const Iv v = iv_primitive(J.ops[k].code, J.ops[k].f, bl, bh);
-    P.super_iv[s * P.list_stride + k] = make_double2(v.lo, v.hi);
-}
 
-// ---------------------------------------------------------------------------------
-// k_sp_prune_fold: the super-tile lists of programs that are left folds of unions and
-// smooth unions (P0 P1 op1 P2 op2 ..., op in {UNION, SMOOTH_UNION with k > 0}), one wave
-// per super-tile, without a sequential walk: lane q evaluates op q's interval, and
-// primitive P_m (m >= 1) is dropped with its operator when
+// prune_fold: the super-tile list of a program that is a left fold of unions and smooth
+// unions (P0 P1 op1 P2 op2 ..., op in {UNION, SMOOTH_UNION with k > 0}), without a
+// sequential walk: lane q evaluates op q's interval, and primitive P_m (m >= 1) is dropped
+// with its operator when
 //     lo(P_m) >= U_{m-1} + k_m + slack,   U_{m-1} = min over j < m of hi(P_j),
 // a prefix minimum over the lanes.  The accumulated value after m - 1 steps never exceeds
 // min_j p_j by more than the rounding of its fp32 operations (smooth union <= min of its
@@ -408,20 +398,11 @@ __global__ __launch_bounds__(64) void k_sp_prune_prims(SpPass P, uint32_t chunks
 // changes acc, so later bounds stay valid.  The super-tile keeps one sign when
 // min_j hi(P_j) + slack < 0 (acc < 0), or when min over the kept P_j of lo(P_j) - the kept
 // smooth radii / 4 - slack > 0 (smooth union >= min of its operands - k / 4).
-// ---------------------------------------------------------------------------------
-__global__ __launch_bounds__(64) void k_sp_prune_fold(SpPass P)
+__device__ __forceinline__ uint32_t prune_fold(const SpJob& J, const double* bl, const double* bh, uint32_t ln,
+                                               uint16_t* out)
 {
-    const uint64_t s = blockIdx.x;
-    const uint32_t ln = thread_id() & 63u;
-    const SpJob& J = P.jobs[__builtin_amdgcn_readfirstlane(job_of(P, s, true))];
-    if (!J.union_fold) return;
-    uint32_t t0[3], t1[3];
-    super_tiles(J, s, t0, t1);
-    double bl[3], bh[3];
-    tiles_box(J, t0, t1, bl, bh);
     const s2m_op* ops = J.ops;
     const uint32_t nops = J.nops;
-    uint16_t* out = P.super_lists + s * P.list_stride;
     double carry_u = kHuge;    // min hi(P_j) over the primitives so far
     double carry_mag = 0.0;    // sum of |P_j| + k_j over the primitives so far
     double carry_max = 0.0;    // max of |P_j| + k_j so far
@@ -497,48 +478,65 @@ __global__ __launch_bounds__(64) void k_sp_prune_fold(SpPass P)
     }
     const double slack = kMargin * (carry_mag + carry_cnt * (carry_max + carry_ka));
     const bool one_sign = (carry_u + slack < 0.0) || (carry_lo > -kHuge && carry_lo - carry_k4 - slack > 0.0);
-    if (ln == 0) P.super_lens[s] = one_sign ? kSingleSign : nkept;
+    return one_sign ? kSingleSign : nkept;
 }
 
-constexpr uint32_t kSuperChunk = 16;  // ops of a lane's program staged in LDS at a time
-
-__global__ __launch_bounds__(64) void k_sp_prune_super(SpPass P)
+// Op q's code and smoothing radius, and the interval of a primitive on the box.
+__device__ __forceinline__ void prim_intervals(const SpJob& J, const double* bl, const double* bh, uint32_t ln, double2* iv,
+                                               uint32_t* codes, uint32_t* radii)
 {
-    extern __shared__ double prune_lds[];
-    __shared__ double2 civ[kSuperChunk][64];   // primitive intervals
-    __shared__ uint32_t ccode[kSuperChunk][64];
-    __shared__ float ck[kSuperChunk][64];      // operator smoothing radius
-    const uint32_t D = P.prune_depth, ln = thread_id() & 63u;
-    const PruneStack S = PruneStack::at(prune_lds, D);
-    const uint64_t s = (uint64_t)blockIdx.x * 64u + ln;
-    if (s >= P.nsuper) return;
-    const SpJob& J = P.jobs[job_of(P, s, true)];
-    if (J.union_fold) return;  // k_sp_prune_fold
-    const s2m_op* ops = J.ops;
-    const uint32_t nops = J.nops;
-    const double2* iv = P.super_iv + s * P.list_stride;
-    uint16_t* out = P.super_lists + s * P.list_stride;
-    PruneWalk w;
-    for (uint32_t q0 = 0; q0 < nops; q0 += kSuperChunk) {
-        // the lane's next ops and intervals: all loads in flight at once (each lane reads
-        // back only its own column)
-        const uint32_t m = min(kSuperChunk, nops - q0);
-        for (uint32_t j = 0; j < m; ++j) {
-            ccode[j][ln] = ops[q0 + j].code;
-            ck[j][ln] = ops[q0 + j].f[0];
-            civ[j][ln] = iv[q0 + j];  // operators' entries are unused
+    for (uint32_t q = ln; q < J.nops; q += 64u) {
+        const s2m_op& o = J.ops[q];
+        const uint32_t code = o.code;
+        if (codes) {
+            codes[q] = code;
+            radii[q] = __float_as_uint(o.f[0]);
         }
-        for (uint32_t j = 0; j < m; ++j) {
-            const uint32_t q = q0 + j, code = ccode[j][ln];
-            if (code < S2M_OP_UNION) {
-                const double2 v = civ[j][ln];
-                w.prim(q, q, Iv{v.x, v.y, v.x > -kHuge}, out, S, ln);  // known iff lo > -kHuge
-            } else {
-                w.op(q, code, ck[j][ln], out, S, ln);
-            }
+        if (code >= S2M_OP_UNION) continue;
+        const Iv v = iv_primitive(code, o.f, bl, bh);
+        iv[q] = make_double2(v.lo, v.hi);
+    }
+}
+
+// The job's program walked in order on those intervals; every lane takes the same steps
+// and writes the same list.
+__device__ __forceinline__ uint32_t walk_super(const SpJob& J, const double2* iv, const uint32_t* codes,
+                                               const uint32_t* radii, const PruneStack& S, uint32_t ln, uint16_t* out)
+{
+    PruneWalk w;
+    for (uint32_t q = 0; q < J.nops; ++q) {
+        const uint32_t code = __builtin_amdgcn_readfirstlane(codes ? codes[q] : J.ops[q].code);
+        if (code < S2M_OP_UNION) {
+            const double2 v = iv[q];
+            w.prim(q, q, Iv{v.x, v.y, v.x > -kHuge}, out, S, ln);  // known iff lo > -kHuge
+        } else {
+            w.op(q, code, codes ? __uint_as_float(radii[q]) : J.ops[q].f[0], out, S, ln);
         }
     }
-    P.super_lens[s] = w.one_sign() ? kSingleSign : w.len;
+    return w.one_sign() ? kSingleSign : w.len;
+}
+
+// What the pass's later kernels count into, cleared (by all blocks): the job rows and
+// counters of a job's first pass (for a later pass the totals so far become its first
+// indices), work queues with the statistics beside them, chunk sums, and before a
+// multi-pass job the boundary plane (no vertex carried yet).  kSlotsUsed and kStageUsed,
+// which this kernel and the tile kernels count, are zero already (k_sp_rowdown).
+__device__ __forceinline__ void clear_pass(const SpPass& P)
+{
+    const uint32_t t = blockIdx.x * 64u + (thread_id() & 63u), step = gridDim.x * 64u;
+    for (uint32_t i = t; i < P.nclear; i += step)
+        if (i != kSlotsUsed && i != kStageUsed) P.counters[i] = 0;
+    if (P.nclear == 0 && t == 0) {
+        P.counters[kVtxPrev] = P.counters[kVtxTotal];
+        P.counters[kTriPrev] = P.counters[kTriTotal];
+    }
+    constexpr uint32_t kLines = kQueues * kQueueGroups;
+    for (uint32_t i = t; i < kLines; i += step) P.queues[i * 32u] = 0;
+    if (P.nclear)  // the statistics are the whole job's
+        for (uint32_t i = t; i < 3u * kQueueGroups; i += step)
+            reinterpret_cast<uint64_t*>(P.queues)[(i % kQueueGroups) * 16u + 1u + i / kQueueGroups] = 0;
+    for (uint32_t i = t; i < P.nbsum; i += step) P.bsum[i * kChunkSumStride] = 0;
+    for (uint32_t i = t; i < P.nbnd; i += step) P.jobs[0].boundary[i] = kNone;
 }
 
 __global__ __launch_bounds__(64) void k_sp_prune(SpPass P)
@@ -547,19 +545,37 @@ __global__ __launch_bounds__(64) void k_sp_prune(SpPass P)
     __shared__ StagedTape T;          // the super-tile's list (at most kStageOps ops)
     __shared__ uint16_t idx[kStageOps];  // op index of each staged op
     __shared__ uint32_t sums[kStageOps];  // its flops | kFoldBit for primitives other than the Mandelbulb
+    static_assert(sizeof T.f >= kStageOps * sizeof(double2), "intervals share the staged operands' space");
+    clear_pass(P);
     const uint32_t D = P.prune_depth, ln = thread_id() & 63u;
     const PruneStack S = PruneStack::at(prune_lds, D);
     const uint64_t s = blockIdx.x;
     const uint32_t jid = __builtin_amdgcn_readfirstlane(job_of(P, s, true));
     const SpJob& J = P.jobs[jid];
-    const uint32_t sl = __builtin_amdgcn_readfirstlane(P.super_lens[s]);
+    const bool small = J.nops <= kStageOps;
+    uint16_t* in = small ? idx : P.super_lists + s * P.list_stride;
     uint32_t t0[3], t1[3];
     super_tiles(J, s, t0, t1);
+    uint32_t sl;
+    {
+        double bl[3], bh[3];
+        tiles_box(J, t0, t1, bl, bh);
+        if (J.union_fold) {
+            sl = prune_fold(J, bl, bh, ln, in);
+        } else {
+            double2* iv = small ? reinterpret_cast<double2*>(T.f) : P.super_iv + s * P.list_stride;
+            uint32_t *codes = small ? T.code : nullptr, *radii = small ? T.iarg : nullptr;
+            prim_intervals(J, bl, bh, ln, iv, codes, radii);
+            __syncthreads();  // visible to all lanes
+            sl = walk_super(J, iv, codes, radii, S, ln, in);
+        }
+        sl = __builtin_amdgcn_readfirstlane(sl);
+    }
+    __syncthreads();  // the list is visible
     const uint32_t tx = t0[0] + (ln & 3u), ty = t0[1] + ((ln >> 2) & 3u), tz = t0[2] + (ln >> 4);
     const bool valid = tx <= t1[0] && ty <= t1[1] && tz <= t1[2];
     const uint64_t tile = J.tile_base + ((uint64_t)(tz - J.tz0) * J.nty + ty) * J.ntx + tx;
     const s2m_op* ops = J.ops;
-    const uint16_t* in = P.super_lists + s * P.list_stride;
     const bool staged = sl != kSingleSign && sl <= kStageOps;
     auto op_sum = [&](uint32_t i) {
         const uint32_t c = ops[i].code;
@@ -568,8 +584,9 @@ __global__ __launch_bounds__(64) void k_sp_prune(SpPass P)
     if (staged) {
         stage_tape(T, ops, in, sl);
         for (uint32_t k = ln; k < sl; k += 64u) {
-            idx[k] = in[k];
-            sums[k] = op_sum(in[k]);
+            const uint32_t i = in[k];
+            if (!small) idx[k] = (uint16_t)i;
+            sums[k] = op_sum(i);
         }
     }
     __syncthreads();
@@ -1202,11 +1219,11 @@ __device__ __forceinline__ void tiles_body(const SpPass& P)
             flops_done += (uint64_t)evaluated * tile_flops;
         }
     }
-    if (thread_id() == 0 && tiles_done) {  // the block's own entry (no shared address): k_sp_job_end sums them
-        uint64_t* st = P.block_stats + 3u * blockIdx.x;
-        st[0] += tiles_done;
-        st[1] += points_done;
-        st[2] += flops_done;
+    if (thread_id() == 0 && tiles_done) {  // the job's statistics, one set per queue group (k_sp_emit sums them)
+        unsigned long long* st = reinterpret_cast<unsigned long long*>(P.queues) + (blockIdx.x % kQueueGroups) * 16u + 1u;
+        atomicAdd(&st[0], (unsigned long long)tiles_done);
+        atomicAdd(&st[1], (unsigned long long)points_done);
+        atomicAdd(&st[2], (unsigned long long)flops_done);
     }
 }
 
@@ -1324,13 +1341,39 @@ __global__ __launch_bounds__(64) void k_sp_quadcount(SpPass P, MeshBufs b)
 // slots whose program is a left fold, LINEAR = 0 the others (launched only when a program
 // of the pass is not a left fold; its stack interpreter needs more registers).
 // ---------------------------------------------------------------------------------
+// Block 0 of k_sp_emit<1>: the totals so far and the pass's use of the slot and staging
+// capacities to P.snap, so that the host can copy the pass's finished vertices and
+// triangles while later passes run; after a job's last pass the statistics summed and
+// counters[0 .. nback) to P.back (both in mapped host memory, NULL: not wanted).  Nothing
+// in the kernel changes them.
+__device__ __forceinline__ void report(const SpPass& P)
+{
+    const uint32_t ln = lane();
+    if (P.snap && ln == 0) {
+        P.snap[0] = P.counters[kVtxTotal];
+        P.snap[1] = P.counters[kTriTotal];
+        P.snap[2] = P.counters[kSlotsNow];
+        P.snap[3] = P.counters[kStageNow];
+    }
+    if (!P.back) return;
+    static_assert(kQueueGroups == 64, "one statistics line per lane");
+    const uint64_t* st = reinterpret_cast<const uint64_t*>(P.queues) + ln * 16u + 1u;
+    uint64_t sum[3] = {st[0], st[1], st[2]};
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+        for (int d = 32; d >= 1; d >>= 1) sum[q] += __shfl_xor(sum[q], d, 64);
+    for (uint32_t i = ln; i < P.nback; i += 64u)
+        P.back[i] = i == kTilesActive ? sum[0] : i == kEvalPoints ? sum[1] : i == kEvalFlops ? sum[2] : P.counters[i];
+}
+
 template <int LINEAR>
 __global__ __launch_bounds__(64) void k_sp_emit(SpPass P, MeshBufs b)
 {
     __shared__ StagedTape T;      // programs that are not left folds (left folds: read in place)
     __shared__ uint32_t nb[729];  // vertex of cell (8tx-1+i, 8ty-1+j, 8tz-1+k) at nb[(k*9+j)*9+i]
     __shared__ uint32_t tc[128];  // triangles of cell c in byte c % 4 of tc[c / 4]
-    const uint32_t nslots = active_slots(P);
+    if (LINEAR && blockIdx.x == 0) report(P);
+    const uint32_t nslots = active_slots(P, kSlotsNow);
     for (uint32_t slot = blockIdx.x; slot < nslots; slot += gridDim.x) {
         const SlotHdr& H = P.slot_hdr[slot];
         const uint64_t tile = __builtin_amdgcn_readfirstlane(H.tile);
@@ -1484,8 +1527,9 @@ constexpr uint32_t kScanPer = 16;                  // consecutive rows per threa
 constexpr uint32_t kScanChunk = 256 * kScanPer;
 static_assert(kScanChunk == kRowChunk, "rows per chunk of the offset scan");
 
-__global__ __launch_bounds__(64) void k_sp_rowsum(SpPass P, uint32_t* __restrict__ bsum)
+__global__ __launch_bounds__(64) void k_sp_rowsum(SpPass P)
 {
+    uint32_t* bsum = P.bsum;
     const uint64_t tr = blockIdx.x;
     uint32_t lo = 0, hi = P.njobs - 1;  // last job whose first tile row <= tr
     while (lo < hi) {
@@ -1571,8 +1615,9 @@ __global__ __launch_bounds__(64) void k_sp_rowsum(SpPass P, uint32_t* __restrict
 // Exclusive offsets of the rows, block b = rows b * kScanChunk ...: the pass's first index
 // (kVtxPrev / kTriPrev) plus the chunk sums of the blocks before it (bsum) plus the
 // block-local scan.  The last block writes the totals after the pass (kVtxTotal / kTriTotal).
-__global__ __launch_bounds__(256) void k_sp_rowdown(SpPass P, const uint32_t* __restrict__ bsum)
+__global__ __launch_bounds__(256) void k_sp_rowdown(SpPass P)
 {
+    const uint32_t* bsum = P.bsum;
     __shared__ uint32_t lds[2][4];
     __shared__ uint32_t pre[2][4];
     const uint64_t base = (uint64_t)blockIdx.x * kScanChunk + thread_id() * kScanPer;
@@ -1619,6 +1664,14 @@ __global__ __launch_bounds__(256) void k_sp_rowdown(SpPass P, const uint32_t* __
     if (blockIdx.x + 1 == gridDim.x && thread_id() == 0) {  // after the pass
         P.counters[kVtxTotal] = bv + lds[0][0] + lds[0][1] + lds[0][2] + lds[0][3];
         P.counters[kTriTotal] = bt + lds[1][0] + lds[1][1] + lds[1][2] + lds[1][3];
+        // the pass's slots and staging: kept, folded into their maxima, reset
+        for (uint32_t q = 0; q < 2; ++q) {
+            const uint32_t used = q ? kStageUsed : kSlotsUsed, most = q ? kStageMax : kSlotsMax;
+            const uint64_t n = P.counters[used];
+            P.counters[q ? kStageNow : kSlotsNow] = n;
+            if (n > P.counters[most]) P.counters[most] = n;
+            P.counters[used] = 0;
+        }
     }
     uint32_t rv = bv + iv - sv, rt = bt + it - st;
     for (uint32_t w = 0; w < (thread_id() >> 6); ++w) {
@@ -1653,108 +1706,6 @@ __global__ __launch_bounds__(256) void k_sp_boundary(SpPass P)
     J.boundary[i] = vertex_at(P, J, i % J.rx, i / J.rx, J.z0 + J.nz - 1);
 }
 
-// Per-pass reset of the slot counter; the largest count seen is kept for the host's
-// capacity check (a kernel rather than a memset, so a pass can be graph-captured).
-__global__ void k_sp_pass_begin(uint64_t* counters, uint32_t* queues, uint32_t* bsum, uint32_t nbsum)
-{
-    if (thread_id() == 0 && blockIdx.x == 0) {
-        const uint64_t used = counters[kSlotsUsed];
-        if (used > counters[kSlotsMax]) counters[kSlotsMax] = used;
-        counters[kSlotsUsed] = 0;
-        if (counters[kStageUsed] > counters[kStageMax]) counters[kStageMax] = counters[kStageUsed];
-        counters[kStageUsed] = 0;
-        counters[kVtxPrev] = counters[kVtxTotal];  // the next pass's first vertex and triangle
-        counters[kTriPrev] = counters[kTriTotal];
-    }
-    for (uint32_t i = thread_id(); i < kQueues * kQueueGroups; i += blockDim.x) queues[i * 32u] = 0;
-    for (uint32_t i = thread_id(); i < nbsum; i += blockDim.x) bsum[i * kChunkSumStride] = 0;
-}
-
-// After a pass (or a dense slab): the totals so far and the pass's use of the slot and
-// staging capacities, written to `out` (host memory mapped for the device) so that the
-// host can copy the pass's finished vertices and triangles while later passes run.
-__global__ void k_snapshot(const uint64_t* counters, uint64_t* out)
-{
-    if (thread_id() == 0 && blockIdx.x == 0) {
-        out[0] = counters[kVtxTotal];
-        out[1] = counters[kTriTotal];
-        out[2] = counters[kSlotsUsed];
-        out[3] = counters[kStageUsed];
-    }
-}
-
-__global__ __launch_bounds__(256) void k_sp_job_begin(uint64_t* counters, uint32_t n, uint32_t* queues,
-                                                      uint32_t* bsum, uint32_t nbsum, uint64_t* stats,
-                                                      uint32_t nstats, uint32_t* boundary, uint32_t nbnd)
-{
-    if (blockIdx.x == 0) {
-        for (uint32_t i = thread_id(); i < n; i += blockDim.x) counters[i] = 0;
-        for (uint32_t i = thread_id(); i < 3u * nstats; i += blockDim.x) stats[i] = 0;
-        for (uint32_t i = thread_id(); i < kQueues * kQueueGroups; i += blockDim.x) queues[i * 32u] = 0;
-        for (uint32_t i = thread_id(); i < nbsum; i += blockDim.x) bsum[i * kChunkSumStride] = 0;
-    }
-    // a multi-pass job's boundary plane: no vertex carried yet
-    for (uint32_t i = blockIdx.x * blockDim.x + thread_id(); i < nbnd; i += gridDim.x * blockDim.x)
-        boundary[i] = 0xffffffffu;
-}
-
-// After a job's last pass: the pass folded into the maxima as k_sp_pass_begin does, then
-// counters[0 .. n) copied to `out` (host memory mapped for the device).
-__global__ __launch_bounds__(256) void k_sp_job_end(uint64_t* counters, uint32_t n, uint64_t* out,
-                                                    const uint64_t* stats, uint32_t nstats)
-{
-    __shared__ uint64_t part[4][3];
-    uint64_t sum[3] = {0, 0, 0};  // the tile blocks' tiles, points and flops
-    for (uint32_t i = thread_id(); i < nstats; i += blockDim.x)
-        for (int k = 0; k < 3; ++k) sum[k] += stats[3u * i + k];
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-        for (int d = 32; d >= 1; d >>= 1) sum[k] += __shfl_xor(sum[k], d, 64);
-    if (lane() == 0)
-        for (int k = 0; k < 3; ++k) part[thread_id() >> 6][k] = sum[k];
-    __syncthreads();
-    if (thread_id() == 0) {
-        if (counters[kSlotsUsed] > counters[kSlotsMax]) counters[kSlotsMax] = counters[kSlotsUsed];
-        if (counters[kStageUsed] > counters[kStageMax]) counters[kStageMax] = counters[kStageUsed];
-        counters[kTilesActive] = part[0][0] + part[1][0] + part[2][0] + part[3][0];
-        counters[kEvalPoints] = part[0][1] + part[1][1] + part[2][1] + part[3][1];
-        counters[kEvalFlops] = part[0][2] + part[1][2] + part[2][2] + part[3][2];
-    }
-    __syncthreads();
-    for (uint32_t i = thread_id(); i < n; i += blockDim.x) out[i] = counters[i];
-}
-
-// ---------------------------------------------------------------------------------
-hipError_t launch_sparse_job_end(hipStream_t s, uint64_t* counters, uint32_t n, uint64_t* out,
-                                 const uint64_t* stats, uint32_t nstats)
-{
-    hipLaunchKernelGGL(k_sp_job_end, dim3(1), dim3(256), 0, s, counters, n, out, stats, nstats);
-    return hipGetLastError();
-}
-
-hipError_t launch_snapshot(hipStream_t s, const uint64_t* counters, uint64_t* out)
-{
-    hipLaunchKernelGGL(k_snapshot, dim3(1), dim3(64), 0, s, counters, out);
-    return hipGetLastError();
-}
-
-hipError_t launch_sparse_pass_begin(hipStream_t s, uint64_t* counters, uint32_t* queues, uint32_t* bsum,
-                                    uint32_t nbsum)
-{
-    hipLaunchKernelGGL(k_sp_pass_begin, dim3(1), dim3(256), 0, s, counters, queues, bsum, nbsum);
-    return hipGetLastError();
-}
-
-hipError_t launch_sparse_job_begin(hipStream_t s, uint64_t* counters, uint32_t n, uint32_t* queues,
-                                   uint32_t* bsum, uint32_t nbsum, uint64_t* stats, uint32_t nstats,
-                                   uint32_t* boundary, uint32_t nbnd)
-{
-    const uint32_t blocks = std::max<uint32_t>(1u, std::min<uint32_t>((nbnd + 255u) / 256u, 256u));
-    hipLaunchKernelGGL(k_sp_job_begin, dim3(blocks), dim3(256), 0, s, counters, n, queues, bsum, nbsum, stats,
-                       nstats, boundary, nbnd);
-    return hipGetLastError();
-}
-
 // Blocks of a persistent launch: as many as the device holds at once (at most `cap`),
 // so no block starts only when others end.  The occupancy query is slow (tens of
 // microseconds), so its answer is cached per (kernel, block size, LDS bytes).
@@ -1786,8 +1737,7 @@ static uint32_t resident_blocks(K kernel, int threads, size_t smem, int cus, uin
 }
 
 hipError_t launch_sparse_pass(hipStream_t s, const SpPass& P, const MeshBufs& b, int cus,
-                              uint32_t tile_blocks, bool general_tiles, bool fold_jobs, bool other_jobs,
-                              int boundary_plane, hipEvent_t* marks)
+                              uint32_t tile_blocks, bool general_tiles, int boundary_plane, hipEvent_t* marks)
 {
     if (P.ntiles == 0) return hipSuccess;
     const uint64_t nsb64 = (P.nrows + kScanChunk - 1) / kScanChunk;
@@ -1798,14 +1748,8 @@ hipError_t launch_sparse_pass(hipStream_t s, const SpPass& P, const MeshBufs& b,
         if (marks && marks[i]) (void)hipEventRecord(marks[i], s);
     };
     const size_t prune_smem = PruneStack::bytes(P.prune_depth);
-    const uint32_t chunks = (P.list_stride + 63) / 64;
-    if (P.nsuper * chunks > 0x7fffffffull) return hipErrorInvalidValue;
+    if (P.nsuper > 0x7fffffffull) return hipErrorInvalidValue;
     mark(0);
-    if (fold_jobs) hipLaunchKernelGGL(k_sp_prune_fold, dim3((uint32_t)P.nsuper), dim3(64), 0, s, P);
-    if (other_jobs) {
-        hipLaunchKernelGGL(k_sp_prune_prims, dim3((uint32_t)(P.nsuper * chunks)), dim3(64), 0, s, P, chunks);
-        hipLaunchKernelGGL(k_sp_prune_super, dim3((uint32_t)((P.nsuper + 63) / 64)), dim3(64), prune_smem, s, P);
-    }
     hipLaunchKernelGGL(k_sp_prune, dim3((uint32_t)P.nsuper), dim3(64), prune_smem, s, P);
     hipLaunchKernelGGL(k_sp_bricks, dim3(resident_blocks(k_sp_bricks, 64, 0, cus, big)), dim3(64), 0, s, P);
     mark(1);
@@ -1819,9 +1763,8 @@ hipError_t launch_sparse_pass(hipStream_t s, const SpPass& P, const MeshBufs& b,
     hipLaunchKernelGGL(k_sp_quadcount, dim3(resident_blocks(k_sp_quadcount, 64, 0, cus, big)), dim3(64), 0, s,
                        P, b);
     mark(3);
-    // b.bcount: the chunk sums (2 x nsb, cleared by the pass's begin kernel)
-    if (P.ntrows) hipLaunchKernelGGL(k_sp_rowsum, dim3((uint32_t)P.ntrows), dim3(64), 0, s, P, b.bcount);
-    if (nsb) hipLaunchKernelGGL(k_sp_rowdown, dim3(nsb), dim3(256), 0, s, P, b.bcount);
+    if (P.ntrows) hipLaunchKernelGGL(k_sp_rowsum, dim3((uint32_t)P.ntrows), dim3(64), 0, s, P);
+    if (nsb) hipLaunchKernelGGL(k_sp_rowdown, dim3(nsb), dim3(256), 0, s, P);
     mark(4);
     hipLaunchKernelGGL((k_sp_emit<1>), dim3(resident_blocks(k_sp_emit<1>, 64, 0, cus, big)), dim3(64), 0, s, P, b);
     if (general_tiles)
