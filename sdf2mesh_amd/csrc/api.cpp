@@ -168,7 +168,8 @@ struct s2m_ctx {
     // dense slabs: the signs of slab k + 1 are evaluated on eval_stream while slab k is
     // contoured on `stream`
     hipStream_t eval_stream = nullptr;
-    PinnedBuf host_snap;                 // per pass: k_snapshot's totals and capacity use
+    PinnedBuf host_snap;                 // per pass: its totals and capacity use (kSnapWords)
+    PinnedBuf host_land;                 // land_mesh's staging of arrays too small to page-lock
     // captured graphs of repeated one-pass jobs, most recent first, and the keys of jobs
     // seen once (run_graph)
     static constexpr size_t kGraphs = 8, kSeen = 16;
@@ -506,11 +507,12 @@ struct SpRange {
     uint64_t v0, nv, t0, nt, invalid;
 };
 
-// Host arrays one job's mesh is copied into while the job runs (s2m_mesh).  After each
-// pass of the sparse pipeline (or slab of the dense one) the compute stream records a
-// snapshot of the totals (k_snapshot, into mapped host memory) and an event;
-// readback_pass waits for a pass's event and queues the copy of that pass's vertices and
-// triangles on the copy stream.  The host calls it for pass k right after queueing pass
+// Host arrays one job's mesh is copied into while the job runs (s2m_mesh).  In each pass of
+// the sparse pipeline (or slab of the dense one) the kernel that knows the totals writes
+// them to mapped host memory, and an event follows the pass's last kernel; readback_pass
+// polls for the totals and queues the copy of that pass's vertices and triangles on the
+// copy stream, behind the event.  A small job of one pass lands in arrays of its exact size
+// from a kernel on its own stream (land_mesh).  The host calls it for pass k right after queueing pass
 // k + 1, so the copy of pass k starts as soon as pass k ends and overlaps the computation
 // of pass k + 1 (waiting until every pass is queued would delay the first copy by the
 // launches of all later passes).  Vertices and triangles are appended in pass order and
@@ -525,6 +527,8 @@ struct Readback {
     uint64_t v_done = 0, t_done = 0;  // copies queued so far
     uint32_t passes_done = 0;         // passes whose copies are queued (or that stopped them)
     bool stopped = false;             // a pass overflowed a capacity: the attempt repeats
+    bool landed = false;              // land_mesh queued the whole mesh's copies
+    CopyList staged{};                // parts that pass through the context's staging memory
     hipEvent_t first = nullptr, last = nullptr;  // profiling: around the copies
 
     void release()
@@ -571,11 +575,108 @@ int readback_begin(s2m_ctx* ctx, Readback& rb, uint64_t vcap, uint64_t tcap)
     rb.v_done = rb.t_done = 0;
     rb.passes_done = 0;
     rb.stopped = false;
+    rb.landed = false;
     rb.first = rb.last = nullptr;
     return S2M_OK;
 }
 
-// After pass (or slab) k's kernels (the last of which writes its snapshot): its event.
+// Page-locked memory for the totals of `npass` passes, none of them valid yet.
+int snapshots_begin(s2m_ctx* ctx, uint32_t npass, uint64_t** dev)
+{
+    HIP_TRY(ctx->host_snap.ensure((size_t)npass * kSnapWords * sizeof(uint64_t)));
+    std::memset(ctx->host_snap.p, 0, (size_t)npass * kSnapWords * sizeof(uint64_t));
+    void* d = nullptr;
+    HIP_TRY(hipHostGetDevicePointer(&d, ctx->host_snap.p, 0));
+    *dev = static_cast<uint64_t*>(d);
+    return S2M_OK;
+}
+
+// Pass k's totals, waiting for the device to write them.  The wait ends with the stream:
+// a stream that is idle (or failed) without having written them is an error.
+int snapshot_wait(s2m_ctx* ctx, uint32_t k, uint64_t (&v)[kSnapWords])
+{
+    const volatile uint64_t* s = ctx->host_snap.as<uint64_t>() + (size_t)k * kSnapWords;
+    bool ended = false;
+    for (uint32_t spins = 1;; ++spins) {
+        uint32_t valid = 0;
+        for (uint32_t i = 0; i < kSnapWords; ++i) {
+            const uint64_t w = s[i];
+            if (w & kSnapValid) ++valid;
+            v[i] = w & ~kSnapValid;
+        }
+        if (valid == kSnapWords) return S2M_OK;
+        if (ended) return fail(S2M_E_HIP, "a pass ended without its totals");
+        if (spins % 256u == 0) {
+            const hipError_t e = hipStreamQuery(ctx->stream);
+            if (e == hipSuccess) ended = true;  // look once more
+            else if (e != hipErrorNotReady) HIP_TRY(e);
+        }
+#if defined(__x86_64__)
+        __builtin_ia32_pause();
+#endif
+    }
+}
+
+// A one-pass job of nv vertices and nt triangles whose last kernels are still running, up to
+// kLandKernel bytes in all: host arrays of that size, and a kernel queued behind the others
+// that writes them, those too small to be page-locked through staging memory, from which
+// land_finish copies them once the stream has ended.  Larger meshes are copied by DMA after
+// the stream has ended (a DMA copy queued behind a kernel starts no sooner).
+constexpr size_t kLandKernel = 2u << 20;
+constexpr size_t kLandStage = 256u << 10;  // >= any array that host_alloc does not page-lock
+
+int land_mesh(s2m_ctx* ctx, Readback& rb, uint64_t nv, uint64_t nt)
+{
+    const size_t bytes[4] = {nv * 6 * sizeof(float), nt * 3 * sizeof(uint32_t), rb.want_keys ? nv * sizeof(uint64_t) : 0,
+                             rb.want_keys ? (size_t)nv : 0};
+    if (bytes[0] + bytes[1] + bytes[2] + bytes[3] > kLandKernel) return S2M_OK;
+    rb.release();
+    rb.vcap = nv;
+    rb.tcap = nt;
+    rb.vtx = static_cast<float*>(host_alloc(std::max<uint64_t>(nv, 1) * 6 * sizeof(float)));
+    rb.tri = static_cast<uint32_t*>(host_alloc(std::max<uint64_t>(nt, 1) * 3 * sizeof(uint32_t)));
+    if (rb.want_keys) {
+        rb.keys = static_cast<uint64_t*>(host_alloc(std::max<uint64_t>(nv, 1) * sizeof(uint64_t)));
+        rb.signs = static_cast<uint8_t*>(host_alloc(std::max<uint64_t>(nv, 1)));
+    }
+    if (!rb.vtx || !rb.tri || (rb.want_keys && (!rb.keys || !rb.signs)))
+        return fail(S2M_E_OOM, "host allocation of %llu vertices / %llu triangles failed", (unsigned long long)nv,
+                    (unsigned long long)nt);
+    const void* src[4] = {ctx->vtx.p, ctx->tri.p, ctx->keys.p, ctx->signs.p};
+    void* dst[4] = {rb.vtx, rb.tri, rb.keys, rb.signs};
+    CopyList list{};
+    rb.staged = CopyList{};
+    for (int k = 0; k < 4; ++k) {
+        if (!bytes[k]) continue;
+        void* to = dst[k];
+        if (!host_is_pinned(to)) {
+            if (bytes[k] > kLandStage) return S2M_OK;  // page-locking failed: by DMA
+            HIP_TRY(ctx->host_land.ensure(4 * kLandStage));
+            to = ctx->host_land.as<uint8_t>() + k * kLandStage;
+            rb.staged.src[k] = to;
+            rb.staged.dst[k] = dst[k];
+            rb.staged.bytes[k] = bytes[k];
+        }
+        HIP_TRY(hipHostGetDevicePointer(&list.dst[k], to, 0));
+        list.src[k] = src[k];
+        list.bytes[k] = bytes[k];
+    }
+    HIP_TRY(launch_copy_out(ctx->stream, list));
+    rb.v_done = nv;
+    rb.t_done = nt;
+    rb.landed = true;
+    return S2M_OK;
+}
+
+// After the stream has ended: the staged parts.
+void land_finish(Readback& rb)
+{
+    for (int k = 0; k < 4; ++k)
+        if (rb.staged.bytes[k]) std::memcpy(rb.staged.dst[k], rb.staged.src[k], rb.staged.bytes[k]);
+    rb.staged = CopyList{};
+}
+
+// After pass (or slab) k's kernels: its event.
 int readback_mark(s2m_ctx* ctx, uint32_t k)
 {
     hipEvent_t e = ctx->pass_event(k);
@@ -612,16 +713,17 @@ int readback_copy(s2m_ctx* ctx, Readback& rb, uint64_t nv, uint64_t nt)
     return S2M_OK;
 }
 
-// Pass rb.passes_done is queued and followed by readback_mark: once it finishes, queue
-// the copies of its vertices and triangles.  A pass whose totals or capacity use exceed
+// Pass rb.passes_done is queued and followed by readback_mark: once its totals are known,
+// queue the copies of its vertices and triangles behind its event.  A pass whose totals or capacity use exceed
 // the attempt's capacities stops the copies (the attempt will repeat).
 int readback_pass(s2m_ctx* ctx, Readback& rb, uint64_t vcap, uint64_t tcap, uint64_t slot_cap, uint64_t stage_cap)
 {
     const uint32_t k = rb.passes_done++;
     if (rb.stopped) return S2M_OK;
-    const volatile uint64_t* snap = ctx->host_snap.as<uint64_t>();
-    HIP_TRY(hipEventSynchronize(ctx->pass_done[k]));
-    const uint64_t nv = snap[4 * k], nt = snap[4 * k + 1], slots = snap[4 * k + 2], staged = snap[4 * k + 3];
+    uint64_t snap[kSnapWords];
+    const int wrc = snapshot_wait(ctx, k, snap);
+    if (wrc) return wrc;
+    const uint64_t nv = snap[0], nt = snap[1], slots = snap[2], staged = snap[3];
     if (nv > vcap || nt > tcap || nv > rb.vcap || nt > rb.tcap || slots > slot_cap || staged > stage_cap ||
         nv < rb.v_done || nt < rb.t_done) {
         rb.stopped = true;
@@ -646,6 +748,10 @@ int readback_passes(s2m_ctx* ctx, Readback& rb, uint32_t npass, uint64_t vcap, u
 // pass stopped the streaming) and every copy finished.
 int readback_finish(s2m_ctx* ctx, Readback& rb, uint64_t nv, uint64_t nt)
 {
+    if (rb.landed) {  // (the stream has been synchronised)
+        land_finish(rb);
+        return S2M_OK;
+    }
     if (!rb.vtx || nv > rb.vcap || nt > rb.tcap) {  // not streamed, or larger than its arrays
         HIP_TRY(hipStreamSynchronize(ctx->copy_stream));
         rb.release();
@@ -919,7 +1025,8 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
         while (layers > 1 && pass_bytes(layers) > (1ull << 30)) layers = (layers + 1) / 2;
     }
     const uint32_t npass = n == 1 ? (tabs[0].nt[2] + layers - 1) / std::max(layers, 1u) : 1;
-    if (npass == 1) rb = nullptr;  // nothing to overlap: the caller copies the finished mesh
+    Readback* const land = npass == 1 && !ctx->profiling ? rb : nullptr;  // copied at its end (land_mesh)
+    if (npass == 1) rb = nullptr;  // no passes to overlap
     const uint64_t tiles_pass = n == 1 ? (uint64_t)tabs[0].nt[0] * tabs[0].nt[1] * layers : ntiles_all;
     const uint64_t rows_pass = n == 1 ? (uint64_t)layers * kTile * jobs[0].res[1] : nrows_all;
     if (tiles_pass > 0x7fffffffull || rows_pass > 0xffffffffull || plane_max > 0xffffffffull ||
@@ -1051,13 +1158,13 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
     uint64_t want_s = std::min<uint64_t>(tiles_pass, std::max<uint64_t>({4096, tiles_pass / 4, ctx->slot_cap}));
     const uint64_t tile_blocks = (uint64_t)std::max(1, ctx->cus) * kTileBlocksPerCU;
     uint64_t stage_cap = ctx->stage_cap;
-    void* snap_dev = nullptr;
-    if (rb) {
-        HIP_TRY(ctx->host_snap.ensure((size_t)npass * 4 * sizeof(uint64_t)));
-        HIP_TRY(hipHostGetDevicePointer(&snap_dev, ctx->host_snap.p, 0));
-    }
 
     for (int attempt = 0; attempt < 4; ++attempt) {
+        uint64_t* snap_dev = nullptr;
+        if (rb || land) {
+            const int src = snapshots_begin(ctx, npass, &snap_dev);
+            if (src) return src;
+        }
         HIP_TRY(ctx->vtx.ensure(want_v * 6 * sizeof(float)));
         HIP_TRY(ctx->keys.ensure(want_v * sizeof(uint64_t)));
         HIP_TRY(ctx->signs.ensure(want_v));
@@ -1169,7 +1276,7 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
             P.nbnd = pass == 0 && n == 1 && npass > 1 ? (uint32_t)plane_max : 0u;
             P.nback = nback;
             P.back = pass + 1 == npass ? static_cast<uint64_t*>(back_dev) : nullptr;
-            P.snap = rb ? static_cast<uint64_t*>(snap_dev) + 4 * (size_t)pass : nullptr;
+            P.snap = snap_dev ? snap_dev + kSnapWords * (size_t)pass : nullptr;
             const int boundary = (n == 1 && pass + 1 < npass) ? 1 : 0;
             HIP_TRY(launch_sparse_pass(ctx->stream, P, b, ctx->cus, (uint32_t)tile_blocks, general_tiles, boundary,
                                        ctx->profiling ? m : nullptr));
@@ -1205,7 +1312,7 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
                                     &ctx->sp_super_act, &ctx->sp_boundary})
                 put(&d->p, sizeof d->p);
             const uint64_t scal[] = {want_v, want_t, want_s, stage_cap, tile_blocks, nsb_max, list_stride,
-                                     prune_depth, box_stride, (uint64_t)general_tiles, n, (uint64_t)(uintptr_t)back_dev};
+                                     prune_depth, box_stride, (uint64_t)general_tiles, n, (uint64_t)(uintptr_t)back_dev, (uint64_t)(uintptr_t)snap_dev};
             put(scal, sizeof scal);
             const int grc = run_graph(ctx, key, enqueue);
             if (grc) return grc;
@@ -1234,6 +1341,14 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
         if (rb) {  // copies of each pass's mesh while the later passes run
             const int rrc = readback_passes(ctx, *rb, npass, want_v, want_t, want_s, stage_cap);
             if (rrc) return rrc;
+        }
+        if (land) {  // a small mesh's copy behind its last kernel
+            uint64_t t[kSnapWords];
+            int lrc = snapshot_wait(ctx, 0, t);
+            land->landed = false;
+            if (!lrc && t[0] <= want_v && t[1] <= want_t && t[2] <= want_s && t[3] <= stage_cap)
+                lrc = land_mesh(ctx, *land, t[0], t[1]);
+            if (lrc) return lrc;
         }
         HIP_TRY(hipStreamSynchronize(ctx->stream));
         if (ctx->profiling) {
@@ -1426,12 +1541,8 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
     }
     const bool normals = prog && !(p->flags & S2M_NO_NORMALS);
     const uint32_t nslabs = (j.nz_cells + T - 1) / T;
-    if (nslabs == 1) rb = nullptr;  // nothing to overlap: the caller copies the finished mesh
-    void* snap_dev = nullptr;
-    if (rb) {
-        HIP_TRY(ctx->host_snap.ensure((size_t)nslabs * 4 * sizeof(uint64_t)));
-        HIP_TRY(hipHostGetDevicePointer(&snap_dev, ctx->host_snap.p, 0));
-    }
+    Readback* const land = nslabs == 1 && !ctx->profiling ? rb : nullptr;  // copied at its end (land_mesh)
+    if (nslabs == 1) rb = nullptr;  // no slabs to overlap
     hipStream_t es = piped ? ctx->eval_stream : ctx->stream;
     void* back_dev = nullptr;  // mapped host memory for the counters
     if (!fx) {
@@ -1501,6 +1612,11 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
         if (rb) {  // host arrays for this job's own estimate, not the context's largest job
             const int rrc = readback_begin(ctx, *rb, std::min(want_v, est_v), std::min(want_t, 3 * est_v));
             if (rrc) return rrc;
+        }
+        uint64_t* snap_dev = nullptr;
+        if (rb || land) {
+            const int src = snapshots_begin(ctx, nslabs, &snap_dev);
+            if (src) return src;
         }
 
         HIP_TRY(launch_dense_begin(ctx->stream, b.counters, act_buf[0],
@@ -1629,11 +1745,10 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
             if (h_corners) HIP_TRY(launch_cells_from_corners(ctx->stream, a, src, bs, 1));
             else HIP_TRY(emit_prog(ctx->stream, prog, A));
             if (m[3]) HIP_TRY(hipEventRecord(m[3], ctx->stream));
-            HIP_TRY(launch_quads(ctx->stream, a, bs, prev));
-            // the other activity words cleared for the next slab; the totals for the host
+            HIP_TRY(launch_quads(ctx->stream, a, bs, prev, snap_dev ? snap_dev + kSnapWords * slabs : nullptr));
+            // the other activity words cleared for the next slab
             HIP_TRY(launch_slab_end(ctx->stream, b.counters, act_buf[cur ^ 1],
                                     (uint32_t)(plane * std::min(T, j.nz_cells - z1)), base_buf[cur ^ 1],
-                                    rb ? static_cast<uint64_t*>(snap_dev) + 4 * slabs : nullptr,
                                     z1 == j.nz_cells ? static_cast<uint64_t*>(back_dev) : nullptr));
             if (m[4]) HIP_TRY(hipEventRecord(m[4], ctx->stream));
             if (rb) {  // the slab's vertices and triangles are final; the copies of the slab two
@@ -1652,6 +1767,13 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
         if (rb) {  // copies of each slab's mesh while the later slabs run
             const int rrc = readback_passes(ctx, *rb, (uint32_t)slabs, want_v, want_t, ~0ull, ~0ull);
             if (rrc) return rrc;
+        }
+        if (land) {  // a small mesh's copy behind its last kernel
+            uint64_t t[kSnapWords];
+            int lrc = snapshot_wait(ctx, 0, t);
+            land->landed = false;
+            if (!lrc && t[0] <= want_v && t[1] <= want_t) lrc = land_mesh(ctx, *land, t[0], t[1]);
+            if (lrc) return lrc;
         }
         uint64_t cnt[kNumCounters];
         if (fx) HIP_TRY(hipMemcpyAsync(cnt, b.counters, sizeof cnt, hipMemcpyDeviceToHost, ctx->stream));
@@ -1848,6 +1970,7 @@ void s2m_destroy(s2m_ctx* ctx)
     ctx->host_img.release();
     ctx->host_back.release();
     ctx->host_snap.release();
+    ctx->host_land.release();
     for (hipEvent_t e : ctx->events) (void)hipEventDestroy(e);
     for (hipEvent_t e : ctx->pass_done) (void)hipEventDestroy(e);
     for (auto& g : ctx->graphs) (void)hipGraphExecDestroy(g.second);
@@ -1996,8 +2119,11 @@ int s2m_mesh(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* params, in
     rb.want_keys = want_keys;
     int rc = mesh_one(ctx, prog, params, &rb);
     if (rc == S2M_OK) rc = readback_finish(ctx, rb, ctx->last_nvtx, ctx->last_ntri);
-    if (rc) {
-        (void)hipStreamSynchronize(ctx->copy_stream);
+    if (rc) {  // no copy may still be writing the arrays
+        if (ctx) {
+            (void)hipStreamSynchronize(ctx->stream);
+            (void)hipStreamSynchronize(ctx->copy_stream);
+        }
         rb.release();
         return rc;
     }

@@ -99,6 +99,14 @@ void* host_alloc_shared(size_t bytes, uint32_t refs)
 
 void* host_alloc(size_t bytes) { return host_alloc_shared(bytes, 1); }
 
+bool host_is_pinned(const void* p)
+{
+    Pool& P = pool();
+    std::lock_guard<std::mutex> g(P.mu);
+    auto it = P.live.find(reinterpret_cast<uintptr_t>(p));
+    return it != P.live.end() && it->second.pinned;
+}
+
 void host_release(void* p)
 {
     if (!p) return;

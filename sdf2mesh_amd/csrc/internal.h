@@ -27,6 +27,19 @@ struct FastDiv {
 };
 FastDiv make_fastdiv(uint32_t d);
 
+// A pass's (slab's) totals for the host, written before its mesh is complete: vertices and
+// triangles so far, slots and staged cells in use, each with kSnapValid set (the host polls
+// for it, so the words need no order among them).
+constexpr uint32_t kSnapWords = 4;
+constexpr uint64_t kSnapValid = 1ull << 63;
+
+// Arrays copied by one kernel (k_copy_out); addresses are 16-byte aligned.
+struct CopyList {
+    const void* src[4];
+    void* dst[4];
+    uint64_t bytes[4];
+};
+
 // Device counters of one job (u64 each).
 enum Counter : uint32_t {
     kVtxTotal = 0,   // vertices emitted so far (all slabs)
@@ -180,7 +193,7 @@ struct SpPass {
     uint32_t nback;            // words of `back`
     uint64_t* back;            // mapped host memory for the counters and job rows after a job's last
                                // pass, else NULL
-    uint64_t* snap;            // mapped host memory for the pass's totals, or NULL
+    uint64_t* snap;            // mapped host memory for the pass's totals (kSnapWords), or NULL
     uint64_t* job_out;         // [job][kJobOut]
 };
 
@@ -217,8 +230,9 @@ hipError_t launch_ranks(hipStream_t s, const MeshBufs& b, uint32_t ncells);
 hipError_t launch_dense_begin(hipStream_t s, uint64_t* counters, uint64_t* words, uint32_t ncells,
                               const void* host_tables, void* tables, size_t bytes, uint32_t* cbase);
 hipError_t launch_slab_end(hipStream_t s, uint64_t* counters, uint64_t* words, uint32_t ncells, uint32_t* cbase,
-                           uint64_t* snap, uint64_t* back);
-hipError_t launch_quads(hipStream_t s, const SlabArgs& a, const MeshBufs& b, const SlabBits& prev);
+                           uint64_t* back);
+hipError_t launch_copy_out(hipStream_t s, const CopyList& c);
+hipError_t launch_quads(hipStream_t s, const SlabArgs& a, const MeshBufs& b, const SlabBits& prev, uint64_t* snap);
 // cnt[0..4) (zeroed by the caller): k_sincos_check's mismatch counts.
 hipError_t launch_sincos_check(hipStream_t s, uint64_t* cnt);
 // cnt[0..2) (zeroed by the caller): k_bailout_check's comparisons and disagreements.
@@ -248,6 +262,8 @@ hipError_t noalloc_scratch(int device, void** ptr);
 // Host memory for a result array: page-locked and recycled when large, malloc otherwise.
 // Returned to the pool (or freed) by host_release; any other pointer is passed to free().
 void* host_alloc(size_t bytes);
+// Whether the device can write the block host_alloc returned (page-locked).
+bool host_is_pinned(const void* p);
 // A page-locked block shared by `refs` results: each points somewhere inside it and is
 // released with host_release; the block returns to the pool after the last release.
 void* host_alloc_shared(size_t bytes, uint32_t refs);

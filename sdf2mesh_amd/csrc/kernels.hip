@@ -413,10 +413,20 @@ __device__ __forceinline__ uint32_t vertex_groups(const uint64_t* counters, uint
     return end > beg ? (uint32_t)((end - beg + kBlock - 1u) / kBlock) : 0u;
 }
 
+// A slab's or pass's totals to mapped host memory (kSnapWords): past the device's caches, so
+// that a polling host sees them while the kernels after this one run.
+__device__ __forceinline__ void write_snapshot(uint64_t* snap, uint64_t nv, uint64_t nt, uint64_t slots, uint64_t staged)
+{
+    const uint64_t v[kSnapWords] = {nv, nt, slots, staged};
+    for (uint32_t i = 0; i < kSnapWords; ++i)
+        __hip_atomic_store(snap + i, v[i] | kSnapValid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // The groups' triangle counts (k_quads<0>) into their offsets, and the running total, by one
 // workgroup: a slab's 600 K vertices are 2 400 groups, one round.
 __global__ __launch_bounds__(1024) void k_tri_offsets(const uint32_t* __restrict__ tcount, uint32_t* __restrict__ toffset,
-                                                      uint64_t* __restrict__ counters, uint64_t vcap)
+                                                      uint64_t* __restrict__ counters, uint64_t vcap,
+                                                      uint64_t* snap)
 {
     __shared__ uint32_t wsum[16];
     const uint32_t groups = vertex_groups(counters, vcap), t = threadIdx.x;
@@ -457,6 +467,7 @@ __global__ __launch_bounds__(1024) void k_tri_offsets(const uint32_t* __restrict
     if (t == 0) {
         counters[kTriPrev] = prev;
         counters[kTriTotal] = run;
+        if (snap) write_snapshot(snap, counters[kVtxTotal], run, 0, 0);
     }
 }
 
@@ -762,12 +773,10 @@ __global__ __launch_bounds__(256) void k_dense_begin(uint64_t* __restrict__ coun
 
 // After a slab's quad pass: the staging use folded into its maximum, the allocation
 // counter reset, and the other activity words and chunk bases (the previous slab's, read
-// for the last time by this slab's quads) set up for the next slab.  snap: the totals so far, for the
-// host to copy the slab's finished mesh (as k_snapshot); back: after the last slab, all
-// counters (both in mapped host memory, NULL: not wanted).
+// for the last time by this slab's quads) set up for the next slab.  back: after the last
+// slab, all counters (mapped host memory, NULL: not wanted).
 __global__ __launch_bounds__(256) void k_slab_end(uint64_t* __restrict__ counters, uint64_t* __restrict__ words,
-                                                  uint32_t nwords, uint32_t* __restrict__ cbase, uint64_t* snap,
-                                                  uint64_t* back)
+                                                  uint32_t nwords, uint32_t* __restrict__ cbase, uint64_t* back)
 {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t < kRankChunks) cbase[t] = (uint32_t)counters[kVtxTotal];
@@ -776,11 +785,6 @@ __global__ __launch_bounds__(256) void k_slab_end(uint64_t* __restrict__ counter
         const uint64_t used = counters[kBrickAlloc] >> 32;
         if (used > counters[kStageMax]) counters[kStageMax] = used;
         counters[kBrickAlloc] = 0;
-        if (snap) {
-            snap[0] = counters[kVtxTotal];
-            snap[1] = counters[kTriTotal];
-            snap[2] = snap[3] = 0;
-        }
         if (back)
             for (uint32_t i = 0; i < kNumCounters; ++i) back[i] = counters[i];
     }
@@ -798,21 +802,49 @@ hipError_t launch_dense_begin(hipStream_t s, uint64_t* counters, uint64_t* words
 }
 
 hipError_t launch_slab_end(hipStream_t s, uint64_t* counters, uint64_t* words, uint32_t ncells, uint32_t* cbase,
-                           uint64_t* snap, uint64_t* back)
+                           uint64_t* back)
 {
     const uint32_t n = (ncells + 63u) / 64u;
     hipLaunchKernelGGL(k_slab_end, dim3(std::max(1u, std::min((n + 255u) / 256u, 2048u))), dim3(256), 0, s, counters,
-                       words, n, cbase, snap, back);
+                       words, n, cbase, back);
     return hipGetLastError();
 }
 
-hipError_t launch_quads(hipStream_t s, const SlabArgs& a, const MeshBufs& b, const SlabBits& prev)
+// Up to four arrays to page-locked host memory (16-byte words, then the last bytes): for
+// small meshes one launch right after the job's last kernel in place of a DMA copy per
+// array (each about 10 us beside its transfer).  Large ones go by DMA: a copying kernel
+// reaches the same 55 GB/s but its queued stores hold up every other kernel's.
+__global__ __launch_bounds__(256) void k_copy_out(CopyList c)
+{
+    const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (uint64_t)gridDim.x * blockDim.x;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const uint64_t n16 = c.bytes[k] >> 4, rest = c.bytes[k] & 15u;
+        const uint4* s = static_cast<const uint4*>(c.src[k]);
+        uint4* d = static_cast<uint4*>(c.dst[k]);
+        for (uint64_t i = t; i < n16; i += step) d[i] = s[i];
+        if (t < rest) reinterpret_cast<uint8_t*>(d + n16)[t] = reinterpret_cast<const uint8_t*>(s + n16)[t];
+    }
+}
+
+hipError_t launch_copy_out(hipStream_t s, const CopyList& c)
+{
+    uint64_t most = 0;
+    for (uint64_t b : c.bytes) most = std::max(most, b);
+    if (most == 0) return hipSuccess;
+    const uint32_t blocks = (uint32_t)std::min<uint64_t>((most / 16u + 255u) / 256u + 1u, 128u);
+    hipLaunchKernelGGL(k_copy_out, dim3(blocks), dim3(256), 0, s, c);
+    return hipGetLastError();
+}
+
+hipError_t launch_quads(hipStream_t s, const SlabArgs& a, const MeshBufs& b, const SlabBits& prev,
+                        uint64_t* snap)
 {
     if (a.ncells == 0) return hipSuccess;
     const uint32_t groups = (a.ncells + kBlock - 1u) / kBlock;  // if every cell had a vertex
     const dim3 grid(std::min(groups, 2048u));
     hipLaunchKernelGGL((k_quads<0>), grid, dim3(kBlock), 0, s, a, b, prev);
-    hipLaunchKernelGGL(k_tri_offsets, dim3(1), dim3(1024), 0, s, b.tcount, b.toffset, b.counters, b.vcap);
+    hipLaunchKernelGGL(k_tri_offsets, dim3(1), dim3(1024), 0, s, b.tcount, b.toffset, b.counters, b.vcap, snap);
     hipLaunchKernelGGL((k_quads<1>), grid, dim3(kBlock), 0, s, a, b, prev);
     return hipGetLastError();
 }

@@ -31,7 +31,7 @@
 //                   4-tap normals (the tile's pruned program), then the triangles of
 //                   their quads, vertex indices relative to the job's first vertex
 //   k_sp_boundary   (multi-slab single job) cell -> vertex map of the slab's last plane
-// The totals go to mapped host memory from the last kernel, k_sp_emit<1>: a pass of folds is
+// The totals go to mapped host memory from k_sp_rowdown and k_sp_emit<1>: a pass of folds is
 // seven launches (of about 4.5 us each at any small size).
 // The per-slot kernels are persistent (as many blocks as the device holds) and draw slots
 // from a work queue.  A cell's vertex index is never stored: it is the first index of its row segment plus
@@ -1341,20 +1341,12 @@ __global__ __launch_bounds__(64) void k_sp_quadcount(SpPass P, MeshBufs b)
 // slots whose program is a left fold, LINEAR = 0 the others (launched only when a program
 // of the pass is not a left fold; its stack interpreter needs more registers).
 // ---------------------------------------------------------------------------------
-// Block 0 of k_sp_emit<1>: the totals so far and the pass's use of the slot and staging
-// capacities to P.snap, so that the host can copy the pass's finished vertices and
-// triangles while later passes run; after a job's last pass the statistics summed and
-// counters[0 .. nback) to P.back (both in mapped host memory, NULL: not wanted).  Nothing
-// in the kernel changes them.
+// Block 0 of k_sp_emit<1> after a job's last pass: the statistics summed and
+// counters[0 .. nback) to P.back (mapped host memory, NULL: not wanted).  Nothing in the
+// kernel changes them.
 __device__ __forceinline__ void report(const SpPass& P)
 {
     const uint32_t ln = lane();
-    if (P.snap && ln == 0) {
-        P.snap[0] = P.counters[kVtxTotal];
-        P.snap[1] = P.counters[kTriTotal];
-        P.snap[2] = P.counters[kSlotsNow];
-        P.snap[3] = P.counters[kStageNow];
-    }
     if (!P.back) return;
     static_assert(kQueueGroups == 64, "one statistics line per lane");
     const uint64_t* st = reinterpret_cast<const uint64_t*>(P.queues) + ln * 16u + 1u;
@@ -1671,6 +1663,14 @@ __global__ __launch_bounds__(256) void k_sp_rowdown(SpPass P)
             P.counters[q ? kStageNow : kSlotsNow] = n;
             if (n > P.counters[most]) P.counters[most] = n;
             P.counters[used] = 0;
+        }
+        // for the host, which allocates and queues the copies of the pass's mesh while
+        // k_sp_emit writes it
+        if (P.snap) {
+            const uint64_t v[kSnapWords] = {P.counters[kVtxTotal], P.counters[kTriTotal], P.counters[kSlotsNow],
+                                            P.counters[kStageNow]};
+            for (uint32_t q = 0; q < kSnapWords; ++q)
+                __hip_atomic_store(P.snap + q, v[q] | kSnapValid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
     }
     uint32_t rv = bv + iv - sv, rt = bt + it - st;
