@@ -146,7 +146,7 @@ struct s2m_ctx {
     PassSet pset[2];
     DevBuf vtx, keys, signs, tri, corners;
     DevBuf tile_tab, tile_lists, tile_lens, tile_flops;
-    DevBuf sp_slot_of_tile, sp_tile_of_slot, sp_job_of_slot, sp_cellbits, sp_slot_rows, sp_boundary;
+    DevBuf sp_slot_of_tile, sp_tile_of_slot, sp_job_of_slot, sp_gen_slots, sp_cellbits, sp_slot_rows, sp_boundary;
     DevBuf sp_stage, sp_slot_nb, sp_slot_stage, sp_slot_live, sp_slot_hdr, sp_slot_rec;
     DevBuf sp_queues, sp_super_iv, sp_super_lists, sp_super_act, sp_rows;
     bool sp_dirty = false;  // a sparse pass was not queued to its end: `counters` may not be zero
@@ -975,7 +975,7 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
     std::vector<SpTables> tabs(n);
     std::vector<size_t> tab_off(n);
     size_t tab_bytes = 0;
-    uint32_t list_stride = 1, box_stride = 1, prune_depth = 1;
+    uint32_t list_stride = 1, box_stride = 1, prune_depth = 1, walk_ops = 0;
     bool general_tiles = false;  // a tile's pruned program may not be a left fold
     uint64_t ntiles_all = 0, nrows_all = 0, plane_max = 0, cells_all = 0, planes_sum = 0;
     for (uint32_t i = 0; i < n; ++i) {
@@ -983,7 +983,10 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
         tab_off[i] = tab_bytes;
         tab_bytes += (tabs[i].bytes.size() + 255) & ~size_t(255);
         list_stride = std::max(list_stride, progs[i]->n);
-        if (!left_fold_program(progs[i]->ops)) general_tiles = true;
+        if (!left_fold_program(progs[i]->ops)) {
+            general_tiles = true;
+            if (progs[i]->n <= kStageOps) walk_ops = std::max(walk_ops, progs[i]->n);
+        }
         box_stride = std::max(box_stride, tabs[i].bmax[0] * tabs[i].bmax[1] * tabs[i].bmax[2]);
         uint32_t depth = 0;  // operand stack entries below the top (k_sp_prune's LDS stack)
         for (const s2m_op& o : progs[i]->ops) {
@@ -1171,6 +1174,7 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
         HIP_TRY(ctx->tri.ensure(want_t * 3 * sizeof(uint32_t)));
         HIP_TRY(ctx->sp_tile_of_slot.ensure(want_s * sizeof(uint32_t)));
         HIP_TRY(ctx->sp_job_of_slot.ensure(want_s * sizeof(uint32_t)));
+        HIP_TRY(ctx->sp_gen_slots.ensure(want_s * sizeof(uint32_t)));
         HIP_TRY(ctx->sp_cellbits.ensure(want_s * 16 * sizeof(uint32_t)));
         HIP_TRY(ctx->sp_slot_rows.ensure(want_s * 4 * 64 * sizeof(uint32_t)));
         // staged cells are reserved 8 per live brick of a slot, in per-block chunks: about
@@ -1223,6 +1227,7 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
             P.njobs = n == 1 ? 1 : n;
             P.list_stride = list_stride;
             P.prune_depth = prune_depth;
+            P.walk_ops = walk_ops;
             if (n == 1) {
                 const SpJob& J = desc[pass];
                 P.ntiles = (uint64_t)J.ntx * J.nty * ((J.nz + kTile - 1) / kTile);
@@ -1246,6 +1251,7 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
             P.slot_of_tile = ctx->sp_slot_of_tile.as<int32_t>();
             P.tile_of_slot = ctx->sp_tile_of_slot.as<uint32_t>();
             P.job_of_slot = ctx->sp_job_of_slot.as<uint32_t>();
+            P.gen_slots = ctx->sp_gen_slots.as<uint32_t>();
             P.slot_cap = (uint32_t)want_s;
             P.box_stride = box_stride;
             P.cellbits = ctx->sp_cellbits.as<uint32_t>();
@@ -1306,13 +1312,13 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
             for (const DevBuf* d : {&ctx->vtx, &ctx->keys, &ctx->signs, &ctx->tri, &ctx->counters, &ctx->bcount,
                                     &ctx->sp_queues, &ctx->tile_tab, &ctx->tile_lists,
                                     &ctx->tile_lens, &ctx->tile_flops, &ctx->sp_slot_of_tile, &ctx->sp_tile_of_slot,
-                                    &ctx->sp_job_of_slot, &ctx->sp_cellbits, &ctx->sp_stage, &ctx->sp_slot_stage,
+                                    &ctx->sp_job_of_slot, &ctx->sp_gen_slots, &ctx->sp_cellbits, &ctx->sp_stage, &ctx->sp_slot_stage,
                                     &ctx->sp_slot_live, &ctx->sp_slot_hdr, &ctx->sp_slot_nb, &ctx->sp_slot_rec,
                                     &ctx->sp_slot_rows, &ctx->sp_rows, &ctx->sp_super_iv, &ctx->sp_super_lists,
                                     &ctx->sp_super_act, &ctx->sp_boundary})
                 put(&d->p, sizeof d->p);
             const uint64_t scal[] = {want_v, want_t, want_s, stage_cap, tile_blocks, nsb_max, list_stride,
-                                     prune_depth, box_stride, (uint64_t)general_tiles, n, (uint64_t)(uintptr_t)back_dev, (uint64_t)(uintptr_t)snap_dev};
+                                     prune_depth, walk_ops, box_stride, (uint64_t)general_tiles, n, (uint64_t)(uintptr_t)back_dev, (uint64_t)(uintptr_t)snap_dev};
             put(scal, sizeof scal);
             const int grc = run_graph(ctx, key, enqueue);
             if (grc) return grc;
@@ -1954,7 +1960,7 @@ void s2m_destroy(s2m_ctx* ctx)
                       &ctx->tables, &ctx->vtx, &ctx->keys, &ctx->signs, &ctx->tri, &ctx->corners,
                       &ctx->tile_tab, &ctx->tile_lists, &ctx->tile_lens,
                       &ctx->tile_flops, &ctx->sp_slot_of_tile, &ctx->sp_tile_of_slot,
-                      &ctx->sp_job_of_slot, &ctx->sp_cellbits, &ctx->sp_slot_rows,
+                      &ctx->sp_job_of_slot, &ctx->sp_gen_slots, &ctx->sp_cellbits, &ctx->sp_slot_rows,
                       &ctx->sp_boundary, &ctx->sp_queues, &ctx->sp_super_iv,
                       &ctx->sp_super_lists, &ctx->sp_super_act, &ctx->sp_rows,
                       &ctx->sp_stage, &ctx->sp_slot_nb, &ctx->sp_slot_stage, &ctx->sp_slot_live, &ctx->sp_slot_hdr, &ctx->sp_slot_rec})

@@ -3,16 +3,19 @@
 // Every lane of a block evaluates the same pruned program (one tile per block), so the
 // opcode is read once per op for the whole wave (readfirstlane) and the dispatch is a
 // scalar branch; operands are LDS broadcasts.  Programs whose postfix form is a left fold
-// of library primitives (P0 P1 op1 P2 op2 ...: CSG built by accumulation, and every
-// pruned sub-program of one) run without an operand stack, several points per lane
-// sharing each op's decode; other programs run on a uniform-depth stack.  Values are
-// bit-identical to tape_eval (device_sdf.h): the same functions in the same order.
+// of library primitives (P0 P1 op1 P2 op2 ...: CSG built by accumulation, every pruned
+// sub-program of one, and any tree whose operators each have a primitive operand, its
+// operators marked where that is the first one) run without an operand stack, several
+// points per lane sharing each op's decode; other programs run on a uniform-depth stack.
+// Values are bit-identical to tape_eval (device_sdf.h): the same functions of the same
+// operands.
 #pragma once
 #include "device_sdf.h"
 #include "internal.h"
 
 namespace s2m {
 
+constexpr uint32_t kSwapCode = 0x80u;           // staged op code: the operands are swapped (kSwapped)
 constexpr uint32_t kLinearFlag = 0x80000000u;  // SpPass::lens: the program is a left fold
 
 template <uint32_t CAP>
@@ -75,8 +78,8 @@ __device__ __forceinline__ void stage_tape(StagedTapeN<CAP>& T, const s2m_op* __
                                            uint32_t t = threadIdx.x, uint32_t nt = blockDim.x)
 {
     for (uint32_t k = t; k < n; k += nt) {
-        const s2m_op& o = ops[L[k]];
-        T.code[k] = o.code;
+        const s2m_op& o = ops[L[k] & (kSwapped - 1u)];
+        T.code[k] = o.code | (L[k] & kSwapped ? kSwapCode : 0u);
         T.iarg[k] = o.iarg;
 #pragma unroll
         for (int j = 0; j < 8; ++j) T.f[k][j] = o.f[j];
@@ -90,8 +93,8 @@ __device__ __forceinline__ void stage_tape(StagedFoldN<CAP>& T, const s2m_op* __
                                            uint32_t t = threadIdx.x, uint32_t nt = blockDim.x)
 {
     for (uint32_t k = t; k < n; k += nt) {
-        const s2m_op& o = ops[L[k]];
-        T.code[k] = (uint8_t)o.code;
+        const s2m_op& o = ops[L[k] & (kSwapped - 1u)];
+        T.code[k] = (uint8_t)(o.code | (L[k] & kSwapped ? kSwapCode : 0u));
         if ((k & 1u) || k == 0) {
 #pragma unroll
             for (int j = 0; j < 7; ++j) T.f[(k + 1u) >> 1][j] = o.f[j];
@@ -157,7 +160,8 @@ __device__ __forceinline__ void staged_prim(const TT& T, uint32_t k, uint32_t co
     }
 }
 
-// acc = op(acc, d) at NP points (code is wave-uniform)
+// acc = op(acc, d) at NP points, op(d, acc) with kSwapCode (code is wave-uniform; union and
+// intersection are never marked)
 template <int NP>
 __device__ __forceinline__ void staged_op(uint32_t code, float k, float (&acc)[NP], const float (&d)[NP])
 {
@@ -182,6 +186,22 @@ __device__ __forceinline__ void staged_op(uint32_t code, float k, float (&acc)[N
 #pragma unroll
         for (int p = 0; p < NP; ++p) acc[p] = op_smooth_intersection(acc[p], d[p], k);
         break;
+    case S2M_OP_SUBTRACTION | kSwapCode:
+#pragma unroll
+        for (int p = 0; p < NP; ++p) acc[p] = fmaxf(-d[p], acc[p]);
+        break;
+    case S2M_OP_SMOOTH_UNION | kSwapCode:
+#pragma unroll
+        for (int p = 0; p < NP; ++p) acc[p] = op_smooth_union(d[p], acc[p], k);
+        break;
+    case S2M_OP_SMOOTH_INTERSECTION | kSwapCode:
+#pragma unroll
+        for (int p = 0; p < NP; ++p) acc[p] = op_smooth_intersection(d[p], acc[p], k);
+        break;
+    case S2M_OP_SMOOTH_SUBTRACTION | kSwapCode:
+#pragma unroll
+        for (int p = 0; p < NP; ++p) acc[p] = op_smooth_subtraction(d[p], acc[p], k);
+        break;
     default:
 #pragma unroll
         for (int p = 0; p < NP; ++p) acc[p] = op_smooth_subtraction(acc[p], d[p], k);
@@ -202,29 +222,45 @@ __device__ __forceinline__ void run_linear(const TT& T, uint32_t n, const float 
     }
 }
 
-// Any valid program: the postfix stack machine of tape_eval with a wave-uniform depth.
-template <class TT>
-__device__ __forceinline__ float run_general(const TT& T, uint32_t n, float px, float py, float pz)
+// Any valid program, at NP points: the postfix stack machine of tape_eval with a
+// wave-uniform depth, several points per lane sharing each op's decode (the latency of a
+// tile's program, not its arithmetic, bounds the few tiles that come here).  An operator
+// right after a primitive takes it without a push.  Deeper entries go to `stack`: entry e
+// of the lane's point p at stack[(e * NP + p) * stride].  MANDEL: the program may hold a
+// Mandelbulb.
+template <int NP, bool MANDEL, class TT>
+__device__ __forceinline__ void run_general(const TT& T, uint32_t n, const float (&x)[NP], const float (&y)[NP],
+                                            const float (&z)[NP], float (&acc)[NP], float* stack, uint32_t stride)
 {
-    float st[S2M_MAX_STACK];
-    float acc = 0.0f;
     uint32_t sp = 0;
-    const float x[1] = {px}, y[1] = {py}, z[1] = {pz};
     for (uint32_t k = 0; k < n; ++k) {
         const uint32_t code = uniform_code(T, k);
-        if (code < S2M_OP_UNION) {
-            float d[1];
-            staged_prim<1, true>(T, k, code, x, y, z, d);
-            if (k != 0) st[sp++] = acc;
-            acc = d[0];
+        if ((code & ~kSwapCode) < S2M_OP_UNION) {
+            float d[NP];
+            staged_prim<NP, MANDEL>(T, k, code, x, y, z, d);
+            const uint32_t next = k + 1 < n && k != 0 ? uniform_code(T, k + 1) : 0u;
+            if ((next & ~kSwapCode) >= S2M_OP_UNION) {
+                staged_op<NP>(next, T.f_at(k + 1)[0], acc, d);
+                ++k;
+                continue;
+            }
+            if (k != 0) {
+#pragma unroll
+                for (int p = 0; p < NP; ++p) stack[(sp * NP + p) * stride] = acc[p];
+                ++sp;
+            }
+#pragma unroll
+            for (int p = 0; p < NP; ++p) acc[p] = d[p];
         } else {
-            float a[1] = {st[--sp]};
-            const float d[1] = {acc};
-            staged_op<1>(code, T.f_at(k)[0], a, d);
-            acc = a[0];
+            float a[NP];
+            --sp;
+#pragma unroll
+            for (int p = 0; p < NP; ++p) a[p] = stack[(sp * NP + p) * stride];
+            staged_op<NP>(code, T.f_at(k)[0], a, acc);
+#pragma unroll
+            for (int p = 0; p < NP; ++p) acc[p] = a[p];
         }
     }
-    return acc;
 }
 
 }  // namespace s2m

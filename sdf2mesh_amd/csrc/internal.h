@@ -57,7 +57,9 @@ enum Counter : uint32_t {
     kSlotsNow = 13,    // sparse pass: its slots and staged cells, once they are final
     kStageNow = 14,
     kStageMax = 12,    // largest kStageUsed of the job so far
-    kNumCounters = 16
+    kGenUsed = 15,     // sparse pass: slots whose program is no fold, being counted and final
+    kGenNow = 16,
+    kNumCounters = 20
 };
 
 // Everything the cell kernels need to address one slab of cells [z0, z0+nz).
@@ -91,6 +93,10 @@ struct SlabBits {
 
 constexpr uint32_t kTile = 8;  // cells per tile edge (sparse pipeline)
 constexpr uint32_t kSuper = 4;  // tiles per super-tile edge (first pruning level)
+// A pruned list's operator entry with this bit applies its operator with the operands
+// swapped: the stack's top is its first (sparse.hip, PruneWalk).
+constexpr uint32_t kSwapped = 0x8000u;
+static_assert(S2M_MAX_TAPE <= kSwapped, "op indices leave the bit free");
 constexpr uint32_t kStageOps = 128;  // longest program staged in LDS (device_staged.h)
 constexpr uint32_t kSingleSign = 0xffffffffu;  // a super-tile's list length: the SDF keeps one sign there
 constexpr uint32_t kStageChunkHost = 1024;  // staged-cell allocation chunk (sparse.hip)
@@ -154,6 +160,7 @@ struct SpPass {
     uint32_t njobs;
     uint32_t list_stride;      // >= nops of every job
     uint32_t prune_depth;      // >= 1, >= the deepest operand stack of any job's program - 1
+    uint32_t walk_ops;         // longest program of a job that is no left fold, if at most kStageOps
     uint64_t ntiles;           // tiles of the pass
     uint64_t nrows;            // rows (z, y) of the pass
     uint64_t ntrows;           // tile rows (tile layer, ty) of the pass
@@ -168,6 +175,7 @@ struct SpPass {
     int32_t* slot_of_tile;     // [tile], -1: no active cell
     uint32_t* tile_of_slot;    // [slot]
     uint32_t* job_of_slot;     // [slot]
+    uint32_t* gen_slots;       // the slots whose program is no fold (kGenUsed of them)
     uint32_t slot_cap;
     uint32_t box_stride;       // floats of a tile's lattice box (LDS)
     uint32_t* cellbits;        // [slot][16] bit c: cell c of the tile has a vertex (row r = c / 8

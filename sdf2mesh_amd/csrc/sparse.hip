@@ -204,21 +204,35 @@ struct PruneStack {
 };
 
 constexpr uint32_t kComposite = 0xffffu;
-constexpr uint32_t kFoldBit = 0x80000000u;  // PruneWalk sums: the subtree is a left fold
+constexpr uint32_t kFoldBit = 0x80000000u;  // PruneWalk sums: the subtree's list is a left fold
 
+// A tile's list while it is walked, in LDS: lane ln's entry k.  (A walk reads entries back when
+// it drops or turns a subtree; from global memory each such step waits for the memory.)
+struct LdsList {
+    uint16_t* p;
+    uint32_t ln;
+    __device__ __forceinline__ uint16_t& operator[](uint32_t k) const { return p[k * 64u + ln]; }
+};
+
+// kTurn: an operator between a primitive and a longer fold is written as a fold too, the
+// fold first, then the primitive, then the operator marked kSwapped (union and
+// intersection need no mark): any tree whose operators each keep a primitive operand
+// becomes a left fold, which the tile kernels run without an operand stack.
+template <bool kTurn>
 struct PruneWalk {
     Iv top = iv_unknown();
     uint32_t top_start = 0, depth = 0, len = 0;  // depth: entries below `top`
     uint32_t top_single = kComposite;  // op index when `top` is one primitive
-    // flops of the kept ops of the top subtree (op_flops), | kFoldBit when that subtree is a
-    // left fold of library primitives (a primitive other than the Mandelbulb, or a left
-    // fold, such a primitive and an operator): the tile's flops and left-fold flag without
-    // reading its list back
+    // flops of the kept ops of the top subtree (op_flops), | kFoldBit when its list is a left
+    // fold of library primitives (a primitive other than the Mandelbulb, or a left fold,
+    // such a primitive and an operator): the tile's flops and left-fold flag without reading
+    // its list back
     uint32_t top_sum = 0;
 
     // The primitive with op index i, interval v (q: its position in the program; sum: its
     // flops | kFoldBit unless it is a Mandelbulb).
-    __device__ __forceinline__ void prim(uint32_t q, uint32_t i, const Iv& v, uint16_t* out, const PruneStack& S,
+    template <class List>
+    __device__ __forceinline__ void prim(uint32_t q, uint32_t i, const Iv& v, const List& out, const PruneStack& S,
                                          uint32_t ln, uint32_t sum = 0)
     {
         if (q != 0) {  // push the previous top
@@ -237,7 +251,8 @@ struct PruneWalk {
     }
 
     // Operator i (code, smoothing radius k, flops fl) on the two topmost values.
-    __device__ __forceinline__ void op(uint32_t i, uint32_t code, float k, uint16_t* out, const PruneStack& S,
+    template <class List>
+    __device__ __forceinline__ void op(uint32_t i, uint32_t code, float k, const List& out, const PruneStack& S,
                                        uint32_t ln, uint32_t fl = 0)
     {
         const Iv B = top;
@@ -250,8 +265,15 @@ struct PruneWalk {
         int keep;
         const Iv r = iv_op(code, A, B, k, keep);
         if (keep == kKeepBoth) {
-            out[len++] = (uint16_t)i;
-            const bool fold = (sumA & kFoldBit) && top_single != kComposite && (top_sum & kFoldBit);
+            bool fold = (sumA & kFoldBit) && top_single != kComposite && (top_sum & kFoldBit);
+            uint32_t mark = 0;
+            if (kTurn && !fold && (sumA & kFoldBit) && singleA != kComposite && (top_sum & kFoldBit)) {
+                for (uint32_t j = sB; j < len; ++j) out[j - 1u] = out[j];  // A is the one entry before B
+                out[len - 1u] = (uint16_t)singleA;
+                mark = code == S2M_OP_UNION || code == S2M_OP_INTERSECTION ? 0u : kSwapped;
+                fold = true;
+            }
+            out[len++] = (uint16_t)(i | mark);
             top_sum = ((sumA & ~kFoldBit) + (top_sum & ~kFoldBit) + fl) | (fold ? kFoldBit : 0u);
             top = r;
             top_single = kComposite;
@@ -380,8 +402,10 @@ __device__ __forceinline__ void super_tiles(const SpJob& J, uint64_t s, uint32_t
 //     (every lane walks the same list: wave-uniform op dispatch).  Tiles that keep one sign
 //     are dropped, the others get a slot in the pool shared by all jobs (and a flag when
 //     their list is a left fold).
-// Dynamic LDS: the prune stack (P.prune_depth entries per lane).  Lists and intervals of
-// programs of at most kStageOps ops live in LDS, of longer ones in super_lists / super_iv.
+// Dynamic LDS: the prune stack (P.prune_depth entries per lane), then P.walk_ops list entries
+// per lane for the tiles' walks of programs that are no left folds.  Lists and intervals of
+// programs of at most kStageOps ops live in LDS, of longer ones in lists, super_lists and
+// super_iv.
 // ---------------------------------------------------------------------------------
 
 // prune_fold: the super-tile list of a program that is a left fold of unions and smooth
@@ -503,7 +527,7 @@ __device__ __forceinline__ void prim_intervals(const SpJob& J, const double* bl,
 __device__ __forceinline__ uint32_t walk_super(const SpJob& J, const double2* iv, const uint32_t* codes,
                                                const uint32_t* radii, const PruneStack& S, uint32_t ln, uint16_t* out)
 {
-    PruneWalk w;
+    PruneWalk<false> w;  // the tiles' walks take its list in the program's order
     for (uint32_t q = 0; q < J.nops; ++q) {
         const uint32_t code = __builtin_amdgcn_readfirstlane(codes ? codes[q] : J.ops[q].code);
         if (code < S2M_OP_UNION) {
@@ -519,13 +543,13 @@ __device__ __forceinline__ uint32_t walk_super(const SpJob& J, const double2* iv
 // What the pass's later kernels count into, cleared (by all blocks): the job rows and
 // counters of a job's first pass (for a later pass the totals so far become its first
 // indices), work queues with the statistics beside them, chunk sums, and before a
-// multi-pass job the boundary plane (no vertex carried yet).  kSlotsUsed and kStageUsed,
-// which this kernel and the tile kernels count, are zero already (k_sp_rowdown).
+// multi-pass job the boundary plane (no vertex carried yet).  kSlotsUsed, kGenUsed and
+// kStageUsed, which this kernel and the tile kernels count, are zero already (k_sp_rowdown).
 __device__ __forceinline__ void clear_pass(const SpPass& P)
 {
     const uint32_t t = blockIdx.x * 64u + (thread_id() & 63u), step = gridDim.x * 64u;
     for (uint32_t i = t; i < P.nclear; i += step)
-        if (i != kSlotsUsed && i != kStageUsed) P.counters[i] = 0;
+        if (i != kSlotsUsed && i != kStageUsed && i != kGenUsed) P.counters[i] = 0;
     if (P.nclear == 0 && t == 0) {
         P.counters[kVtxPrev] = P.counters[kVtxTotal];
         P.counters[kTriPrev] = P.counters[kTriTotal];
@@ -600,7 +624,7 @@ __global__ __launch_bounds__(64) void k_sp_prune(SpPass P)
         double bl[3], bh[3];
         tiles_box(J, tt, tt, bl, bh);
         uint16_t* L = P.lists + (size_t)tile * P.list_stride;
-        auto walk = [&](auto& w) {
+        auto walk = [&](auto& w, auto L) {
             if (staged) {  // every lane walks the same list: wave-uniform dispatch
                 for (uint32_t q = 0; q < sl; ++q) {
                     const uint32_t code = uniform_code(T, q), i = idx[q], sum = sums[q];
@@ -624,10 +648,16 @@ __global__ __launch_bounds__(64) void k_sp_prune(SpPass P)
         };
         if (J.left_fold) {  // the super-tile's list is a left fold too
             FoldWalk w;
-            walk(w);
+            walk(w, L);
+        } else if (J.nops <= P.walk_ops) {
+            PruneWalk<true> w;
+            const LdsList list{reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(prune_lds) + PruneStack::bytes(D)), ln};
+            walk(w, list);
+            if (surface)
+                for (uint32_t q = 0; q < w.len; ++q) L[q] = list[q];
         } else {
-            PruneWalk w;
-            walk(w);
+            PruneWalk<true> w;
+            walk(w, L);
         }
     }
     // slots for the surviving tiles: one counter update per wave
@@ -645,6 +675,14 @@ __global__ __launch_bounds__(64) void k_sp_prune(SpPass P)
         }
     }
     if (valid) P.slot_of_tile[tile] = slot;
+    // the slots that are no folds, listed for k_sp_tiles<0> and k_sp_emit<0>
+    const uint64_t g = __ballot(slot >= 0 && !(lens & kLinearFlag));
+    if (g) {
+        uint64_t gbase = 0;
+        if (ln == 0) gbase = atomicAdd((unsigned long long*)&P.counters[kGenUsed], (unsigned long long)__builtin_popcountll(g));
+        gbase = __shfl(gbase, 0, 64);
+        if ((g >> ln) & 1ull) P.gen_slots[gbase + (uint64_t)__builtin_popcountll(g & ((1ull << ln) - 1ull))] = (uint32_t)slot;
+    }
     const uint64_t act = __ballot(slot >= 0);  // bit l: tile l of the super-tile has a slot
     if (ln == 0) P.super_act[s] = act;
 
@@ -700,6 +738,7 @@ struct TileGen {  // k_sp_tiles<0>: the same parts, staged per slot
     StagedTape T;
     TileAxes A;
     float pc[3][16];
+    uint32_t mandel;  // the program holds a Mandelbulb
 };
 
 // ---------------------------------------------------------------------------------
@@ -830,7 +869,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
         for (uint32_t k = 1; k + 1 < n; k += 2) {
             const Iv d = iv_primitive(uniform_code(T, k), T.f_at(k), bl, bh);
             int keep;
-            acc = iv_op(uniform_code(T, k + 1), acc, d, T.f_at(k + 1)[0], keep);
+            const uint32_t code = uniform_code(T, k + 1);
+            if (code & kSwapCode) acc = iv_op(code & ~kSwapCode, d, acc, T.f_at(k + 1)[0], keep);
+            else acc = iv_op(code, acc, d, T.f_at(k + 1)[0], keep);
         }
         const bool may_cross = !(acc.known && (acc.lo > 0.0 || acc.hi < 0.0));
         const uint64_t m = __ballot(may_cross);
@@ -855,6 +896,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
 constexpr uint32_t kStageChunk = kStageChunkHost;
 constexpr uint32_t kTileThreads = 256;  // threads of a k_sp_tiles block (one tile at a time)
 constexpr int kLinearPoints = 2;        // points per lane sharing each op's decode (left folds)
+constexpr int kGeneralPoints = 4;       // (other programs: a box of up to 1024 points in one round,
+constexpr uint32_t kWideDepth = 8;      // their operand stacks within 32 KB of LDS; deeper ones
+                                        // take one point at a time)
 static_assert(kRecVec - kRecPre <= kTileThreads, "one thread per record word past the read-ahead");
 
 struct ContourLds {  // block-shared state of contour_tile (and `cand`, 512 entries: the cells
@@ -1012,12 +1056,12 @@ static_assert(kTileThreads >= kBoxAxis * kBoxAxis, "one box row per thread");
 // LDS, at the lattice points of its closed box that the tile's cells need (all points for
 // programs that are not left folds), into an LDS box; then the tile's cells are contoured
 // from it (contour_tile).  LINEAR = 1 runs the slots whose program is a left fold (two
-// points per lane), LINEAR = 0 the others; both launches walk all slots and skip the
-// other kind.
+// points per lane) and skips the others, LINEAR = 0 the others (gen_slots).
 template <int LINEAR>
 __device__ __forceinline__ void tiles_body(const SpPass& P)
 {
-    extern __shared__ float box[];  // P.box_stride floats
+    extern __shared__ float box[];  // P.box_stride floats; LINEAR = 0: then the operand stacks
+                                    // (P.prune_depth entries per thread and point)
     // left folds: the slot's record (k_sp_bricks); other programs: staged here
     __shared__ std::conditional_t<LINEAR != 0, TileRec, TileGen> R;
     // points to evaluate; then the contour's candidate cells (contour_tile's `cand`)
@@ -1026,7 +1070,8 @@ __device__ __forceinline__ void tiles_body(const SpPass& P)
     __shared__ ContourLds L;
     __shared__ uint32_t sh_slot, sh_next;
     __shared__ uint8_t lb[64];  // the live bricks of the slot (contour_tile)
-    const uint32_t nslots = active_slots(P);
+    // LINEAR = 0: indices into the list of the slots that are no folds
+    const uint32_t nslots = active_slots(P, LINEAR ? kSlotsUsed : kGenUsed);
     constexpr uint32_t kQueue = LINEAR ? 0u : 1u;
     if (thread_id() == 0) L.left = 0;  // published by the first slot's barriers
     uint64_t tiles_done = 0, points_done = 0, flops_done = 0;  // thread 0: this block's share
@@ -1049,8 +1094,8 @@ __device__ __forceinline__ void tiles_body(const SpPass& P)
         if (thread_id() == 0) sh_slot = next;
         if (LINEAR && thread_id() < kRecPre) reinterpret_cast<uint4*>(&R)[thread_id()] = pre;
         __syncthreads();
-        const uint32_t slot = sh_slot;
-        if (slot >= nslots) break;
+        if (sh_slot >= nslots) break;
+        const uint32_t slot = LINEAR ? sh_slot : P.gen_slots[sh_slot];
         if (thread_id() == 0) next = queue_take(P, kQueue, blockIdx.x, gridDim.x);  // prefetched
         const SlotHdr& H = [&]() -> const SlotHdr& {
             if constexpr (LINEAR != 0) return R.H;
@@ -1195,13 +1240,43 @@ __device__ __forceinline__ void tiles_body(const SpPass& P)
                 const float* c = a == 0 ? J.cx + x0 : a == 1 ? J.cy + y0 : J.cz + z0;
                 if (i < (a == 0 ? nx : a == 1 ? ny : nz)) R.pc[a][i] = c[i];
             }
+            if (thread_id() == 0) R.mandel = 0;
             __syncthreads();
-            for (uint32_t q = thread_id(); q < npts; q += kTileThreads) {
+            if (staged)
+                for (uint32_t q = thread_id(); q < n; q += kTileThreads)
+                    if (R.T.code[q] == S2M_OP_MANDELBULB) R.mandel = 1;
+            __syncthreads();
+            auto point = [&](uint32_t q, float& x, float& y, float& z) {  // its entry in the box
                 const uint32_t iz = div16(q, nxy, mxy), r = q - iz * nxy;
                 const uint32_t iy = div16(r, nx, mx), ix = r - iy * nx;
-                const float x = R.pc[0][ix], y = R.pc[1][iy], z = R.pc[2][iz];
-                box[(iz * by + iy) * bx + ix] =
-                    staged ? run_general(R.T, n, x, y, z) : tape_eval_list(J.ops, Lst, n, x, y, z);
+                x = R.pc[0][ix];
+                y = R.pc[1][iy];
+                z = R.pc[2][iz];
+                return (iz * by + iy) * bx + ix;
+            };
+            float* stack = box + P.box_stride + thread_id();
+            if (staged && !R.mandel && P.prune_depth <= kWideDepth) {
+                for (uint32_t q0 = thread_id(); q0 < npts; q0 += kGeneralPoints * kTileThreads) {
+                    float x[kGeneralPoints], y[kGeneralPoints], z[kGeneralPoints], v[kGeneralPoints];
+                    uint32_t at[kGeneralPoints];
+#pragma unroll
+                    for (int p = 0; p < kGeneralPoints; ++p) {
+                        const uint32_t q = q0 + p * kTileThreads;
+                        at[p] = point(q < npts ? q : q0, x[p], y[p], z[p]);
+                    }
+                    run_general<kGeneralPoints, false>(R.T, n, x, y, z, v, stack, kTileThreads);
+#pragma unroll
+                    for (int p = 0; p < kGeneralPoints; ++p)
+                        if (q0 + p * kTileThreads < npts) box[at[p]] = v[p];
+                }
+            } else {
+                for (uint32_t q = thread_id(); q < npts; q += kTileThreads) {
+                    float x[1], y[1], z[1], v[1];
+                    const uint32_t at = point(q, x[0], y[0], z[0]);
+                    if (staged) run_general<1, true>(R.T, n, x, y, z, v, stack, kTileThreads);
+                    else v[0] = tape_eval_list(J.ops, Lst, n, x[0], y[0], z[0]);
+                    box[at] = v[0];
+                }
             }
             evaluated = npts;
         }
@@ -1362,11 +1437,14 @@ template <int LINEAR>
 __global__ __launch_bounds__(64) void k_sp_emit(SpPass P, MeshBufs b)
 {
     __shared__ StagedTape T;      // programs that are not left folds (left folds: read in place)
+    __shared__ uint32_t mandel;   // such a program holds a Mandelbulb
+    extern __shared__ float taps[];  // their operand stacks: P.prune_depth entries of 4 per lane
     __shared__ uint32_t nb[729];  // vertex of cell (8tx-1+i, 8ty-1+j, 8tz-1+k) at nb[(k*9+j)*9+i]
     __shared__ uint32_t tc[128];  // triangles of cell c in byte c % 4 of tc[c / 4]
     if (LINEAR && blockIdx.x == 0) report(P);
-    const uint32_t nslots = active_slots(P, kSlotsNow);
-    for (uint32_t slot = blockIdx.x; slot < nslots; slot += gridDim.x) {
+    const uint32_t nslots = active_slots(P, LINEAR ? kSlotsNow : kGenNow);
+    for (uint32_t turn = blockIdx.x; turn < nslots; turn += gridDim.x) {
+        const uint32_t slot = LINEAR ? turn : P.gen_slots[turn];
         const SlotHdr& H = P.slot_hdr[slot];
         const uint64_t tile = __builtin_amdgcn_readfirstlane(H.tile);
         const SpJob& J = P.jobs[__builtin_amdgcn_readfirstlane(H.job)];
@@ -1383,7 +1461,13 @@ __global__ __launch_bounds__(64) void k_sp_emit(SpPass P, MeshBufs b)
         const bool linear = (lens & kLinearFlag) != 0, staged = len <= kStageOps;
         if (linear != (LINEAR != 0)) continue;  // the other launch's slot
         __syncthreads();  // the previous slot's readers of T, nb, tc are done
-        if (!LINEAR && normals && staged) stage_tape(T, J.ops, Lst, len);
+        if (!LINEAR && normals && staged) {
+            if (thread_id() == 0) mandel = 0;
+            stage_tape(T, J.ops, Lst, len);
+            __syncthreads();
+            for (uint32_t q = thread_id(); q < len; q += 64u)
+                if (T.code[q] == S2M_OP_MANDELBULB) mandel = 1;
+        }
         // left folds: the program as staged in the slot's record, read in place
         const ScalarFold TS =
             ScalarFold::at(reinterpret_cast<const char*>(P.slot_rec + (size_t)slot * kRecVec) + offsetof(TileRec, T));
@@ -1439,11 +1523,16 @@ __global__ __launch_bounds__(64) void k_sp_emit(SpPass P, MeshBufs b)
             float d[4];
             if constexpr (LINEAR != 0) {
                 run_linear<4>(TS, len, tx4, ty4, tz4, d);
+            } else if (staged && !mandel) {
+                run_general<4, false>(T, len, tx4, ty4, tz4, d, taps + thread_id(), 64u);
             } else {
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-                    d[t] = staged ? run_general(T, len, tx4[t], ty4[t], tz4[t])
-                                  : tape_eval_list(J.ops, Lst, len, tx4[t], ty4[t], tz4[t]);
+                for (int t = 0; t < 4; ++t) {
+                    const float x[1] = {tx4[t]}, y[1] = {ty4[t]}, z[1] = {tz4[t]};
+                    float v[1];
+                    if (staged) run_general<1, true>(T, len, x, y, z, v, taps + thread_id(), 64u);
+                    else v[0] = tape_eval_list(J.ops, Lst, len, x[0], y[0], z[0]);
+                    d[t] = v[0];
+                }
             }
             const float d1 = d[0], d2 = d[1], d3 = d[2], d4 = d[3];
             const float gx = ((d1 + (-d2)) + (-d3)) + d4;
@@ -1657,6 +1746,8 @@ __global__ __launch_bounds__(256) void k_sp_rowdown(SpPass P)
         P.counters[kVtxTotal] = bv + lds[0][0] + lds[0][1] + lds[0][2] + lds[0][3];
         P.counters[kTriTotal] = bt + lds[1][0] + lds[1][1] + lds[1][2] + lds[1][3];
         // the pass's slots and staging: kept, folded into their maxima, reset
+        P.counters[kGenNow] = P.counters[kGenUsed];
+        P.counters[kGenUsed] = 0;
         for (uint32_t q = 0; q < 2; ++q) {
             const uint32_t used = q ? kStageUsed : kSlotsUsed, most = q ? kStageMax : kSlotsMax;
             const uint64_t n = P.counters[used];
@@ -1747,7 +1838,7 @@ hipError_t launch_sparse_pass(hipStream_t s, const SpPass& P, const MeshBufs& b,
     auto mark = [&](int i) {
         if (marks && marks[i]) (void)hipEventRecord(marks[i], s);
     };
-    const size_t prune_smem = PruneStack::bytes(P.prune_depth);
+    const size_t prune_smem = PruneStack::bytes(P.prune_depth) + (size_t)P.walk_ops * 64u * sizeof(uint16_t);
     if (P.nsuper > 0x7fffffffull) return hipErrorInvalidValue;
     mark(0);
     hipLaunchKernelGGL(k_sp_prune, dim3((uint32_t)P.nsuper), dim3(64), prune_smem, s, P);
@@ -1756,9 +1847,12 @@ hipError_t launch_sparse_pass(hipStream_t s, const SpPass& P, const MeshBufs& b,
     const size_t smem = (size_t)P.box_stride * sizeof(float);
     hipLaunchKernelGGL((k_sp_tiles<1>), dim3(resident_blocks(k_sp_tiles<1>, kTileThreads, smem, cus, tile_blocks)),
                        dim3(kTileThreads), smem, s, P);
+    const size_t gsmem = smem + (size_t)P.prune_depth * (P.prune_depth <= kWideDepth ? kGeneralPoints : 1) *
+                                    kTileThreads * sizeof(float);
+    const size_t esmem = (size_t)P.prune_depth * 4u * 64u * sizeof(float);
     if (general_tiles)
-        hipLaunchKernelGGL((k_sp_tiles<0>), dim3(resident_blocks(k_sp_tiles<0>, kTileThreads, smem, cus, tile_blocks)),
-                           dim3(kTileThreads), smem, s, P);
+        hipLaunchKernelGGL((k_sp_tiles<0>), dim3(resident_blocks(k_sp_tiles<0>, kTileThreads, gsmem, cus, tile_blocks)),
+                           dim3(kTileThreads), gsmem, s, P);
     mark(2);
     hipLaunchKernelGGL(k_sp_quadcount, dim3(resident_blocks(k_sp_quadcount, 64, 0, cus, big)), dim3(64), 0, s,
                        P, b);
@@ -1768,7 +1862,8 @@ hipError_t launch_sparse_pass(hipStream_t s, const SpPass& P, const MeshBufs& b,
     mark(4);
     hipLaunchKernelGGL((k_sp_emit<1>), dim3(resident_blocks(k_sp_emit<1>, 64, 0, cus, big)), dim3(64), 0, s, P, b);
     if (general_tiles)
-        hipLaunchKernelGGL((k_sp_emit<0>), dim3(resident_blocks(k_sp_emit<0>, 64, 0, cus, big)), dim3(64), 0, s, P, b);
+        hipLaunchKernelGGL((k_sp_emit<0>), dim3(resident_blocks(k_sp_emit<0>, 64, esmem, cus, big)), dim3(64), esmem, s,
+                           P, b);
     if (boundary_plane) {
         hipLaunchKernelGGL(k_sp_boundary, dim3((uint32_t)((P.boundary_cells + 255) / 256)), dim3(256), 0,
                            s, P);
