@@ -1149,7 +1149,7 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
     HIP_TRY(ctx->sp_queues.ensure((size_t)kQueues * kQueueGroups * 32 * sizeof(uint32_t)));
     const uint64_t nsup_alloc = std::max<uint64_t>(nsuper_pass, 1);
     if (list_stride > kStageOps) {  // super-tile lists and intervals that do not fit LDS
-        HIP_TRY(ctx->sp_super_iv.ensure(nsup_alloc * list_stride * 2 * sizeof(double)));
+        HIP_TRY(ctx->sp_super_iv.ensure(nsup_alloc * list_stride * 2 * sizeof(float)));
         HIP_TRY(ctx->sp_super_lists.ensure(nsup_alloc * list_stride * sizeof(uint16_t)));
     }
     HIP_TRY(ctx->sp_super_act.ensure(nsup_alloc * sizeof(uint64_t)));
@@ -1267,7 +1267,7 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
             P.row_off = P.row_sum + 2 * P.nrows;
             P.counters = b.counters;
             P.queues = ctx->sp_queues.as<uint32_t>();
-            P.super_iv = ctx->sp_super_iv.as<double2>();
+            P.super_iv = ctx->sp_super_iv.as<float2>();
             P.super_lists = ctx->sp_super_lists.as<uint16_t>();
             P.super_act = ctx->sp_super_act.as<uint64_t>();
             P.job_out = job_out;

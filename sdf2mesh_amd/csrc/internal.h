@@ -166,7 +166,7 @@ struct SpPass {
     uint64_t ntrows;           // tile rows (tile layer, ty) of the pass
     uint64_t boundary_cells;   // rx * ry of jobs[0] when a boundary plane is written
     uint64_t nsuper;           // super-tiles of the pass
-    double2* super_iv;         // [super-tile][list_stride] primitive intervals (lo, hi), and pruned op
+    float2* super_iv;         // [super-tile][list_stride] primitive intervals (lo, hi), and pruned op
     uint16_t* super_lists;     // indices, of programs too long for LDS (kStageOps; NULL if none is)
     uint64_t* super_act;       // [super-tile] bit (z * 4 + y) * 4 + x: that tile has a slot
     uint16_t* lists;           // [tile][list_stride] pruned op indices

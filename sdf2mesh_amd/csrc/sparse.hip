@@ -184,8 +184,8 @@ __device__ __forceinline__ uint32_t vertex_at(const SpPass& P, const SpJob& J, u
 // of the interval stack is kept in registers, deeper entries in LDS columns (entry d of
 // lane l at [d * 64 + l]).
 struct PruneStack {
-    double* lo;        // [depth][64]
-    double* hi;        // [depth][64]
+    float* lo;         // [depth][64]
+    float* hi;         // [depth][64]
     uint32_t* sum;     // [depth][64] PruneWalk::top_sum of the entry
     uint16_t* start;   // [depth][64]
     uint16_t* single;  // [depth][64] op index of a one-primitive subtree, else kComposite
@@ -193,9 +193,9 @@ struct PruneStack {
     // LDS bytes of a stack of `depth` entries per lane, and its layout from `base`.
     static constexpr size_t bytes(uint32_t depth)
     {
-        return (size_t)depth * 64u * (2 * sizeof(double) + sizeof(uint32_t) + 2 * sizeof(uint16_t));
+        return (size_t)depth * 64u * (2 * sizeof(float) + sizeof(uint32_t) + 2 * sizeof(uint16_t));
     }
-    __device__ static PruneStack at(double* base, uint32_t depth)
+    __device__ static PruneStack at(float* base, uint32_t depth)
     {
         uint32_t* s32 = reinterpret_cast<uint32_t*>(base + 128u * depth);
         uint16_t* s16 = reinterpret_cast<uint16_t*>(s32 + 64u * depth);
@@ -258,7 +258,7 @@ struct PruneWalk {
         const Iv B = top;
         const uint32_t sB = top_start;
         --depth;
-        const double alo = S.lo[depth * 64u + ln], ahi = S.hi[depth * 64u + ln];
+        const float alo = S.lo[depth * 64u + ln], ahi = S.hi[depth * 64u + ln];
         const Iv A{alo, ahi, alo > -kHuge};  // iv_make / iv_unknown: known iff lo > -kHuge
         const uint32_t sA = S.start[depth * 64u + ln], singleA = S.single[depth * 64u + ln];
         const uint32_t sumA = S.sum[depth * 64u + ln];
@@ -296,7 +296,7 @@ struct PruneWalk {
         top_start = sA;
     }
 
-    __device__ __forceinline__ bool one_sign() const { return top.known && (top.lo > 0.0 || top.hi < 0.0); }
+    __device__ __forceinline__ bool one_sign() const { return top.known && (top.lo > 0.0f || top.hi < 0.0f); }
 };
 
 // PruneWalk for a left fold (P0 P1 op1 P2 op2 ...): the same decisions, list and sums with
@@ -348,7 +348,7 @@ struct FoldWalk {
         }
     }
 
-    __device__ __forceinline__ bool one_sign() const { return top.known && (top.lo > 0.0 || top.hi < 0.0); }
+    __device__ __forceinline__ bool one_sign() const { return top.known && (top.lo > 0.0f || top.hi < 0.0f); }
 };
 
 __device__ __forceinline__ uint32_t job_of(const SpPass& P, uint64_t index, bool super)
@@ -364,15 +364,18 @@ __device__ __forceinline__ uint32_t job_of(const SpPass& P, uint64_t index, bool
 
 }  // namespace
 
-// Padded box of the tiles [t0, t1] (per axis, t1 inclusive; z: tile layers of the job).
-__device__ __forceinline__ void tiles_box(const SpJob& J, const uint32_t t0[3], const uint32_t t1[3], double bl[3],
-                                          double bh[3])
+// Padded box of the tiles [t0, t1] (per axis, t1 inclusive; z: tile layers of the job).  The
+// pad is 1.25 times what the taps and roundings of a vertex need (J.pad), which covers the
+// rounding of the box itself: a quarter of 1e-6 (1 + max |coordinate|) is four half ulps.
+__device__ __forceinline__ void tiles_box(const SpJob& J, const uint32_t t0[3], const uint32_t t1[3], float bl[3],
+                                          float bh[3])
 {
+    const float pad = 1.25f * (float)J.pad;
     const float* e[3] = {J.ext, J.ext + 2 * J.ntx, J.ext + 2 * J.ntx + 2 * J.nty};
     const uint32_t n[3] = {J.ntx, J.nty, J.ntz};
     for (int a = 0; a < 3; ++a) {
-        bl[a] = (double)e[a][t0[a]] - J.pad;
-        bh[a] = (double)e[a][n[a] + t1[a]] + J.pad;
+        bl[a] = e[a][t0[a]] - pad;
+        bh[a] = e[a][n[a] + t1[a]] + pad;
     }
 }
 
@@ -422,18 +425,18 @@ __device__ __forceinline__ void super_tiles(const SpJob& J, uint64_t s, uint32_t
 // changes acc, so later bounds stay valid.  The super-tile keeps one sign when
 // min_j hi(P_j) + slack < 0 (acc < 0), or when min over the kept P_j of lo(P_j) - the kept
 // smooth radii / 4 - slack > 0 (smooth union >= min of its operands - k / 4).
-__device__ __forceinline__ uint32_t prune_fold(const SpJob& J, const double* bl, const double* bh, uint32_t ln,
+__device__ __forceinline__ uint32_t prune_fold(const SpJob& J, const float* bl, const float* bh, uint32_t ln,
                                                uint16_t* out)
 {
     const s2m_op* ops = J.ops;
     const uint32_t nops = J.nops;
-    double carry_u = kHuge;    // min hi(P_j) over the primitives so far
-    double carry_mag = 0.0;    // sum of |P_j| + k_j over the primitives so far
-    double carry_max = 0.0;    // max of |P_j| + k_j so far
-    double carry_ka = 0.0;     // sum of k_j / 4 so far
-    double carry_cnt = 0.0;    // primitives so far
-    double carry_lo = kHuge;   // min lo(P_j) over the kept primitives
-    double carry_k4 = 0.0;     // sum of the kept smooth radii / 4
+    float carry_u = kHuge;    // min hi(P_j) over the primitives so far
+    float carry_mag = 0.0f;    // sum of |P_j| + k_j over the primitives so far
+    float carry_max = 0.0f;    // max of |P_j| + k_j so far
+    float carry_ka = 0.0f;     // sum of k_j / 4 so far
+    float carry_cnt = 0.0f;    // primitives so far
+    float carry_lo = kHuge;   // min lo(P_j) over the kept primitives
+    float carry_k4 = 0.0f;     // sum of the kept smooth radii / 4
     uint32_t nkept = 0;
     bool prev_kept = true;     // was the last primitive of the previous chunk kept?
     for (uint32_t c0 = 0; c0 < nops; c0 += 64u) {
@@ -441,36 +444,36 @@ __device__ __forceinline__ uint32_t prune_fold(const SpJob& J, const double* bl,
         const bool valid = q < nops;
         const bool prim = valid && (q == 0 || (q & 1u));  // a left fold: P0, then P_m at odd q
         // the operator after primitive q (q >= 1) and its smoothing radius
-        double kk = 0.0;
-        if (prim && q >= 1 && ops[q + 1].code == S2M_OP_SMOOTH_UNION) kk = (double)ops[q + 1].f[0];
+        float kk = 0.0f;
+        if (prim && q >= 1 && ops[q + 1].code == S2M_OP_SMOOTH_UNION) kk = ops[q + 1].f[0];
         Iv B = iv_unknown();
         if (prim) B = iv_primitive(ops[q].code, ops[q].f, bl, bh);
-        const double mag = prim ? fmax(fabs(B.lo), fabs(B.hi)) + kk : 0.0;
+        const float mag = prim ? fmaxf(fabsf(B.lo), fabsf(B.hi)) + kk : 0.0f;
         // prefix scans over the lanes (inclusive): min hi, sum and max of the magnitudes,
         // sum of k / 4, count of primitives
-        double u_ex = prim ? B.hi : kHuge, m_in = mag, x_in = mag, ka_in = 0.25 * kk, c_in = prim ? 1.0 : 0.0;
+        float u_ex = prim ? B.hi : kHuge, m_in = mag, x_in = mag, ka_in = 0.25f * kk, c_in = prim ? 1.0f : 0.0f;
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) {
-            const double uo = __shfl_up(u_ex, d, 64), mo = __shfl_up(m_in, d, 64);
-            const double xo = __shfl_up(x_in, d, 64), ko = __shfl_up(ka_in, d, 64), co = __shfl_up(c_in, d, 64);
+            const float uo = __shfl_up(u_ex, d, 64), mo = __shfl_up(m_in, d, 64);
+            const float xo = __shfl_up(x_in, d, 64), ko = __shfl_up(ka_in, d, 64), co = __shfl_up(c_in, d, 64);
             if (ln >= (uint32_t)d) {
-                u_ex = fmin(u_ex, uo);
+                u_ex = fminf(u_ex, uo);
                 m_in += mo;
-                x_in = fmax(x_in, xo);
+                x_in = fmaxf(x_in, xo);
                 ka_in += ko;
                 c_in += co;
             }
         }
-        const double u_in = u_ex;  // inclusive
+        const float u_in = u_ex;  // inclusive
         u_ex = __shfl_up(u_in, 1, 64);
         if (ln == 0) u_ex = kHuge;
-        u_ex = fmin(u_ex, carry_u);
+        u_ex = fminf(u_ex, carry_u);
         m_in += carry_mag;
-        x_in = fmax(x_in, carry_max);
+        x_in = fmaxf(x_in, carry_max);
         ka_in += carry_ka;
         c_in += carry_cnt;
-        const double slack = kMargin * (m_in + c_in * (x_in + ka_in));
-        const double tiny = 1e-12 * (fabs(u_ex) + fabs(B.lo) + fabs(B.hi) + kk);
+        const float slack = kMargin * (m_in + c_in * (x_in + ka_in));
+        const float tiny = kUlps * (fabsf(u_ex) + fabsf(B.lo) + fabsf(B.hi) + kk);
         const bool drop = prim && q >= 1 && B.known && u_ex < kHuge && B.lo >= u_ex + kk + tiny + slack;
         // an operator (even q >= 2) is kept with its primitive q - 1
         const uint64_t pk = __ballot(prim && !drop);
@@ -480,16 +483,16 @@ __device__ __forceinline__ uint32_t prune_fold(const SpJob& J, const double* bl,
         if (kept) out[nkept + (uint32_t)__builtin_popcountll(km & ((1ull << ln) - 1ull))] = (uint16_t)q;
         nkept += (uint32_t)__builtin_popcountll(km);
         // one-sign bounds over the kept primitives
-        double lo_k = (prim && !drop) ? B.lo : kHuge;
-        double k4 = (prim && !drop) ? 0.25 * kk : 0.0;
+        float lo_k = (prim && !drop) ? B.lo : kHuge;
+        float k4 = (prim && !drop) ? 0.25f * kk : 0.0f;
 #pragma unroll
         for (int d = 32; d >= 1; d >>= 1) {
-            lo_k = fmin(lo_k, __shfl_xor(lo_k, d, 64));
+            lo_k = fminf(lo_k, __shfl_xor(lo_k, d, 64));
             k4 += __shfl_xor(k4, d, 64);
         }
-        carry_lo = fmin(carry_lo, lo_k);
+        carry_lo = fminf(carry_lo, lo_k);
         carry_k4 += k4;
-        carry_u = fmin(carry_u, __shfl(u_in, 63, 64));
+        carry_u = fminf(carry_u, __shfl(u_in, 63, 64));
         carry_mag = __shfl(m_in, 63, 64);
         carry_max = __shfl(x_in, 63, 64);
         carry_ka = __shfl(ka_in, 63, 64);
@@ -500,13 +503,13 @@ __device__ __forceinline__ uint32_t prune_fold(const SpJob& J, const double* bl,
         const uint32_t lastp = (c0 + last) & 1u ? last : (last ? last - 1u : 0u);
         prev_kept = ((pk >> lastp) & 1ull) != 0;
     }
-    const double slack = kMargin * (carry_mag + carry_cnt * (carry_max + carry_ka));
-    const bool one_sign = (carry_u + slack < 0.0) || (carry_lo > -kHuge && carry_lo - carry_k4 - slack > 0.0);
+    const float slack = kMargin * (carry_mag + carry_cnt * (carry_max + carry_ka));
+    const bool one_sign = (carry_u + slack < 0.0f) || (carry_lo > -kHuge && carry_lo - carry_k4 - slack > 0.0f);
     return one_sign ? kSingleSign : nkept;
 }
 
 // Op q's code and smoothing radius, and the interval of a primitive on the box.
-__device__ __forceinline__ void prim_intervals(const SpJob& J, const double* bl, const double* bh, uint32_t ln, double2* iv,
+__device__ __forceinline__ void prim_intervals(const SpJob& J, const float* bl, const float* bh, uint32_t ln, float2* iv,
                                                uint32_t* codes, uint32_t* radii)
 {
     for (uint32_t q = ln; q < J.nops; q += 64u) {
@@ -518,20 +521,20 @@ __device__ __forceinline__ void prim_intervals(const SpJob& J, const double* bl,
         }
         if (code >= S2M_OP_UNION) continue;
         const Iv v = iv_primitive(code, o.f, bl, bh);
-        iv[q] = make_double2(v.lo, v.hi);
+        iv[q] = make_float2(v.lo, v.hi);
     }
 }
 
 // The job's program walked in order on those intervals; every lane takes the same steps
 // and writes the same list.
-__device__ __forceinline__ uint32_t walk_super(const SpJob& J, const double2* iv, const uint32_t* codes,
+__device__ __forceinline__ uint32_t walk_super(const SpJob& J, const float2* iv, const uint32_t* codes,
                                                const uint32_t* radii, const PruneStack& S, uint32_t ln, uint16_t* out)
 {
     PruneWalk<false> w;  // the tiles' walks take its list in the program's order
     for (uint32_t q = 0; q < J.nops; ++q) {
         const uint32_t code = __builtin_amdgcn_readfirstlane(codes ? codes[q] : J.ops[q].code);
         if (code < S2M_OP_UNION) {
-            const double2 v = iv[q];
+            const float2 v = iv[q];
             w.prim(q, q, Iv{v.x, v.y, v.x > -kHuge}, out, S, ln);  // known iff lo > -kHuge
         } else {
             w.op(q, code, codes ? __uint_as_float(radii[q]) : J.ops[q].f[0], out, S, ln);
@@ -565,11 +568,11 @@ __device__ __forceinline__ void clear_pass(const SpPass& P)
 
 __global__ __launch_bounds__(64) void k_sp_prune(SpPass P)
 {
-    extern __shared__ double prune_lds[];
+    extern __shared__ float prune_lds[];
     __shared__ StagedTape T;          // the super-tile's list (at most kStageOps ops)
     __shared__ uint16_t idx[kStageOps];  // op index of each staged op
     __shared__ uint32_t sums[kStageOps];  // its flops | kFoldBit for primitives other than the Mandelbulb
-    static_assert(sizeof T.f >= kStageOps * sizeof(double2), "intervals share the staged operands' space");
+    static_assert(sizeof T.f >= kStageOps * sizeof(float2), "intervals share the staged operands' space");
     clear_pass(P);
     const uint32_t D = P.prune_depth, ln = thread_id() & 63u;
     const PruneStack S = PruneStack::at(prune_lds, D);
@@ -582,12 +585,12 @@ __global__ __launch_bounds__(64) void k_sp_prune(SpPass P)
     super_tiles(J, s, t0, t1);
     uint32_t sl;
     {
-        double bl[3], bh[3];
+        float bl[3], bh[3];
         tiles_box(J, t0, t1, bl, bh);
         if (J.union_fold) {
             sl = prune_fold(J, bl, bh, ln, in);
         } else {
-            double2* iv = small ? reinterpret_cast<double2*>(T.f) : P.super_iv + s * P.list_stride;
+            float2* iv = small ? reinterpret_cast<float2*>(T.f) : P.super_iv + s * P.list_stride;
             uint32_t *codes = small ? T.code : nullptr, *radii = small ? T.iarg : nullptr;
             prim_intervals(J, bl, bh, ln, iv, codes, radii);
             __syncthreads();  // visible to all lanes
@@ -621,7 +624,7 @@ __global__ __launch_bounds__(64) void k_sp_prune(SpPass P)
         P.flops[tile] = 0;
     } else if (valid) {
         const uint32_t tt[3] = {tx, ty, tz};
-        double bl[3], bh[3];
+        float bl[3], bh[3];
         tiles_box(J, tt, tt, bl, bh);
         uint16_t* L = P.lists + (size_t)tile * P.list_stride;
         auto walk = [&](auto& w, auto L) {
@@ -860,10 +863,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
         }
         // brick b: cells c, c + 1 per axis; the first cell's lo corner, the second's hi corner
         const uint32_t c[3] = {(b & 3u) * 2u, ((b >> 2) & 3u) * 2u, (b >> 4) * 2u};
-        double bl[3], bh[3];
+        float bl[3], bh[3];
         for (int a = 0; a < 3; ++a) {
-            bl[a] = (double)A.clo[a][c[a]];
-            bh[a] = (double)A.chi[a][c[a] + 1];
+            bl[a] = A.clo[a][c[a]];
+            bh[a] = A.chi[a][c[a] + 1];
         }
         Iv acc = iv_primitive(uniform_code(T, 0), T.f_at(0), bl, bh);
         for (uint32_t k = 1; k + 1 < n; k += 2) {
@@ -873,7 +876,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
             if (code & kSwapCode) acc = iv_op(code & ~kSwapCode, d, acc, T.f_at(k + 1)[0], keep);
             else acc = iv_op(code, acc, d, T.f_at(k + 1)[0], keep);
         }
-        const bool may_cross = !(acc.known && (acc.lo > 0.0 || acc.hi < 0.0));
+        const bool may_cross = !(acc.known && (acc.lo > 0.0f || acc.hi < 0.0f));
         const uint64_t m = __ballot(may_cross);
         if (b == 0) P.slot_live[slot] = RG.live = m;
     }
