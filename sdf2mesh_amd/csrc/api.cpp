@@ -781,6 +781,12 @@ uint32_t stream_passes(uint32_t tile_layers)
     return std::max<uint32_t>(1, std::min<uint32_t>(4, tile_layers / 16));
 }
 
+// Most bytes a pass of a single sparse job holds per tile and row; larger grids take several
+// passes.  Every pass pays the tails of its kernels, their latency and the test of its last
+// cell plane for the next: CSG-64 1024^3 takes 1389 us in four passes (1 GiB each) and 1084
+// in one.  2.3 GB of 288 there; the next power of two is split in four.
+constexpr uint64_t kSparsePassBytes = 4ull << 30;
+
 // Is the program a left fold of library primitives (P0 P1 op1 P2 op2 ...) short enough to
 // be staged (sparse.hip, kStageOps = 128)?  Every pruned sub-program of one is one too:
 // pruning keeps either the accumulated value or the right operand, a single primitive.
@@ -1008,7 +1014,7 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
         if (tabs[i].bmax[0] > 16 || tabs[i].bmax[1] > 16 || tabs[i].bmax[2] > 16)
             return fail(S2M_E_ARG, "tile box of %u x %u x %u lattice points", tabs[i].bmax[0], tabs[i].bmax[1],
                         tabs[i].bmax[2]);
-    // slabs (single job only): whole tile layers, per-pass buffers bounded to ~1 GiB
+    // slabs (single job only): whole tile layers, per-pass buffers bounded
     uint32_t layers = tabs[0].nt[2];
     if (n == 1) {
         if (ps[0]->slab) layers = std::max<uint32_t>(1, (ps[0]->slab + kTile - 1) / kTile);
@@ -1021,11 +1027,17 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
             layers = (tabs[0].nt[2] + passes - 1) / passes;
         }
         layers = std::min(layers, std::max<uint32_t>(tabs[0].nt[2], 1));
+        const uint64_t slot = kTileRecBytes + 16 * 68 + sizeof(SlotHdr) + 64;  // a quarter of the tiles get one
         auto pass_bytes = [&](uint64_t L) {
             const uint64_t t = (uint64_t)tabs[0].nt[0] * tabs[0].nt[1] * L;
-            return t * (list_stride * 2 + 12) + 16ull * L * kTile * jobs[0].res[1] * tabs[0].nt[0];
+            return t * (list_stride * 2 + 12 + slot / 4) + 16ull * L * kTile * jobs[0].res[1];
         };
-        while (layers > 1 && pass_bytes(layers) > (1ull << 30)) layers = (layers + 1) / 2;
+        auto pass_fits = [&](uint64_t L) {
+            return pass_bytes(L) <= kSparsePassBytes &&
+                   (uint64_t)tabs[0].nt[0] * tabs[0].nt[1] * L <= 0x7fffffffull &&
+                   L * kTile * jobs[0].res[1] <= (uint64_t)kMaxScanBlocks * kRowChunk;
+        };
+        while (layers > 1 && !pass_fits(layers)) layers = (layers + 1) / 2;
     }
     const uint32_t npass = n == 1 ? (tabs[0].nt[2] + layers - 1) / std::max(layers, 1u) : 1;
     Readback* const land = npass == 1 && !ctx->profiling ? rb : nullptr;  // copied at its end (land_mesh)
