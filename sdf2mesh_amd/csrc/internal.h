@@ -104,7 +104,7 @@ constexpr uint32_t kTileBlocksPerCU = 8;    // most k_sp_tiles blocks per comput
 constexpr uint32_t kTileRecBytes = 2720;    // per slot: k_sp_tiles' staged record (sparse.hip)
 constexpr uint32_t kRowChunk = 4096;        // rows per chunk of the row offset scan (sparse.hip)
 constexpr uint32_t kChunkSumStride = 32;    // words between chunk sums (one 128-byte line each)
-constexpr uint32_t kQueues = 2;        // work queues of a pass (k_sp_tiles<1>, k_sp_tiles<0>)
+constexpr uint32_t kQueues = 4;        // work queues of a pass (k_sp_tiles<1/0>, k_sp_emit<1/0>)
 constexpr uint32_t kQueueGroups = 64;  // counters per queue, 32 u32 (128 bytes) apart
 // Profiling marks of one sparse pass: prune (tiles, bricks) | eval+contour | quad count |
 // scan | emission

@@ -84,6 +84,17 @@ __device__ __forceinline__ uint32_t queue_take(const SpPass& P, uint32_t q, uint
     return (uint32_t)(slot < 0xffffffffull ? slot : 0xffffffffull);
 }
 
+// Neighbouring slots are mostly neighbouring tiles: runs of kTurnRun of them go to one XCD (the
+// hardware deals blocks to XCDs in turn), so rows and output lines they share stay in one L2.
+// Slot of draw `j` of group g; increasing in j, every slot once.
+constexpr uint32_t kTurnRun = 16;
+__device__ __forceinline__ uint32_t turn_of(uint32_t j, uint32_t g, uint32_t G)
+{
+    if (G != kQueueGroups) return j * G + g;
+    const uint32_t m = j * (kQueueGroups / 8u) + (g >> 3);
+    return ((m / kTurnRun) * 8u + (g & 7u)) * kTurnRun + m % kTurnRun;
+}
+
 // Row segment of row (zl, y) and tile column tx of job J.
 // Per-slot row data: array k (kRowVtx, kRowTri: counts; kRowVtxOff, kRowTriOff: first
 // vertex / triangle of the row segment within its row) of slot `slot`, row r = (z % 8) * 8
@@ -144,21 +155,24 @@ __device__ uint32_t nb_row(const SpPass& P, const SpJob& J, uint32_t tx, uint32_
     const uint32_t zl = (uint32_t)z - J.z0;
     const uint32_t nsel = ((tz - ((uint32_t)z >> 3)) * 2u + (ty - ((uint32_t)y >> 3))) * 2u;
     const uint32_t r = ((uint32_t)z & 7u) * 8u + ((uint32_t)y & 7u);
-    for (uint32_t c = 0; c < 2; ++c) {  // c = 0: the tile column's own cells, 1: the cell before it
-        const int32_t slot = ns[nsel + c];
-        if (slot < 0) continue;
-        const uint32_t b8 = slot_row_bits(P, slot, r);
-        if (c ? !(b8 & 0x80u) : !b8) continue;
-        bits |= c ? 1u : b8 << 1;
-        if (INDEX) {
-            const uint32_t first = slot_row(P, kRowVtxOff, (uint32_t)slot)[r] + P.row_off[row_index(J, zl, (uint32_t)y)];
-            if (c) {
-                idx[0] = first + (uint32_t)__builtin_popcount(b8 & 0x7fu);
-            } else {
-                for (uint32_t i = 0; i < 8; ++i)
-                    if ((b8 >> i) & 1u) idx[i + 1] = first + (uint32_t)__builtin_popcount(b8 & ((1u << i) - 1u));
-            }
-        }
+    // the tile column's own cells and the cell before it; every load without a branch (slot 0
+    // for a tile without one), so that they are in flight together
+    const int32_t s0 = ns[nsel], s1 = ns[nsel + 1u];
+    const int32_t a0 = max(s0, 0), a1 = max(s1, 0);
+    uint32_t b0 = slot_row_bits(P, a0, r), b1 = slot_row_bits(P, a1, r);
+    uint32_t f0 = 0, f1 = 0;
+    if (INDEX) {
+        const uint32_t row = P.row_off[row_index(J, zl, (uint32_t)y)];
+        f0 = slot_row(P, kRowVtxOff, (uint32_t)a0)[r] + row;
+        f1 = slot_row(P, kRowVtxOff, (uint32_t)a1)[r] + row;
+    }
+    b0 = s0 < 0 ? 0u : b0;
+    b1 = s1 < 0 ? 0u : b1;
+    bits = b0 << 1 | b1 >> 7;
+    if (INDEX) {
+        if (b1 & 0x80u) idx[0] = f1 + (uint32_t)__builtin_popcount(b1 & 0x7fu);
+        for (uint32_t i = 0; i < 8; ++i)
+            if ((b0 >> i) & 1u) idx[i + 1] = f0 + (uint32_t)__builtin_popcount(b0 & ((1u << i) - 1u));
     }
     return bits;
 }
@@ -1418,6 +1432,14 @@ __global__ __launch_bounds__(64) void k_sp_quadcount(SpPass P, MeshBufs b)
 // Triangle vertex indices are relative to the job's first vertex.  LINEAR = 1 handles the
 // slots whose program is a left fold, LINEAR = 0 the others (launched only when a program
 // of the pass is not a left fold; its stack interpreter needs more registers).
+//
+// A slot is a chain of dependent loads (header, neighbours' rows, staged vertices, tape), four
+// folds per vertex and scattered stores of rows a few vertices long: bound by latency and by
+// instruction issue alike (half of the issue slots), the 228 MB of a CSG-64 1024^3 mesh take
+// 50 us at copy speed.  So the loads of a slot are issued together (no branch between them),
+// rows are stored 8 bytes at a time, and blocks draw slots: with slots dealt out in advance
+// a block's share of vertices varies twofold and half of the waves idled at the end.
+// 325 -> 243 us there (69 k slots, 4.0 M vertices).
 // ---------------------------------------------------------------------------------
 // Block 0 of k_sp_emit<1> after a job's last pass: the statistics summed and
 // counters[0 .. nback) to P.back (mapped host memory, NULL: not wanted).  Nothing in the
@@ -1444,9 +1466,16 @@ __global__ __launch_bounds__(64) void k_sp_emit(SpPass P, MeshBufs b)
     extern __shared__ float taps[];  // their operand stacks: P.prune_depth entries of 4 per lane
     __shared__ uint32_t nb[729];  // vertex of cell (8tx-1+i, 8ty-1+j, 8tz-1+k) at nb[(k*9+j)*9+i]
     __shared__ uint32_t tc[128];  // triangles of cell c in byte c % 4 of tc[c / 4]
+    __shared__ uint32_t trow[64];  // first triangle of row segment c >> 3
     if (LINEAR && blockIdx.x == 0) report(P);
     const uint32_t nslots = active_slots(P, LINEAR ? kSlotsNow : kGenNow);
-    for (uint32_t turn = blockIdx.x; turn < nslots; turn += gridDim.x) {
+    // the first turn is the block's own, the others are drawn, one ahead
+    const uint32_t G = min(kQueueGroups, gridDim.x), g = blockIdx.x % G;
+    uint32_t* const queue = P.queues + ((LINEAR ? 2u : 3u) * kQueueGroups + g) * 32u;
+    const uint32_t own = (gridDim.x - g + G - 1u) / G;  // blocks of the group
+    uint32_t turn = turn_of(blockIdx.x / G, g, G), drawn = 0;
+    for (; turn < nslots; turn = turn_of(own + (uint32_t)__builtin_amdgcn_readfirstlane(drawn), g, G)) {
+        if (thread_id() == 0) drawn = atomicAdd(queue, 1u);
         const uint32_t slot = LINEAR ? turn : P.gen_slots[turn];
         const SlotHdr& H = P.slot_hdr[slot];
         const uint64_t tile = __builtin_amdgcn_readfirstlane(H.tile);
@@ -1477,18 +1506,27 @@ __global__ __launch_bounds__(64) void k_sp_emit(SpPass P, MeshBufs b)
         int32_t ns[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) ns[i] = P.slot_nb[(size_t)slot * 8u + i];
+        // the first round's vertex and the segments' triangle offsets, read beside the rows
+        float4 e0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (thread_id() < n && (uint64_t)base + thread_id() < P.stage_cap) e0 = P.stage[(uint64_t)base + thread_id()];
+        {
+            const uint32_t r = thread_id(), zl = tzl * 8u + (r >> 3), y = ty * 8u + (r & 7u);
+            uint32_t t = 0;
+            if (zl < J.nz && y < J.ry)
+                t = slot_row(P, kRowTriOff, slot)[r] + P.row_off[P.nrows + row_index(J, zl, y)];
+            trow[r] = t;
+        }
         for (uint32_t t = thread_id(); t < 81u; t += 64u)
             (void)nb_row<true>(P, J, tx, ty, J.tz0 + tzl, ns, (int)(ty * 8u + t % 9u) - 1,
                                (int)(J.z0 + tzl * 8u + t / 9u) - 1, nb + 9u * t);
         for (uint32_t w = thread_id(); w < 128u; w += 64u) tc[w] = 0;
         __syncthreads();
-        // vertices, and each cell's triangle count (the first round's cell, quads and row
-        // triangle offset are kept for the triangle loop)
-        uint32_t meta0 = 0, nq0 = 0;
-        uint64_t trow0 = 0;
+        // vertices, and each cell's triangle count (the first round's quads are kept for the
+        // triangle loop)
+        uint32_t nq0 = 0;
         for (uint32_t k = thread_id(); k < n; k += 64u) {
             if ((uint64_t)base + k >= P.stage_cap) break;
-            const float4 e = P.stage[(uint64_t)base + k];
+            const float4 e = k == thread_id() ? e0 : P.stage[(uint64_t)base + k];
             const uint32_t meta = __float_as_uint(e.w);
             const uint32_t c = meta & 511u, sg = meta >> 12;
             const uint32_t cxl = c & 7u, cyl = (c >> 3) & 7u, czl = c >> 6;
@@ -1498,24 +1536,17 @@ __global__ __launch_bounds__(64) void k_sp_emit(SpPass P, MeshBufs b)
             const uint32_t nq =
                 cell_quads(sg, tx * 8u + cxl, ty * 8u + cyl, J.z0 + tzl * 8u + czl, lag, exists, invalid);
             if (nq) atomicOr(&tc[c >> 2], (2u * (uint32_t)__builtin_popcount(nq)) << ((c & 3u) * 8u));
-            if (k == thread_id()) {
-                meta0 = meta;
-                nq0 = nq;
-                if (nq)
-                    trow0 = (uint64_t)slot_row(P, kRowTriOff, slot)[c >> 3] +
-                            P.row_off[P.nrows + row_index(J, tzl * 8u + czl, ty * 8u + cyl)];
-            }
+            if (k == thread_id()) nq0 = nq;
             const uint64_t vi = nb[at];
             if (vi >= b.vcap) continue;
-            float* o = b.vtx + 6 * vi;
-            o[0] = e.x;
-            o[1] = e.y;
-            o[2] = e.z;
+            float2* o = reinterpret_cast<float2*>(b.vtx + 6 * vi);
+            o[0] = make_float2(e.x, e.y);
             b.keys[vi] = (uint64_t)(tx * 8u + cxl) | ((uint64_t)(ty * 8u + cyl) << 16) |
                          ((uint64_t)(J.z0 + tzl * 8u + czl) << 32);
             b.signs[vi] = (uint8_t)sg;
             if (!normals) {
-                o[3] = o[4] = o[5] = 0.0f;
+                o[1] = make_float2(e.z, 0.0f);
+                o[2] = make_float2(0.0f, 0.0f);
                 continue;
             }
             const float px = e.x, py = e.y, pz = e.z, eps = J.eps;
@@ -1542,28 +1573,26 @@ __global__ __launch_bounds__(64) void k_sp_emit(SpPass P, MeshBufs b)
             const float gy = (((-d1) + (-d2)) + d3) + d4;
             const float gz = (((-d1) + d2) + (-d3)) + d4;
             const float ln = sqrtf((gx * gx + gy * gy) + gz * gz);
-            o[3] = canonical_nan(gx / ln);
-            o[4] = canonical_nan(gy / ln);
-            o[5] = canonical_nan(gz / ln);
+            o[1] = make_float2(e.z, canonical_nan(gx / ln));
+            o[2] = make_float2(canonical_nan(gy / ln), canonical_nan(gz / ln));
         }
         __syncthreads();  // every cell's triangle count is in tc
         // triangles, in vertex order: each quad (q2, q1, q0), (q0, q3, q2)
         for (uint32_t k = thread_id(); k < n; k += 64u) {
             if ((uint64_t)base + k >= P.stage_cap) break;
             const bool first = k == thread_id();
-            const uint32_t meta = first ? meta0 : __float_as_uint(P.stage[(uint64_t)base + k].w);
+            const uint32_t meta = __float_as_uint(first ? e0.w : P.stage[(uint64_t)base + k].w);
             const uint32_t c = meta & 511u, sg = meta >> 12;
             const uint32_t cxl = c & 7u, cyl = (c >> 3) & 7u, czl = c >> 6;
             const uint32_t at = ((czl + 1) * 9u + (cyl + 1)) * 9u + (cxl + 1);
             auto nbv = [&](int dx, int dy, int dz) { return nb[(int)at + (dz * 9 + dy) * 9 + dx]; };
             auto exists = [&](int dx, int dy, int dz) { return nbv(dx, dy, dz) != kNone; };
             uint32_t invalid = 0;
-            const uint32_t y = ty * 8u + cyl, zl = tzl * 8u + czl;
-            const uint32_t nq = first ? nq0 : cell_quads(sg, tx * 8u + cxl, y, J.z0 + zl, lag, exists, invalid);
+            const uint32_t nq = first ? nq0 : cell_quads(sg, tx * 8u + cxl, ty * 8u + cyl, J.z0 + tzl * 8u + czl, lag,
+                                                         exists, invalid);
             if (!nq) continue;
             const uint64_t row2 = ((uint64_t)tc[(c >> 3) * 2u + 1] << 32) | tc[(c >> 3) * 2u];  // 8 counts
-            uint64_t t = first ? trow0
-                               : (uint64_t)slot_row(P, kRowTriOff, slot)[c >> 3] + P.row_off[P.nrows + row_index(J, zl, y)];
+            uint64_t t = trow[c >> 3];
             for (uint32_t i = 0; i < cxl; ++i) t += (row2 >> (8u * i)) & 0xffu;
             const uint32_t v = nbv(0, 0, 0);
             const bool c0 = sg & 1u, c1 = (sg >> 1) & 1u, c2 = (sg >> 2) & 1u;
@@ -1582,13 +1611,11 @@ __global__ __launch_bounds__(64) void k_sp_emit(SpPass P, MeshBufs b)
                 uint32_t qv[4];
                 for (int i = 0; i < 4; ++i) qv[i] = (rev ? f[3 - i] : f[i]) - vbase;
                 if (t + 1 < b.tcap) {
-                    uint32_t* o = b.tri + 3 * t;
-                    o[0] = qv[2];
-                    o[1] = qv[1];
-                    o[2] = qv[0];
-                    o[3] = qv[0];
-                    o[4] = qv[3];
-                    o[5] = qv[2];
+                    // t is even: triangles come in pairs
+                    uint2* o = reinterpret_cast<uint2*>(b.tri + 3 * t);
+                    o[0] = make_uint2(qv[2], qv[1]);
+                    o[1] = make_uint2(qv[0], qv[0]);
+                    o[2] = make_uint2(qv[3], qv[2]);
                 }
                 t += 2;
             }
