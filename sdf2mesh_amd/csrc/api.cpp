@@ -145,8 +145,8 @@ struct s2m_ctx {
     };
     PassSet pset[2];
     DevBuf vtx, keys, signs, tri, corners;
-    DevBuf tile_tab, tile_lists, tile_lens, tile_flops;
-    DevBuf sp_slot_of_tile, sp_tile_of_slot, sp_job_of_slot, sp_gen_slots, sp_cellbits, sp_slot_rows, sp_boundary;
+    DevBuf tile_tab, tile_lists, sp_slot_info;
+    DevBuf sp_gen_slots, sp_cellbits, sp_slot_rows, sp_boundary;
     DevBuf sp_stage, sp_slot_nb, sp_slot_stage, sp_slot_live, sp_slot_hdr, sp_slot_rec;
     DevBuf sp_queues, sp_super_iv, sp_super_lists, sp_super_act, sp_rows;
     bool sp_dirty = false;  // a sparse pass was not queued to its end: `counters` may not be zero
@@ -1027,10 +1027,11 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
             layers = (tabs[0].nt[2] + passes - 1) / passes;
         }
         layers = std::min(layers, std::max<uint32_t>(tabs[0].nt[2], 1));
-        const uint64_t slot = kTileRecBytes + 16 * 68 + sizeof(SlotHdr) + 64;  // a quarter of the tiles get one
+        // per slot (a quarter of the tiles get one)
+        const uint64_t slot = kTileRecBytes + 16 * 68 + sizeof(SlotHdr) + 64 + 2 * list_stride;
         auto pass_bytes = [&](uint64_t L) {
             const uint64_t t = (uint64_t)tabs[0].nt[0] * tabs[0].nt[1] * L;
-            return t * (list_stride * 2 + 12 + slot / 4) + 16ull * L * kTile * jobs[0].res[1];
+            return t * (slot / 4 + (list_stride > kStageOps ? 2 * list_stride : 0)) + 16ull * L * kTile * jobs[0].res[1];
         };
         auto pass_fits = [&](uint64_t L) {
             return pass_bytes(L) <= kSparsePassBytes &&
@@ -1142,10 +1143,6 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
     }
     const SpJob* ddesc = reinterpret_cast<const SpJob*>(dimg + desc_off);
 
-    HIP_TRY(ctx->tile_lists.ensure(tiles_pass * list_stride * sizeof(uint16_t)));
-    HIP_TRY(ctx->tile_lens.ensure(tiles_pass * sizeof(uint32_t)));
-    HIP_TRY(ctx->tile_flops.ensure(tiles_pass * sizeof(uint32_t)));
-    HIP_TRY(ctx->sp_slot_of_tile.ensure(tiles_pass * sizeof(int32_t)));
     HIP_TRY(ctx->sp_rows.ensure(std::max<uint64_t>(nrows_pass, 1) * 4 * sizeof(uint32_t)));
     const uint32_t nsb_max = (uint32_t)((nrows_pass + kRowChunk - 1) / kRowChunk) + 1;  // vertex and triangle sums
     HIP_TRY(ctx->bcount.ensure((size_t)2 * nsb_max * kChunkSumStride * sizeof(uint32_t)));
@@ -1160,11 +1157,12 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
     }
     HIP_TRY(ctx->sp_queues.ensure((size_t)kQueues * kQueueGroups * 32 * sizeof(uint32_t)));
     const uint64_t nsup_alloc = std::max<uint64_t>(nsuper_pass, 1);
+    const bool lists_by_tile = list_stride > kStageOps;
     if (list_stride > kStageOps) {  // super-tile lists and intervals that do not fit LDS
         HIP_TRY(ctx->sp_super_iv.ensure(nsup_alloc * list_stride * 2 * sizeof(float)));
         HIP_TRY(ctx->sp_super_lists.ensure(nsup_alloc * list_stride * sizeof(uint16_t)));
     }
-    HIP_TRY(ctx->sp_super_act.ensure(nsup_alloc * sizeof(uint64_t)));
+    HIP_TRY(ctx->sp_super_act.ensure(nsup_alloc * sizeof(SuperSlots)));
 
     // a closed surface crosses O(res^2) cells: start from 6 per row-plane cell
     const uint64_t est_v = std::min<uint64_t>(cells_all, std::max<uint64_t>(65536, 6 * planes_sum));
@@ -1184,8 +1182,8 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
         HIP_TRY(ctx->keys.ensure(want_v * sizeof(uint64_t)));
         HIP_TRY(ctx->signs.ensure(want_v));
         HIP_TRY(ctx->tri.ensure(want_t * 3 * sizeof(uint32_t)));
-        HIP_TRY(ctx->sp_tile_of_slot.ensure(want_s * sizeof(uint32_t)));
-        HIP_TRY(ctx->sp_job_of_slot.ensure(want_s * sizeof(uint32_t)));
+        HIP_TRY(ctx->tile_lists.ensure((lists_by_tile ? tiles_pass : want_s) * list_stride * sizeof(uint16_t)));
+        HIP_TRY(ctx->sp_slot_info.ensure(want_s * sizeof(uint4)));
         HIP_TRY(ctx->sp_gen_slots.ensure(want_s * sizeof(uint32_t)));
         HIP_TRY(ctx->sp_cellbits.ensure(want_s * 16 * sizeof(uint32_t)));
         HIP_TRY(ctx->sp_slot_rows.ensure(want_s * 4 * 64 * sizeof(uint32_t)));
@@ -1258,11 +1256,8 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
                 P.nsuper = nsuper_pass;
             }
             P.lists = ctx->tile_lists.as<uint16_t>();
-            P.lens = ctx->tile_lens.as<uint32_t>();
-            P.flops = ctx->tile_flops.as<uint32_t>();
-            P.slot_of_tile = ctx->sp_slot_of_tile.as<int32_t>();
-            P.tile_of_slot = ctx->sp_tile_of_slot.as<uint32_t>();
-            P.job_of_slot = ctx->sp_job_of_slot.as<uint32_t>();
+            P.lists_by_tile = lists_by_tile ? 1u : 0u;
+            P.slot_info = ctx->sp_slot_info.as<uint4>();
             P.gen_slots = ctx->sp_gen_slots.as<uint32_t>();
             P.slot_cap = (uint32_t)want_s;
             P.box_stride = box_stride;
@@ -1281,7 +1276,7 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
             P.queues = ctx->sp_queues.as<uint32_t>();
             P.super_iv = ctx->sp_super_iv.as<float2>();
             P.super_lists = ctx->sp_super_lists.as<uint16_t>();
-            P.super_act = ctx->sp_super_act.as<uint64_t>();
+            P.super_act = ctx->sp_super_act.as<SuperSlots>();
             P.job_out = job_out;
             hipEvent_t m[kSparseMarks] = {};
             if (ctx->profiling >= 2)
@@ -1322,9 +1317,8 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
             std::string key(reinterpret_cast<const char*>(img), img_bytes);
             auto put = [&key](const void* q, size_t m) { key.append(static_cast<const char*>(q), m); };
             for (const DevBuf* d : {&ctx->vtx, &ctx->keys, &ctx->signs, &ctx->tri, &ctx->counters, &ctx->bcount,
-                                    &ctx->sp_queues, &ctx->tile_tab, &ctx->tile_lists,
-                                    &ctx->tile_lens, &ctx->tile_flops, &ctx->sp_slot_of_tile, &ctx->sp_tile_of_slot,
-                                    &ctx->sp_job_of_slot, &ctx->sp_gen_slots, &ctx->sp_cellbits, &ctx->sp_stage, &ctx->sp_slot_stage,
+                                    &ctx->sp_queues, &ctx->tile_tab, &ctx->tile_lists, &ctx->sp_slot_info,
+                                    &ctx->sp_gen_slots, &ctx->sp_cellbits, &ctx->sp_stage, &ctx->sp_slot_stage,
                                     &ctx->sp_slot_live, &ctx->sp_slot_hdr, &ctx->sp_slot_nb, &ctx->sp_slot_rec,
                                     &ctx->sp_slot_rows, &ctx->sp_rows, &ctx->sp_super_iv, &ctx->sp_super_lists,
                                     &ctx->sp_super_act, &ctx->sp_boundary})
@@ -1970,9 +1964,8 @@ void s2m_destroy(s2m_ctx* ctx)
     (void)hipStreamSynchronize(ctx->eval_stream);
     for (DevBuf* b : {&ctx->lattice, &ctx->dense, &ctx->bcount, &ctx->check, &ctx->counters,
                       &ctx->tables, &ctx->vtx, &ctx->keys, &ctx->signs, &ctx->tri, &ctx->corners,
-                      &ctx->tile_tab, &ctx->tile_lists, &ctx->tile_lens,
-                      &ctx->tile_flops, &ctx->sp_slot_of_tile, &ctx->sp_tile_of_slot,
-                      &ctx->sp_job_of_slot, &ctx->sp_gen_slots, &ctx->sp_cellbits, &ctx->sp_slot_rows,
+                      &ctx->tile_tab, &ctx->tile_lists, &ctx->sp_slot_info,
+                      &ctx->sp_gen_slots, &ctx->sp_cellbits, &ctx->sp_slot_rows,
                       &ctx->sp_boundary, &ctx->sp_queues, &ctx->sp_super_iv,
                       &ctx->sp_super_lists, &ctx->sp_super_act, &ctx->sp_rows,
                       &ctx->sp_stage, &ctx->sp_slot_nb, &ctx->sp_slot_stage, &ctx->sp_slot_live, &ctx->sp_slot_hdr, &ctx->sp_slot_rec})

@@ -155,6 +155,13 @@ struct SlotHdr {
     uint32_t box[3]; // per axis: first lattice index of the tile's box | points << 24
 };
 
+// The slots of a super-tile's tiles: bit (z * 4 + y) * 4 + x of `act` says that the tile has one,
+// and they are numbered from `first` in bit order.
+struct SuperSlots {
+    uint64_t act;
+    uint32_t first, unused;
+};
+
 struct SpPass {
     const SpJob* jobs;
     uint32_t njobs;
@@ -168,13 +175,11 @@ struct SpPass {
     uint64_t nsuper;           // super-tiles of the pass
     float2* super_iv;         // [super-tile][list_stride] primitive intervals (lo, hi), and pruned op
     uint16_t* super_lists;     // indices, of programs too long for LDS (kStageOps; NULL if none is)
-    uint64_t* super_act;       // [super-tile] bit (z * 4 + y) * 4 + x: that tile has a slot
-    uint16_t* lists;           // [tile][list_stride] pruned op indices
-    uint32_t* lens;            // [tile]
-    uint32_t* flops;           // [tile] flops per point of the pruned tape
-    int32_t* slot_of_tile;     // [tile], -1: no active cell
-    uint32_t* tile_of_slot;    // [slot]
-    uint32_t* job_of_slot;     // [slot]
+    SuperSlots* super_act;     // [super-tile]
+    uint16_t* lists;           // [slot][list_stride] pruned op indices ([tile] with lists_by_tile: programs
+                               // longer than kStageOps are listed before their tile has a slot)
+    uint32_t lists_by_tile;
+    uint4* slot_info;          // [slot] tile, job, pruned length (| kLinearFlag), its flops per point
     uint32_t* gen_slots;       // the slots whose program is no fold (kGenUsed of them)
     uint32_t slot_cap;
     uint32_t box_stride;       // floats of a tile's lattice box (LDS)

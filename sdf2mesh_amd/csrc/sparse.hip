@@ -121,6 +121,22 @@ __device__ __forceinline__ void tile_xyz(const SpJob& J, uint64_t tile, uint32_t
     tzl = t / (J.ntx * J.nty);
 }
 
+// The slot of tile (tx, ty, tile layer tzl of the pass) of job J, -1 without one.
+__device__ __forceinline__ int32_t slot_at(const SpPass& P, const SpJob& J, uint32_t tx, uint32_t ty, uint32_t tzl)
+{
+    static_assert(kSuper == 4, "64 tiles per super-tile");
+    const SuperSlots S = P.super_act[J.super_base + ((uint64_t)(tzl >> 2) * J.nsy + (ty >> 2)) * J.nsx + (tx >> 2)];
+    const uint32_t bit = ((tzl & 3u) * 4u + (ty & 3u)) * 4u + (tx & 3u);
+    if (!((S.act >> bit) & 1ull)) return -1;
+    return (int32_t)(S.first + (uint32_t)__builtin_popcountll(S.act & ((1ull << bit) - 1ull)));
+}
+
+// The pruned op indices of a slot.
+__device__ __forceinline__ uint16_t* slot_list(const SpPass& P, uint32_t slot, uint64_t tile)
+{
+    return P.lists + (size_t)(P.lists_by_tile ? tile : slot) * P.list_stride;
+}
+
 // Existence bits of row r (= z % 8 * 8 + y % 8) of a tile with a slot: bit x % 8.
 __device__ __forceinline__ uint32_t slot_row_bits(const SpPass& P, int32_t slot, uint32_t r)
 {
@@ -183,9 +199,7 @@ __device__ __forceinline__ uint32_t vertex_at(const SpPass& P, const SpJob& J, u
                                               uint32_t z)
 {
     if (z < J.z0) return J.boundary[(size_t)y * J.rx + x];
-    const uint64_t tile =
-        J.tile_base + ((uint64_t)((z >> 3) - J.tz0) * J.nty + (y >> 3)) * J.ntx + (x >> 3);
-    const int32_t slot = P.slot_of_tile[tile];
+    const int32_t slot = slot_at(P, J, x >> 3, y >> 3, (z >> 3) - J.tz0);
     if (slot < 0) return kNone;
     const uint32_t b8 = slot_row_bits(P, slot, (z & 7u) * 8u + (y & 7u)), i = x & 7u;
     if (!((b8 >> i) & 1u)) return kNone;
@@ -362,6 +376,51 @@ struct FoldWalk {
         }
     }
 
+    __device__ __forceinline__ bool one_sign() const { return top.known && (top.lo > 0.0f || top.hi < 0.0f); }
+};
+
+// FoldWalk for a staged list (at most kStageOps ops): the kept primitives (each with the operator
+// behind it) as a bit mask in place of a list, bit (q + 1) / 2 for the primitive at position q;
+// the list is written once the tile has a slot.
+struct FoldMask {
+    Iv top = iv_unknown();
+    uint64_t kept = 0;
+    uint32_t top_sum = 0;
+    Iv b = iv_unknown();
+    uint32_t b_sum = 0;
+
+    __device__ __forceinline__ void prim(uint32_t q, const Iv& v, uint32_t sum)
+    {
+        static_assert(kStageOps <= 128, "one bit per primitive");
+        if (q == 0) {
+            top = v;
+            top_sum = sum;
+            kept = 1ull;
+        } else {
+            b = v;
+            b_sum = sum;
+        }
+    }
+
+    // The operator at position q >= 2.
+    __device__ __forceinline__ void op(uint32_t q, uint32_t code, float k, uint32_t fl)
+    {
+        int keep;
+        const Iv r = iv_op(code, top, b, k, keep);
+        const uint64_t bit = 1ull << (q >> 1);
+        if (keep == kKeepBoth) {
+            kept |= bit;
+            const bool fold = (top_sum & kFoldBit) && (b_sum & kFoldBit);
+            top_sum = ((top_sum & ~kFoldBit) + (b_sum & ~kFoldBit) + fl) | (fold ? kFoldBit : 0u);
+            top = r;
+        } else if (keep != kKeepA) {  // the list is the primitive
+            kept = bit;
+            top = b;
+            top_sum = b_sum;
+        }
+    }
+
+    __device__ __forceinline__ uint32_t len() const { return 2u * (uint32_t)__builtin_popcountll(kept) - 1u; }
     __device__ __forceinline__ bool one_sign() const { return top.known && (top.lo > 0.0f || top.hi < 0.0f); }
 };
 
@@ -632,15 +691,20 @@ __global__ __launch_bounds__(64) void k_sp_prune(SpPass P)
     }
     __syncthreads();
     bool surface = false;
-    uint32_t lens = 0;
-    if (valid && sl == kSingleSign) {  // no surface anywhere in the super-tile
-        P.lens[tile] = 0;
-        P.flops[tile] = 0;
-    } else if (valid) {
+    uint32_t lens = 0, flops = 0;
+    uint64_t kept = 0;  // the tile's list of a staged fold (FoldMask)
+    const LdsList list{reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(prune_lds) + PruneStack::bytes(D)), ln};
+    const bool in_lds = !J.left_fold && J.nops <= P.walk_ops;
+    if (valid && sl != kSingleSign) {
         const uint32_t tt[3] = {tx, ty, tz};
         float bl[3], bh[3];
         tiles_box(J, tt, tt, bl, bh);
-        uint16_t* L = P.lists + (size_t)tile * P.list_stride;
+        auto done = [&](bool one_sign, uint32_t len, uint32_t sum) {
+            // the pruned program is one subtree: its flops and whether it is a left fold
+            surface = !one_sign;
+            lens = len | (surface && (sum & kFoldBit) && len <= kStageOps ? kLinearFlag : 0u);
+            flops = sum & ~kFoldBit;
+        };
         auto walk = [&](auto& w, auto L) {
             if (staged) {  // every lane walks the same list: wave-uniform dispatch
                 for (uint32_t q = 0; q < sl; ++q) {
@@ -656,25 +720,26 @@ __global__ __launch_bounds__(64) void k_sp_prune(SpPass P)
                     else w.op(i, code, ops[i].f[0], L, S, ln, sum);
                 }
             }
-            surface = !w.one_sign();
-            // the pruned program is one subtree: its flops and whether it is a left fold
-            const bool fold = (w.top_sum & kFoldBit) && w.len <= kStageOps;
-            lens = w.len | (surface && fold ? kLinearFlag : 0u);
-            P.lens[tile] = lens;
-            P.flops[tile] = w.top_sum & ~kFoldBit;
+            done(w.one_sign(), w.len, w.top_sum);
         };
-        if (J.left_fold) {  // the super-tile's list is a left fold too
+        if (J.left_fold && staged) {  // the super-tile's list is a left fold too
+            FoldMask w;
+            for (uint32_t q = 0; q < sl; ++q) {
+                const uint32_t code = uniform_code(T, q), sum = sums[q];
+                if (code < S2M_OP_UNION) w.prim(q, iv_primitive(code, T.f[q], bl, bh), sum);
+                else w.op(q, code, T.f[q][0], sum);
+            }
+            done(w.one_sign(), w.len(), w.top_sum);
+            kept = w.kept;
+        } else if (J.left_fold) {
             FoldWalk w;
-            walk(w, L);
-        } else if (J.nops <= P.walk_ops) {
+            walk(w, P.lists + (size_t)tile * P.list_stride);
+        } else if (in_lds) {
             PruneWalk<true> w;
-            const LdsList list{reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(prune_lds) + PruneStack::bytes(D)), ln};
             walk(w, list);
-            if (surface)
-                for (uint32_t q = 0; q < w.len; ++q) L[q] = list[q];
         } else {
             PruneWalk<true> w;
-            walk(w, L);
+            walk(w, P.lists + (size_t)tile * P.list_stride);
         }
     }
     // slots for the surviving tiles: one counter update per wave
@@ -687,11 +752,23 @@ __global__ __launch_bounds__(64) void k_sp_prune(SpPass P)
         const uint64_t sidx = wbase + (uint64_t)__builtin_popcountll(m & ((1ull << ln) - 1ull));
         if (sidx < P.slot_cap) {
             slot = (int32_t)sidx;
-            P.tile_of_slot[sidx] = (uint32_t)tile;
-            P.job_of_slot[sidx] = jid;
+            P.slot_info[sidx] = make_uint4((uint32_t)tile, jid, lens, flops);
+            uint16_t* L = slot_list(P, (uint32_t)sidx, tile);
+            uint32_t k = 0;
+            for (; kept; kept &= kept - 1ull) {
+                const uint32_t q = 2u * (uint32_t)__builtin_ctzll(kept);
+                if (k) {  // the primitive at q - 1 and its operator
+                    L[k] = idx[q - 1u];
+                    L[k + 1] = idx[q];
+                    k += 2;
+                } else {
+                    L[k++] = idx[q ? q - 1u : 0u];
+                }
+            }
+            if (in_lds)
+                for (uint32_t q = 0; q < (lens & ~kLinearFlag); ++q) L[q] = list[q];
         }
     }
-    if (valid) P.slot_of_tile[tile] = slot;
     // the slots that are no folds, listed for k_sp_tiles<0> and k_sp_emit<0>
     const uint64_t g = __ballot(slot >= 0 && !(lens & kLinearFlag));
     if (g) {
@@ -701,8 +778,7 @@ __global__ __launch_bounds__(64) void k_sp_prune(SpPass P)
         if ((g >> ln) & 1ull) P.gen_slots[gbase + (uint64_t)__builtin_popcountll(g & ((1ull << ln) - 1ull))] = (uint32_t)slot;
     }
     const uint64_t act = __ballot(slot >= 0);  // bit l: tile l of the super-tile has a slot
-    if (ln == 0) P.super_act[s] = act;
-
+    if (ln == 0) P.super_act[s] = SuperSlots{act, (uint32_t)wbase, 0u};
 }
 
 // Per-axis corner tables of a tile's 8 cells: box-relative lattice index and coordinate
@@ -783,33 +859,21 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
     __shared__ StagedFold T;
     __shared__ TileAxes A;
     const uint32_t nslots = active_slots(P);
-    // The slots' tile, job and list length are read ahead (tile and job two slots ahead,
-    // the length one slot ahead) with per-lane loads, which barriers do not wait for.
+    // The slots' tile, job and list length are read two slots ahead with per-lane loads,
+    // which barriers do not wait for.
     const uint32_t z = thread_id() & 0u;  // a per-lane zero: vector loads
     const uint32_t G = gridDim.x;
-    uint32_t t1 = 0, j1 = 0, l1 = 0, t2 = 0, j2 = 0;
-    if (blockIdx.x < nslots) {
-        t1 = P.tile_of_slot[blockIdx.x + z];
-        j1 = P.job_of_slot[blockIdx.x + z];
-        l1 = P.lens[__builtin_amdgcn_readfirstlane(t1) + z];
-    }
-    if (blockIdx.x + G < nslots) {
-        t2 = P.tile_of_slot[blockIdx.x + G + z];
-        j2 = P.job_of_slot[blockIdx.x + G + z];
-    }
+    uint4 i1 = make_uint4(0u, 0u, 0u, 0u), i2 = i1;
+    if (blockIdx.x < nslots) i1 = P.slot_info[blockIdx.x + z];
+    if (blockIdx.x + G < nslots) i2 = P.slot_info[blockIdx.x + G + z];
     for (uint32_t slot = blockIdx.x; slot < nslots; slot += G) {
         const uint32_t b = thread_id();
-        const uint64_t tile = __builtin_amdgcn_readfirstlane(t1);
-        const uint32_t lens = __builtin_amdgcn_readfirstlane(l1);
+        const uint64_t tile = __builtin_amdgcn_readfirstlane(i1.x);
+        const uint32_t lens = __builtin_amdgcn_readfirstlane(i1.z);
         const uint32_t n = lens & ~kLinearFlag;
-        const uint32_t jid = __builtin_amdgcn_readfirstlane(j1);
-        t1 = t2;
-        j1 = j2;
-        if (slot + G < nslots) l1 = P.lens[__builtin_amdgcn_readfirstlane(t1) + z];
-        if (slot + 2u * G < nslots) {
-            t2 = P.tile_of_slot[slot + 2u * G + z];
-            j2 = P.job_of_slot[slot + 2u * G + z];
-        }
+        const uint32_t jid = __builtin_amdgcn_readfirstlane(i1.y);
+        i1 = i2;
+        if (slot + 2u * G < nslots) i2 = P.slot_info[slot + 2u * G + z];
         const SpJob& J = P.jobs[jid];
         uint32_t tx, ty, tzl;
         tile_xyz(J, tile, tx, ty, tzl);
@@ -846,7 +910,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
             const uint32_t i = b - 48u, dx = i & 1u, dy = (i >> 1) & 1u, dz = i >> 2;
             int32_t ns = -1;
             if (tx >= dx && ty >= dy && tzl >= dz)
-                ns = P.slot_of_tile[J.tile_base + ((uint64_t)(tzl - dz) * J.nty + (ty - dy)) * J.ntx + (tx - dx)];
+                ns = slot_at(P, J, tx - dx, ty - dy, tzl - dz);
             P.slot_nb[(size_t)slot * 8u + i] = ns;
         }
         if (!(lens & kLinearFlag) || n > kStageOps) {  // every brick is kept
@@ -854,7 +918,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
             continue;
         }
         __syncthreads();  // the previous slot's readers of T and A are done
-        stage_tape(T, J.ops, P.lists + (size_t)tile * P.list_stride, n);
+        stage_tape(T, J.ops, slot_list(P, slot, tile), n);
         if (b < 24) load_tile_axes(A, J, tx, ty, J.tz0 + tzl, b);
         __syncthreads();
         {  // the record's axes and program (codes and the rows in use)
@@ -1133,7 +1197,7 @@ __device__ __forceinline__ void tiles_body(const SpPass& P)
         const uint64_t tile = __builtin_amdgcn_readfirstlane(H.tile);
         // thread 0's flop count for the block statistics, read now so that the load has
         // landed when the tile ends
-        const uint32_t tile_flops = thread_id() == 0 ? P.flops[tile] : 0u;
+        const uint32_t tile_flops = thread_id() == 0 ? P.slot_info[slot].w : 0u;
         const uint32_t n = lens & ~kLinearFlag;
         const SpJob& J = P.jobs[__builtin_amdgcn_readfirstlane(H.job)];
         const uint32_t txy = __builtin_amdgcn_readfirstlane(H.txy);
@@ -1143,7 +1207,7 @@ __device__ __forceinline__ void tiles_body(const SpPass& P)
         const uint32_t nx = bxh >> 24, ny = byh >> 24, nz = bzh >> 24;
         const TileGrid G = tile_grid(J);
         const uint32_t bx = G.bx, by = G.by;
-        const uint16_t* Lst = P.lists + (size_t)tile * P.list_stride;
+        const uint16_t* Lst = slot_list(P, slot, tile);
         uint64_t lv = ~0ull;
         uint32_t evaluated = 0;
         contour_reset(L);
@@ -1487,7 +1551,7 @@ __global__ __launch_bounds__(64) void k_sp_emit(SpPass P, MeshBufs b)
         const bool normals = !(J.flags & S2M_NO_NORMALS);
         const bool lag = (J.flags & S2M_COMPAT_DROP_LAST_SLICE) != 0;
         const uint32_t vbase = (uint32_t)P.job_out[(size_t)J.out_index * kJobOut + 0];
-        const uint16_t* Lst = P.lists + (size_t)tile * P.list_stride;
+        const uint16_t* Lst = slot_list(P, slot, tile);
         const uint32_t lens = __builtin_amdgcn_readfirstlane(H.lens);
         const uint32_t len = lens & ~kLinearFlag;
         const bool linear = (lens & kLinearFlag) != 0, staged = len <= kStageOps;
@@ -1654,16 +1718,23 @@ __global__ __launch_bounds__(64) void k_sp_rowsum(SpPass P)
     const bool row_ok = zl < J.nz && y < J.ry;
     const uint64_t srow = J.super_base + ((uint64_t)(tzl / kSuper) * J.nsy + ty / kSuper) * J.nsx;
     const uint32_t bit0 = ((tzl % kSuper) * kSuper + ty % kSuper) * kSuper;
-    const uint64_t trow_tile = J.tile_base + ((uint64_t)tzl * J.nty + ty) * J.ntx;  // tile (0, ty, tzl)
     uint32_t sv = 0, st = 0;
     for (uint32_t sx0 = 0; sx0 < J.nsx; sx0 += 16u) {
         // active tiles 4 * sx0 .. 4 * sx0 + 63: lane l < 16 reads super-tile sx0 + l's word
-        uint64_t m = 0;
-        if (lane() < 16u && sx0 + lane() < J.nsx)
-            m = ((P.super_act[srow + sx0 + lane()] >> bit0) & 0xfull) << (4u * lane());
+        // and the slot of the first of its active tiles in this tile row
+        uint64_t mine = 0;
+        uint32_t first = 0;
+        if (lane() < 16u && sx0 + lane() < J.nsx) {
+            const SuperSlots S = P.super_act[srow + sx0 + lane()];
+            mine = ((S.act >> bit0) & 0xfull) << (4u * lane());
+            first = S.first + (uint32_t)__builtin_popcountll(S.act & ((1ull << bit0) - 1ull));
+        }
 #pragma unroll
-        for (int d = 8; d >= 1; d >>= 1) m |= __shfl_xor(m, d, 64);
-        m = __shfl(m, 0, 64);
+        for (int d = 8; d >= 1; d >>= 1) mine |= __shfl_xor(mine, d, 64);
+        const uint32_t m0 = __builtin_amdgcn_readfirstlane((uint32_t)mine);
+        const uint32_t m1 = __builtin_amdgcn_readfirstlane((uint32_t)(mine >> 32));
+        uint64_t m = (uint64_t)m1 << 32 | m0;
+        const uint64_t all = m;
         // the active tiles' row counts (one 256-byte row of each slot), 8 tiles at a time
         while (m) {
             uint32_t slots[8], v[8], t[8];
@@ -1672,9 +1743,10 @@ __global__ __launch_bounds__(64) void k_sp_rowsum(SpPass P)
             for (uint32_t k = 0; k < 8u; ++k) {
                 slots[k] = 0;
                 if (m) {
-                    const uint32_t tx = 4u * sx0 + (uint32_t)__builtin_ctzll(m);
+                    const uint32_t t = (uint32_t)__builtin_ctzll(m), l = t >> 2;
                     m &= m - 1ull;
-                    slots[k] = (uint32_t)__builtin_amdgcn_readfirstlane(P.slot_of_tile[trow_tile + tx]);
+                    slots[k] = (uint32_t)__builtin_amdgcn_readlane((int)first, (int)l) +
+                               (uint32_t)__builtin_popcountll((all >> (4u * l)) & ((1ull << (t & 3u)) - 1ull));
                     nb = k + 1;
                 }
             }
