@@ -185,7 +185,7 @@ struct SpPass {
     uint32_t box_stride;       // floats of a tile's lattice box (LDS)
     uint32_t* cellbits;        // [slot][16] bit c: cell c of the tile has a vertex (row r = c / 8
                                // in byte r % 4 of word r / 4)
-    float4* stage;             // [stage_cap] active cells: position, cell | rank << 9 | signs << 12
+    float4* stage;             // [stage_cap] active cells: position, cell | signs << 12
     uint64_t stage_cap;
     uint32_t* slot_stage;      // [slot][2] first staged cell, staged cells
     uint64_t* slot_live;       // [slot] bricks (2x2x2 cells) that may hold an active cell

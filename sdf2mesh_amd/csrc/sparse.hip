@@ -835,16 +835,10 @@ struct TileGen {  // k_sp_tiles<0>: the same parts, staged per slot
 };
 
 // ---------------------------------------------------------------------------------
-// n / d for n, d < 2^16 with m = ceil(2^32 / d): the error term n * (m*d - 2^32) / 2^32 / d
-// stays below 1/d, so it never reaches the next integer.
-__device__ __forceinline__ uint32_t magic16(uint32_t d)
-{
-    return d <= 1u ? 0u : (uint32_t)((0x100000000ull + d - 1u) / d);
-}
-__device__ __forceinline__ uint32_t div16(uint32_t n, uint32_t d, uint32_t m)
-{
-    return d <= 1u ? n : __umulhi(n, m);
-}
+// n / d for n < 2^16 and d <= 256, r = recip(d): (n + 0.5) / d is at least 1 / (2 d) from an
+// integer, and its error (three roundings of one ulp) below (n + 1) / d * 2^-21.
+__device__ __forceinline__ float recip(uint32_t d) { return __builtin_amdgcn_rcpf((float)d); }
+__device__ __forceinline__ uint32_t div_by(uint32_t n, float r) { return (uint32_t)(((float)n + 0.5f) * r); }
 
 // ---------------------------------------------------------------------------------
 // Bricks: the 4x4x4 blocks of 2x2x2 cells of a tile, brick (bx, by, bz) = bit
@@ -965,22 +959,25 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
 // three steps: the cells whose 8 corners change sign are listed (cells of bricks outside
 // `live` are skipped: their corner values keep one sign and were not evaluated); each
 // listed cell gets its vertex (dualcontour.wgsl:72-131) and sign bits (:57-69); the
-// cells with a vertex are staged compactly for k_sp_emit with their rank in their row
-// segment, their bits go to the slot's `cellbits` and each row segment's count to the
-// slot's kRowVtx row.  Contains barriers.
+// cells with a vertex are staged compactly for k_sp_emit, their bits go to the slot's
+// `cellbits` and each row segment's count to the slot's kRowVtx row.  Contains barriers.
 // ---------------------------------------------------------------------------------
 // Staged cells are allocated in chunks of kStageChunk per block (one counter update per
-// chunk).  Each slot reserves 8 entries per live brick (its cells) when its tile starts,
-// so a slot's cells are contiguous; a chunk with fewer entries left than a slot reserves
-// is abandoned.  Hence at most 2 x (reserved entries) + blocks x kStageChunk are used; the
-// host grows the buffer from the device count if that exceeds it.
+// chunk).  A slot needs room for 8 entries per live brick (its cells) when its tile starts, so
+// that its cells are contiguous, and takes what it has used; a chunk with less room left is
+// abandoned.  Hence at most (staged cells) + (room needed by the slots that open a chunk) +
+// blocks x kStageChunk are used; the host grows the buffer from the device count if that
+// exceeds it.
 constexpr uint32_t kStageChunk = kStageChunkHost;
-constexpr uint32_t kTileThreads = 256;  // threads of a k_sp_tiles block (one tile at a time)
-constexpr int kLinearPoints = 2;        // points per lane sharing each op's decode (left folds)
-constexpr int kGeneralPoints = 4;       // (other programs: a box of up to 1024 points in one round,
+// Threads of a k_sp_tiles block (one tile at a time).  128 would share a tile's fixed work
+// among fewer waves, but then half of the waves fit (the box of the worst tile, 16^3 points,
+// and the rest take 21 KB of LDS: seven blocks per compute unit either way): 318 against 300 us
+// at CSG-64 1024^3, 201 against 153 at 512^3.
+constexpr uint32_t kTileThreads = 256;
+static_assert(kRecVec - kRecPre <= kTileThreads, "one thread per record word past the read-ahead");
+constexpr int kGeneralPoints = 4;       // (k_sp_tiles<0>: a box of up to 1024 points in one round,
 constexpr uint32_t kWideDepth = 8;      // their operand stacks within 32 KB of LDS; deeper ones
                                         // take one point at a time)
-static_assert(kRecVec - kRecPre <= kTileThreads, "one thread per record word past the read-ahead");
 
 struct ContourLds {  // block-shared state of contour_tile (and `cand`, 512 entries: the cells
                      // with a sign change among their corners)
@@ -997,7 +994,8 @@ __device__ __forceinline__ void contour_reset(ContourLds& L)
 }
 
 // Thread 0: staging space for the slot's cells with a vertex, at most `cells` (8 per live
-// brick), from the block's chunk; published by the barriers before contour_tile.
+// brick), from the block's chunk; published by the barriers before contour_tile, which takes
+// what the slot has used from the chunk.
 __device__ __forceinline__ void contour_reserve(const SpPass& P, ContourLds& L, uint32_t cells)
 {
     if (L.left < cells) {
@@ -1005,7 +1003,6 @@ __device__ __forceinline__ void contour_reserve(const SpPass& P, ContourLds& L, 
         L.left = kStageChunk;
     }
     L.slot_base = L.base + (kStageChunk - L.left);
-    L.left -= cells;
 }
 
 __device__ __forceinline__ void tile_corners(const float* box, const TileAxes& A, uint32_t bx, uint32_t by,
@@ -1044,8 +1041,9 @@ __device__ __forceinline__ void contour_tile(const SpPass& P, const TileGrid& G,
 {
     // 1. cells with a sign change: the 8 cells of each live brick (lb: the live bricks,
     // nlive of them), one per thread
-    for (uint32_t k0 = 0; k0 < nlive * 8u; k0 += kTileThreads) {
-        const uint32_t k = k0 + thread_id();
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(thread_id() >> 6) * 64u;
+    for (uint32_t k0 = wave; k0 < nlive * 8u; k0 += kTileThreads) {
+        const uint32_t k = k0 + lane();
         uint32_t c = 0;
         bool cand_c = false;
         if (k < nlive * 8u) {
@@ -1070,43 +1068,44 @@ __device__ __forceinline__ void contour_tile(const SpPass& P, const TileGrid& G,
         if (cand_c) cand[wbase + (uint32_t)__builtin_popcountll(w & ((1ull << lane()) - 1ull))] = (uint16_t)c;
     }
     __syncthreads();
-    // 2. vertex and sign bits of each listed cell
-    const uint32_t ncand = L.ncand;
-    bool act[2] = {false, false};
-    float pos[2][3];
-    uint32_t cell[2] = {0, 0}, sg[2] = {0, 0}, k_at[2] = {0, 0};
-#pragma unroll
-    for (uint32_t r = 0; r < 2; ++r) {
-        const uint32_t k = r * kTileThreads + thread_id();
+    // 2. vertex and sign bits of each listed cell, staged at the space reserved by
+    // contour_reserve
+    const uint32_t ncand = L.ncand, stage_base = L.slot_base;
+    for (uint32_t k0 = wave; k0 < ncand; k0 += kTileThreads) {
+        const uint32_t k = k0 + lane();
+        bool act = false;
+        float pos[3];
+        uint32_t c = 0, sg = 0;
         if (k < ncand) {
-            const uint32_t c = cand[k];
+            c = cand[k];
             const uint32_t cxl = c & 7u, cyl = (c >> 3) & 7u, czl = c >> 6;
             float cv[8];
             tile_corners(box, A, G.bx, G.by, c, cv);
             const float lo[3] = {A.clo[0][cxl], A.clo[1][cyl], A.clo[2][czl]};
             const float hi[3] = {A.chi[0][cxl], A.chi[1][cyl], A.chi[2][czl]};
-            act[r] = contour_cell(cv, lo, hi, pos[r]);
-            cell[r] = c;
+            act = contour_cell(cv, lo, hi, pos);
             // cell_sign_changes (dualcontour.wgsl:57-69)
-            sg[r] = (uint32_t)(cv[1] > 0.0f) | ((uint32_t)(cv[2] > 0.0f) << 1) |
-                    ((uint32_t)(cv[4] > 0.0f) << 2) | ((uint32_t)(cv[0] > 0.0f) << 3);
+            sg = (uint32_t)(cv[1] > 0.0f) | ((uint32_t)(cv[2] > 0.0f) << 1) | ((uint32_t)(cv[4] > 0.0f) << 2) |
+                 ((uint32_t)(cv[0] > 0.0f) << 3);
         }
-        const uint64_t w = __ballot(act[r]);
-        const uint32_t lead = (uint32_t)__builtin_ctzll(w | (1ull << 63));
+        const uint64_t w = __ballot(act);
+        if (!w) continue;
+        const uint32_t lead = (uint32_t)__builtin_ctzll(w);
         uint32_t wbase = 0;
-        if (w && lane() == lead) wbase = atomicAdd(&L.nact, (uint32_t)__builtin_popcountll(w));
+        if (lane() == lead) wbase = atomicAdd(&L.nact, (uint32_t)__builtin_popcountll(w));
         wbase = (uint32_t)__builtin_amdgcn_readlane((int)wbase, (int)lead);
-        if (act[r]) {
-            k_at[r] = wbase + (uint32_t)__builtin_popcountll(w & ((1ull << lane()) - 1ull));
-            atomicOr(&L.rows[cell[r] >> 3], 1u << (cell[r] & 7u));
+        if (act) {
+            atomicOr(&L.rows[c >> 3], 1u << (c & 7u));
+            const uint64_t at = (uint64_t)stage_base + wbase + (uint32_t)__builtin_popcountll(w & ((1ull << lane()) - 1ull));
+            if (at < P.stage_cap) P.stage[at] = make_float4(pos[0], pos[1], pos[2], __uint_as_float(c | (sg << 12)));
         }
     }
     __syncthreads();
-    // 3. the staged cells (at the space reserved by contour_reserve), row segment counts
-    // and the slot's cell bits
+    // 3. row segment counts and the slot's cell bits
     if (thread_id() == 0) {
-        P.slot_stage[2 * slot] = L.slot_base;
+        P.slot_stage[2 * slot] = stage_base;
         P.slot_stage[2 * slot + 1] = L.nact;
+        L.left -= L.nact;
     }
     if (thread_id() < 64) {
         const uint32_t row = thread_id();
@@ -1114,16 +1113,6 @@ __device__ __forceinline__ void contour_tile(const SpPass& P, const TileGrid& G,
         if (row < 16)
             P.cellbits[(size_t)slot * 16u + row] = L.rows[4 * row] | (L.rows[4 * row + 1] << 8) |
                                                    (L.rows[4 * row + 2] << 16) | (L.rows[4 * row + 3] << 24);
-    }
-    const uint32_t stage_base = L.slot_base;
-#pragma unroll
-    for (uint32_t r = 0; r < 2; ++r) {
-        if (!act[r]) continue;
-        const uint32_t c = cell[r];
-        const uint32_t rank = (uint32_t)__builtin_popcount(L.rows[c >> 3] & ((1u << (c & 7u)) - 1u));
-        const uint64_t at = (uint64_t)stage_base + k_at[r];
-        if (at < P.stage_cap)
-            P.stage[at] = make_float4(pos[r][0], pos[r][1], pos[r][2], __uint_as_float(c | (rank << 9) | (sg[r] << 12)));
     }
 }
 
@@ -1136,8 +1125,12 @@ static_assert(kTileThreads >= kBoxAxis * kBoxAxis, "one box row per thread");
 // program, staged in
 // LDS, at the lattice points of its closed box that the tile's cells need (all points for
 // programs that are not left folds), into an LDS box; then the tile's cells are contoured
-// from it (contour_tile).  LINEAR = 1 runs the slots whose program is a left fold (two
-// points per lane) and skips the others, LINEAR = 0 the others (gen_slots).
+// from it (contour_tile).  LINEAR = 1 runs the slots whose program is a left fold and skips
+// the others, LINEAR = 0 the others (gen_slots).
+// Bound by instruction issue (three quarters of the issue slots at CSG-64 1024^3: 69.5 k slots,
+// 258 points and 57 vertices each): of 300 us there, 60 evaluate, 42 place vertices, 28 look for
+// sign changes, the rest is the fixed work of a tile.  355 us with the points dealt to all
+// lanes, half of them twice, and a 64-bit division per row.
 template <int LINEAR>
 __device__ __forceinline__ void tiles_body(const SpPass& P)
 {
@@ -1236,38 +1229,42 @@ __device__ __forceinline__ void tiles_body(const SpPass& P)
             // its rows' points in `list` with one atomic; entries are iz << 10 | iy << 5 | ix.
             // The list is evaluated window by window (one window unless more than kList points).
             if (thread_id() == 0) contour_reserve(P, L, 8u * (uint32_t)__builtin_popcountll(lv));
-            const uint32_t q = thread_id();
-            uint32_t M = 0, code = 0;
-            if (q < ny * nz) {
-                const uint32_t iz = div16(q, ny, magic16(ny)), iy = q - iz * ny;
-                // rm = OR over the z-bricks bz and y-bricks by that use the row of the live
-                // bits of x-bricks (bz, by, 0..3): the used z layers of lv ORed (16 bits,
-                // by * 4 + bx), then the used y rows of that
-                const uint32_t mz = R.bm[1][iz], my = R.bm[0][iy];
-                uint32_t layers = 0, rm = 0;
+            const uint32_t nrow = ny * nz;
+            const float rny = recip(ny);
+            uint32_t M = 0, code = 0, off = 0, cnt = 0;
+            if ((thread_id() & ~63u) < nrow) {  // the wave has rows
+                const uint32_t q = thread_id();
+                if (q < nrow) {
+                    const uint32_t iz = div_by(q, rny), iy = q - iz * ny;
+                    // rm = OR over the z-bricks bz and y-bricks by that use the row of the live
+                    // bits of x-bricks (bz, by, 0..3): the used z layers of lv ORed (16 bits,
+                    // by * 4 + bx), then the used y rows of that
+                    const uint32_t mz = R.bm[1][iz], my = R.bm[0][iy];
+                    uint32_t layers = 0, rm = 0;
 #pragma unroll
-                for (uint32_t bz = 0; bz < 4; ++bz)
-                    if ((mz >> bz) & 1u) layers |= (uint32_t)(lv >> (16u * bz)) & 0xffffu;
+                    for (uint32_t bz = 0; bz < 4; ++bz)
+                        if ((mz >> bz) & 1u) layers |= (uint32_t)(lv >> (16u * bz)) & 0xffffu;
 #pragma unroll
-                for (uint32_t by = 0; by < 4; ++by)
-                    if ((my >> by) & 1u) rm |= (layers >> (4u * by)) & 0xfu;
-                M = ((rm & 1u) ? R.xb[0] : 0u) | ((rm & 2u) ? R.xb[1] : 0u) | ((rm & 4u) ? R.xb[2] : 0u) |
-                    ((rm & 8u) ? R.xb[3] : 0u);
-                code = (iz << 10) | (iy << 5);
+                    for (uint32_t by = 0; by < 4; ++by)
+                        if ((my >> by) & 1u) rm |= (layers >> (4u * by)) & 0xfu;
+                    M = ((rm & 1u) ? R.xb[0] : 0u) | ((rm & 2u) ? R.xb[1] : 0u) | ((rm & 4u) ? R.xb[2] : 0u) |
+                           ((rm & 8u) ? R.xb[3] : 0u);
+                    code = (iz << 10) | (iy << 5);
+                }
+                // the exclusive prefix sum of cnt (<= 16, 5 bits) over the wave's lanes, bit by
+                // bit: lanes below with the bit set (mbcnt over its ballot) times its weight
+                cnt = (uint32_t)__builtin_popcount(M);
+                uint32_t below = 0, wtotal = 0;
+#pragma unroll
+                for (uint32_t b = 0; b < 5; ++b) {
+                    const uint64_t m = __ballot((int)((cnt >> b) & 1u));
+                    below += __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u)) << b;
+                    wtotal += (uint32_t)__builtin_popcountll(m) << b;
+                }
+                uint32_t wbase = 0;
+                if (lane() == 0 && wtotal) wbase = atomicAdd(&nlist, wtotal);
+                off = (uint32_t)__builtin_amdgcn_readlane((int)wbase, 0) + below;
             }
-            // the exclusive prefix sum of cnt (<= 16, 5 bits) over the wave's lanes, bit by
-            // bit: lanes below with the bit set (mbcnt over its ballot) times its weight
-            const uint32_t cnt = (uint32_t)__builtin_popcount(M);
-            uint32_t below = 0, wtotal = 0;
-#pragma unroll
-            for (uint32_t b = 0; b < 5; ++b) {
-                const uint64_t m = __ballot((int)((cnt >> b) & 1u));
-                below += __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u)) << b;
-                wtotal += (uint32_t)__builtin_popcountll(m) << b;
-            }
-            uint32_t wbase = 0;
-            if (lane() == 0 && wtotal) wbase = atomicAdd(&nlist, wtotal);
-            const uint32_t off = (uint32_t)__builtin_amdgcn_readlane((int)wbase, 0) + below;
             if (kr < need) reinterpret_cast<uint4*>(&R)[kr] = rest;
             // window 0 is filled at once (every wave has its offsets); the total is read
             // after the barrier that completes it
@@ -1286,23 +1283,30 @@ __device__ __forceinline__ void tiles_body(const SpPass& P)
                 __syncthreads();
                 if (w0 == 0) total = nlist;  // reset for the next slot after the box is complete
                 const uint32_t m = min(kList, total - w0);
-                for (uint32_t i0 = thread_id(); i0 < m; i0 += kLinearPoints * kTileThreads) {
-                    float x[kLinearPoints], y[kLinearPoints], z[kLinearPoints], v[kLinearPoints];
-                    uint32_t at[kLinearPoints];
+                // a wave takes 128 points in a row, two per lane sharing each op's decode, or the
+                // last 64 or fewer one per lane: whole waves have nothing left, instead of
+                // every lane half of its points
+                auto points = [&](auto np, uint32_t i0) {
+                    constexpr int NP = decltype(np)::value;
+                    float x[NP], y[NP], z[NP], v[NP];
+                    uint32_t at[NP];
 #pragma unroll
-                    for (int p = 0; p < kLinearPoints; ++p) {
-                        const uint32_t i = i0 + p * kTileThreads;
-                        const uint32_t e = list[i < m ? i : i0];
+                    for (int p = 0; p < NP; ++p) {
+                        const uint32_t e = list[min(i0 + p * 64u + lane(), m - 1u)];
                         const uint32_t ix = e & 31u, iy = (e >> 5) & 31u, iz = e >> 10;
                         x[p] = R.pc[0][ix];
                         y[p] = R.pc[1][iy];
                         z[p] = R.pc[2][iz];
                         at[p] = (iz * by + iy) * bx + ix;
                     }
-                    run_linear<kLinearPoints>(R.T, n, x, y, z, v);
+                    run_linear<NP>(R.T, n, x, y, z, v);
 #pragma unroll
-                    for (int p = 0; p < kLinearPoints; ++p)
-                        if (i0 + p * kTileThreads < m) box[at[p]] = v[p];
+                    for (int p = 0; p < NP; ++p)
+                        if (i0 + p * 64u + lane() < m) box[at[p]] = v[p];
+                };
+                for (uint32_t i0 = __builtin_amdgcn_readfirstlane(thread_id() >> 6) * 128u; i0 < m; i0 += 2u * kTileThreads) {
+                    if (m - i0 > 64u) points(std::integral_constant<int, 2>{}, i0);
+                    else points(std::integral_constant<int, 1>{}, i0);
                 }
                 if (w0 + kList >= total) break;
             }
@@ -1311,7 +1315,7 @@ __device__ __forceinline__ void tiles_body(const SpPass& P)
         } else {
             const uint32_t x0 = bxh & 0xffffffu, y0 = byh & 0xffffffu, z0 = bzh & 0xffffffu;
             const uint32_t nxy = nx * ny, npts = nxy * nz;
-            const uint32_t mx = magic16(nx), mxy = magic16(nxy);
+            const float rx = recip(nx), rxy = recip(nxy);
             const bool staged = n <= kStageOps;
             if (thread_id() == 0) contour_reserve(P, L, 8u * 8u * 8u);
             if (staged) stage_tape(R.T, J.ops, Lst, n);
@@ -1328,8 +1332,8 @@ __device__ __forceinline__ void tiles_body(const SpPass& P)
                     if (R.T.code[q] == S2M_OP_MANDELBULB) R.mandel = 1;
             __syncthreads();
             auto point = [&](uint32_t q, float& x, float& y, float& z) {  // its entry in the box
-                const uint32_t iz = div16(q, nxy, mxy), r = q - iz * nxy;
-                const uint32_t iy = div16(r, nx, mx), ix = r - iy * nx;
+                const uint32_t iz = div_by(q, rxy), r = q - iz * nxy;
+                const uint32_t iy = div_by(r, rx), ix = r - iy * nx;
                 x = R.pc[0][ix];
                 y = R.pc[1][iy];
                 z = R.pc[2][iz];
