@@ -1264,6 +1264,7 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
             P.cellbits = ctx->sp_cellbits.as<uint32_t>();
             P.stage = ctx->sp_stage.as<float4>();
             P.stage_cap = stage_cap;
+            P.tile_blocks = (uint32_t)tile_blocks;
             P.slot_stage = ctx->sp_slot_stage.as<uint32_t>();
             P.slot_live = ctx->sp_slot_live.as<uint64_t>();
             P.slot_hdr = ctx->sp_slot_hdr.as<SlotHdr>();

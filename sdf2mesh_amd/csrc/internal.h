@@ -187,6 +187,8 @@ struct SpPass {
                                // in byte r % 4 of word r / 4)
     float4* stage;             // [stage_cap] active cells: position, cell | signs << 12
     uint64_t stage_cap;
+    uint32_t tile_blocks;      // most blocks of a k_sp_tiles launch: the first 2 * tile_blocks staging chunks
+                               // are theirs without being counted
     uint32_t* slot_stage;      // [slot][2] first staged cell, staged cells
     uint64_t* slot_live;       // [slot] bricks (2x2x2 cells) that may hold an active cell
     SlotHdr* slot_hdr;         // [slot]

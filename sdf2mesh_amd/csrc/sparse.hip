@@ -71,29 +71,37 @@ __device__ __forceinline__ uint32_t active_slots(const SpPass& P, uint32_t count
     return (uint32_t)(n < P.slot_cap ? n : P.slot_cap);
 }
 
-// Work queues of a persistent launch: worker b of nid draws slots g, g + G, g + 2G, ... (g =
-// b mod G, G = min(kQueueGroups, nid)) one at a time from its group's counter, so blocks that
-// draw cheap tiles take more of them.  One counter per group, each on its own 128-byte
-// line: updates of one address are serialised by the memory system, so a single counter
-// for all blocks would throttle them.
-__device__ __forceinline__ uint32_t queue_take(const SpPass& P, uint32_t q, uint32_t id, uint32_t nid)
-{
-    const uint32_t G = min(kQueueGroups, nid), g = id % G;
-    const uint32_t j = atomicAdd(&P.queues[(q * kQueueGroups + g) * 32u], 1u);
-    const uint64_t slot = (uint64_t)j * G + g;
-    return (uint32_t)(slot < 0xffffffffull ? slot : 0xffffffffull);
-}
-
+// Work queues of a persistent launch: block b draws turns from the counter of its group g = b
+// mod G, G = min(kQueueGroups, blocks), so blocks that draw cheap tiles take more of them.
+// One counter per group, each on its own 128-byte line: updates of one address are serialised
+// by the memory system (some 25 ns each), so a single counter for all blocks would throttle
+// them.  A block's first turn is its own, without a draw.
 // Neighbouring slots are mostly neighbouring tiles: runs of kTurnRun of them go to one XCD (the
 // hardware deals blocks to XCDs in turn), so rows and output lines they share stay in one L2.
-// Slot of draw `j` of group g; increasing in j, every slot once.
-constexpr uint32_t kTurnRun = 16;
-__device__ __forceinline__ uint32_t turn_of(uint32_t j, uint32_t g, uint32_t G)
-{
-    if (G != kQueueGroups) return j * G + g;
-    const uint32_t m = j * (kQueueGroups / 8u) + (g >> 3);
-    return ((m / kTurnRun) * 8u + (g & 7u)) * kTurnRun + m % kTurnRun;
-}
+struct Turns {
+    uint32_t* queue;
+    uint32_t G, g, own;  // own: blocks of the group
+
+    __device__ Turns(const SpPass& P, uint32_t q)
+    {
+        G = min(kQueueGroups, gridDim.x);
+        g = blockIdx.x % G;
+        own = (gridDim.x - g + G - 1u) / G;
+        queue = P.queues + (q * kQueueGroups + g) * 32u;
+    }
+    __device__ __forceinline__ uint32_t first() const { return turn(blockIdx.x / G); }
+    // One lane's draw; turn(own + draw()) increases with every draw of the group.
+    __device__ __forceinline__ uint32_t draw() const { return atomicAdd(queue, 1u); }
+    __device__ __forceinline__ uint32_t drawn(uint32_t d) const { return turn(own + d); }
+    // Turn j of group g: every index once.
+    __device__ __forceinline__ uint32_t turn(uint32_t j) const
+    {
+        if (G != kQueueGroups) return j * G + g;
+        const uint32_t m = j * (kQueueGroups / 8u) + (g >> 3);
+        return ((m / kTurnRun) * 8u + (g & 7u)) * kTurnRun + m % kTurnRun;
+    }
+    static constexpr uint32_t kTurnRun = 16;
+};
 
 // Row segment of row (zl, y) and tile column tx of job J.
 // Per-slot row data: array k (kRowVtx, kRowTri: counts; kRowVtxOff, kRowTriOff: first
@@ -962,8 +970,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
 // cells with a vertex are staged compactly for k_sp_emit, their bits go to the slot's
 // `cellbits` and each row segment's count to the slot's kRowVtx row.  Contains barriers.
 // ---------------------------------------------------------------------------------
-// Staged cells are allocated in chunks of kStageChunk per block (one counter update per
-// chunk).  A slot needs room for 8 entries per live brick (its cells) when its tile starts, so
+// Staged cells are allocated in chunks of kStageChunk per block: the block's own, then one
+// counter update per chunk (with the first ones counted too, the blocks of a launch wait for
+// each other's update of one address: up to 15 us of a launch of 1792).  A slot needs room for 8 entries per live brick (its cells) when its tile starts, so
 // that its cells are contiguous, and takes what it has used; a chunk with less room left is
 // abandoned.  Hence at most (staged cells) + (room needed by the slots that open a chunk) +
 // blocks x kStageChunk are used; the host grows the buffer from the device count if that
@@ -999,7 +1008,8 @@ __device__ __forceinline__ void contour_reset(ContourLds& L)
 __device__ __forceinline__ void contour_reserve(const SpPass& P, ContourLds& L, uint32_t cells)
 {
     if (L.left < cells) {
-        L.base = (uint32_t)atomicAdd((unsigned long long*)&P.counters[kStageUsed], (unsigned long long)kStageChunk);
+        L.base = 2u * P.tile_blocks * kStageChunk +
+                 (uint32_t)atomicAdd((unsigned long long*)&P.counters[kStageUsed], (unsigned long long)kStageChunk);
         L.left = kStageChunk;
     }
     L.slot_base = L.base + (kStageChunk - L.left);
@@ -1147,9 +1157,13 @@ __device__ __forceinline__ void tiles_body(const SpPass& P)
     // LINEAR = 0: indices into the list of the slots that are no folds
     const uint32_t nslots = active_slots(P, LINEAR ? kSlotsUsed : kGenUsed);
     constexpr uint32_t kQueue = LINEAR ? 0u : 1u;
-    if (thread_id() == 0) L.left = 0;  // published by the first slot's barriers
+    if (thread_id() == 0) {  // the block's first staging chunk; published by the first slot's barriers
+        L.base = (blockIdx.x + (LINEAR ? 0u : P.tile_blocks)) * kStageChunk;
+        L.left = kStageChunk;
+    }
     uint64_t tiles_done = 0, points_done = 0, flops_done = 0;  // thread 0: this block's share
-    uint32_t next = thread_id() == 0 ? queue_take(P, kQueue, blockIdx.x, gridDim.x) : 0u;
+    const Turns Q(P, kQueue);
+    uint32_t next = Q.first();  // thread 0's counts
     // Left folds: threads < kRecPre hold the first kRecPre x 16 bytes of the next slot's
     // record, read while the current slot is contoured and stored to R at the loop's top.
     uint4 pre = make_uint4(0u, 0u, 0u, 0u);
@@ -1170,7 +1184,7 @@ __device__ __forceinline__ void tiles_body(const SpPass& P)
         __syncthreads();
         if (sh_slot >= nslots) break;
         const uint32_t slot = LINEAR ? sh_slot : P.gen_slots[sh_slot];
-        if (thread_id() == 0) next = queue_take(P, kQueue, blockIdx.x, gridDim.x);  // prefetched
+        if (thread_id() == 0) next = Q.drawn(Q.draw());  // prefetched
         const SlotHdr& H = [&]() -> const SlotHdr& {
             if constexpr (LINEAR != 0) return R.H;
             else return P.slot_hdr[__builtin_amdgcn_readfirstlane(slot)];
@@ -1537,13 +1551,11 @@ __global__ __launch_bounds__(64) void k_sp_emit(SpPass P, MeshBufs b)
     __shared__ uint32_t trow[64];  // first triangle of row segment c >> 3
     if (LINEAR && blockIdx.x == 0) report(P);
     const uint32_t nslots = active_slots(P, LINEAR ? kSlotsNow : kGenNow);
-    // the first turn is the block's own, the others are drawn, one ahead
-    const uint32_t G = min(kQueueGroups, gridDim.x), g = blockIdx.x % G;
-    uint32_t* const queue = P.queues + ((LINEAR ? 2u : 3u) * kQueueGroups + g) * 32u;
-    const uint32_t own = (gridDim.x - g + G - 1u) / G;  // blocks of the group
-    uint32_t turn = turn_of(blockIdx.x / G, g, G), drawn = 0;
-    for (; turn < nslots; turn = turn_of(own + (uint32_t)__builtin_amdgcn_readfirstlane(drawn), g, G)) {
-        if (thread_id() == 0) drawn = atomicAdd(queue, 1u);
+    // the turns after the first are drawn one ahead
+    const Turns Q(P, LINEAR ? 2u : 3u);
+    uint32_t drawn = 0;
+    for (uint32_t turn = Q.first(); turn < nslots; turn = Q.drawn((uint32_t)__builtin_amdgcn_readfirstlane(drawn))) {
+        if (thread_id() == 0) drawn = Q.draw();
         const uint32_t slot = LINEAR ? turn : P.gen_slots[turn];
         const SlotHdr& H = P.slot_hdr[slot];
         const uint64_t tile = __builtin_amdgcn_readfirstlane(H.tile);
@@ -1856,7 +1868,7 @@ __global__ __launch_bounds__(256) void k_sp_rowdown(SpPass P)
         P.counters[kGenUsed] = 0;
         for (uint32_t q = 0; q < 2; ++q) {
             const uint32_t used = q ? kStageUsed : kSlotsUsed, most = q ? kStageMax : kSlotsMax;
-            const uint64_t n = P.counters[used];
+            const uint64_t n = P.counters[used] + (q ? 2ull * P.tile_blocks * kStageChunk : 0ull);
             P.counters[q ? kStageNow : kSlotsNow] = n;
             if (n > P.counters[most]) P.counters[most] = n;
             P.counters[used] = 0;
