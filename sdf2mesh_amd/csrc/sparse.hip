@@ -15,7 +15,7 @@
 //                   left fold on the brick (bricks that keep one sign are not evaluated),
 //                   and the slot's record: header, live bricks, axis tables, box
 //                   coordinates and the program in k_sp_tiles' LDS layout
-//   k_sp_tiles<1/0> per slot (one block): the pruned program in LDS (left folds: from the
+//   k_sp_tiles      per slot (one block): the pruned program in LDS (left folds: from the
 //                   record, read while the block contours the slot before), at the
 //                   lattice points the tile's live bricks use (left folds) or at all
 //                   points of its box (other programs), into an LDS box; then the tile's
@@ -27,11 +27,11 @@
 //                   VertexList order (job after job, then z, y, tile x): per row, the
 //                   segments of its active tiles; then a scan over rows, which also gives
 //                   each job's first vertex and triangle index
-//   k_sp_emit<1/0>  per slot: the staged vertices at their ordered index with their
+//   k_sp_emit       per slot: the staged vertices at their ordered index with their
 //                   4-tap normals (the tile's pruned program), then the triangles of
 //                   their quads, vertex indices relative to the job's first vertex
 //   k_sp_boundary   (multi-slab single job) cell -> vertex map of the slab's last plane
-// The totals go to mapped host memory from k_sp_rowdown and k_sp_emit<1>: a pass of folds is
+// The totals go to mapped host memory from k_sp_rowdown and k_sp_emit: a pass of folds is
 // seven launches (of about 4.5 us each at any small size).
 // The per-slot kernels are persistent (as many blocks as the device holds) and draw slots
 // from a work queue.  A cell's vertex index is never stored: it is the first index of its row segment plus
@@ -80,16 +80,17 @@ __device__ __forceinline__ uint32_t active_slots(const SpPass& P, uint32_t count
 // hardware deals blocks to XCDs in turn), so rows and output lines they share stay in one L2.
 struct Turns {
     uint32_t* queue;
-    uint32_t G, g, own;  // own: blocks of the group
+    uint32_t G, g, own, mine;  // own: blocks of the group
 
-    __device__ Turns(const SpPass& P, uint32_t q)
+    __device__ Turns(const SpPass& P, uint32_t q, uint32_t block, uint32_t blocks)
     {
-        G = min(kQueueGroups, gridDim.x);
-        g = blockIdx.x % G;
-        own = (gridDim.x - g + G - 1u) / G;
+        G = min(kQueueGroups, blocks);
+        g = block % G;
+        own = (blocks - g + G - 1u) / G;
         queue = P.queues + (q * kQueueGroups + g) * 32u;
+        mine = block / G;
     }
-    __device__ __forceinline__ uint32_t first() const { return turn(blockIdx.x / G); }
+    __device__ __forceinline__ uint32_t first() const { return turn(mine); }
     // One lane's draw; turn(own + draw()) increases with every draw of the group.
     __device__ __forceinline__ uint32_t draw() const { return atomicAdd(queue, 1u); }
     __device__ __forceinline__ uint32_t drawn(uint32_t d) const { return turn(own + d); }
@@ -102,6 +103,18 @@ struct Turns {
     }
     static constexpr uint32_t kTurnRun = 16;
 };
+
+// Launches that run both kinds of slots (kBothKinds): the first blocks take the slots that are
+// no folds, a share by their number and cost (a tile of them costs some two of a fold: every
+// point of its box is evaluated).
+constexpr uint32_t kGeneralCost = 2;
+__device__ __forceinline__ uint32_t general_blocks(uint32_t general, uint32_t slots)
+{
+    if (general == 0) return 0;
+    const uint64_t w = (uint64_t)kGeneralCost * general;
+    const uint32_t n = (uint32_t)(gridDim.x * w / (w + (slots - min(slots, general))));
+    return min(max(n, 1u), gridDim.x - 1u);
+}
 
 // Row segment of row (zl, y) and tile column tx of job J.
 // Per-slot row data: array k (kRowVtx, kRowTri: counts; kRowVtxOff, kRowTriOff: first
@@ -1142,7 +1155,7 @@ static_assert(kTileThreads >= kBoxAxis * kBoxAxis, "one box row per thread");
 // sign changes, the rest is the fixed work of a tile.  355 us with the points dealt to all
 // lanes, half of them twice, and a 64-bit division per row.
 template <int LINEAR>
-__device__ __forceinline__ void tiles_body(const SpPass& P)
+__device__ __forceinline__ void tiles_body(const SpPass& P, uint32_t block, uint32_t blocks)
 {
     extern __shared__ float box[];  // P.box_stride floats; LINEAR = 0: then the operand stacks
                                     // (P.prune_depth entries per thread and point)
@@ -1158,11 +1171,11 @@ __device__ __forceinline__ void tiles_body(const SpPass& P)
     const uint32_t nslots = active_slots(P, LINEAR ? kSlotsUsed : kGenUsed);
     constexpr uint32_t kQueue = LINEAR ? 0u : 1u;
     if (thread_id() == 0) {  // the block's first staging chunk; published by the first slot's barriers
-        L.base = (blockIdx.x + (LINEAR ? 0u : P.tile_blocks)) * kStageChunk;
+        L.base = (block + (LINEAR ? 0u : P.tile_blocks)) * kStageChunk;
         L.left = kStageChunk;
     }
     uint64_t tiles_done = 0, points_done = 0, flops_done = 0;  // thread 0: this block's share
-    const Turns Q(P, kQueue);
+    const Turns Q(P, kQueue, block, blocks);
     uint32_t next = Q.first();  // thread 0's counts
     // Left folds: threads < kRecPre hold the first kRecPre x 16 bytes of the next slot's
     // record, read while the current slot is contoured and stored to R at the loop's top.
@@ -1401,17 +1414,33 @@ __device__ __forceinline__ void tiles_body(const SpPass& P)
     }
 }
 
-template <int LINEAR>
+// Kinds of slots a launch runs: those that are no folds, folds, or both, each by a share of the
+// blocks.  Two launches leave most of the device idle while a small pass's few slots of the
+// one kind run, each some 15 to 30 us of latency; in one launch the folds are held to the
+// registers of the other kind (four waves per SIMD instead of seven), which costs more than it
+// saves from some 130 k tiles on.  Three trees, one launch against two, us: 160^3 182 / 222,
+// 256^3 168 / 195, 352^3 249 / 273, 384^3 279 / 287, 448^3 297 / 298, 640^3 478 / 441.
+enum Kind : int { kGeneralKind = 0, kFoldKind = 1, kBothKinds = 2 };
+constexpr uint64_t kBothTiles = 128u << 10;
+
+template <int KIND>
 __global__ void k_sp_tiles(SpPass P);
 template <>
-__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_sp_tiles<1>(SpPass P)
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_sp_tiles<kFoldKind>(SpPass P)
 {
-    tiles_body<1>(P);
+    tiles_body<1>(P, blockIdx.x, gridDim.x);
 }
 template <>
-__global__ __launch_bounds__(kTileThreads) void k_sp_tiles<0>(SpPass P)
+__global__ __launch_bounds__(kTileThreads) void k_sp_tiles<kGeneralKind>(SpPass P)
 {
-    tiles_body<0>(P);
+    tiles_body<0>(P, blockIdx.x, gridDim.x);
+}
+template <>
+__global__ __launch_bounds__(kTileThreads) void k_sp_tiles<kBothKinds>(SpPass P)
+{
+    const uint32_t general = general_blocks(active_slots(P, kGenUsed), active_slots(P, kSlotsUsed));
+    if (blockIdx.x >= general) tiles_body<1>(P, blockIdx.x - general, gridDim.x - general);
+    else tiles_body<0>(P, blockIdx.x, general);
 }
 
 // ---------------------------------------------------------------------------------
@@ -1523,7 +1552,7 @@ __global__ __launch_bounds__(64) void k_sp_quadcount(SpPass P, MeshBufs b)
 // a block's share of vertices varies twofold and half of the waves idled at the end.
 // 325 -> 243 us there (69 k slots, 4.0 M vertices).
 // ---------------------------------------------------------------------------------
-// Block 0 of k_sp_emit<1> after a job's last pass: the statistics summed and
+// The first fold block of k_sp_emit after a job's last pass: the statistics summed and
 // counters[0 .. nback) to P.back (mapped host memory, NULL: not wanted).  Nothing in the
 // kernel changes them.
 __device__ __forceinline__ void report(const SpPass& P)
@@ -1541,7 +1570,7 @@ __device__ __forceinline__ void report(const SpPass& P)
 }
 
 template <int LINEAR>
-__global__ __launch_bounds__(64) void k_sp_emit(SpPass P, MeshBufs b)
+__device__ __forceinline__ void emit_body(const SpPass& P, const MeshBufs& b, uint32_t block, uint32_t blocks)
 {
     __shared__ StagedTape T;      // programs that are not left folds (left folds: read in place)
     __shared__ uint32_t mandel;   // such a program holds a Mandelbulb
@@ -1549,10 +1578,10 @@ __global__ __launch_bounds__(64) void k_sp_emit(SpPass P, MeshBufs b)
     __shared__ uint32_t nb[729];  // vertex of cell (8tx-1+i, 8ty-1+j, 8tz-1+k) at nb[(k*9+j)*9+i]
     __shared__ uint32_t tc[128];  // triangles of cell c in byte c % 4 of tc[c / 4]
     __shared__ uint32_t trow[64];  // first triangle of row segment c >> 3
-    if (LINEAR && blockIdx.x == 0) report(P);
+    if (LINEAR && block == 0) report(P);
     const uint32_t nslots = active_slots(P, LINEAR ? kSlotsNow : kGenNow);
     // the turns after the first are drawn one ahead
-    const Turns Q(P, LINEAR ? 2u : 3u);
+    const Turns Q(P, LINEAR ? 2u : 3u, block, blocks);
     uint32_t drawn = 0;
     for (uint32_t turn = Q.first(); turn < nslots; turn = Q.drawn((uint32_t)__builtin_amdgcn_readfirstlane(drawn))) {
         if (thread_id() == 0) drawn = Q.draw();
@@ -1700,6 +1729,18 @@ __global__ __launch_bounds__(64) void k_sp_emit(SpPass P, MeshBufs b)
                 t += 2;
             }
         }
+    }
+}
+
+template <int KIND>
+__global__ __launch_bounds__(64) void k_sp_emit(SpPass P, MeshBufs b)
+{
+    if constexpr (KIND != kBothKinds) {
+        emit_body<KIND>(P, b, blockIdx.x, gridDim.x);
+    } else {
+        const uint32_t general = general_blocks(active_slots(P, kGenNow), active_slots(P, kSlotsNow));
+        if (blockIdx.x >= general) emit_body<1>(P, b, blockIdx.x - general, gridDim.x - general);
+        else emit_body<0>(P, b, blockIdx.x, general);
     }
 }
 
@@ -1963,14 +2004,23 @@ hipError_t launch_sparse_pass(hipStream_t s, const SpPass& P, const MeshBufs& b,
     hipLaunchKernelGGL(k_sp_bricks, dim3(resident_blocks(k_sp_bricks, 64, 0, cus, big)), dim3(64), 0, s, P);
     mark(1);
     const size_t smem = (size_t)P.box_stride * sizeof(float);
-    hipLaunchKernelGGL((k_sp_tiles<1>), dim3(resident_blocks(k_sp_tiles<1>, kTileThreads, smem, cus, tile_blocks)),
-                       dim3(kTileThreads), smem, s, P);
     const size_t gsmem = smem + (size_t)P.prune_depth * (P.prune_depth <= kWideDepth ? kGeneralPoints : 1) *
                                     kTileThreads * sizeof(float);
     const size_t esmem = (size_t)P.prune_depth * 4u * 64u * sizeof(float);
-    if (general_tiles)
-        hipLaunchKernelGGL((k_sp_tiles<0>), dim3(resident_blocks(k_sp_tiles<0>, kTileThreads, gsmem, cus, tile_blocks)),
-                           dim3(kTileThreads), gsmem, s, P);
+    const bool both = general_tiles && P.ntiles <= kBothTiles;
+    auto tiles = [&](auto kernel, size_t lds) {
+        hipLaunchKernelGGL(kernel, dim3(resident_blocks(kernel, kTileThreads, lds, cus, tile_blocks)), dim3(kTileThreads),
+                           lds, s, P);
+    };
+    auto emit = [&](auto kernel, size_t lds) {
+        hipLaunchKernelGGL(kernel, dim3(resident_blocks(kernel, 64, lds, cus, big)), dim3(64), lds, s, P, b);
+    };
+    if (both) {
+        tiles(k_sp_tiles<kBothKinds>, gsmem);
+    } else {
+        tiles(k_sp_tiles<kFoldKind>, smem);
+        if (general_tiles) tiles(k_sp_tiles<kGeneralKind>, gsmem);
+    }
     mark(2);
     hipLaunchKernelGGL(k_sp_quadcount, dim3(resident_blocks(k_sp_quadcount, 64, 0, cus, big)), dim3(64), 0, s,
                        P, b);
@@ -1978,10 +2028,12 @@ hipError_t launch_sparse_pass(hipStream_t s, const SpPass& P, const MeshBufs& b,
     if (P.ntrows) hipLaunchKernelGGL(k_sp_rowsum, dim3((uint32_t)P.ntrows), dim3(64), 0, s, P);
     if (nsb) hipLaunchKernelGGL(k_sp_rowdown, dim3(nsb), dim3(256), 0, s, P);
     mark(4);
-    hipLaunchKernelGGL((k_sp_emit<1>), dim3(resident_blocks(k_sp_emit<1>, 64, 0, cus, big)), dim3(64), 0, s, P, b);
-    if (general_tiles)
-        hipLaunchKernelGGL((k_sp_emit<0>), dim3(resident_blocks(k_sp_emit<0>, 64, esmem, cus, big)), dim3(64), esmem, s,
-                           P, b);
+    if (both) {
+        emit(k_sp_emit<kBothKinds>, esmem);
+    } else {
+        emit(k_sp_emit<kFoldKind>, 0);
+        if (general_tiles) emit(k_sp_emit<kGeneralKind>, esmem);
+    }
     if (boundary_plane) {
         hipLaunchKernelGGL(k_sp_boundary, dim3((uint32_t)((P.boundary_cells + 255) / 256)), dim3(256), 0,
                            s, P);
