@@ -773,12 +773,18 @@ int readback_finish(s2m_ctx* ctx, Readback& rb, uint64_t nv, uint64_t nt)
     return S2M_OK;
 }
 
-// Passes of a single sparse job whose mesh is streamed to host memory: enough that the
-// copy of one pass overlaps the next pass's work (copying a CSG-64 512^3 mesh over PCIe
-// takes about twice its device time), few enough that every pass keeps the device busy.
+// Passes of a single sparse job whose mesh is streamed to host memory: the copy of one pass
+// overlaps the next pass's work, but a pass costs about 110 us beside its tiles and its copies
+// some 30.  One per 256 cell planes, 2 to 4 from 256 planes on (at 256^3 one would do, but a
+// job of that size is expected to be streamed); us in 1 / 2 / 3 / 4 passes:
+//             CSG-64 (much to copy)          a tree                      a torus
+//   256^3     456 / 486 / 544 / 620     214 / 282 / 361 / 417     208 / 232 / 277 / 334
+//   384^3     812 / 736 / 816 / 855     323 / 363 / 414 / 480     355 / 358 / 391 / 416
+//   512^3    1222 / 1107 / 1105 / 1142  441 / 423 / 493 / 542     536 / 529 / 529 / 570
+//   1024^3   4225 / 3820 / 3715 / 3647  1341 / 1199 / 1198 / 1273 1764 / 1670 / 1636 / 1622
 uint32_t stream_passes(uint32_t tile_layers)
 {
-    return std::max<uint32_t>(1, std::min<uint32_t>(4, tile_layers / 16));
+    return tile_layers < 32 ? 1u : std::max<uint32_t>(2, std::min<uint32_t>(4, (tile_layers + 16) / 32));
 }
 
 // Most bytes a pass of a single sparse job holds per tile and row; larger grids take several
@@ -791,7 +797,7 @@ constexpr uint64_t kSparsePassBytes = 4ull << 30;
 // be staged (sparse.hip, kStageOps = 128)?  Every pruned sub-program of one is one too:
 // pruning keeps either the accumulated value or the right operand, a single primitive.
 // Is the program a left fold of unions and smooth unions (k > 0) of library primitives
-// other than the Mandelbulb (k_sp_prune_fold)?
+// other than the Mandelbulb (prune_fold)?
 bool union_fold_program(const std::vector<s2m_op>& ops)
 {
     const size_t n = ops.size();
