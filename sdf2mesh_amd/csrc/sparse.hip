@@ -1569,15 +1569,21 @@ __device__ __forceinline__ void report(const SpPass& P)
         P.back[i] = i == kTilesActive ? sum[0] : i == kEvalPoints ? sum[1] : i == kEvalFlops ? sum[2] : P.counters[i];
 }
 
+struct EmitLds {
+    uint32_t nb[729];     // vertex of cell (8tx-1+i, 8ty-1+j, 8tz-1+k) at nb[(k*9+j)*9+i]
+    uint32_t tc[128];     // triangles of cell c in byte c % 4 of tc[c / 4]
+    uint32_t trow[64];    // first triangle of row segment c >> 3
+    uint16_t quads[512];  // staged cell k: cell | signs << 9 | valid quads << 13
+};
+
 template <int LINEAR>
-__device__ __forceinline__ void emit_body(const SpPass& P, const MeshBufs& b, uint32_t block, uint32_t blocks)
+__device__ __forceinline__ void emit_body(const SpPass& P, const MeshBufs& b, EmitLds& E, uint32_t block, uint32_t blocks)
 {
     __shared__ StagedTape T;      // programs that are not left folds (left folds: read in place)
     __shared__ uint32_t mandel;   // such a program holds a Mandelbulb
     extern __shared__ float taps[];  // their operand stacks: P.prune_depth entries of 4 per lane
-    __shared__ uint32_t nb[729];  // vertex of cell (8tx-1+i, 8ty-1+j, 8tz-1+k) at nb[(k*9+j)*9+i]
-    __shared__ uint32_t tc[128];  // triangles of cell c in byte c % 4 of tc[c / 4]
-    __shared__ uint32_t trow[64];  // first triangle of row segment c >> 3
+    uint32_t *const nb = E.nb, *const tc = E.tc, *const trow = E.trow;
+    uint16_t* const quads = E.quads;
     if (LINEAR && block == 0) report(P);
     const uint32_t nslots = active_slots(P, LINEAR ? kSlotsNow : kGenNow);
     // the turns after the first are drawn one ahead
@@ -1630,12 +1636,13 @@ __device__ __forceinline__ void emit_body(const SpPass& P, const MeshBufs& b, ui
                                (int)(J.z0 + tzl * 8u + t / 9u) - 1, nb + 9u * t);
         for (uint32_t w = thread_id(); w < 128u; w += 64u) tc[w] = 0;
         __syncthreads();
-        // vertices, and each cell's triangle count (the first round's quads are kept for the
-        // triangle loop)
-        uint32_t nq0 = 0;
+        // vertices, and each cell's triangle count.  A load waits for the stores before it, so
+        // the next round's vertex is loaded before this round's stores and the triangle loop
+        // loads nothing.
         for (uint32_t k = thread_id(); k < n; k += 64u) {
             if ((uint64_t)base + k >= P.stage_cap) break;
-            const float4 e = k == thread_id() ? e0 : P.stage[(uint64_t)base + k];
+            const float4 e = e0;
+            if (k + 64u < n && (uint64_t)base + k + 64u < P.stage_cap) e0 = P.stage[(uint64_t)base + k + 64u];
             const uint32_t meta = __float_as_uint(e.w);
             const uint32_t c = meta & 511u, sg = meta >> 12;
             const uint32_t cxl = c & 7u, cyl = (c >> 3) & 7u, czl = c >> 6;
@@ -1645,7 +1652,7 @@ __device__ __forceinline__ void emit_body(const SpPass& P, const MeshBufs& b, ui
             const uint32_t nq =
                 cell_quads(sg, tx * 8u + cxl, ty * 8u + cyl, J.z0 + tzl * 8u + czl, lag, exists, invalid);
             if (nq) atomicOr(&tc[c >> 2], (2u * (uint32_t)__builtin_popcount(nq)) << ((c & 3u) * 8u));
-            if (k == thread_id()) nq0 = nq;
+            quads[k] = (uint16_t)(c | (sg << 9) | (nq << 13));
             const uint64_t vi = nb[at];
             if (vi >= b.vcap) continue;
             float2* o = reinterpret_cast<float2*>(b.vtx + 6 * vi);
@@ -1689,17 +1696,11 @@ __device__ __forceinline__ void emit_body(const SpPass& P, const MeshBufs& b, ui
         // triangles, in vertex order: each quad (q2, q1, q0), (q0, q3, q2)
         for (uint32_t k = thread_id(); k < n; k += 64u) {
             if ((uint64_t)base + k >= P.stage_cap) break;
-            const bool first = k == thread_id();
-            const uint32_t meta = __float_as_uint(first ? e0.w : P.stage[(uint64_t)base + k].w);
-            const uint32_t c = meta & 511u, sg = meta >> 12;
+            const uint32_t word = quads[k], c = word & 511u, sg = (word >> 9) & 15u, nq = word >> 13;
+            if (!nq) continue;
             const uint32_t cxl = c & 7u, cyl = (c >> 3) & 7u, czl = c >> 6;
             const uint32_t at = ((czl + 1) * 9u + (cyl + 1)) * 9u + (cxl + 1);
             auto nbv = [&](int dx, int dy, int dz) { return nb[(int)at + (dz * 9 + dy) * 9 + dx]; };
-            auto exists = [&](int dx, int dy, int dz) { return nbv(dx, dy, dz) != kNone; };
-            uint32_t invalid = 0;
-            const uint32_t nq = first ? nq0 : cell_quads(sg, tx * 8u + cxl, ty * 8u + cyl, J.z0 + tzl * 8u + czl, lag,
-                                                         exists, invalid);
-            if (!nq) continue;
             const uint64_t row2 = ((uint64_t)tc[(c >> 3) * 2u + 1] << 32) | tc[(c >> 3) * 2u];  // 8 counts
             uint64_t t = trow[c >> 3];
             for (uint32_t i = 0; i < cxl; ++i) t += (row2 >> (8u * i)) & 0xffu;
@@ -1735,12 +1736,13 @@ __device__ __forceinline__ void emit_body(const SpPass& P, const MeshBufs& b, ui
 template <int KIND>
 __global__ __launch_bounds__(64) void k_sp_emit(SpPass P, MeshBufs b)
 {
+    __shared__ EmitLds E;
     if constexpr (KIND != kBothKinds) {
-        emit_body<KIND>(P, b, blockIdx.x, gridDim.x);
+        emit_body<KIND>(P, b, E, blockIdx.x, gridDim.x);
     } else {
         const uint32_t general = general_blocks(active_slots(P, kGenNow), active_slots(P, kSlotsNow));
-        if (blockIdx.x >= general) emit_body<1>(P, b, blockIdx.x - general, gridDim.x - general);
-        else emit_body<0>(P, b, blockIdx.x, general);
+        if (blockIdx.x >= general) emit_body<1>(P, b, E, blockIdx.x - general, gridDim.x - general);
+        else emit_body<0>(P, b, E, blockIdx.x, general);
     }
 }
 
