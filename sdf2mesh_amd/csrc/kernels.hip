@@ -21,6 +21,7 @@
 #include <mutex>
 
 #include "device_dense.h"
+#include "device_scan.h"
 #include "device_sdf.h"
 #include "internal.h"
 
@@ -224,15 +225,7 @@ __global__ __launch_bounds__(256) void k_find_bricks(BrickArgs a)
         recs += mask[k] != 0ull ? 1u : 0u;
         cells += (uint32_t)__popcll(mask[k]);
     }
-    uint32_t ir = recs, ic = cells;  // inclusive prefixes over the wave
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t t = __shfl_up(ir, d, 64), u = __shfl_up(ic, d, 64);
-        if (lane_id() >= (uint32_t)d) {
-            ir += t;
-            ic += u;
-        }
-    }
+    const uint32_t ir = wave_scan(recs), ic = wave_scan(cells);
     const uint32_t w = threadIdx.x >> 6;
     if (lane_id() == 63u) {
         wrecs[w] = ir;
@@ -374,23 +367,12 @@ __global__ __launch_bounds__(1024) void k_ranks(const uint64_t* __restrict__ bit
 #pragma unroll
     for (uint32_t k = 0; k < 16u; ++k) {
         const uint32_t i = w0 + k * 1024u + t, n = (uint32_t)__popcll(word[k]);
-        uint32_t upto = n;
-#pragma unroll
-        for (int d = 1; d < 16; d <<= 1) {
-            const uint32_t v = __shfl_up(upto, d, 16);
-            if (l >= (uint32_t)d) upto += v;
-        }
+        const uint32_t upto = row_scan(n);
         if (i < nwords) wpre[i] = (uint16_t)(upto - n);
         if (l == 15u) count[k * 64u + (t >> 4)] = upto;
     }
     __syncthreads();
-    const uint32_t mine = count[t];
-    uint32_t upto = mine;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t v = __shfl_up(upto, d, 64);
-        if (lane_id() >= (uint32_t)d) upto += v;
-    }
+    const uint32_t mine = count[t], upto = wave_scan(mine);
     if (lane_id() == 63u) wsum[t >> 6] = upto;
     __syncthreads();
     uint32_t before = 0, all = 0;
@@ -440,12 +422,7 @@ __global__ __launch_bounds__(1024) void k_tri_offsets(const uint32_t* __restrict
             n[k] = g < groups ? tcount[g] : 0u;
             sum += n[k];
         }
-        uint32_t upto = sum;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const uint32_t v = __shfl_up(upto, d, 64);
-            if (lane_id() >= (uint32_t)d) upto += v;
-        }
+        const uint32_t upto = wave_scan(sum);
         __syncthreads();  // the previous round's readers of wsum
         if (lane_id() == 63u) wsum[t >> 6] = upto;
         __syncthreads();

@@ -43,6 +43,7 @@
 
 #include "device_dense.h"
 #include "device_interval.h"
+#include "device_scan.h"
 #include "device_sdf.h"
 #include "device_staged.h"
 #include "internal.h"
@@ -1858,18 +1859,6 @@ __global__ __launch_bounds__(64) void k_sp_rowsum(SpPass P)
 // Exclusive offsets of the rows, block b = rows b * kScanChunk ...: the pass's first index
 // (kVtxPrev / kTriPrev) plus the chunk sums of the blocks before it (bsum) plus the
 // block-local scan.  The last block writes the totals after the pass (kVtxTotal / kTriTotal).
-// Inclusive prefix sum over the wave's lanes (row shifts, then the row totals passed on).
-__device__ __forceinline__ uint32_t wave_scan(uint32_t x)
-{
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false);  // row_shr:1
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);  // row_bcast:15
-    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);  // row_bcast:31
-    return x;
-}
-
 // Wave w of a block takes rows w * 1024 ... of its chunk, 64 at a time (a thread with 16 rows
 // in a row made every load and store of a wave touch 64 lines).  Bound by latency: all that
 // does not depend on something else is read at the start.  10.2 -> 4.7 us at tree 256^3,
