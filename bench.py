@@ -19,9 +19,8 @@ latency, against one-at-a-time meshing of the same stream).  ``--workload NAME -
 runs one of them alone (profiling runs).
 
   roofline      the SDF evaluation kernel (k_sp_tiles on the tile-pruned path: the pruned
-                program at each live tile's lattice points fused with contouring;
-                k_eval_lattice, or k_eval_mandelbulb for a one-op Mandelbulb tape, on the
-                dense path): executed pruned-program fp32 flops per
+                program at each live tile's lattice points fused with contouring; k_signs
+                on the dense path): executed pruned-program fp32 flops per
                 launch (static op count of the program each tile runs x the lattice points
                 it evaluates, counted on the device) / mean launch time from HIP events
                 recorded around the launches on the library's stream during the timed
@@ -255,7 +254,7 @@ def single_job(name: str, args, ctx, headline: bool) -> dict:
     tiled = agg["tiles_total"] > 0
     ops = node.tape()
     one_mandelbulb = len(ops) == 1 and int(ops[0]["code"]) == tape.MANDELBULB
-    kernel = "k_sp_tiles" if tiled else ("k_eval_mandelbulb" if one_mandelbulb else "k_eval_lattice")
+    kernel = "k_sp_tiles" if tiled else "k_signs"
     d2h_bytes = nvtx * 24 + ntri * 12
     d2h_ms = agg["d2h_ms"] / args.steps
     cfg = {**cfg, "eval": "tile-pruned (exact)" if tiled else
@@ -301,6 +300,10 @@ def single_job(name: str, args, ctx, headline: bool) -> dict:
             "points_per_launch": agg["lattice_points"] / launches,
         },
     }
+    if one_mandelbulb and not tiled:  # priced at the estimator's full count
+        out["roofline"]["frac_of_issue_ceiling"] = None
+        out["roofline"]["note"] = ("flops of the whole estimator at every point; the sign pass ends an orbit "
+                                   "once its sign is certain and executes fewer")
     if headline:
         # stage split (every stage bracketed by events), outside the timed steps
         ctx.set_profiling(2)

@@ -179,11 +179,11 @@ typedef struct s2m_device_mesh {
  * so level 2 costs a little device time).  Counts are filled at every level. */
 typedef struct s2m_timing {
     double total_ms;    /* first kernel start to last kernel end                   */
-    double eval_ms;     /* lattice evaluation kernels                               */
-    double contour_ms;  /* active-cell count, scan (and vertex emission when dense);
+    double eval_ms;     /* lattice evaluation (dense: sign) kernels                 */
+    double contour_ms;  /* dense: bricks at the surface, contouring, ranks;
                            pruned path: the vertex and triangle offset scans        */
-    double normal_ms;   /* 4-tap normals (pruned path: vertex, normal and triangle
-                           emission)                                                */
+    double normal_ms;   /* vertex emission with 4-tap normals (pruned path: and
+                           triangle emission)                                       */
     double quad_ms;     /* quad count, scan, triangle emission (pruned path: the
                            quad count)                                              */
     double d2h_ms;      /* device-to-host copies (s2m_mesh only)                    */
@@ -279,8 +279,8 @@ void s2m_mesh_free(s2m_mesh_out* out);
 /* No counterpart in the reference.  For callers that cannot allocate device memory
  * (serving loops that must not call hipMalloc, harnesses that forbid it): the mesh of
  * s2m_mesh_device, computed by the dense-path kernels, written into the caller's device
- * buffers.  Every working buffer (coordinate tables, lattice slab, cell -> vertex planes,
- * block counts, activity bits, counters) is carved from one static device array of
+ * buffers.  Every working buffer (coordinate tables, the slab's sign words, bricks and staged
+ * vertices, block counts, activity bits, counters) is carved from one static device array of
  * S2M_NOALLOC_SCRATCH_BYTES that each GPU the library runs on holds until the process
  * ends; slabs shrink until they fit it.  The call performs no hipMalloc, hipFree or
  * other allocating HIP call.  Errors: S2M_E_ARG when one cell plane per slab does not fit
