@@ -167,6 +167,9 @@ struct s2m_ctx {
     hipStream_t copy_stream = nullptr;
     // dense slabs: the signs of slab k + 1 are evaluated on eval_stream while slab k is
     // contoured on `stream`
+    // created by the first such job: the device runs a process's streams on four hardware
+    // queues, and a stream nobody uses can still put two busy ones on the same queue (a server's
+    // three contexts: 24 requests in 4.5 - 4.9 ms, 5.3 - 7.1 with a third stream for each)
     hipStream_t eval_stream = nullptr;
     PinnedBuf host_snap;                 // per pass: its totals and capacity use (kSnapWords)
     PinnedBuf host_land;                 // land_mesh's staging of arrays too small to page-lock
@@ -1562,6 +1565,7 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
     const uint32_t nslabs = (j.nz_cells + T - 1) / T;
     Readback* const land = nslabs == 1 && !ctx->profiling ? rb : nullptr;  // copied at its end (land_mesh)
     if (nslabs == 1) rb = nullptr;  // no slabs to overlap
+    if (piped && !ctx->eval_stream) HIP_TRY(hipStreamCreateWithFlags(&ctx->eval_stream, hipStreamNonBlocking));
     hipStream_t es = piped ? ctx->eval_stream : ctx->stream;
     void* back_dev = nullptr;  // mapped host memory for the counters
     if (!fx) {
@@ -1946,7 +1950,6 @@ s2m_ctx* s2m_create(int device)
     }
     e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&ctx->copy_stream, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipStreamCreateWithFlags(&ctx->eval_stream, hipStreamNonBlocking);
     if (e != hipSuccess) {
         fail(S2M_E_HIP, "hipStreamCreate: %s", hipGetErrorString(e));
         if (ctx->copy_stream) (void)hipStreamDestroy(ctx->copy_stream);
@@ -1968,7 +1971,7 @@ void s2m_destroy(s2m_ctx* ctx)
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
     (void)hipStreamSynchronize(ctx->copy_stream);
-    (void)hipStreamSynchronize(ctx->eval_stream);
+    if (ctx->eval_stream) (void)hipStreamSynchronize(ctx->eval_stream);
     for (DevBuf* b : {&ctx->lattice, &ctx->dense, &ctx->bcount, &ctx->check, &ctx->counters,
                       &ctx->tables, &ctx->vtx, &ctx->keys, &ctx->signs, &ctx->tri, &ctx->corners,
                       &ctx->tile_tab, &ctx->tile_lists, &ctx->sp_slot_info,
@@ -1992,7 +1995,7 @@ void s2m_destroy(s2m_ctx* ctx)
     for (hipEvent_t e : ctx->events) (void)hipEventDestroy(e);
     for (hipEvent_t e : ctx->pass_done) (void)hipEventDestroy(e);
     for (auto& g : ctx->graphs) (void)hipGraphExecDestroy(g.second);
-    (void)hipStreamDestroy(ctx->eval_stream);
+    if (ctx->eval_stream) (void)hipStreamDestroy(ctx->eval_stream);
     (void)hipStreamDestroy(ctx->copy_stream);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
