@@ -446,6 +446,7 @@ int upload_tables(s2m_ctx* ctx, const Job& j, DeviceTables& t, void* dst, void**
 struct SpTables {
     std::vector<uint8_t> bytes;
     size_t off_c[3], off_lo[3], off_hi[3], off_ext, off_ibox, off_flops;
+    uint32_t levels;
     uint32_t nt[3];
     uint32_t bmax[3];
     double pad;
@@ -499,6 +500,21 @@ void build_sp_tables(const Job& j, const s2m_program* prog, float eps, SpTables&
     T.off_ibox = put(ibox.data(), next * 4);
     std::vector<uint32_t> fl(prog->n);
     for (uint32_t i = 0; i < prog->n; ++i) fl[i] = op_flops(prog->ops[i]);
+    T.levels = 0;
+    if (prog->n <= kStageOps) {  // the tree (SpJob::op_flops)
+        std::vector<std::pair<uint32_t, uint32_t>> st;  // op and level of each value on the stack
+        for (uint32_t i = 0; i < prog->n; ++i) {
+            uint32_t place = 0, level = 0;
+            if (prog->ops[i].code >= S2M_OP_UNION) {
+                level = 1 + std::max(st[st.size() - 2].second, st.back().second);
+                place = st[st.size() - 2].first | level << 16;
+                st.resize(st.size() - 2);
+            }
+            fl.push_back(place);
+            st.push_back({i, level});
+            T.levels = level;
+        }
+    }
     T.off_flops = put(fl.data(), fl.size() * 4);
     // tile boxes must also hold the normal taps p +- eps of vertices in their cells and
     // absorb the fp32 rounding of p + eps and of the vertex position
@@ -1136,6 +1152,7 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
         J.ext = reinterpret_cast<const float*>(base + T.off_ext);
         J.ibox = reinterpret_cast<const uint32_t*>(base + T.off_ibox);
         J.op_flops = reinterpret_cast<const uint32_t*>(base + T.off_flops);
+        J.levels = T.levels;
         J.boundary = ctx->sp_boundary.as<uint32_t>();
         desc[d] = J;
     }

@@ -143,7 +143,9 @@ struct SpJob {
     const uint32_t* hiz;
     const float* ext;          // tile coordinate extents: xmin[ntx] xmax[ntx] ymin.. zmax[ntz]
     const uint32_t* ibox;      // tile lattice index boxes, same layout
-    const uint32_t* op_flops;
+    const uint32_t* op_flops;  // [nops], then for programs of at most kStageOps ops [nops] op q's place in the
+                               // tree: left operand (the right one is q - 1) | level << 16, primitives 0
+    uint32_t levels;           // of the root
     uint32_t* boundary;        // [ry][rx] vertex of cell plane z0 - 1 (multi-slab job)
 };
 

@@ -494,8 +494,8 @@ __device__ __forceinline__ void super_tiles(const SpJob& J, uint64_t s, uint32_t
 //  1. the super-tile's list: the job's program exactly pruned on its padded box, or
 //     kSingleSign when the SDF keeps one sign there.  Left folds of unions: prune_fold, a
 //     lane per op.  Other programs: a lane per primitive for its interval on the box
-//     (prim_intervals), then every lane walks the program in order (walk_super; the walk is
-//     serial, so the lanes take the same steps).
+//     (prim_intervals), then a lane per op up and down the tree (prune_levels); of more than
+//     kStageOps ops: every lane walks the program in order (walk_super).
 //  2. lane l = its tile (l % 4, l / 4 % 4, l / 16): the list pruned on the tile's padded box
 //     (every lane walks the same list: wave-uniform op dispatch).  Tiles that keep one sign
 //     are dropped, the others get a slot in the pool shared by all jobs (and a flag when
@@ -603,36 +603,87 @@ __device__ __forceinline__ uint32_t prune_fold(const SpJob& J, const float* bl, 
     return one_sign ? kSingleSign : nkept;
 }
 
-// Op q's code and smoothing radius, and the interval of a primitive on the box.
-__device__ __forceinline__ void prim_intervals(const SpJob& J, const float* bl, const float* bh, uint32_t ln, float2* iv,
-                                               uint32_t* codes, uint32_t* radii)
+// The intervals of the job's primitives on the box, a lane per op.
+__device__ __forceinline__ void prim_intervals(const SpJob& J, const float* bl, const float* bh, uint32_t ln, float2* iv)
 {
     for (uint32_t q = ln; q < J.nops; q += 64u) {
         const s2m_op& o = J.ops[q];
         const uint32_t code = o.code;
-        if (codes) {
-            codes[q] = code;
-            radii[q] = __float_as_uint(o.f[0]);
-        }
         if (code >= S2M_OP_UNION) continue;
         const Iv v = iv_primitive(code, o.f, bl, bh);
         iv[q] = make_float2(v.lo, v.hi);
     }
 }
 
-// The job's program walked in order on those intervals; every lane takes the same steps
-// and writes the same list.
-__device__ __forceinline__ uint32_t walk_super(const SpJob& J, const float2* iv, const uint32_t* codes,
-                                               const uint32_t* radii, const PruneStack& S, uint32_t ln, uint16_t* out)
+// The super-tile's list of a program of at most kStageOps ops from its primitives' intervals: a
+// lane per op, level by level up the tree (an op when its operands are done), then down it for
+// the ops no operator above has dropped.  A walk in the program's order takes some 700 cycles
+// per op; a tree of 39 ops has six to eight levels.  `alive`: a word per op.
+__device__ __forceinline__ uint32_t prune_levels(const SpJob& J, float2* iv, uint32_t* alive, uint32_t ln, uint16_t* out)
+{
+    static_assert(kStageOps <= 128, "two ops per lane");
+    const uint32_t n = J.nops, levels = J.levels;
+    const uint32_t* tree = J.op_flops + n;
+    uint32_t code[2] = {0, 0}, place[2] = {0, 0};
+    float k[2] = {0.0f, 0.0f};
+    int keep[2] = {kKeepBoth, kKeepBoth};
+#pragma unroll
+    for (uint32_t s = 0; s < 2; ++s) {
+        const uint32_t q = ln + 64u * s;
+        if (q >= n) continue;
+        code[s] = J.ops[q].code;
+        k[s] = J.ops[q].f[0];
+        place[s] = tree[q];
+        alive[q] = q + 1u == n ? 1u : 0u;
+    }
+    __syncthreads();  // the intervals are visible
+    for (uint32_t h = 1; h <= levels; ++h) {
+#pragma unroll
+        for (uint32_t s = 0; s < 2; ++s) {
+            if (place[s] >> 16 != h) continue;
+            const uint32_t q = ln + 64u * s;
+            const float2 a = iv[place[s] & 0xffffu], b = iv[q - 1u];  // known iff lo > -kHuge
+            const Iv r = iv_op(code[s], Iv{a.x, a.y, a.x > -kHuge}, Iv{b.x, b.y, b.x > -kHuge}, k[s], keep[s]);
+            iv[q] = make_float2(r.lo, r.hi);
+        }
+        __syncthreads();
+    }
+    for (uint32_t h = levels; h >= 1; --h) {
+#pragma unroll
+        for (uint32_t s = 0; s < 2; ++s) {
+            const uint32_t q = ln + 64u * s;
+            if (place[s] >> 16 != h || !alive[q]) continue;
+            alive[place[s] & 0xffffu] = keep[s] != kKeepB;
+            alive[q - 1u] = keep[s] != kKeepA;
+        }
+        __syncthreads();
+    }
+    uint32_t len = 0;
+#pragma unroll
+    for (uint32_t s = 0; s < 2; ++s) {
+        const uint32_t q = ln + 64u * s;
+        const bool in = q < n && alive[q] && keep[s] == kKeepBoth;
+        const uint64_t w = __ballot(in);
+        if (in) out[len + (uint32_t)__builtin_popcountll(w & ((1ull << ln) - 1ull))] = (uint16_t)q;
+        len += (uint32_t)__builtin_popcountll(w);
+    }
+    const float2 top = iv[n - 1u];
+    return top.x > -kHuge && (top.x > 0.0f || top.y < 0.0f) ? kSingleSign : len;
+}
+
+// A longer program walked in order on those intervals; every lane takes the same steps and
+// writes the same list.
+__device__ __forceinline__ uint32_t walk_super(const SpJob& J, const float2* iv, const PruneStack& S, uint32_t ln,
+                                               uint16_t* out)
 {
     PruneWalk<false> w;  // the tiles' walks take its list in the program's order
     for (uint32_t q = 0; q < J.nops; ++q) {
-        const uint32_t code = __builtin_amdgcn_readfirstlane(codes ? codes[q] : J.ops[q].code);
+        const uint32_t code = __builtin_amdgcn_readfirstlane(J.ops[q].code);
         if (code < S2M_OP_UNION) {
             const float2 v = iv[q];
             w.prim(q, q, Iv{v.x, v.y, v.x > -kHuge}, out, S, ln);  // known iff lo > -kHuge
         } else {
-            w.op(q, code, codes ? __uint_as_float(radii[q]) : J.ops[q].f[0], out, S, ln);
+            w.op(q, code, J.ops[q].f[0], out, S, ln);
         }
     }
     return w.one_sign() ? kSingleSign : w.len;
@@ -686,10 +737,13 @@ __global__ __launch_bounds__(64) void k_sp_prune(SpPass P)
             sl = prune_fold(J, bl, bh, ln, in);
         } else {
             float2* iv = small ? reinterpret_cast<float2*>(T.f) : P.super_iv + s * P.list_stride;
-            uint32_t *codes = small ? T.code : nullptr, *radii = small ? T.iarg : nullptr;
-            prim_intervals(J, bl, bh, ln, iv, codes, radii);
-            __syncthreads();  // visible to all lanes
-            sl = walk_super(J, iv, codes, radii, S, ln, in);
+            prim_intervals(J, bl, bh, ln, iv);
+            if (small) {
+                sl = prune_levels(J, iv, sums, ln, in);
+            } else {
+                __syncthreads();  // visible to all lanes
+                sl = walk_super(J, iv, S, ln, in);
+            }
         }
         sl = __builtin_amdgcn_readfirstlane(sl);
     }
