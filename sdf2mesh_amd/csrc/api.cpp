@@ -357,11 +357,14 @@ uint32_t pick_slab(const s2m_params* p, const Job& j, bool streamed)
     // tables allow (64M cells; Mandelbulb 1024^3 left on the device: 8.0 ms at 16 planes per
     // slab, 6.1 at 32, 5.3 at 63).  Streamed to host memory, a slab's copy runs beside the next
     // slab's work: 16 slabs of at least 8M cells (Mandelbulb 512^3: 3.28 ms in 2 slabs, 2.63
-    // in 16; 256^3: 1.02 ms in 1 slab, 0.98 in 2, but a compiled CSG program with a third of
-    // the vertices 0.385 in 1, 0.389 in 2, 0.454 in 4).
+    // in 16), two from 6M cells on.  us in 1 / 2 / 3 slabs, Mandelbulb, a compiled CSG program
+    // and a GLSL estimator: 160^3 383 / 381 / 408, 232 / 265 / 301, 934 / 942 / 926; 200^3 552 /
+    // 524 / 520, 452 / 429 / 462, 1440 / 1398 / 1355; 250^3 669 / 646 / 637, 685 / 669 / 691,
+    // 1366 / 1256 / 1239.
     const uint64_t cells = plane * j.nz_cells;
-    const uint64_t slab_cells = streamed ? std::min<uint64_t>(std::max<uint64_t>(cells / 16, 8ull << 20), 64ull << 20)
-                                         : 64ull << 20;
+    uint64_t slab_cells = 64ull << 20;
+    if (streamed && cells >= (6ull << 20))
+        slab_cells = std::min(slab_cells, std::max(cells / 16, std::min<uint64_t>(8ull << 20, cells / 2)));
     if (t == 0) t = std::max<uint64_t>(1, (slab_cells + plane - 1) / plane);
     // keep the per-slab block count within one scan block
     const uint64_t max_t = std::max<uint64_t>(1, ((uint64_t)kMaxScanBlocks * kCellsPerBlock) / plane);
