@@ -800,10 +800,10 @@ int readback_finish(s2m_ctx* ctx, Readback& rb, uint64_t nv, uint64_t nt)
 // some 30.  One per 256 cell planes, 2 to 4 from 256 planes on (at 256^3 one would do, but a
 // job of that size is expected to be streamed); us in 1 / 2 / 3 / 4 passes:
 //             CSG-64 (much to copy)          a tree                      a torus
-//   256^3     456 / 486 / 544 / 620     214 / 282 / 361 / 417     208 / 232 / 277 / 334
-//   384^3     812 / 736 / 816 / 855     323 / 363 / 414 / 480     355 / 358 / 391 / 416
-//   512^3    1222 / 1107 / 1105 / 1142  441 / 423 / 493 / 542     536 / 529 / 529 / 570
-//   1024^3   4225 / 3820 / 3715 / 3647  1341 / 1199 / 1198 / 1273 1764 / 1670 / 1636 / 1622
+//   256^3     453 / 477 / 528 / 601     199 / 248 / 316 / 359     204 / 223 / 261 / 303
+//   384^3     810 / 729 / 803 / 840     300 / 327 / 380 / 428     349 / 352 / 377 / 409
+//   512^3    1219 / 1102 / 1097 / 1130  410 / 404 / 454 / 487     531 / 521 / 522 / 557
+//   1024^3   4216 / 3815 / 3707 / 3640  1186 / 1121 / 1083 / 1191 1753 / 1662 / 1627 / 1615
 uint32_t stream_passes(uint32_t tile_layers)
 {
     return tile_layers < 32 ? 1u : std::max<uint32_t>(2, std::min<uint32_t>(4, (tile_layers + 16) / 32));
@@ -811,8 +811,8 @@ uint32_t stream_passes(uint32_t tile_layers)
 
 // Most bytes a pass of a single sparse job holds per tile and row; larger grids take several
 // passes.  Every pass pays the tails of its kernels, their latency and the test of its last
-// cell plane for the next: CSG-64 1024^3 takes 1389 us in four passes (1 GiB each) and 1084
-// in one.  2.3 GB of 288 there; the next power of two is split in four.
+// cell plane for the next: CSG-64 1024^3 takes 1081 us in four passes (1 GiB each) and 828 in
+// one.  2.3 GB of 288 there; the next power of two is split in four.
 constexpr uint64_t kSparsePassBytes = 4ull << 30;
 
 // Is the program a left fold of library primitives (P0 P1 op1 P2 op2 ...) short enough to

@@ -1040,16 +1040,16 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
 // ---------------------------------------------------------------------------------
 // Staged cells are allocated in chunks of kStageChunk per block: the block's own, then one
 // counter update per chunk (with the first ones counted too, the blocks of a launch wait for
-// each other's update of one address: up to 15 us of a launch of 1792).  A slot needs room for 8 entries per live brick (its cells) when its tile starts, so
-// that its cells are contiguous, and takes what it has used; a chunk with less room left is
-// abandoned.  Hence at most (staged cells) + (room needed by the slots that open a chunk) +
-// blocks x kStageChunk are used; the host grows the buffer from the device count if that
-// exceeds it.
+// each other's update of one address: up to 15 us of a launch of 1792).  A slot needs room for
+// 8 entries per live brick (its cells) when its tile starts, so that its cells are contiguous,
+// and takes what it has used; a chunk with less room left is abandoned.  Hence at most (staged
+// cells) + (room needed by the slots that open a chunk) + blocks x kStageChunk are used; the
+// host grows the buffer from the device count if that exceeds it.
 constexpr uint32_t kStageChunk = kStageChunkHost;
 // Threads of a k_sp_tiles block (one tile at a time).  128 would share a tile's fixed work
 // among fewer waves, but then half of the waves fit (the box of the worst tile, 16^3 points,
 // and the rest take 21 KB of LDS: seven blocks per compute unit either way): 318 against 300 us
-// at CSG-64 1024^3, 201 against 153 at 512^3.
+// at CSG-64 1024^3, 201 against 153 at 512^3 (before the first chunks were the blocks' own).
 constexpr uint32_t kTileThreads = 256;
 static_assert(kRecVec - kRecPre <= kTileThreads, "one thread per record word past the read-ahead");
 constexpr int kGeneralPoints = 4;       // (k_sp_tiles<0>: a box of up to 1024 points in one round,
@@ -1206,9 +1206,10 @@ static_assert(kTileThreads >= kBoxAxis * kBoxAxis, "one box row per thread");
 // from it (contour_tile).  LINEAR = 1 runs the slots whose program is a left fold and skips
 // the others, LINEAR = 0 the others (gen_slots).
 // Bound by instruction issue (three quarters of the issue slots at CSG-64 1024^3: 69.5 k slots,
-// 258 points and 57 vertices each): of 300 us there, 60 evaluate, 42 place vertices, 28 look for
+// 258 points and 57 vertices each): of 277 us there, 60 evaluate, 42 place vertices, 28 look for
 // sign changes, the rest is the fixed work of a tile.  355 us with the points dealt to all
-// lanes, half of them twice, and a 64-bit division per row.
+// lanes, half of them twice, and a 64-bit division per row; 300 with every block's first
+// staging chunk counted (512^3: 166, 151, now 136).
 template <int LINEAR>
 __device__ __forceinline__ void tiles_body(const SpPass& P, uint32_t block, uint32_t blocks)
 {
@@ -1605,7 +1606,7 @@ __global__ __launch_bounds__(64) void k_sp_quadcount(SpPass P, MeshBufs b)
 // 50 us at copy speed.  So the loads of a slot are issued together (no branch between them),
 // rows are stored 8 bytes at a time, and blocks draw slots: with slots dealt out in advance
 // a block's share of vertices varies twofold and half of the waves idled at the end.
-// 325 -> 243 us there (69 k slots, 4.0 M vertices).
+// 325 -> 243 us there (69 k slots, 4.0 M vertices), 233 since no load waits for stores.
 // ---------------------------------------------------------------------------------
 // The first fold block of k_sp_emit after a job's last pass: the statistics summed and
 // counters[0 .. nback) to P.back (mapped host memory, NULL: not wanted).  Nothing in the
