@@ -25,4 +25,33 @@ __device__ __forceinline__ uint32_t wave_scan(uint32_t x)
     return x;
 }
 
+// The same for another operation on floats, `none` its neutral element.
+template <class Op>
+__device__ __forceinline__ float wave_scan(float x, float none, const Op& op)
+{
+    const int o = (int)__float_as_uint(none);
+    auto from = [&](auto move) { return __uint_as_float((uint32_t)move(o, (int)__float_as_uint(x))); };
+    x = op(x, from([](int n, int v) { return __builtin_amdgcn_update_dpp(n, v, 0x111, 0xf, 0xf, false); }));
+    x = op(x, from([](int n, int v) { return __builtin_amdgcn_update_dpp(n, v, 0x112, 0xf, 0xf, false); }));
+    x = op(x, from([](int n, int v) { return __builtin_amdgcn_update_dpp(n, v, 0x114, 0xf, 0xf, false); }));
+    x = op(x, from([](int n, int v) { return __builtin_amdgcn_update_dpp(n, v, 0x118, 0xf, 0xf, false); }));
+    x = op(x, from([](int n, int v) { return __builtin_amdgcn_update_dpp(n, v, 0x142, 0xa, 0xf, false); }));
+    x = op(x, from([](int n, int v) { return __builtin_amdgcn_update_dpp(n, v, 0x143, 0xc, 0xf, false); }));
+    return x;
+}
+__device__ __forceinline__ float wave_min(float x, float none) { return wave_scan(x, none, [](float a, float b) { return fminf(a, b); }); }
+__device__ __forceinline__ float wave_max(float x, float none) { return wave_scan(x, none, [](float a, float b) { return fmaxf(a, b); }); }
+__device__ __forceinline__ float wave_sum(float x) { return wave_scan(x, 0.0f, [](float a, float b) { return a + b; }); }
+
+// The last lane's value, and the value of the lane below (`none` for lane 0).
+__device__ __forceinline__ float last_lane(float x)
+{
+    return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(x), 63));
+}
+__device__ __forceinline__ float lane_below(float x, float none)
+{
+    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp((int)__float_as_uint(none), (int)__float_as_uint(x), 0x138,
+                                                                 0xf, 0xf, false));  // wave_shr:1
+}
+
 }  // namespace s2m

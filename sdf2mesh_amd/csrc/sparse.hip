@@ -546,22 +546,10 @@ __device__ __forceinline__ uint32_t prune_fold(const SpJob& J, const float* bl, 
         const float mag = prim ? fmaxf(fabsf(B.lo), fabsf(B.hi)) + kk : 0.0f;
         // prefix scans over the lanes (inclusive): min hi, sum and max of the magnitudes,
         // sum of k / 4, count of primitives
-        float u_ex = prim ? B.hi : kHuge, m_in = mag, x_in = mag, ka_in = 0.25f * kk, c_in = prim ? 1.0f : 0.0f;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const float uo = __shfl_up(u_ex, d, 64), mo = __shfl_up(m_in, d, 64);
-            const float xo = __shfl_up(x_in, d, 64), ko = __shfl_up(ka_in, d, 64), co = __shfl_up(c_in, d, 64);
-            if (ln >= (uint32_t)d) {
-                u_ex = fminf(u_ex, uo);
-                m_in += mo;
-                x_in = fmaxf(x_in, xo);
-                ka_in += ko;
-                c_in += co;
-            }
-        }
-        const float u_in = u_ex;  // inclusive
-        u_ex = __shfl_up(u_in, 1, 64);
-        if (ln == 0) u_ex = kHuge;
+        const float u_in = wave_min(prim ? B.hi : kHuge, kHuge);
+        float m_in = wave_sum(mag), x_in = wave_max(mag, 0.0f), ka_in = wave_sum(0.25f * kk);
+        float c_in = (float)__builtin_popcountll(__ballot(prim) & ((2ull << ln) - 1ull));
+        float u_ex = lane_below(u_in, kHuge);
         u_ex = fminf(u_ex, carry_u);
         m_in += carry_mag;
         x_in = fmaxf(x_in, carry_max);
@@ -578,20 +566,13 @@ __device__ __forceinline__ uint32_t prune_fold(const SpJob& J, const float* bl, 
         if (kept) out[nkept + (uint32_t)__builtin_popcountll(km & ((1ull << ln) - 1ull))] = (uint16_t)q;
         nkept += (uint32_t)__builtin_popcountll(km);
         // one-sign bounds over the kept primitives
-        float lo_k = (prim && !drop) ? B.lo : kHuge;
-        float k4 = (prim && !drop) ? 0.25f * kk : 0.0f;
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) {
-            lo_k = fminf(lo_k, __shfl_xor(lo_k, d, 64));
-            k4 += __shfl_xor(k4, d, 64);
-        }
-        carry_lo = fminf(carry_lo, lo_k);
-        carry_k4 += k4;
-        carry_u = fminf(carry_u, __shfl(u_in, 63, 64));
-        carry_mag = __shfl(m_in, 63, 64);
-        carry_max = __shfl(x_in, 63, 64);
-        carry_ka = __shfl(ka_in, 63, 64);
-        carry_cnt = __shfl(c_in, 63, 64);
+        carry_lo = fminf(carry_lo, last_lane(wave_min((prim && !drop) ? B.lo : kHuge, kHuge)));
+        carry_k4 += last_lane(wave_sum((prim && !drop) ? 0.25f * kk : 0.0f));
+        carry_u = fminf(carry_u, last_lane(u_in));
+        carry_mag = last_lane(m_in);
+        carry_max = last_lane(x_in);
+        carry_ka = last_lane(ka_in);
+        carry_cnt = last_lane(c_in);
         // the chunk's last primitive: at the highest odd q of the chunk (q = c0 + 63 when
         // the chunk is full; 64 is even, so lane 63 is odd)
         const uint32_t last = min(nops - c0, 64u) - 1u;
