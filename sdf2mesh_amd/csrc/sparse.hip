@@ -799,9 +799,9 @@ __global__ __launch_bounds__(64) void k_sp_prune(SpPass P)
             walk(w, P.lists + (size_t)tile * P.list_stride);
         }
     }
-    // slots for the surviving tiles: one counter update per wave.  (Some 25 ns each: 3.5 k of
-    // them bound a CSG-64 1024^3 job's 92 us here.  Four super-tiles per block and update took 98:
-    // the block waits for its slowest wave.)
+    // slots for the surviving tiles: one counter update per wave.  (Some 25 ns each, but fewer of
+    // them cost more than they gain: 92 us at CSG-64 1024^3, 98 with four super-tiles per block
+    // and update, the block waiting for its slowest wave, 107 with two per wave in turn.)
     const uint64_t m = __ballot(surface);
     uint64_t wbase = 0;
     if (ln == 0 && m) wbase = atomicAdd((unsigned long long*)&P.counters[kSlotsUsed], (unsigned long long)__builtin_popcountll(m));
