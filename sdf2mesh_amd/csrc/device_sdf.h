@@ -143,7 +143,9 @@ __device__ __forceinline__ float bailout_threshold(float b)
 // 0 <= offset <= 1000, iters >= 1 and gain <= 0.999 * 0.5 ln(bailout) bailout (mandel_gain):
 //   |p|^2 <= kMandelInner: |z| stays below 0.74 (0.74^8 + 0.648 < 0.74), so the last r < 1,
 //     ln r < 0 and the value is negative (or NaN);
-//   r >= bailout with dr * offset <= gain: 0.5 ln(r) r / dr exceeds the offset;
+//   r >= bailout with dr * per <= gain: 0.5 ln(r) r / dr exceeds the offset.  `per` is the
+//     offset, but at least gain / 2^100: past dr = 2^126 the hardware reciprocal is 0, and the
+//     value -offset, which is not positive even with offset 0 (orbits of some 40 steps and more);
 //   r^8 > 1.01 (bailout + |p|): the next |z| >= r^8 - |p| is past the bailout (or, in the
 //     last step, r^8 itself is), with the dr of this step.  The percent covers the
 //     roundings of z' (about 2e-5) where xy2 is not tiny;
@@ -162,11 +164,12 @@ __device__ __forceinline__ float mandelbulb8(float px, float py, float pz, float
                                              float bailout, float gain)
 {
     float zx = px, zy = py, zz = pz;
-    float r = 0.0f, dr = 1.0f, far = 0.0f;
+    float r = 0.0f, dr = 1.0f, far = 0.0f, per = 0.0f;
     bool out = false;
     if (kSign) {
         const float c2 = (px * px + py * py) + pz * pz;
         if (c2 <= kMandelInner) return -1.0f;
+        per = fmaxf(offset, gain * 0x1p-100f);
         far = 1.01f * (bailout + __builtin_amdgcn_sqrtf(c2));
     }
     for (uint32_t i = 0; i < iters; ++i) {
@@ -181,7 +184,7 @@ __device__ __forceinline__ float mandelbulb8(float px, float py, float pz, float
         const float r7 = (r4 * r2) * __builtin_amdgcn_sqrtf(r2);
         dr = __builtin_fmaf(r7 * dr, 8.0f, 1.0f);
         r = r4 * r4;
-        if (kSign && r > far && xy2 >= kMandelAxis && dr * offset <= gain) return 1.0f;
+        if (kSign && r > far && xy2 >= kMandelAxis && dr * per <= gain) return 1.0f;
         if (i + 1u == iters) break;
         const float irho = rsqrt_full(xy2);
         const float rho = xy2 * irho;
@@ -205,7 +208,7 @@ __device__ __forceinline__ float mandelbulb8(float px, float py, float pz, float
     }
     if (kSign) {
         if (!(r >= 1.0f)) return -1.0f;
-        if (out && dr * offset <= gain) return 1.0f;
+        if (out && dr * per <= gain) return 1.0f;
     }
     // 0.5 ln(r) r / dr from the hardware log2 (times ln 2; a denormal r scaled by 2^24
     // first) and reciprocal, each within about an ulp: dr >= 1, and r = 0 gives NaN as

@@ -54,6 +54,17 @@ def test_mandelbulb_signs(ctx, iterations, bailout, offset, swap):
         same(ctx.mesh(ctx.program(m), p), ctx.mesh(ctx.program(tape.union(m, m)), p))
 
 
+# Orbits of many steps: the derivative grows past 2^126, where the reciprocal the value takes is
+# 0.  With offset 0 that decides the sign, so an early positive one would leave cells out.
+@pytest.mark.parametrize("iterations,swap", [(256, True), (1024, False)])
+def test_mandelbulb_signs_of_deep_orbits(ctx, iterations, swap):
+    m = tape.mandelbulb(iterations, bailout=2.0, offset=0.0, swap_yz=swap)
+    p = s2m.Params((-1.25,) * 3, (1.25,) * 3, (160, 160, 160), 1e-4, s2m.DENSE_EVAL)
+    print(f"deep orbits {iterations}", flush=True)
+    a, b = ctx.program(m), ctx.program(tape.union(m, m))
+    same(ctx.mesh(a, p), ctx.mesh(b, p))
+
+
 OPS = [tape.union, tape.intersection, tape.subtraction] + [
     (lambda f: lambda a, b: f(a, b, 0.08))(f)
     for f in (tape.smooth_union, tape.smooth_intersection, tape.smooth_subtraction)]
