@@ -468,9 +468,9 @@ __device__ __forceinline__ void tiles_box(const SpJob& J, const uint32_t t0[3], 
     const float pad = 1.25f * (float)J.pad;
     const float* e[3] = {J.ext, J.ext + 2 * J.ntx, J.ext + 2 * J.ntx + 2 * J.nty};
     const uint32_t n[3] = {J.ntx, J.nty, J.ntz};
-    for (int a = 0; a < 3; ++a) {
-        bl[a] = e[a][t0[a]] - pad;
-        bh[a] = e[a][n[a] + t1[a]] + pad;
+    for (int a = 0; a < 3; ++a) {  // (an axis may run from its maximum to its minimum)
+        bl[a] = fminf(e[a][t0[a]], e[a][t1[a]]) - pad;
+        bh[a] = fmaxf(e[a][n[a] + t0[a]], e[a][n[a] + t1[a]]) + pad;
     }
 }
 
@@ -992,12 +992,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
                 RG.bm[a - 1u][i] = (uint8_t)m;
             }
         }
-        // brick b: cells c, c + 1 per axis; the first cell's lo corner, the second's hi corner
+        // brick b: cells c, c + 1 per axis, from the first cell's lo corner to the second's hi
+        // corner (which lies below it on an axis that runs from its maximum to its minimum)
         const uint32_t c[3] = {(b & 3u) * 2u, ((b >> 2) & 3u) * 2u, (b >> 4) * 2u};
         float bl[3], bh[3];
         for (int a = 0; a < 3; ++a) {
-            bl[a] = A.clo[a][c[a]];
-            bh[a] = A.chi[a][c[a] + 1];
+            const float lo = A.clo[a][c[a]], hi = A.chi[a][c[a] + 1];
+            bl[a] = fminf(lo, hi);
+            bh[a] = fmaxf(lo, hi);
         }
         Iv acc = iv_primitive(uniform_code(T, 0), T.f_at(0), bl, bh);
         for (uint32_t k = 1; k + 1 < n; k += 2) {

@@ -173,3 +173,22 @@ def test_small_meshes_land(ctx, res):
     b = ctx.mesh_to_host(prog, p)
     assert np.array_equal(np.asarray(b.vertices()).view(np.uint32).reshape(-1, 6), a.vertices.view(np.uint32))
     assert np.array_equal(np.asarray(b.triangles()).reshape(-1, 3), a.triangles)
+
+
+# Boxes with an axis (or all) running from its maximum to its minimum: the coordinate tables
+# descend, and the intervals of bricks, tiles and super-tiles are still ordered.
+@pytest.mark.parametrize("axes", [(0,), (1,), (2,), (0, 1, 2)])
+@pytest.mark.parametrize("flags", [0, s2m.CORNERS_EXACT])
+def test_reversed_axes(ctx, axes, flags):
+    a = parts(5, 2)
+    lo, hi = [-1.0, -1.1, -0.9], [1.05, 1.0, 1.1]
+    for k in axes:
+        lo[k], hi[k] = hi[k], lo[k]
+    for node in (tape.sphere((0.0, 0.0, 0.0), 0.5), tape.csg64(), right_nested(a, OPS[::-1]), unfoldable(3, 5)):
+        print(f"reversed {axes} flags={flags} ops={len(node.tape())}", flush=True)
+        p = s2m.Params(tuple(lo), tuple(hi), (70, 66, 72), 1e-4, flags)
+        d = s2m.Params(tuple(lo), tuple(hi), (70, 66, 72), 1e-4, flags | s2m.DENSE_EVAL)
+        m = ctx.mesh(ctx.program(node), p)
+        assert len(m.vertices) > 0
+        same(m, ctx.mesh(ctx.program(node), d))
+        assert_same_mesh(m, reference_mesh(node, p))
