@@ -187,7 +187,7 @@ typedef struct s2m_timing {
     double quad_ms;     /* quad count, scan, triangle emission (pruned path: the
                            quad count)                                              */
     double d2h_ms;      /* device-to-host copies (s2m_mesh only)                    */
-    uint64_t eval_launches;
+    uint64_t eval_launches;  /* dense path: of every attempt, where a buffer overflowed */
     uint64_t lattice_points; /* SDF evaluations done on the lattice                 */
     uint64_t slabs;
     uint64_t tiles_total;    /* tiles of 8^3 cells (pruned path; 0 when dense)       */

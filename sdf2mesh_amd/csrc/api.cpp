@@ -159,6 +159,7 @@ struct s2m_ctx {
     const void* dev_img_at = nullptr;  // ... at this device address
     PinnedBuf host_back;  // device counters and per-job ranges read back after a pass
     uint64_t vcap = 0, tcap = 0;
+    uint64_t dense_stage = 0;  // staged vertices of a dense slab: the most a job has asked for
     uint64_t last_nvtx = 0, last_ntri = 0, last_invalid = 0;
     std::vector<hipEvent_t> events;
     size_t events_used = 0;
@@ -1558,7 +1559,8 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
         want_v = fx->vcap;
         want_t = fx->tcap;
     }
-    uint64_t want_s = fx ? 0 : est_v + est_v / 4;  // staged vertices of a slab (cells with a sign change)
+    // staged vertices of a slab (cells with a sign change)
+    uint64_t want_s = fx ? 0 : std::max<uint64_t>(est_v + est_v / 4, ctx->dense_stage);
     // Several slabs: slab k + 1's signs are evaluated (VALU-bound) on eval_stream, into the
     // other of two sets of sign words (and kept values), while slab k is contoured on the context's stream.
     // Events order it: a slab's bricks are listed after its evaluation, an evaluation waits
@@ -1593,6 +1595,7 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
         HIP_TRY(hipHostGetDevicePointer(&back_dev, ctx->host_back.p, 0));
     }
 
+    uint64_t eval_launches = 0;  // of all attempts
     for (int attempt = 0; attempt < (fx ? 1 : 3); ++attempt) {
         // the working buffers
         if (!fx) {
@@ -1797,7 +1800,7 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
             if (rb) {  // the slab's vertices and triangles are final; the copies of the slab two
                        // before (waiting for it leaves this slab and the next evaluation queued)
                 int rrc = readback_mark(ctx, (uint32_t)slabs);
-                if (!rrc && slabs > 1) rrc = readback_pass(ctx, *rb, want_v, want_t, ~0ull, ~0ull);
+                if (!rrc && slabs > 1) rrc = readback_pass(ctx, *rb, want_v, want_t, ~0ull, L.stage_cap);
                 if (rrc) return rrc;
             }
             if (prof) ev.insert(ev.end(), m, m + 6);
@@ -1808,14 +1811,15 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
             HIP_TRY(hipEventRecord(ev_end, ctx->stream));
         }
         if (rb) {  // copies of each slab's mesh while the later slabs run
-            const int rrc = readback_passes(ctx, *rb, (uint32_t)slabs, want_v, want_t, ~0ull, ~0ull);
+            const int rrc = readback_passes(ctx, *rb, (uint32_t)slabs, want_v, want_t, ~0ull, L.stage_cap);
             if (rrc) return rrc;
         }
         if (land) {  // a small mesh's copy behind its last kernel
             uint64_t t[kSnapWords];
             int lrc = snapshot_wait(ctx, 0, t);
             land->landed = false;
-            if (!lrc && t[0] <= want_v && t[1] <= want_t) lrc = land_mesh(ctx, *land, t[0], t[1]);
+            if (!lrc && t[0] <= want_v && t[1] <= want_t && t[3] <= L.stage_cap)
+                lrc = land_mesh(ctx, *land, t[0], t[1]);
             if (lrc) return lrc;
         }
         uint64_t cnt[kNumCounters];
@@ -1838,7 +1842,8 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
                 ctx->timing.quad_ms += t3;
             }
         }
-        ctx->timing.eval_launches = h_corners ? 0 : slabs;
+        eval_launches += h_corners ? 0 : slabs;
+        ctx->timing.eval_launches = eval_launches;
         ctx->timing.slabs = slabs;
         ctx->timing.lattice_points = lattice_points;
         if (prog) {
@@ -1870,7 +1875,7 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
         if (cnt[kVtxTotal] > want_v) want_t = std::max<uint64_t>(want_t, 3 * (cnt[kVtxTotal] + cnt[kVtxTotal] / 8));
         if (cnt[kVtxTotal] > want_v) want_v = cnt[kVtxTotal] + cnt[kVtxTotal] / 8 + 1024;
         if (cnt[kTriTotal] > want_t) want_t = cnt[kTriTotal] + cnt[kTriTotal] / 8 + 2048;
-        if (!staged) want_s = cnt[kStageMax] + cnt[kStageMax] / 8 + 1024;
+        if (!staged) ctx->dense_stage = want_s = cnt[kStageMax] + cnt[kStageMax] / 8 + 1024;
     }
     return fail(S2M_E_OOM, "output buffers kept overflowing");
 }

@@ -444,7 +444,7 @@ __global__ __launch_bounds__(1024) void k_tri_offsets(const uint32_t* __restrict
     if (t == 0) {
         counters[kTriPrev] = prev;
         counters[kTriTotal] = run;
-        if (snap) write_snapshot(snap, counters[kVtxTotal], run, 0, 0);
+        if (snap) write_snapshot(snap, counters[kVtxTotal], run, 0, counters[kBrickAlloc] >> 32);
     }
 }
 

@@ -192,3 +192,31 @@ def test_reversed_axes(ctx, axes, flags):
         assert len(m.vertices) > 0
         same(m, ctx.mesh(ctx.program(node), d))
         assert_same_mesh(m, reference_mesh(node, p))
+
+
+# A dense job with more sign changes per slab than the first estimate of the staging buffer
+# repeats once with the device's count; the context keeps that size, so the same job runs once
+# when it comes again.  A cube in one slab, one in slabs, and one streamed to host memory.
+@pytest.mark.parametrize("res,slab", [(64, 0), (96, 40), (188, 0)])
+def test_staging_capacity_kept(res, slab):
+    wave = """use sdf3d::*;
+fn sdf3d(p: vec3f) -> f32 {
+    let q = p * %s;
+    return sin(q.x) * cos(q.y) + sin(q.y) * cos(q.z) + sin(q.z) * cos(q.x);
+}
+""" % tape.wgsl_float(0.6 * res)
+    with s2m.Context(0) as fresh:
+        prog = fresh.program_from_source(wave)
+        p = s2m.Params.reference(res, 2.0, flags=0)
+        p.slab = slab
+        print(f"staging {res} slab={slab}", flush=True)
+        first = fresh.mesh(prog, p)
+        t = fresh.last_timing()
+        assert t["eval_launches"] > t["slabs"]  # more than the estimate holds
+        for _ in range(2):
+            same(first, fresh.mesh(prog, p))
+            t = fresh.last_timing()
+            assert t["eval_launches"] == t["slabs"]
+        fresh.mesh(prog, s2m.Params.reference(32, 2.0))
+        same(first, fresh.mesh(prog, p))
+        assert fresh.last_timing()["eval_launches"] == t["slabs"]
