@@ -292,7 +292,7 @@ void s2m_mesh_free(s2m_mesh_out* out);
  * synchronises the stream. */
 #define S2M_NOALLOC_SCRATCH_BYTES (64u << 20)
 typedef struct s2m_mesh_buffers {
-    float* vtx;          /* device: 6 floats per vertex, vcap vertices                    */
+    float* vtx;          /* device: 6 floats per vertex, vcap vertices (4-byte aligned)   */
     uint64_t* cell_keys; /* device: vcap keys (working storage of the quad pass too)      */
     uint8_t* signs;      /* device: vcap sign bytes (read by the quad pass)               */
     uint64_t vcap;

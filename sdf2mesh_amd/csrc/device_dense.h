@@ -322,7 +322,7 @@ __device__ __forceinline__ float quad_lane(float v)
 // bricks at a time per block of 256, their vertices listed together.  LibraryNormal: four
 // lanes per vertex, one per tap (sdf3d_normal.wgsl:4-9: v1=(1,-1,-1), v2=(-1,-1,1),
 // v3=(-1,1,-1), v4=(1,1,1) at p + v * eps, summed left to right, normalized), so the SDF is
-// inlined once; three of them store the vertex as 8-byte pairs.  Otherwise N(px, py, pz,
+// inlined once; three of them store the vertex as 8-byte pairs where vtx allows it.  Otherwise N(px, py, pz,
 // eps, o) writes o[3..5], one lane per vertex.
 template <class F, class N>
 __device__ __forceinline__ void emit_bricks(const F& sdf, const N& normal, const BrickArgs& a)
@@ -332,6 +332,7 @@ __device__ __forceinline__ void emit_bricks(const F& sdf, const N& normal, const
     constexpr bool kTaps = __is_same(N, LibraryNormal);
     const uint32_t l = threadIdx.x & 63u, w = threadIdx.x >> 6, nrec = (uint32_t)*a.alloc;
     const uint32_t tap = kTaps ? l & 3u : 0u;
+    const bool pairs = ((size_t)a.vtx & 7u) == 0;  // a caller's buffer may be 4-byte aligned
     for (uint32_t r0 = blockIdx.x * 4u; r0 < nrec; r0 += gridDim.x * 4u) {  // block-uniform
         const bool mine = r0 + w < nrec;
         const BrickRec* R = a.recs + (mine ? r0 + w : r0);
@@ -382,10 +383,14 @@ __device__ __forceinline__ void emit_bricks(const F& sdf, const N& normal, const
                     write_unit(nrm, ((d1 + (-d2)) + (-d3)) + d4, (((-d1) + (-d2)) + d3) + d4,
                                (((-d1) + d2) + (-d3)) + d4);
                 }
-                if (tap < 3u)
-                    *reinterpret_cast<float2*>(o + 2 * tap) =
-                        make_float2(tap == 0u ? nrm[0] : tap == 1u ? nrm[2] : nrm[4],
-                                    tap == 0u ? nrm[1] : tap == 1u ? nrm[3] : nrm[5]);
+                const float n0 = tap == 0u ? nrm[0] : tap == 1u ? nrm[2] : nrm[4];
+                const float n1 = tap == 0u ? nrm[1] : tap == 1u ? nrm[3] : nrm[5];
+                if (tap < 3u && pairs) {
+                    *reinterpret_cast<float2*>(o + 2 * tap) = make_float2(n0, n1);
+                } else if (tap < 3u) {
+                    o[2 * tap] = n0;
+                    o[2 * tap + 1] = n1;
+                }
             } else {
                 o[0] = px;
                 o[1] = py;

@@ -130,3 +130,20 @@ def test_noalloc_reports_sizes_and_limits(ctx):
         assert e.value.code == s2m.E_ARG
     finally:
         one.free()
+
+
+@pytest.mark.parametrize("node,bounds", [(tape.csg64(), 2.0), (tape.mandelbulb(5), 2.5)])
+def test_noalloc_vertices_at_any_float_address(ctx, node, bounds):
+    # the caller's vertex buffer needs the alignment of its floats only
+    prog = ctx.program(node)
+    p = s2m.Params.reference(64, bounds, flags=0)
+    bufs = DeviceBuffers(100_000, 200_000)
+    base = bufs.ptr["vtx"]
+    try:
+        for shift in (4, 8, 12):
+            print(f"noalloc: vertices {shift} bytes past an aligned address", flush=True)
+            bufs.ptr["vtx"], bufs.vcap = base + shift, 99_999
+            check_same(ctx, prog, p, bufs)
+    finally:
+        bufs.ptr["vtx"] = base
+        bufs.free()
