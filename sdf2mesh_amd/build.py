@@ -40,7 +40,7 @@ SOURCES = ["kernels.hip", "sparse.hip", "api.cpp", "hostmem.cpp", "tune.cpp", "s
 # Device headers a program compiled at run time includes, in order; written into one
 # string (rtc_source.inc) that hiprtc receives ahead of the generated code.
 RTC_HEADERS = [PKG.parent / "include" / "sdf2mesh.h", CSRC / "device_sdf.h", CSRC / "dense_args.h",
-               CSRC / "device_dense.h",               CSRC / "rtc_prelude.h"]
+               CSRC / "device_dense.h", CSRC / "rtc_prelude.h"]
 RTC_TYPES = """typedef __hip_internal::uint8_t uint8_t;
 typedef __hip_internal::uint16_t uint16_t;
 typedef __hip_internal::uint32_t uint32_t;

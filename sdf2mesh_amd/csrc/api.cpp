@@ -119,7 +119,7 @@ struct s2m_program {
     bool owns_device_copy = true;  // false: d_ops points into a caller-owned arena
     // compiled programs (hiprtc code object): dense-path kernels instead of a tape
     hipModule_t module = nullptr;
-    hipFunction_t k_lattice = nullptr, k_signs = nullptr, k_contour = nullptr, k_emit = nullptr;
+    hipFunction_t k_lattice = nullptr, k_signs = nullptr, k_normals = nullptr;
 };
 
 struct s2m_ctx {
@@ -1441,18 +1441,15 @@ hipError_t signs_prog(hipStream_t s, const s2m_program* prog, BrickArgs a)
     return hipModuleLaunchKernel(prog->k_signs, g.x, g.y, g.z, 256, 1, 1, 0, s, args, nullptr);
 }
 
-hipError_t contour_prog(hipStream_t s, const s2m_program* prog, BrickArgs a)
+// A compiled program's normals of the slab's vertices (a tape's are k_emit's).
+hipError_t normals_prog(hipStream_t s, const s2m_program* prog, float eps, const MeshBufs& b)
 {
-    if (!prog->module) return launch_contour(s, a, prog->ops.data(), prog->d_ops, prog->n);
-    void* args[] = {&a};
-    return hipModuleLaunchKernel(prog->k_contour, kBrickBlocks, 1, 1, 256, 1, 1, 0, s, args, nullptr);
-}
-
-hipError_t emit_prog(hipStream_t s, const s2m_program* prog, BrickArgs a)
-{
-    if (!prog->module) return launch_emit(s, a, prog->ops.data(), prog->d_ops, prog->n);
-    void* args[] = {&a};
-    return hipModuleLaunchKernel(prog->k_emit, kBrickBlocks, 1, 1, 256, 1, 1, 0, s, args, nullptr);
+    if (!prog->module) return hipSuccess;
+    float* vtx = b.vtx;
+    const uint64_t* counters = b.counters;
+    uint64_t vcap = b.vcap;
+    void* args[] = {&eps, &vtx, &counters, &vcap};
+    return hipModuleLaunchKernel(prog->k_normals, kBrickBlocks, 1, 1, 256, 1, 1, 0, s, args, nullptr);
 }
 
 // Buffers of a dense job that must not allocate (s2m_mesh_device_noalloc): every working
@@ -1474,6 +1471,8 @@ struct FixedBufs {
 // slab read the slab before).
 struct DenseLayout {
     uint32_t T, nx, ny, nbx, nby, max_nzl, max_blocks;
+    uint32_t strip, nstrips;  // brick rows per strip: the words and values of a strip (and of its
+                              // successor's first row) are held at a time
     size_t stage_cap;
     size_t tables, words, vals, recs, stage, stage_sign, actbits, wpre, blocks, chunks, tblocks, counters;
     bool piped;   // two sets of words and values
@@ -1487,9 +1486,10 @@ struct DenseLayout {
     }
 };
 
-// stage_cap: vertices staged per slab, 0 for one per cell.  vals: the values of bricks with
-// both signs are kept.
-DenseLayout dense_layout(const Job& j, uint32_t T, bool bricks, bool piped, uint64_t stage_cap, bool vals)
+// stage_cap: vertices staged per slab, 0 for one per cell.  vals: the values of bricks (with
+// both signs, or all) are kept.  strip: 0 for one strip.
+DenseLayout dense_layout(const Job& j, uint32_t T, bool bricks, bool piped, uint64_t stage_cap, bool vals,
+                         uint32_t strip = 0)
 {
     DenseLayout L{};
     const uint64_t plane = (uint64_t)j.res[0] * j.res[1];
@@ -1502,13 +1502,16 @@ DenseLayout dense_layout(const Job& j, uint32_t T, bool bricks, bool piped, uint
         const uint32_t z1 = std::min(z0 + T, j.nz_cells);
         L.max_nzl = std::max(L.max_nzl, j.ax[2].hi[z1 - 1] - j.ax[2].lo[z0] + 1);
     }
+    L.strip = strip ? std::min(strip, L.nby) : L.nby;
+    L.nstrips = (L.nby + std::max(L.strip, 1u) - 1u) / std::max(L.strip, 1u);
+    const size_t rows = std::min(L.strip + 1u, L.nby);  // of the words and values
     const size_t nbricks = bricks ? (size_t)L.nbx * L.nby * ((L.max_nzl + 3u) / 4u) : 0;
     L.max_blocks = (uint32_t)((plane * T + kCellsPerBlock - 1) / kCellsPerBlock);
     L.stage_cap = bricks ? (size_t)(stage_cap ? std::min<uint64_t>(stage_cap, plane * T) : plane * T) : 0;
     L.piped = piped;
     L.tables = tables_bytes(j);
-    L.words = nbricks * sizeof(uint64_t);
-    L.vals = vals ? nbricks * 64 * sizeof(float) : 0;
+    L.words = bricks ? L.nbx * rows * ((L.max_nzl + 3u) / 4u) * sizeof(uint64_t) : 0;
+    L.vals = vals ? L.nbx * rows * 16 * L.max_nzl * sizeof(float) : 0;  // brick_vals
     L.recs = nbricks * sizeof(BrickRec);
     L.stage = L.stage_cap * 3 * sizeof(float);
     L.stage_sign = L.stage_cap;
@@ -1517,7 +1520,7 @@ DenseLayout dense_layout(const Job& j, uint32_t T, bool bricks, bool piped, uint
     L.wpre = (size_t)L.max_blocks * (kCellsPerBlock / 64) * sizeof(uint16_t);
     L.tblocks = (size_t)((plane * T + kBlock - 1) / kBlock) * sizeof(uint32_t);
     L.chunks = kRankChunks * sizeof(uint32_t);
-    L.counters = kNumCounters * sizeof(uint64_t);
+    L.counters = (kNumCounters + (L.nstrips > 1 ? L.nstrips : 0)) * sizeof(uint64_t);  // and the strips' kBrickAlloc
     return L;
 }
 
@@ -1567,10 +1570,14 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
     // until the slab two before has contoured its bricks (the last reader of its words and
     // kept values), and the first evaluation waits for the tables queued before it.
     const bool piped = !fx && !h_corners && slab < j.nz_cells;
-    const bool keep_vals = prog && !fx && !h_corners && !sign_early(prog->ops.data(), prog->n);
+    // the values a compiled program's vertices are placed from; a tape's are evaluated where
+    // they are not kept
+    const bool keep_vals = prog && !h_corners && (prog->module || (!fx && !sign_early(prog->ops.data(), prog->n)));
     DenseLayout L = dense_layout(j, slab, !h_corners, piped, want_s, keep_vals);
     if (fx) {  // the largest slab (at most the usual one) whose buffers fit the scratch
-        while (L.T > 1 && L.carved() > fx->scratch_bytes) L = dense_layout(j, L.T - 1, true, false, 0, false);
+        while (L.T > 1 && L.carved() > fx->scratch_bytes) L = dense_layout(j, L.T - 1, true, false, 0, keep_vals);
+        while (keep_vals && L.strip > 1 && L.carved() > fx->scratch_bytes)  // one cell plane in strips
+            L = dense_layout(j, 1, true, false, 0, true, (L.strip + 1) / 2);
         if (L.carved() > fx->scratch_bytes)
             return fail(S2M_E_ARG, "a %u x %u grid needs %llu bytes of working memory per cell plane; "
                                    "the no-allocation scratch holds %llu",
@@ -1665,7 +1672,8 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
             if (src) return src;
         }
 
-        HIP_TRY(launch_dense_begin(ctx->stream, b.counters, act_buf[0],
+        const uint32_t ncounters = (uint32_t)(L.counters / sizeof(uint64_t));
+        HIP_TRY(launch_dense_begin(ctx->stream, b.counters, ncounters, act_buf[0],
                                    (uint32_t)(plane * std::min(T, j.nz_cells)), tables_from, tables_at,
                                    tables_from ? L.tables : 0, base_buf[0]));
 
@@ -1734,9 +1742,8 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
             A.nzl = nzl;
             A.lz0 = lz0;
             A.nbx = L.nbx;
-            A.nby = L.nby;
+            A.nby = A.own = L.nby;
             A.nbz = (nzl + 3u) / 4u;
-            A.run = sign_run((uint64_t)A.nbx * A.nby * A.nbz);
             A.rx = a.rx;
             A.ry = a.ry;
             A.z0 = z0;
@@ -1758,6 +1765,21 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
             A.vcap = b.vcap;
             A.eps = p->eps;
             A.normals = normals ? 1u : 0u;
+            A.run = sign_run((uint64_t)A.nbx * A.nby * A.nbz);
+            auto strip = [&](uint32_t k) {  // brick rows k * L.strip ..: its own records and staging space
+                BrickArgs B = A;
+                if (L.nstrips == 1) return B;
+                B.by0 = k * L.strip;
+                B.own = std::min(L.strip, L.nby - B.by0);
+                B.nby = std::min(B.own + 1u, L.nby - B.by0);
+                B.run = sign_run((uint64_t)B.nbx * B.nby * B.nbz);
+                B.recs = recs + (size_t)B.by0 * B.nbx * B.nbz;
+                B.alloc = b.counters + kNumCounters + k;
+                const std::vector<uint32_t>& lo = j.ax[1].lo;  // ascending
+                const size_t rows = std::lower_bound(lo.begin(), lo.end(), 4u * B.by0) - lo.begin();
+                B.stage0 = (uint32_t)(rows * a.rx * nzc);
+                return B;
+            };
 
             hipEvent_t m[6] = {};
             if (prof)
@@ -1765,7 +1787,7 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
             if (piped && words_free[cur]) HIP_TRY(hipStreamWaitEvent(es, words_free[cur], 0));
             if (m[0]) HIP_TRY(hipEventRecord(m[0], es));
             if (!h_corners) {
-                HIP_TRY(signs_prog(es, prog, A));
+                HIP_TRY(signs_prog(es, prog, strip(0)));
                 lattice_points += (uint64_t)L.nx * L.ny * nzl;
             }
             if (m[1]) HIP_TRY(hipEventRecord(m[1], es));
@@ -1776,11 +1798,16 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
             }
             if (m[5]) HIP_TRY(hipEventRecord(m[5], ctx->stream));
             const float* src = h_corners ? ctx->corners.as<float>() + (size_t)z0 * plane * 8 : nullptr;
+            const uint32_t tape_ops = prog && !prog->module ? prog->n : 0u;
+            const s2m_op* host_ops = tape_ops ? prog->ops.data() : nullptr;
             if (h_corners) {
                 HIP_TRY(launch_cells_from_corners(ctx->stream, a, src, bs, 0));
             } else {
-                HIP_TRY(launch_find_bricks(ctx->stream, A));
-                HIP_TRY(contour_prog(ctx->stream, prog, A));
+                for (uint32_t k = 0; k < L.nstrips; ++k) {
+                    if (k) HIP_TRY(signs_prog(ctx->stream, prog, strip(k)));
+                    HIP_TRY(launch_find_bricks(ctx->stream, strip(k)));
+                    HIP_TRY(launch_contour(ctx->stream, strip(k), host_ops, prog->d_ops, tape_ops));
+                }
                 if (piped) {
                     words_free[cur] = mark(ctx->stream);
                     if (!words_free[cur]) return fail(S2M_E_HIP, "event record failed");
@@ -1789,11 +1816,13 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
             HIP_TRY(launch_ranks(ctx->stream, bs, a.ncells));
             if (m[2]) HIP_TRY(hipEventRecord(m[2], ctx->stream));
             if (h_corners) HIP_TRY(launch_cells_from_corners(ctx->stream, a, src, bs, 1));
-            else HIP_TRY(emit_prog(ctx->stream, prog, A));
+            for (uint32_t k = 0; !h_corners && k < L.nstrips; ++k)
+                HIP_TRY(launch_emit(ctx->stream, strip(k), host_ops, prog->d_ops, tape_ops));
+            if (!h_corners && normals) HIP_TRY(normals_prog(ctx->stream, prog, p->eps, b));
             if (m[3]) HIP_TRY(hipEventRecord(m[3], ctx->stream));
             HIP_TRY(launch_quads(ctx->stream, a, bs, prev, snap_dev ? snap_dev + kSnapWords * slabs : nullptr));
             // the other activity words cleared for the next slab
-            HIP_TRY(launch_slab_end(ctx->stream, b.counters, act_buf[cur ^ 1],
+            HIP_TRY(launch_slab_end(ctx->stream, b.counters, ncounters, act_buf[cur ^ 1],
                                     (uint32_t)(plane * std::min(T, j.nz_cells - z1)), base_buf[cur ^ 1],
                                     z1 == j.nz_cells ? static_cast<uint64_t*>(back_dev) : nullptr));
             if (m[4]) HIP_TRY(hipEventRecord(m[4], ctx->stream));
@@ -2837,8 +2866,7 @@ int program_from_code_object(s2m_ctx* ctx, const void* code, size_t size, s2m_pr
     hipError_t e = hipModuleLoadData(&p->module, code);
     if (e == hipSuccess) e = hipModuleGetFunction(&p->k_lattice, p->module, "s2m_c_eval_lattice");
     if (e == hipSuccess) e = hipModuleGetFunction(&p->k_signs, p->module, "s2m_c_signs");
-    if (e == hipSuccess) e = hipModuleGetFunction(&p->k_contour, p->module, "s2m_c_contour");
-    if (e == hipSuccess) e = hipModuleGetFunction(&p->k_emit, p->module, "s2m_c_emit");
+    if (e == hipSuccess) e = hipModuleGetFunction(&p->k_normals, p->module, "s2m_c_normals");
     if (e != hipSuccess) {
         if (p->module) (void)hipModuleUnload(p->module);
         delete p;

@@ -1,16 +1,16 @@
-// device_dense.h - bodies of the dense path's kernels that evaluate the SDF, templated on
-// it.  The tape interpreter's kernels (kernels.hip) and the kernels of programs compiled at
-// run time by hiprtc instantiate the same bodies, so both paths run identical per-point
-// code around their SDF.
+// device_dense.h - bodies of the dense path's kernels that evaluate the SDF at given points,
+// templated on it.  The tape interpreter's kernels (kernels.hip) and the kernels of programs
+// compiled at run time by hiprtc instantiate the same bodies, so both paths run identical
+// per-point code around their SDF.  What else the dense path does (device_bricks.h) is
+// compiled once, in the library: in every program's module it took half of the 130 ms that
+// compiling one takes otherwise.
 //
 // A slab's corner lattice is handled in bricks of 4 x 4 x 4 points.  sign_words evaluates
-// every point but keeps only `value > 0`, one 64-bit word per brick; bricks whose cells
-// change sign are listed (k_find_bricks), and contour_bricks needs the values at just the
-// corners of those cells.  Those inside bricks with both signs are kept by sign_words (a
-// 256-byte line per brick), the others evaluated again.  Against a lattice of floats
-// written to memory and read back by the contour pass, this moves about 1/20 of the bytes;
-// the values computed twice are some of the corners of cells at the surface (well under
-// 1 % of the points at 512^3).
+// every point and keeps `value > 0`, one 64-bit word per brick; bricks whose cells change
+// sign are listed (k_find_bricks), and contour_bricks needs the values at just the corners
+// of those cells.  A compiled program's values are all kept (4 bytes a point beside a whole
+// program each).  Of a tape's, those inside bricks with both signs are kept (a 256-byte line
+// per brick), the others evaluated again: well under 1 % of the points at 512^3.
 #pragma once
 #ifndef __HIPCC_RTC__
 #include <hip/hip_runtime.h>
@@ -56,12 +56,21 @@ __device__ __forceinline__ void write_unit(float* o, float gx, float gy, float g
 
 __device__ __forceinline__ uint32_t clamp_to(uint32_t i, uint32_t n) { return i < n ? i : n - 1u; }
 
+// Where the values of brick (bx, by, bz), by counted from by0, start: 16 per lattice plane of
+// the slab in it, bricks of one layer after each other.
+__device__ __forceinline__ size_t brick_vals(const BrickArgs& a, uint32_t bx, uint32_t by, uint32_t bz)
+{
+    const uint32_t planes = a.nzl - 4u * bz < 4u ? a.nzl - 4u * bz : 4u;
+    return 16u * ((size_t)bz * 4u * a.nby * a.nbx + ((size_t)by * a.nbx + bx) * planes);
+}
+
 // Sign of an SDF at a point as that of its value, without a test on whole bricks.
-template <class F>
+template <class F, bool KEEP_ALL>
 struct PointSign {
     F sdf;
-    static constexpr bool kBricks = false;  // brick() decides whole bricks
-    static constexpr bool kValue = true;    // operator() returns the value itself
+    static constexpr bool kBricks = false;   // brick() decides whole bricks
+    static constexpr bool kValue = true;     // operator() returns the value itself
+    static constexpr bool kAll = KEEP_ALL;   // every brick's values are kept
     __device__ float operator()(float x, float y, float z) const { return sdf(x, y, z); }
     __device__ int brick(float, float, float, float, float, float) const { return -1; }
 };
@@ -79,10 +88,12 @@ __device__ __forceinline__ void sign_words(const S& sign, const BrickArgs& a)
     const uint32_t b0 = blockIdx.x * a.run, by = blockIdx.y * 4u + w, bz = blockIdx.z;
     if (by >= a.nby) return;
     const float xr = a.cx[clamp_to(b0 * 4u + l, a.nx)];
-    const float y = a.cy[clamp_to(by * 4u + ((l >> 2) & 3u), a.ny)];
+    const float y = a.cy[clamp_to((a.by0 + by) * 4u + ((l >> 2) & 3u), a.ny)];
     const float z = a.cz[a.lz0 + clamp_to(bz * 4u + (l >> 4), a.nzl)];
     const uint32_t nb = min(a.run, a.nbx - b0);
     const size_t row = ((size_t)bz * a.nby + by) * a.nbx + b0;
+    const uint32_t planes16 = 16u * min(a.nzl - 4u * bz, 4u);  // values of a brick
+    float* const vals = a.vals ? a.vals + brick_vals(a, b0, by, bz) : nullptr;
     uint64_t word = 0;  // lane b: brick b's
     uint32_t todo = (1u << nb) - 1u;
     if constexpr (S::kBricks) {
@@ -105,211 +116,12 @@ __device__ __forceinline__ void sign_words(const S& sign, const BrickArgs& a)
         const float v = sign(x, y, z);
         const uint64_t m = __ballot(v > 0.0f);
         if (l == b) word = m;
-        if (S::kValue && a.vals && m != 0ull && m != ~0ull) a.vals[(row + b) * 64u + l] = v;
+        if constexpr (S::kValue) {
+            if ((S::kAll || (a.vals && m != 0ull && m != ~0ull)) && l < planes16) vals[b * planes16 + l] = v;
+        }
     }
     if (l < nb) a.words[row + l] = word;
 }
-
-// dualcontour.wgsl:72-131: crossings on the 12 edges in the reference's order (z-, y-, then
-// x-edges), counted iff the sign changes and the crossing is not at the cell origin;
-// the centroid if at least two count.  c in corner order 000,100,010,110,001,101,011,111.
-__device__ __forceinline__ bool contour_cell(const float c[8], const float lo[3], const float hi[3], float pos[3])
-{
-    // (corner a, corner b, axis of t, fixed x, fixed y, fixed z)
-    constexpr uint8_t E[12][6] = {{0, 4, 2, 0, 0, 0}, {2, 6, 2, 0, 1, 0}, {1, 5, 2, 1, 0, 0},
-                                  {3, 7, 2, 1, 1, 0}, {0, 2, 1, 0, 0, 0}, {4, 6, 1, 0, 0, 1},
-                                  {1, 3, 1, 1, 0, 0}, {5, 7, 1, 1, 0, 1}, {0, 1, 0, 0, 0, 0},
-                                  {4, 5, 0, 0, 0, 1}, {2, 3, 0, 0, 1, 0}, {6, 7, 0, 0, 1, 1}};
-    uint32_t pm = 0;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) pm |= (uint32_t)(c[k] > 0.0f) << k;
-    if (pm == 0u || pm == 0xffu) return false;
-    float ax = 0.0f, ay = 0.0f, az = 0.0f, cnt = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 12; ++e) {
-        const float v0 = c[E[e][0]], v1 = c[E[e][1]];
-        const float t = (0.0f - v0) / (v1 - v0);
-        float x = E[e][3], y = E[e][4], z = E[e][5];
-        if (E[e][2] == 0) x = t;
-        else if (E[e][2] == 1) y = t;
-        else z = t;
-        if ((v0 > 0.0f) == (v1 > 0.0f)) x = y = z = 0.0f;
-        if (x > 0.0f || y > 0.0f || z > 0.0f) {
-            ax = ax + x;
-            ay = ay + y;
-            az = az + z;
-            cnt = cnt + 1.0f;
-        }
-    }
-    if (cnt <= 1.0f) return false;
-    pos[0] = canonical_nan(lo[0] + ((hi[0] - lo[0]) * ax) / cnt);
-    pos[1] = canonical_nan(lo[1] + ((hi[1] - lo[1]) * ay) / cnt);
-    pos[2] = canonical_nan(lo[2] + ((hi[2] - lo[2]) * az) / cnt);
-    return true;
-}
-
-// contour_cell for a cell of a 5 x 5 x 5 block of values (val: its corner 000), over the
-// edges that change sign only, with one copy of the division: fewer of them run, and a
-// program compiled at run time is compiled in two thirds of the time that twelve take.
-// pm: the corners > 0.  Edge e goes from corner `a` (3 bits of kEdgeA) along axis 2 - e / 4.
-__device__ __forceinline__ bool contour_block(const float* val, uint32_t pm, const float lo[3], const float hi[3],
-                                              float pos[3])
-{
-    constexpr uint64_t kEdgeA = 0ull | 2ull << 3 | 1ull << 6 | 3ull << 9 | 0ull << 12 | 4ull << 15 | 1ull << 18 |
-                                5ull << 21 | 0ull << 24 | 4ull << 27 | 2ull << 30 | 6ull << 33;
-    uint32_t todo = 0;
-#pragma unroll
-    for (uint32_t e = 0; e < 12; ++e) {
-        const uint32_t a = (uint32_t)(kEdgeA >> (3u * e)) & 7u, b = a + (4u >> (e >> 2));
-        todo |= (((pm >> a) ^ (pm >> b)) & 1u) << e;
-    }
-    float ax = 0.0f, ay = 0.0f, az = 0.0f, cnt = 0.0f;
-    while (todo) {
-        const uint32_t e = (uint32_t)__builtin_ctz(todo), axis = 2u - (e >> 2);
-        todo &= todo - 1u;
-        const uint32_t a = (uint32_t)(kEdgeA >> (3u * e)) & 7u;
-        const float* p = val + (a >> 2) * 25u + ((a >> 1) & 1u) * 5u + (a & 1u);
-        const float v0 = p[0], v1 = p[axis == 0u ? 1 : axis == 1u ? 5 : 25];
-        const float t = (0.0f - v0) / (v1 - v0);
-        const float x = axis == 0u ? t : (float)(a & 1u), y = axis == 1u ? t : (float)((a >> 1) & 1u);
-        const float z = axis == 2u ? t : (float)(a >> 2);
-        if (x > 0.0f || y > 0.0f || z > 0.0f) {
-            ax = ax + x;
-            ay = ay + y;
-            az = az + z;
-            cnt = cnt + 1.0f;
-        }
-    }
-    if (cnt <= 1.0f) return false;
-    const float s[3] = {ax, ay, az};
-    for (int k = 0; k < 3; ++k) pos[k] = canonical_nan(lo[k] + ((hi[k] - lo[k]) * s[k]) / cnt);
-    return true;
-}
-
-// Sign bits of a cell (dualcontour.wgsl:57-69).
-__device__ __forceinline__ uint32_t sign_bits(const float c[8])
-{
-    return (uint32_t)(c[1] > 0.0f) | ((uint32_t)(c[2] > 0.0f) << 1) | ((uint32_t)(c[4] > 0.0f) << 2) |
-           ((uint32_t)(c[0] > 0.0f) << 3);
-}
-
-// The listed bricks, four at a time per block of 256 (one wave each).  The SDF at the
-// corners of the cells with a sign change (at most 5 x 5 x 5 points per brick) goes into
-// LDS: kept values are read, the four bricks' other points listed together so that the
-// evaluating waves are full; then one lane per cell, the vertex rule.  Vertices are staged (position, sign bits) at
-// the record's base in cell order, the record's mask becomes the cells with a vertex and
-// their bits are set in `actbits` (zero on entry).
-template <class F>
-__device__ __forceinline__ void contour_bricks(const F& sdf, const BrickArgs& a)
-{
-    __shared__ float val[4 * 125];
-    __shared__ uint16_t list[4 * 125];  // brick * 125 + point
-    __shared__ uint32_t count[4], org[4][3];
-    const uint32_t l = threadIdx.x & 63u, w = threadIdx.x >> 6, nrec = (uint32_t)*a.alloc;
-    for (uint32_t r0 = blockIdx.x * 4u; r0 < nrec; r0 += gridDim.x * 4u) {  // block-uniform
-        const bool mine = r0 + w < nrec;
-        BrickRec* R = a.recs + (mine ? r0 + w : r0);
-        const uint64_t mask = mine ? R->mask : 0ull;
-        const uint32_t ix0 = R->bx * 4u, iy0 = R->by * 4u, iz0 = a.lz0 + R->bz * 4u;
-        // points p = (z * 5 + y) * 5 + x used by a cell of the mask: of the cells x - 1, x (and
-        // so on), as a 64-bit product of the three axes' pairs
-        uint32_t kept = 0;  // bit dz * 4 + dy * 2 + dx: the brick there has its values kept
-        size_t brick = 0;   // lane's brick of the eight
-        if (a.vals) {
-            const uint32_t d = l & 7u, bx = R->bx + (d & 1u), by = R->by + ((d >> 1) & 1u), bz = R->bz + (d >> 2);
-            brick = ((size_t)bz * a.nby + by) * a.nbx + bx;
-            const uint64_t word = l < 8u && bx < a.nbx && by < a.nby && bz < a.nbz ? a.words[brick] : 0ull;
-            kept = (uint32_t)__ballot(word != 0ull && word != ~0ull);
-        }
-        uint64_t need[2];
-        uint32_t n = 0;
-#pragma unroll
-        for (uint32_t h = 0; h < 2; ++h) {
-            const uint32_t p = h * 64u + l, pz = p / 25u, py = (p / 5u) % 5u, px = p % 5u;
-            const uint32_t xm = (3u << px) >> 1 & 15u, ym = (3u << py) >> 1 & 15u, zm = (3u << pz) >> 1 & 15u;
-            const uint32_t rows = ((ym & 1u) | (ym & 2u) << 3 | (ym & 4u) << 6 | (ym & 8u) << 9) * xm;
-            const uint64_t cells = (zm & 1u ? (uint64_t)rows : 0ull) | (zm & 2u ? (uint64_t)rows << 16 : 0ull) |
-                                   (zm & 4u ? (uint64_t)rows << 32 : 0ull) | (zm & 8u ? (uint64_t)rows << 48 : 0ull);
-            bool used = p < 125u && (mask & cells) != 0ull;
-            const uint32_t d = (px >> 2) | (py >> 2) << 1 | (pz >> 2) << 2;
-            const size_t at = (size_t)__shfl((long long)brick, (int)(d & 7u), 64);
-            if (used && ((kept >> d) & 1u)) {
-                val[w * 125u + p] = a.vals[at * 64u + (pz & 3u) * 16u + (py & 3u) * 4u + (px & 3u)];
-                used = false;
-            }
-            need[h] = __ballot(used);
-            n += (uint32_t)__popcll(need[h]);
-        }
-        if (l == 0) {
-            count[w] = n;
-            org[w][0] = ix0;
-            org[w][1] = iy0;
-            org[w][2] = iz0;
-        }
-        __syncthreads();
-        uint32_t at = 0, total = 0;
-#pragma unroll
-        for (uint32_t k = 0; k < 4; ++k) {
-            at += k < w ? count[k] : 0u;
-            total += count[k];
-        }
-#pragma unroll
-        for (uint32_t h = 0; h < 2; ++h) {
-            if ((need[h] >> l) & 1ull)
-                list[at + (uint32_t)__popcll(need[h] & ((1ull << l) - 1ull))] = (uint16_t)(w * 125u + h * 64u + l);
-            at += (uint32_t)__popcll(need[h]);
-        }
-        __syncthreads();
-        for (uint32_t i = threadIdx.x; i < total; i += 256u) {
-            const uint32_t q = list[i], b = q / 125u, p = q - b * 125u;
-            val[q] = sdf(a.cx[org[b][0] + p % 5u], a.cy[org[b][1] + (p / 5u) % 5u], a.cz[org[b][2] + p / 25u]);
-        }
-        __syncthreads();
-        const uint32_t x = l & 3u, y = (l >> 2) & 3u, z = l >> 4;
-        bool act = false;
-        float pos[3] = {0.0f, 0.0f, 0.0f};
-        uint32_t sg = 0;
-        if ((mask >> l) & 1ull) {
-            const float* c = val + w * 125u + (z * 5u + y) * 5u + x;
-            uint32_t pm = 0;
-#pragma unroll
-            for (uint32_t k = 0; k < 8; ++k) pm |= (uint32_t)(c[(k >> 2) * 25u + ((k >> 1) & 1u) * 5u + (k & 1u)] > 0.0f) << k;
-            const float lo[3] = {a.cx[ix0 + x], a.cy[iy0 + y], a.cz[iz0 + z]};
-            const float hi[3] = {a.cx[ix0 + x + 1u], a.cy[iy0 + y + 1u], a.cz[iz0 + z + 1u]};
-            act = contour_block(c, pm, lo, hi, pos);
-            sg = ((pm >> 1) & 3u) | ((pm >> 2) & 4u) | ((pm & 1u) << 3);  // sign_bits
-        }
-        const uint64_t m = __ballot(act);
-        if (act) {
-            const uint64_t cell =
-                ((uint64_t)(a.coz[iz0 + z] - a.z0) * a.ry + a.coy[iy0 + y]) * a.rx + a.cox[ix0 + x];
-            atomicOr(&a.actbits[cell >> 6], 1ull << (cell & 63u));
-            const uint64_t to = (uint64_t)R->base + (uint32_t)__popcll(m & ((1ull << l) - 1ull));
-            if (to < a.stage_cap) {
-                float* s = a.stage + 3 * to;
-                s[0] = pos[0];
-                s[1] = pos[1];
-                s[2] = pos[2];
-                a.stage_sign[to] = (uint8_t)sg;
-            }
-        }
-        if (mine && l == 0) R->mask = m;
-        // the next round's writes to count, list and val follow barriers that every reader of
-        // this round passes first: count is read before the second, list before the third,
-        // val (own wave's bricks, written by all waves) after it, so one more is needed
-        __syncthreads();
-    }
-}
-
-// Ordered index of the vertex of slab cell `cell` (which has one).
-__device__ __forceinline__ uint32_t vertex_rank(const BrickArgs& a, uint64_t cell)
-{
-    const unsigned long long word = a.actbits[cell >> 6];
-    return a.cbase[cell >> 20] + a.boffset[cell >> 10] + a.wpre[cell >> 6] +
-           (uint32_t)__popcll(word & ((1ull << (cell & 63u)) - 1ull));
-}
-
-struct LibraryNormal {};  // emit_bricks: the 4-tap normal of the SDF
 
 // Lane `k` of each group of four lanes, broadcast to the group.
 template <int K>
@@ -318,92 +130,39 @@ __device__ __forceinline__ float quad_lane(float v)
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), K * 0x55, 0xf, 0xf, true));
 }
 
-// The staged vertices written at their ordered index with key, sign bits and normal, four
-// bricks at a time per block of 256, their vertices listed together.  LibraryNormal: four
-// lanes per vertex, one per tap (sdf3d_normal.wgsl:4-9: v1=(1,-1,-1), v2=(-1,-1,1),
-// v3=(-1,1,-1), v4=(1,1,1) at p + v * eps, summed left to right, normalized), so the SDF is
-// inlined once; three of them store the vertex as 8-byte pairs where vtx allows it.  Otherwise N(px, py, pz,
-// eps, o) writes o[3..5], one lane per vertex.
-template <class F, class N>
-__device__ __forceinline__ void emit_bricks(const F& sdf, const N& normal, const BrickArgs& a)
+// sdf3d_normal (sdf3d_normal.wgsl:4-9) of the vertex at p, by the four lanes of a group, one per
+// tap (v1=(1,-1,-1), v2=(-1,-1,1), v3=(-1,1,-1), v4=(1,1,1) at p + v * eps, summed left to
+// right, normalized), so the SDF is inlined once: o[3..5].
+template <class F>
+__device__ __forceinline__ void tap_normal(const F& sdf, float px, float py, float pz, float eps, uint32_t tap, float* o)
 {
-    __shared__ uint8_t list[256];  // brick << 6 | cell
-    __shared__ uint32_t count[4], org[4][4];
-    constexpr bool kTaps = __is_same(N, LibraryNormal);
-    const uint32_t l = threadIdx.x & 63u, w = threadIdx.x >> 6, nrec = (uint32_t)*a.alloc;
-    const uint32_t tap = kTaps ? l & 3u : 0u;
-    const bool pairs = ((size_t)a.vtx & 7u) == 0;  // a caller's buffer may be 4-byte aligned
-    for (uint32_t r0 = blockIdx.x * 4u; r0 < nrec; r0 += gridDim.x * 4u) {  // block-uniform
-        const bool mine = r0 + w < nrec;
-        const BrickRec* R = a.recs + (mine ? r0 + w : r0);
-        const uint64_t mask = mine ? R->mask : 0ull;
-        if (l == 0) {
-            count[w] = (uint32_t)__popcll(mask);
-            org[w][0] = R->bx * 4u;
-            org[w][1] = R->by * 4u;
-            org[w][2] = a.lz0 + R->bz * 4u;
-            org[w][3] = R->base;
+    const float ex = (tap == 0u || tap == 3u) ? eps : -eps;
+    const float ey = tap >= 2u ? eps : -eps;
+    const float ez = (tap == 1u || tap == 3u) ? eps : -eps;
+    const float d = sdf(px + ex, py + ey, pz + ez);
+    const float d1 = quad_lane<0>(d), d2 = quad_lane<1>(d), d3 = quad_lane<2>(d), d4 = quad_lane<3>(d);
+    write_unit(o, ((d1 + (-d2)) + (-d3)) + d4, (((-d1) + (-d2)) + d3) + d4, (((-d1) + d2) + (-d3)) + d4);
+}
+
+// A compiled program's normals: the vertices the slab has written, [counters[kDenseVtxPrev],
+// counters[kDenseVtxTotal]) below vcap, their positions in place.  LIB: the library's
+// normal of the SDF F, else F(px, py, pz, eps, o) writes o[3..5].
+constexpr uint32_t kDenseVtxTotal = 0, kDenseVtxPrev = 1;  // Counter (internal.h)
+template <bool LIB, class F>
+__device__ __forceinline__ void vertex_normals(const F& f, float eps, float* vtx, const uint64_t* counters, uint64_t vcap)
+{
+    constexpr uint32_t kLanes = LIB ? 4u : 1u;
+    const uint64_t beg = counters[kDenseVtxPrev], end = min(counters[kDenseVtxTotal], vcap);
+    const uint32_t tap = LIB ? threadIdx.x & 3u : 0u;
+    for (uint64_t v = beg + ((uint64_t)blockIdx.x * 256u + threadIdx.x) / kLanes; v < end; v += gridDim.x * (256u / kLanes)) {
+        float* o = vtx + 6 * v;
+        if constexpr (LIB) {
+            float n[6];
+            tap_normal(f, o[0], o[1], o[2], eps, tap, n);
+            if (tap < 3u) o[3u + tap] = tap == 0u ? n[3] : tap == 1u ? n[4] : n[5];
+        } else {
+            f(o[0], o[1], o[2], eps, o);
         }
-        __syncthreads();
-        uint32_t first[4], total = 0;  // the bricks' first list entries
-#pragma unroll
-        for (uint32_t k = 0; k < 4; ++k) {
-            first[k] = total;
-            total += count[k];
-        }
-        const uint32_t at0 = w == 0 ? first[0] : w == 1 ? first[1] : w == 2 ? first[2] : first[3];
-        if ((mask >> l) & 1ull) list[at0 + (uint32_t)__popcll(mask & ((1ull << l) - 1ull))] = (uint8_t)(w << 6 | l);
-        __syncthreads();
-        for (uint32_t e = kTaps ? threadIdx.x >> 2 : threadIdx.x; e < total; e += kTaps ? 64u : 256u) {
-            const uint32_t q = list[e], b = q >> 6, c = q & 63u;
-            const uint32_t f = b == 0 ? first[0] : b == 1 ? first[1] : b == 2 ? first[2] : first[3];
-            const uint32_t X = a.cox[org[b][0] + (c & 3u)], Y = a.coy[org[b][1] + ((c >> 2) & 3u)];
-            const uint32_t Z = a.coz[org[b][2] + (c >> 4)];
-            const uint32_t v = vertex_rank(a, ((uint64_t)(Z - a.z0) * a.ry + Y) * a.rx + X);
-            const uint64_t at = (uint64_t)org[b][3] + (e - f);
-            if (v >= a.vcap) continue;  // the job is repeated with larger buffers
-            if (at >= a.stage_cap) {    // likewise, but the quad pass reads this vertex's key: without sign
-                                        // changes it forms no quads
-                if (tap == 0u) {
-                    a.keys[v] = (uint64_t)X | ((uint64_t)Y << 16) | ((uint64_t)Z << 32);
-                    a.signs[v] = 0;
-                }
-                continue;
-            }
-            const float px = a.stage[3 * at], py = a.stage[3 * at + 1], pz = a.stage[3 * at + 2];
-            float* o = a.vtx + 6 * (size_t)v;
-            if constexpr (kTaps) {
-                float nrm[6] = {px, py, pz, 0.0f, 0.0f, 0.0f};
-                if (a.normals) {
-                    const float ex = (tap == 0u || tap == 3u) ? a.eps : -a.eps;
-                    const float ey = tap >= 2u ? a.eps : -a.eps;
-                    const float ez = (tap == 1u || tap == 3u) ? a.eps : -a.eps;
-                    const float d = sdf(px + ex, py + ey, pz + ez);
-                    const float d1 = quad_lane<0>(d), d2 = quad_lane<1>(d), d3 = quad_lane<2>(d), d4 = quad_lane<3>(d);
-                    write_unit(nrm, ((d1 + (-d2)) + (-d3)) + d4, (((-d1) + (-d2)) + d3) + d4,
-                               (((-d1) + d2) + (-d3)) + d4);
-                }
-                const float n0 = tap == 0u ? nrm[0] : tap == 1u ? nrm[2] : nrm[4];
-                const float n1 = tap == 0u ? nrm[1] : tap == 1u ? nrm[3] : nrm[5];
-                if (tap < 3u && pairs) {
-                    *reinterpret_cast<float2*>(o + 2 * tap) = make_float2(n0, n1);
-                } else if (tap < 3u) {
-                    o[2 * tap] = n0;
-                    o[2 * tap + 1] = n1;
-                }
-            } else {
-                o[0] = px;
-                o[1] = py;
-                o[2] = pz;
-                if (a.normals) normal(px, py, pz, a.eps, o);
-                else o[3] = o[4] = o[5] = 0.0f;
-            }
-            if (tap == 0u) {
-                a.keys[v] = (uint64_t)X | ((uint64_t)Y << 16) | ((uint64_t)Z << 32);
-                a.signs[v] = a.stage_sign[at];
-            }
-        }
-        __syncthreads();  // list, count and org are read
     }
 }
 

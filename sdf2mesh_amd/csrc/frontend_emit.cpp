@@ -802,7 +802,7 @@ bool emit_hip(const Module& m, Lang lang, const std::string& entry, std::string&
     o << "\nstruct s2m_user_fn {\n"
          "    __device__ float operator()(float x, float y, float z) const { return s2m_entry(s2m::rtc::vf3{{x, y, z}}); }\n"
          "};\n"
-         "// the kernels that evaluate few points share one copy of the program\n"
+         "// the kernels beside s2m_c_signs share one copy of the program\n"
          "__device__ __attribute__((noinline)) float s2m_entry_shared(float x, float y, float z)\n{\n"
          "    return s2m_user_fn{}(x, y, z);\n}\n"
          "struct s2m_shared_fn {\n"
@@ -813,18 +813,16 @@ bool emit_hip(const Module& m, Lang lang, const std::string& entry, std::string&
          "    uint32_t nzl, uint32_t pitch, float* __restrict__ lat)\n{\n"
          "    s2m::eval_lattice_point(s2m_shared_fn{}, cx, cy, cz, nx, ny, lz0, nzl, pitch, lat);\n}\n"
          "extern \"C\" __global__ __launch_bounds__(256) void s2m_c_signs(s2m::BrickArgs a)\n{\n"
-         "    s2m::sign_words(s2m::PointSign<s2m_user_fn>{}, a);\n}\n"
-         "extern \"C\" __global__ __launch_bounds__(256) void s2m_c_contour(s2m::BrickArgs a)\n{\n"
-         "    s2m::contour_bricks(s2m_shared_fn{}, a);\n}\n";
+         "    s2m::sign_words(s2m::PointSign<s2m_user_fn, true>{}, a);\n}\n";
     if (user_normal)
         o << "struct s2m_user_normal {\n"
              "    __device__ void operator()(float px, float py, float pz, float eps, float* o) const\n    {\n"
              "        const s2m::rtc::vf3 g = u_sdf3d_normal(s2m::rtc::vf3{{px, py, pz}}, eps);\n"
              "        s2m::write_unit(o, g.v[0], g.v[1], g.v[2]);\n    }\n};\n";
-    else
-        o << "using s2m_user_normal = s2m::LibraryNormal;\n";
-    o << "extern \"C\" __global__ __launch_bounds__(256) void s2m_c_emit(s2m::BrickArgs a)\n{\n"
-         "    s2m::emit_bricks(s2m_shared_fn{}, s2m_user_normal{}, a);\n}\n";
+    o << "extern \"C\" __global__ __launch_bounds__(256) void s2m_c_normals(float eps, float* vtx,\n"
+         "    const uint64_t* counters, uint64_t vcap)\n{\n"
+      << (user_normal ? "    s2m::vertex_normals<false>(s2m_user_normal{}, eps, vtx, counters, vcap);\n}\n"
+                      : "    s2m::vertex_normals<true>(s2m_shared_fn{}, eps, vtx, counters, vcap);\n}\n");
     hip = o.str();
     return true;
 }

@@ -232,8 +232,8 @@ struct MeshBufs {
 hipError_t launch_eval_lattice(hipStream_t s, const s2m_op* ops, uint32_t nops, const float* cx,
                                const float* cy, const float* cz, uint32_t nx, uint32_t ny,
                                uint32_t lz0, uint32_t nzl, uint32_t pitch, float* lat);
-// The dense slab's kernels (kernels.hip, bodies in device_dense.h).  host_ops: the host copy
-// of the tape (it selects the kernel).
+// The dense slab's kernels (kernels.hip, bodies in device_dense.h and device_bricks.h).  host_ops: the host copy
+// of the tape (it selects the kernel); nops = 0: a compiled program, whose values are kept.
 struct BrickArgs;
 bool mandel_power8(const s2m_op* ops, uint32_t n);  // the tape is one power-8 Mandelbulb op
 bool sign_early(const s2m_op* ops, uint32_t n);     // its signs are decided early (no values to keep)
@@ -244,10 +244,10 @@ hipError_t launch_find_bricks(hipStream_t s, const BrickArgs& a);
 hipError_t launch_contour(hipStream_t s, const BrickArgs& a, const s2m_op* host_ops, const s2m_op* ops, uint32_t nops);
 hipError_t launch_emit(hipStream_t s, const BrickArgs& a, const s2m_op* host_ops, const s2m_op* ops, uint32_t nops);
 hipError_t launch_ranks(hipStream_t s, const MeshBufs& b, uint32_t ncells);
-hipError_t launch_dense_begin(hipStream_t s, uint64_t* counters, uint64_t* words, uint32_t ncells,
+hipError_t launch_dense_begin(hipStream_t s, uint64_t* counters, uint32_t ncounters, uint64_t* words, uint32_t ncells,
                               const void* host_tables, void* tables, size_t bytes, uint32_t* cbase);
-hipError_t launch_slab_end(hipStream_t s, uint64_t* counters, uint64_t* words, uint32_t ncells, uint32_t* cbase,
-                           uint64_t* back);
+hipError_t launch_slab_end(hipStream_t s, uint64_t* counters, uint32_t ncounters, uint64_t* words, uint32_t ncells,
+                           uint32_t* cbase, uint64_t* back);
 hipError_t launch_copy_out(hipStream_t s, const CopyList& c);
 hipError_t launch_quads(hipStream_t s, const SlabArgs& a, const MeshBufs& b, const SlabBits& prev, uint64_t* snap);
 // cnt[0..4) (zeroed by the caller): k_sincos_check's mismatch counts.

@@ -2,13 +2,15 @@
 //
 // The dense path meshes programs that interval bounds cannot prune (the Mandelbulb,
 // compiled programs, S2M_DENSE_EVAL).  Per z-slab of cells the host launches, in stream
-// order (bodies of the evaluating kernels: device_dense.h):
+// order (bodies: device_dense.h, device_bricks.h; a compiled program's s2m_c_signs and
+// s2m_c_normals are in its own module):
 //   k_signs            sign of the SDF at every corner-lattice point, one bit each  (VALU bound)
 //   k_find_bricks      the 4x4x4 bricks whose cells change sign
-//   k_contour          their corner values again, the vertex rule, staged vertices, one
-//                      activity bit per cell
+//   k_contour          their cells' corner values (kept by the sign pass or taken again), the
+//                      vertex rule, staged vertices, one activity bit per cell
 //   k_ranks            vertices before each word of 64 cells, block of 1024 cells and chunk
-//   k_emit             staged vertices at their ordered index, with 4-tap normals
+//   k_emit             staged vertices at their ordered index, with 4-tap normals (a compiled
+//                      program's: s2m_c_normals after it)
 //   k_quads<0>, k_tri_offsets, k_quads<1>   triangles per 256 vertices, their offsets, triangles
 //   k_slab_end         the other slab's bits cleared, staging counters folded, the totals
 //                      for the host
@@ -20,6 +22,7 @@
 #include <algorithm>
 #include <mutex>
 
+#include "device_bricks.h"
 #include "device_dense.h"
 #include "device_scan.h"
 #include "device_sdf.h"
@@ -136,22 +139,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
                                                                                          uint32_t nops)
 {
     if constexpr (MANDEL == 2) sign_words(MandelSign(ops), a);
-    else if constexpr (MANDEL == 1) sign_words(PointSign<MandelSdf>{MandelSdf(ops)}, a);
-    else sign_words(PointSign<TapeSdf>{TapeSdf{ops, nops}}, a);
+    else if constexpr (MANDEL == 1) sign_words(PointSign<MandelSdf, false>{MandelSdf(ops)}, a);
+    else sign_words(PointSign<TapeSdf, false>{TapeSdf{ops, nops}}, a);
 }
 
-template <int MANDEL>
+// What the kernels of the listed bricks evaluate: a tape, one power-8 Mandelbulb op, or nothing
+// (a compiled program's kept values).
+enum BrickSdf : int { kTapeSdf = 0, kMandelSdf = 1, kNoSdf = 2 };
+
+template <int SDF>
 __global__ __launch_bounds__(256) void k_contour(BrickArgs a, const s2m_op* ops, uint32_t nops)
 {
-    if constexpr (MANDEL) contour_bricks(MandelSdf(ops), a);
-    else contour_bricks(TapeSdf{ops, nops}, a);
+    if constexpr (SDF == kMandelSdf) contour_bricks(MandelSdf(ops), a);
+    else if constexpr (SDF == kTapeSdf) contour_bricks(TapeSdf{ops, nops}, a);
+    else contour_bricks(KeptValues{}, a);
 }
 
-template <int MANDEL>
+template <int SDF>
 __global__ __launch_bounds__(256) void k_emit(BrickArgs a, const s2m_op* ops, uint32_t nops)
 {
-    if constexpr (MANDEL) emit_bricks(MandelSdf(ops), LibraryNormal{}, a);
-    else emit_bricks(TapeSdf{ops, nops}, LibraryNormal{}, a);
+    if constexpr (SDF == kMandelSdf) emit_bricks(MandelSdf(ops), a);
+    else if constexpr (SDF == kTapeSdf) emit_bricks(TapeSdf{ops, nops}, a);
+    else emit_bricks(KeptValues{}, a);
 }
 
 // ---------------------------------------------------------------------------------
@@ -171,11 +180,11 @@ __device__ __forceinline__ uint64_t mixed_cells(const BrickArgs& a, uint32_t i, 
 {
     const uint32_t row = i / a.nbx;
     bx = i - row * a.nbx;
-    bz = row / a.nby;
-    by = row - bz * a.nby;
+    bz = row / a.own;
+    by = row - bz * a.own;
     const uint32_t dx = bx + 1 < a.nbx ? 1u : 0u;  // past the end: cells that are masked off
     const size_t dy = by + 1 < a.nby ? a.nbx : 0u, dz = bz + 1 < a.nbz ? (size_t)a.nbx * a.nby : 0u;
-    const uint64_t* w = a.words + i;
+    const uint64_t* w = a.words + ((size_t)bz * a.nby + by) * a.nbx + bx;
     uint64_t o[4], n4[4];  // OR / AND along x of the rows (y, z), (y + 1, z), (y, z + 1), (y + 1, z + 1)
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -195,7 +204,7 @@ __device__ __forceinline__ uint64_t mixed_cells(const BrickArgs& a, uint32_t i, 
     uint32_t vx = 0, vy = 0, vz = 0;  // the axes' cells
 #pragma unroll
     for (uint32_t k = 0; k < 4; ++k) {
-        const uint32_t ix = bx * 4u + k, iy = by * 4u + k, iz = bz * 4u + k;
+        const uint32_t ix = bx * 4u + k, iy = (a.by0 + by) * 4u + k, iz = bz * 4u + k;
         if (ix < a.nx && a.cox[ix] != kNoCell) vx |= 1u << k;
         if (iy < a.ny && a.coy[iy] != kNoCell) vy |= 1u << (4u * k);
         if (iz + 1u < a.nzl) {
@@ -212,7 +221,7 @@ __global__ __launch_bounds__(256) void k_find_bricks(BrickArgs a)
 {
     __shared__ uint32_t wrecs[kBlock / 64], wcells[kBlock / 64];
     __shared__ uint64_t base;
-    const uint32_t n = a.nbx * a.nby * a.nbz;
+    const uint32_t n = a.nbx * a.own * a.nbz;
     uint64_t mask[kFindBricks];
     BrickRec rec[kFindBricks];
     uint32_t recs = 0, cells = 0;  // of this thread
@@ -221,7 +230,7 @@ __global__ __launch_bounds__(256) void k_find_bricks(BrickArgs a)
         const uint32_t i = (blockIdx.x * kFindBricks + k) * kBlock + threadIdx.x;
         uint32_t bx = 0, by = 0, bz = 0;
         mask[k] = i < n ? mixed_cells(a, i, bx, by, bz) : 0ull;
-        rec[k] = BrickRec{mask[k], 0u, (uint16_t)bx, (uint16_t)by, (uint16_t)bz, 0};
+        rec[k] = BrickRec{mask[k], 0u, (uint16_t)bx, (uint16_t)(a.by0 + by), (uint16_t)bz, 0};
         recs += mask[k] != 0ull ? 1u : 0u;
         cells += (uint32_t)__popcll(mask[k]);
     }
@@ -659,27 +668,29 @@ hipError_t launch_signs(hipStream_t s, const BrickArgs& a, const s2m_op* host_op
     return hipGetLastError();
 }
 
+template <class K0, class K1, class K2>
+static hipError_t launch_bricks(hipStream_t s, K0 tape, K1 mandel, K2 kept, const BrickArgs& a, const s2m_op* host_ops,
+                                const s2m_op* ops, uint32_t nops)
+{
+    if (nops == 0) hipLaunchKernelGGL(kept, dim3(kBrickBlocks), dim3(256), 0, s, a, ops, nops);
+    else if (mandel_power8(host_ops, nops)) hipLaunchKernelGGL(mandel, dim3(kBrickBlocks), dim3(256), 0, s, a, ops, nops);
+    else hipLaunchKernelGGL(tape, dim3(kBrickBlocks), dim3(256), 0, s, a, ops, nops);
+    return hipGetLastError();
+}
+
 hipError_t launch_contour(hipStream_t s, const BrickArgs& a, const s2m_op* host_ops, const s2m_op* ops, uint32_t nops)
 {
-    if (mandel_power8(host_ops, nops))
-        hipLaunchKernelGGL(k_contour<1>, dim3(kBrickBlocks), dim3(256), 0, s, a, ops, nops);
-    else
-        hipLaunchKernelGGL(k_contour<0>, dim3(kBrickBlocks), dim3(256), 0, s, a, ops, nops);
-    return hipGetLastError();
+    return launch_bricks(s, k_contour<kTapeSdf>, k_contour<kMandelSdf>, k_contour<kNoSdf>, a, host_ops, ops, nops);
 }
 
 hipError_t launch_emit(hipStream_t s, const BrickArgs& a, const s2m_op* host_ops, const s2m_op* ops, uint32_t nops)
 {
-    if (mandel_power8(host_ops, nops))
-        hipLaunchKernelGGL(k_emit<1>, dim3(kBrickBlocks), dim3(256), 0, s, a, ops, nops);
-    else
-        hipLaunchKernelGGL(k_emit<0>, dim3(kBrickBlocks), dim3(256), 0, s, a, ops, nops);
-    return hipGetLastError();
+    return launch_bricks(s, k_emit<kTapeSdf>, k_emit<kMandelSdf>, k_emit<kNoSdf>, a, host_ops, ops, nops);
 }
 
 hipError_t launch_find_bricks(hipStream_t s, const BrickArgs& a)
 {
-    const uint64_t n = (uint64_t)a.nbx * a.nby * a.nbz;
+    const uint64_t n = (uint64_t)a.nbx * a.own * a.nbz;
     if (n > 0x7fffffffull) return hipErrorInvalidValue;
     const uint64_t per = kFindBricks * kBlock;
     hipLaunchKernelGGL(k_find_bricks, dim3((uint32_t)((n + per - 1u) / per)), dim3(kBlock), 0, s, a);
@@ -743,19 +754,21 @@ __global__ __launch_bounds__(256) void k_dense_begin(uint64_t* __restrict__ coun
 {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
     for (uint32_t i = t; i < n16; i += stride) tables[i] = host_tables[i];
-    if (t < n) counters[t] = 0ull;
+    for (uint32_t i = t; i < n; i += stride) counters[i] = 0ull;
     if (t < kRankChunks) cbase[t] = 0u;
     for (uint32_t i = t; i < nwords; i += stride) words[i] = 0ull;
 }
 
 // After a slab's quad pass: the staging use folded into its maximum, the allocation
-// counter reset, and the other activity words and chunk bases (the previous slab's, read
+// counter (of strips: counters) reset, and the other activity words and chunk bases (the previous slab's, read
 // for the last time by this slab's quads) set up for the next slab.  back: after the last
 // slab, all counters (mapped host memory, NULL: not wanted).
-__global__ __launch_bounds__(256) void k_slab_end(uint64_t* __restrict__ counters, uint64_t* __restrict__ words,
-                                                  uint32_t nwords, uint32_t* __restrict__ cbase, uint64_t* back)
+__global__ __launch_bounds__(256) void k_slab_end(uint64_t* __restrict__ counters, uint32_t ncounters,
+                                                  uint64_t* __restrict__ words, uint32_t nwords,
+                                                  uint32_t* __restrict__ cbase, uint64_t* back)
 {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    for (uint32_t i = kNumCounters + t; i < ncounters; i += gridDim.x * blockDim.x) counters[i] = 0ull;
     if (t < kRankChunks) cbase[t] = (uint32_t)counters[kVtxTotal];
     if (t == 0) {
         counters[kVtxPrev] = counters[kVtxTotal];
@@ -768,22 +781,22 @@ __global__ __launch_bounds__(256) void k_slab_end(uint64_t* __restrict__ counter
     for (uint32_t i = t; i < nwords; i += gridDim.x * blockDim.x) words[i] = 0ull;
 }
 
-hipError_t launch_dense_begin(hipStream_t s, uint64_t* counters, uint64_t* words, uint32_t ncells,
+hipError_t launch_dense_begin(hipStream_t s, uint64_t* counters, uint32_t ncounters, uint64_t* words, uint32_t ncells,
                               const void* host_tables, void* tables, size_t bytes, uint32_t* cbase)
 {
     const uint32_t n = (ncells + 63u) / 64u, n16 = (uint32_t)((bytes + 15u) / 16u);
     hipLaunchKernelGGL(k_dense_begin, dim3(std::max(1u, std::min((std::max(n, n16) + 255u) / 256u, 2048u))), dim3(256), 0,
-                       s, counters, (uint32_t)kNumCounters, words, n, static_cast<const uint4*>(host_tables),
+                       s, counters, ncounters, words, n, static_cast<const uint4*>(host_tables),
                        static_cast<uint4*>(tables), n16, cbase);
     return hipGetLastError();
 }
 
-hipError_t launch_slab_end(hipStream_t s, uint64_t* counters, uint64_t* words, uint32_t ncells, uint32_t* cbase,
-                           uint64_t* back)
+hipError_t launch_slab_end(hipStream_t s, uint64_t* counters, uint32_t ncounters, uint64_t* words, uint32_t ncells,
+                           uint32_t* cbase, uint64_t* back)
 {
     const uint32_t n = (ncells + 63u) / 64u;
     hipLaunchKernelGGL(k_slab_end, dim3(std::max(1u, std::min((n + 255u) / 256u, 2048u))), dim3(256), 0, s, counters,
-                       words, n, cbase, back);
+                       ncounters, words, n, cbase, back);
     return hipGetLastError();
 }
 

@@ -41,7 +41,7 @@
 #include <mutex>
 #include <vector>
 
-#include "device_dense.h"
+#include "device_bricks.h"
 #include "device_interval.h"
 #include "device_scan.h"
 #include "device_sdf.h"

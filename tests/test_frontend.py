@@ -19,6 +19,7 @@ Pins:
 from __future__ import annotations
 
 import ctypes as C
+import re
 import subprocess
 import sys
 import tempfile
@@ -181,6 +182,16 @@ def test_non_tape_programs(body, why):
         s2m.translate_tape(src)
     assert e.value.code == s2m.E_WGSL and why in str(e.value)
     assert "s2m_c_eval_lattice" in hip_of(src)
+
+
+def test_module_holds_what_depends_on_the_program():
+    # every kernel in a program's module adds to the time of compiling it: the evaluating ones
+    # only (placing and emitting vertices is the library's), one copy of the SDF beside s2m_c_signs
+    for body in ("return sdf3d_sphere(p * 2.0, 0.5);", "return sdf3d_sphere(p.xzy, 0.5);"):
+        hip = hip_of(f"use sdf3d::*;\nfn sdf3d(p: vec3f) -> f32 {{ {body} }}\n")
+        kernels = re.findall(r"__global__[^{;]*?\b(s2m_c_\w+)\(", hip)
+        assert kernels == ["s2m_c_eval_lattice", "s2m_c_signs", "s2m_c_normals"]
+        assert "contour" not in hip and "emit_bricks" not in hip
 
 
 def test_abstract_and_f32_constant_evaluation():

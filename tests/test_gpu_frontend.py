@@ -164,3 +164,33 @@ fn sdf3d_normal(p: vec3f, eps: f32) -> vec3f { return vec3(p.x, 2.0 * p.y, 0.0);
     nan = np.isnan(want)  # g = 0 on the z axis: NaN on both sides (payload may differ)
     assert np.array_equal(np.isnan(v[:, 3:]), nan)
     assert np.array_equal(v[:, 3:][~nan].view(np.uint32), want[~nan].view(np.uint32))
+
+
+@pytest.mark.parametrize("res", [(1, 1, 1), (2, 3, 5), (3, 4, 8), (5, 9, 7), (17, 33, 12), (64, 65, 9)])
+@pytest.mark.parametrize("flags", [0, s2m.CORNERS_EXACT | s2m.COMPAT_DROP_LAST_SLICE, s2m.NO_NORMALS])
+def test_compiled_bricks(ctx, res, flags):
+    # every value kept by the sign pass, vertices placed by the library's kernels: partial
+    # bricks on every axis, slabs of one and of five cell planes, with and without normals
+    t = ctx.program_from_source(GOLDEN / "random_csg1.sdf3d", path=True)
+    c = ctx.program_from_source(GOLDEN / "random_csg1.sdf3d", path=True, force_compiled=True)
+    for slab in (0, 1, 5):
+        print(f"compiled bricks {res} flags={flags} slab={slab}", flush=True)
+        p = s2m.Params((-1.0, -1.1, -0.9), (1.05, 1.0, 1.1), res, 1e-4, flags | s2m.DENSE_EVAL, slab)
+        same_mesh(ctx.mesh(c, p), ctx.mesh(t, p))
+
+
+@pytest.mark.parametrize("res", [(130, 70, 40), (1750, 1740, 3), (330, 9000, 3)])
+def test_compiled_noalloc(ctx, res):
+    # without allocation: a few slabs; one cell plane per slab whose values do not fit the
+    # scratch at once (strips of brick rows), on square and on long planes
+    from test_zz_no_alloc import DeviceBuffers, check_same
+
+    c = ctx.program_from_source(GOLDEN / "random_csg1.sdf3d", path=True, force_compiled=True)
+    bufs = DeviceBuffers(6_000_000, 12_000_000)
+    try:
+        print(f"compiled noalloc {res}", flush=True)
+        for flags in (0, s2m.NO_NORMALS):
+            p = s2m.Params((-1.0, -1.1, -0.9), (1.05, 1.0, 1.1), res, 1e-4, flags)
+            check_same(ctx, c, p, bufs)
+    finally:
+        bufs.free()
