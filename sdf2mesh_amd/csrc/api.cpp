@@ -1820,11 +1820,11 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
                 HIP_TRY(launch_emit(ctx->stream, strip(k), host_ops, prog->d_ops, tape_ops));
             if (!h_corners && normals) HIP_TRY(normals_prog(ctx->stream, prog, p->eps, b));
             if (m[3]) HIP_TRY(hipEventRecord(m[3], ctx->stream));
-            HIP_TRY(launch_quads(ctx->stream, a, bs, prev, snap_dev ? snap_dev + kSnapWords * slabs : nullptr));
-            // the other activity words cleared for the next slab
-            HIP_TRY(launch_slab_end(ctx->stream, b.counters, ncounters, act_buf[cur ^ 1],
-                                    (uint32_t)(plane * std::min(T, j.nz_cells - z1)), base_buf[cur ^ 1],
-                                    z1 == j.nz_cells ? static_cast<uint64_t*>(back_dev) : nullptr));
+            HIP_TRY(launch_quads(ctx->stream, a, bs, prev, snap_dev ? snap_dev + kSnapWords * slabs : nullptr,
+                                 z1 == j.nz_cells ? static_cast<uint64_t*>(back_dev) : nullptr));
+            if (z1 < j.nz_cells)  // the other activity words cleared for the next slab
+                HIP_TRY(launch_slab_end(ctx->stream, b.counters, ncounters, act_buf[cur ^ 1],
+                                        (uint32_t)(plane * std::min(T, j.nz_cells - z1)), base_buf[cur ^ 1]));
             if (m[4]) HIP_TRY(hipEventRecord(m[4], ctx->stream));
             if (rb) {  // the slab's vertices and triangles are final; the copies of the slab two
                        // before (waiting for it leaves this slab and the next evaluation queued)

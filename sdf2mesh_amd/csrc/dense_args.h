@@ -1,5 +1,6 @@
 // dense_args.h - arguments of the dense path's per-brick kernels (device_dense.h,
-// device_bricks.h), shared by the host runtime, the library's kernels and the programs compiled at run time.
+// device_bricks.h), shared by the host runtime, the library's kernels and the programs
+// compiled at run time.
 #pragma once
 #ifndef __HIPCC_RTC__
 #include <stdint.h>

@@ -247,9 +247,10 @@ hipError_t launch_ranks(hipStream_t s, const MeshBufs& b, uint32_t ncells);
 hipError_t launch_dense_begin(hipStream_t s, uint64_t* counters, uint32_t ncounters, uint64_t* words, uint32_t ncells,
                               const void* host_tables, void* tables, size_t bytes, uint32_t* cbase);
 hipError_t launch_slab_end(hipStream_t s, uint64_t* counters, uint32_t ncounters, uint64_t* words, uint32_t ncells,
-                           uint32_t* cbase, uint64_t* back);
+                           uint32_t* cbase);
 hipError_t launch_copy_out(hipStream_t s, const CopyList& c);
-hipError_t launch_quads(hipStream_t s, const SlabArgs& a, const MeshBufs& b, const SlabBits& prev, uint64_t* snap);
+hipError_t launch_quads(hipStream_t s, const SlabArgs& a, const MeshBufs& b, const SlabBits& prev, uint64_t* snap,
+                        uint64_t* back);
 // cnt[0..4) (zeroed by the caller): k_sincos_check's mismatch counts.
 hipError_t launch_sincos_check(hipStream_t s, uint64_t* cnt);
 // cnt[0..2) (zeroed by the caller): k_bailout_check's comparisons and disagreements.

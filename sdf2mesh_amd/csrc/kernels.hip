@@ -12,8 +12,7 @@
 //   k_emit             staged vertices at their ordered index, with 4-tap normals (a compiled
 //                      program's: s2m_c_normals after it)
 //   k_quads<0>, k_tri_offsets, k_quads<1>   triangles per 256 vertices, their offsets, triangles
-//   k_slab_end         the other slab's bits cleared, staging counters folded, the totals
-//                      for the host
+//   k_slab_end         between slabs: the other slab's bits cleared
 // (with several slabs the signs are evaluated one slab ahead on a second stream; per-cell
 // corner dumps have k_cells<0/1> in place of the brick kernels).  A cell's vertex index is
 // never stored: it is its chunk's first vertex plus the vertices before it in the chunk.  Cells are
@@ -414,10 +413,12 @@ __device__ __forceinline__ void write_snapshot(uint64_t* snap, uint64_t nv, uint
 }
 
 // The groups' triangle counts (k_quads<0>) into their offsets, and the running total, by one
-// workgroup: a slab's 600 K vertices are 2 400 groups, one round.
+// workgroup: a slab's 600 K vertices are 2 400 groups, one round.  The staging use is folded into
+// its maximum here, and after a job's last slab the counters (final then: k_quads<1> changes
+// none) go to `back` (mapped host memory, else NULL), so that no k_slab_end follows it.
 __global__ __launch_bounds__(1024) void k_tri_offsets(const uint32_t* __restrict__ tcount, uint32_t* __restrict__ toffset,
                                                       uint64_t* __restrict__ counters, uint64_t vcap,
-                                                      uint64_t* snap)
+                                                      uint64_t* snap, uint64_t* back)
 {
     __shared__ uint32_t wsum[16];
     const uint32_t groups = vertex_groups(counters, vcap), t = threadIdx.x;
@@ -453,7 +454,11 @@ __global__ __launch_bounds__(1024) void k_tri_offsets(const uint32_t* __restrict
     if (t == 0) {
         counters[kTriPrev] = prev;
         counters[kTriTotal] = run;
-        if (snap) write_snapshot(snap, counters[kVtxTotal], run, 0, counters[kBrickAlloc] >> 32);
+        const uint64_t used = counters[kBrickAlloc] >> 32;
+        if (snap) write_snapshot(snap, counters[kVtxTotal], run, 0, used);
+        if (used > counters[kStageMax]) counters[kStageMax] = used;
+        if (back)
+            for (uint32_t i = 0; i < kNumCounters; ++i) back[i] = counters[i];
     }
 }
 
@@ -759,24 +764,19 @@ __global__ __launch_bounds__(256) void k_dense_begin(uint64_t* __restrict__ coun
     for (uint32_t i = t; i < nwords; i += stride) words[i] = 0ull;
 }
 
-// After a slab's quad pass: the staging use folded into its maximum, the allocation
-// counter (of strips: counters) reset, and the other activity words and chunk bases (the previous slab's, read
-// for the last time by this slab's quads) set up for the next slab.  back: after the last
-// slab, all counters (mapped host memory, NULL: not wanted).
+// After the quad pass of a slab that is not the last: the allocation counter (of strips:
+// counters) reset, and the other activity words and chunk bases (the previous slab's, read for
+// the last time by this slab's quads) set up for the next slab.
 __global__ __launch_bounds__(256) void k_slab_end(uint64_t* __restrict__ counters, uint32_t ncounters,
                                                   uint64_t* __restrict__ words, uint32_t nwords,
-                                                  uint32_t* __restrict__ cbase, uint64_t* back)
+                                                  uint32_t* __restrict__ cbase)
 {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     for (uint32_t i = kNumCounters + t; i < ncounters; i += gridDim.x * blockDim.x) counters[i] = 0ull;
     if (t < kRankChunks) cbase[t] = (uint32_t)counters[kVtxTotal];
     if (t == 0) {
         counters[kVtxPrev] = counters[kVtxTotal];
-        const uint64_t used = counters[kBrickAlloc] >> 32;
-        if (used > counters[kStageMax]) counters[kStageMax] = used;
         counters[kBrickAlloc] = 0;
-        if (back)
-            for (uint32_t i = 0; i < kNumCounters; ++i) back[i] = counters[i];
     }
     for (uint32_t i = t; i < nwords; i += gridDim.x * blockDim.x) words[i] = 0ull;
 }
@@ -792,11 +792,11 @@ hipError_t launch_dense_begin(hipStream_t s, uint64_t* counters, uint32_t ncount
 }
 
 hipError_t launch_slab_end(hipStream_t s, uint64_t* counters, uint32_t ncounters, uint64_t* words, uint32_t ncells,
-                           uint32_t* cbase, uint64_t* back)
+                           uint32_t* cbase)
 {
     const uint32_t n = (ncells + 63u) / 64u;
     hipLaunchKernelGGL(k_slab_end, dim3(std::max(1u, std::min((n + 255u) / 256u, 2048u))), dim3(256), 0, s, counters,
-                       ncounters, words, n, cbase, back);
+                       ncounters, words, n, cbase);
     return hipGetLastError();
 }
 
@@ -828,13 +828,14 @@ hipError_t launch_copy_out(hipStream_t s, const CopyList& c)
 }
 
 hipError_t launch_quads(hipStream_t s, const SlabArgs& a, const MeshBufs& b, const SlabBits& prev,
-                        uint64_t* snap)
+                        uint64_t* snap, uint64_t* back)
 {
     if (a.ncells == 0) return hipSuccess;
     const uint32_t groups = (a.ncells + kBlock - 1u) / kBlock;  // if every cell had a vertex
     const dim3 grid(std::min(groups, 2048u));
     hipLaunchKernelGGL((k_quads<0>), grid, dim3(kBlock), 0, s, a, b, prev);
-    hipLaunchKernelGGL(k_tri_offsets, dim3(1), dim3(1024), 0, s, b.tcount, b.toffset, b.counters, b.vcap, snap);
+    hipLaunchKernelGGL(k_tri_offsets, dim3(1), dim3(1024), 0, s, b.tcount, b.toffset, b.counters, b.vcap, snap,
+                       back);
     hipLaunchKernelGGL((k_quads<1>), grid, dim3(kBlock), 0, s, a, b, prev);
     return hipGetLastError();
 }
