@@ -147,7 +147,7 @@ struct s2m_ctx {
     DevBuf vtx, keys, signs, tri, corners;
     DevBuf tile_tab, tile_lists, sp_slot_info;
     DevBuf sp_gen_slots, sp_cellbits, sp_slot_rows, sp_boundary;
-    DevBuf sp_stage, sp_slot_nb, sp_slot_stage, sp_slot_live, sp_slot_hdr, sp_slot_rec;
+    DevBuf sp_stage, sp_slot_nb, sp_slot_stage, sp_slot_hdr, sp_slot_rec;
     DevBuf sp_queues, sp_super_iv, sp_super_lists, sp_super_act, sp_rows;
     bool sp_dirty = false;  // a sparse pass was not queued to its end: `counters` may not be zero
     uint64_t slot_cap = 0;
@@ -839,7 +839,7 @@ bool union_fold_program(const std::vector<s2m_op>& ops)
 bool left_fold_program(const std::vector<s2m_op>& ops)
 {
     const size_t n = ops.size();
-    if (n == 0 || n > 128 || (n & 1u) == 0) return false;
+    if (n == 0 || n > kStageOps || (n & 1u) == 0) return false;
     for (size_t k = 0; k < n; ++k) {
         const bool prim = ops[k].code < S2M_OP_UNION;
         if (prim != (k == 0 || (k & 1u)) || ops[k].code == S2M_OP_MANDELBULB) return false;
@@ -1223,7 +1223,6 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
         HIP_TRY(ctx->sp_stage.ensure(stage_cap * sizeof(float4)));
         ctx->stage_cap = stage_cap;
         HIP_TRY(ctx->sp_slot_stage.ensure(want_s * 2 * sizeof(uint32_t)));
-        HIP_TRY(ctx->sp_slot_live.ensure(want_s * sizeof(uint64_t)));
         HIP_TRY(ctx->sp_slot_hdr.ensure(want_s * sizeof(SlotHdr)));
         HIP_TRY(ctx->sp_slot_nb.ensure(want_s * 8 * sizeof(int32_t)));
         HIP_TRY(ctx->sp_slot_rec.ensure(want_s * kTileRecBytes));
@@ -1296,7 +1295,6 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
             P.stage_cap = stage_cap;
             P.tile_blocks = (uint32_t)tile_blocks;
             P.slot_stage = ctx->sp_slot_stage.as<uint32_t>();
-            P.slot_live = ctx->sp_slot_live.as<uint64_t>();
             P.slot_hdr = ctx->sp_slot_hdr.as<SlotHdr>();
             P.slot_nb = ctx->sp_slot_nb.as<int32_t>();
             P.slot_rec = ctx->sp_slot_rec.as<uint4>();
@@ -1350,7 +1348,7 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
             for (const DevBuf* d : {&ctx->vtx, &ctx->keys, &ctx->signs, &ctx->tri, &ctx->counters, &ctx->bcount,
                                     &ctx->sp_queues, &ctx->tile_tab, &ctx->tile_lists, &ctx->sp_slot_info,
                                     &ctx->sp_gen_slots, &ctx->sp_cellbits, &ctx->sp_stage, &ctx->sp_slot_stage,
-                                    &ctx->sp_slot_live, &ctx->sp_slot_hdr, &ctx->sp_slot_nb, &ctx->sp_slot_rec,
+                                    &ctx->sp_slot_hdr, &ctx->sp_slot_nb, &ctx->sp_slot_rec,
                                     &ctx->sp_slot_rows, &ctx->sp_rows, &ctx->sp_super_iv, &ctx->sp_super_lists,
                                     &ctx->sp_super_act, &ctx->sp_boundary})
                 put(&d->p, sizeof d->p);
@@ -2032,7 +2030,7 @@ void s2m_destroy(s2m_ctx* ctx)
                       &ctx->sp_gen_slots, &ctx->sp_cellbits, &ctx->sp_slot_rows,
                       &ctx->sp_boundary, &ctx->sp_queues, &ctx->sp_super_iv,
                       &ctx->sp_super_lists, &ctx->sp_super_act, &ctx->sp_rows,
-                      &ctx->sp_stage, &ctx->sp_slot_nb, &ctx->sp_slot_stage, &ctx->sp_slot_live, &ctx->sp_slot_hdr, &ctx->sp_slot_rec})
+                      &ctx->sp_stage, &ctx->sp_slot_nb, &ctx->sp_slot_stage, &ctx->sp_slot_hdr, &ctx->sp_slot_rec})
         b->release();
     for (DevBuf& b : ctx->batch_dense) b.release();
     for (s2m_ctx::PassSet& S : ctx->pset) {

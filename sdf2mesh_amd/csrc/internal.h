@@ -54,8 +54,7 @@ enum Counter : uint32_t {
     kSlotsMax = 9,     // largest kSlotsUsed of the job so far
     kStageUsed = 10,   // staged active cells of the current pass (sparse path)
     kBrickAlloc = 11,  // dense slab: listed bricks (low word), staged vertices (high word)
-    kSlotsNow = 13,    // sparse pass: its slots and staged cells, once they are final
-    kStageNow = 14,
+    kSlotsNow = 13,    // sparse pass: its slots, once they are final
     kStageMax = 12,    // largest kStageUsed of the job so far
     kGenUsed = 15,     // sparse pass: slots whose program is no fold, being counted and final
     kGenNow = 16,
@@ -121,7 +120,7 @@ struct SpJob {
     uint32_t tz0;              // tile layer of plane z0
     uint32_t nops, flags;
     uint32_t union_fold;       // the program is a left fold of unions / smooth unions (k > 0)
-    uint32_t left_fold;        // the program is a left fold of library primitives
+    uint32_t left_fold;        // the program is a left fold of library primitives (at most kStageOps ops)
     uint32_t bx, by;           // lattice box dims of the job's tiles (slot box indexing)
     uint32_t out_index;        // row of the pass's job_out table
     float eps;
@@ -192,7 +191,6 @@ struct SpPass {
     uint32_t tile_blocks;      // most blocks of a k_sp_tiles launch: the first 2 * tile_blocks staging chunks
                                // are theirs without being counted
     uint32_t* slot_stage;      // [slot][2] first staged cell, staged cells
-    uint64_t* slot_live;       // [slot] bricks (2x2x2 cells) that may hold an active cell
     SlotHdr* slot_hdr;         // [slot]
     int32_t* slot_nb;          // [slot][8] slots of the tile (tx - dx, ty - dy, tz - dz) at (dz * 2 + dy) * 2 + dx
     uint4* slot_rec;           // [slot] kTileRecBytes: k_sp_tiles<1>'s staged record

@@ -117,7 +117,6 @@ __device__ __forceinline__ uint32_t general_blocks(uint32_t general, uint32_t sl
     return min(max(n, 1u), gridDim.x - 1u);
 }
 
-// Row segment of row (zl, y) and tile column tx of job J.
 // Per-slot row data: array k (kRowVtx, kRowTri: counts; kRowVtxOff, kRowTriOff: first
 // vertex / triangle of the row segment within its row) of slot `slot`, row r = (z % 8) * 8
 // + y % 8 of the tile.
@@ -349,61 +348,11 @@ struct PruneWalk {
     __device__ __forceinline__ bool one_sign() const { return top.known && (top.lo > 0.0f || top.hi < 0.0f); }
 };
 
-// PruneWalk for a left fold (P0 P1 op1 P2 op2 ...): the same decisions, list and sums with
-// the accumulated value and the latest primitive in registers instead of the LDS stack
-// (every operator's left operand is the accumulated value, which starts the list).
-struct FoldWalk {
-    Iv top = iv_unknown();
-    uint32_t len = 0;
-    uint32_t top_single = kComposite;
-    uint32_t top_sum = 0;
-    Iv b = iv_unknown();  // the latest primitive (the right operand of the next operator)
-    uint32_t b_i = 0, b_sum = 0, b_start = 0;
-
-    __device__ __forceinline__ void prim(uint32_t q, uint32_t i, const Iv& v, uint16_t* out, const PruneStack&,
-                                         uint32_t, uint32_t sum = 0)
-    {
-        if (q == 0) {
-            top = v;
-            top_single = i;
-            top_sum = sum;
-        } else {
-            b = v;
-            b_i = i;
-            b_sum = sum;
-            b_start = len;
-        }
-        out[len++] = (uint16_t)i;
-    }
-
-    __device__ __forceinline__ void op(uint32_t i, uint32_t code, float k, uint16_t* out, const PruneStack&,
-                                       uint32_t, uint32_t fl = 0)
-    {
-        int keep;
-        const Iv r = iv_op(code, top, b, k, keep);
-        if (keep == kKeepBoth) {
-            out[len++] = (uint16_t)i;
-            const bool fold = (top_sum & kFoldBit) && (b_sum & kFoldBit);
-            top_sum = ((top_sum & ~kFoldBit) + (b_sum & ~kFoldBit) + fl) | (fold ? kFoldBit : 0u);
-            top = r;
-            top_single = kComposite;
-        } else if (keep == kKeepA) {
-            len = b_start;  // drop the primitive and the operator
-        } else {            // drop the accumulated value and the operator: the list is the primitive
-            out[0] = (uint16_t)b_i;
-            len = 1;
-            top = b;
-            top_single = b_i;
-            top_sum = b_sum;
-        }
-    }
-
-    __device__ __forceinline__ bool one_sign() const { return top.known && (top.lo > 0.0f || top.hi < 0.0f); }
-};
-
-// FoldWalk for a staged list (at most kStageOps ops): the kept primitives (each with the operator
-// behind it) as a bit mask in place of a list, bit (q + 1) / 2 for the primitive at position q;
-// the list is written once the tile has a slot.
+// PruneWalk for a left fold (P0 P1 op1 P2 op2 ..., at most kStageOps ops): the same decisions and
+// sums with the accumulated value and the latest primitive in registers instead of the LDS
+// stack (every operator's left operand is the accumulated value), and the kept primitives
+// (each with the operator behind it) as a bit mask in place of a list, bit (q + 1) / 2 for the
+// primitive at position q; the list is written once the tile has a slot.
 struct FoldMask {
     Iv top = iv_unknown();
     uint64_t kept = 0;
@@ -779,7 +728,7 @@ __global__ __launch_bounds__(64) void k_sp_prune(SpPass P)
             }
             done(w.one_sign(), w.len, w.top_sum);
         };
-        if (J.left_fold && staged) {  // the super-tile's list is a left fold too
+        if (J.left_fold) {  // the super-tile's list is a left fold too, and staged
             FoldMask w;
             for (uint32_t q = 0; q < sl; ++q) {
                 const uint32_t code = uniform_code(T, q), sum = sums[q];
@@ -788,9 +737,6 @@ __global__ __launch_bounds__(64) void k_sp_prune(SpPass P)
             }
             done(w.one_sign(), w.len(), w.top_sum);
             kept = w.kept;
-        } else if (J.left_fold) {
-            FoldWalk w;
-            walk(w, P.lists + (size_t)tile * P.list_stride);
         } else if (in_lds) {
             PruneWalk<true> w;
             walk(w, list);
@@ -901,7 +847,7 @@ __device__ __forceinline__ uint32_t div_by(uint32_t n, float r) { return (uint32
 
 // ---------------------------------------------------------------------------------
 // Bricks: the 4x4x4 blocks of 2x2x2 cells of a tile, brick (bx, by, bz) = bit
-// (bz * 4 + by) * 4 + bx of the slot's `slot_live`.  Per slot (one 64-lane block
+// (bz * 4 + by) * 4 + bx of its record's `live`.  Per slot (one 64-lane block
 // iteration, lane = brick): interval bounds of the tile's program on the brick's lattice
 // points; a brick whose values provably keep one sign holds no active cell, so its cells
 // are not contoured and its points are not evaluated.  Left-fold programs only (other
@@ -967,7 +913,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
             P.slot_nb[(size_t)slot * 8u + i] = ns;
         }
         if (!(lens & kLinearFlag) || n > kStageOps) {  // every brick is kept
-            if (b == 0) P.slot_live[slot] = RG.live = ~0ull;
+            if (b == 0) RG.live = ~0ull;
             continue;
         }
         __syncthreads();  // the previous slot's readers of T and A are done
@@ -1011,7 +957,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
         }
         const bool may_cross = !(acc.known && (acc.lo > 0.0f || acc.hi < 0.0f));
         const uint64_t m = __ballot(may_cross);
-        if (b == 0) P.slot_live[slot] = RG.live = m;
+        if (b == 0) RG.live = m;
     }
 }
 
@@ -1977,7 +1923,6 @@ __global__ __launch_bounds__(kScanThreads) void k_sp_rowdown(SpPass P)
         P.counters[kGenUsed] = 0;
         P.counters[kSlotsNow] = slots;
         P.counters[kSlotsUsed] = 0;
-        P.counters[kStageNow] = stage;
         P.counters[kStageUsed] = 0;
         if (slots > slots_max) P.counters[kSlotsMax] = slots;
         if (stage > stage_max) P.counters[kStageMax] = stage;
