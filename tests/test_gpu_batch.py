@@ -159,6 +159,30 @@ def test_batch_passes_overflow_and_repeat():
             same(profiled[i], solo)
 
 
+def test_batch_third_pass_after_overflow():
+    # Passes of 128M cells hold eight 256^3 jobs: eighteen and a small one are three passes, so
+    # that the third is queued into the first one's buffer set (after its copy has left it)
+    # while the second is repeated.  Every job equals the job alone.
+    print("three batch passes", flush=True)
+    s2m.tuning_clear()
+    with s2m.Context(0) as fresh:
+        nodes = [stacked_boxes(8, -0.65 + 0.01 * s) for s in range(18)]
+        nodes.insert(3, tape.torus_example())
+        progs = [fresh.program(x) for x in nodes]
+        params = [s2m.Params.reference(256, 2.0) for _ in progs]
+        params[3] = s2m.Params.reference(64, 2.0)
+        first = fresh.mesh_batch(progs, params)
+        assert fresh.last_timing()["slabs"] > 3  # passes and their repetitions
+        second = fresh.mesh_batch(progs, params)
+        assert fresh.last_timing()["slabs"] == 3
+        for i, (p, q) in enumerate(zip(progs, params)):
+            solo = fresh.mesh(p, q)
+            if q.res[0] == 256:  # above its share of the pass's first estimate
+                assert len(solo.vertices) > 6 * 256 * 256
+            same(first[i], solo)
+            same(second[i], solo)
+
+
 def test_batch_nan_results_equal_solo(ctx):
     # A 3-iteration Mandelbulb whose estimator gives NaN at some lattice points, so some
     # vertex positions and normals are NaN: meshed alone it takes the dense path, in a
