@@ -65,10 +65,12 @@ __device__ __forceinline__ uint32_t block_exclusive_256(uint32_t v, uint32_t* ld
 // ---------------------------------------------------------------------------------
 // SDFs of the tape programs, for the dense bodies (device_dense.h).
 // ---------------------------------------------------------------------------------
+// (The kernels take the tape as a __restrict__ argument and the call is inlined, so that the
+// wave-uniform ops are read through the scalar cache beside the kernels' stores.)
 struct TapeSdf {
     const s2m_op* ops;
     uint32_t n;
-    __device__ float operator()(float x, float y, float z) const { return tape_eval(ops, n, x, y, z); }
+    __device__ __forceinline__ float operator()(float x, float y, float z) const { return tape_eval(ops, n, x, y, z); }
 };
 
 // A tape that is one power-8 Mandelbulb op: the estimator called directly with its operands
@@ -134,7 +136,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
 // MANDEL = 1: the tape is one power-8 Mandelbulb op (k_signs<2>: its sign may be decided
 // early as well).
 template <int MANDEL>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_signs(BrickArgs a, const s2m_op* ops,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_signs(BrickArgs a,
+                                                                                         const s2m_op* __restrict__ ops,
                                                                                          uint32_t nops)
 {
     if constexpr (MANDEL == 2) sign_words(MandelSign(ops), a);
@@ -147,7 +150,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
 enum BrickSdf : int { kTapeSdf = 0, kMandelSdf = 1, kNoSdf = 2 };
 
 template <int SDF>
-__global__ __launch_bounds__(256) void k_contour(BrickArgs a, const s2m_op* ops, uint32_t nops)
+__global__ __launch_bounds__(256) void k_contour(BrickArgs a, const s2m_op* __restrict__ ops, uint32_t nops)
 {
     if constexpr (SDF == kMandelSdf) contour_bricks(MandelSdf(ops), a);
     else if constexpr (SDF == kTapeSdf) contour_bricks(TapeSdf{ops, nops}, a);
@@ -155,7 +158,7 @@ __global__ __launch_bounds__(256) void k_contour(BrickArgs a, const s2m_op* ops,
 }
 
 template <int SDF>
-__global__ __launch_bounds__(256) void k_emit(BrickArgs a, const s2m_op* ops, uint32_t nops)
+__global__ __launch_bounds__(256) void k_emit(BrickArgs a, const s2m_op* __restrict__ ops, uint32_t nops)
 {
     if constexpr (SDF == kMandelSdf) emit_bricks(MandelSdf(ops), a);
     else if constexpr (SDF == kTapeSdf) emit_bricks(TapeSdf{ops, nops}, a);

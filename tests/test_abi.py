@@ -97,3 +97,12 @@ def test_tape_flops_match_python_count():
     assert T.torus_example().flops() == 10
     assert T.csg64().flops() == 1774
     assert T.mandelbulb(8).flops() == 245
+
+
+def test_kernels_inline_the_tape_interpreter():
+    # a call per point (its ops then read through flat addresses) made the dense path's kernels
+    # up to 1.7 times as slow: no function of the interpreter may be left in the device code
+    code = Path(s2m.__file__).with_name("libsdf2mesh.so").read_bytes()
+    assert b"k_signs" in code and b"k_eval_lattice" in code
+    for name in (b"TapeSdfclE", b"MandelSdfclE", b"tape_evalE", b"tape_eval_listE"):
+        assert name not in code
