@@ -1439,15 +1439,15 @@ hipError_t signs_prog(hipStream_t s, const s2m_program* prog, BrickArgs a)
     return hipModuleLaunchKernel(prog->k_signs, g.x, g.y, g.z, 256, 1, 1, 0, s, args, nullptr);
 }
 
-// A compiled program's normals of the slab's vertices (a tape's are k_emit's).
+// Normals of the slab's vertices.
 hipError_t normals_prog(hipStream_t s, const s2m_program* prog, float eps, const MeshBufs& b)
 {
-    if (!prog->module) return hipSuccess;
+    if (!prog->module) return launch_normals(s, prog->ops.data(), prog->d_ops, prog->n, eps, b);
     float* vtx = b.vtx;
     const uint64_t* counters = b.counters;
     uint64_t vcap = b.vcap;
     void* args[] = {&eps, &vtx, &counters, &vcap};
-    return hipModuleLaunchKernel(prog->k_normals, kBrickBlocks, 1, 1, 256, 1, 1, 0, s, args, nullptr);
+    return hipModuleLaunchKernel(prog->k_normals, kNormalBlocks, 1, 1, 256, 1, 1, 0, s, args, nullptr);
 }
 
 // Buffers of a dense job that must not allocate (s2m_mesh_device_noalloc): every working
@@ -1469,8 +1469,8 @@ struct FixedBufs {
 // slab read the slab before).
 struct DenseLayout {
     uint32_t T, nx, ny, nbx, nby, max_nzl, max_blocks;
-    uint32_t strip, nstrips;  // brick rows per strip: the words and values of a strip (and of its
-                              // successor's first row) are held at a time
+    uint32_t px, py, nparts;  // bricks of a part per axis: the words and values of a part (and of the
+                              // bricks past it) are held at a time
     size_t stage_cap;
     size_t tables, words, vals, recs, stage, stage_sign, actbits, wpre, blocks, chunks, tblocks, counters;
     bool piped;   // two sets of words and values
@@ -1484,10 +1484,10 @@ struct DenseLayout {
     }
 };
 
-// stage_cap: vertices staged per slab, 0 for one per cell.  vals: the values of bricks (with
-// both signs, or all) are kept.  strip: 0 for one strip.
+// stage_cap: vertices staged per slab, 0 for one per cell.  vals: the values are kept.  px, py: 0
+// for one part.
 DenseLayout dense_layout(const Job& j, uint32_t T, bool bricks, bool piped, uint64_t stage_cap, bool vals,
-                         uint32_t strip = 0)
+                         uint32_t px = 0, uint32_t py = 0)
 {
     DenseLayout L{};
     const uint64_t plane = (uint64_t)j.res[0] * j.res[1];
@@ -1500,16 +1500,17 @@ DenseLayout dense_layout(const Job& j, uint32_t T, bool bricks, bool piped, uint
         const uint32_t z1 = std::min(z0 + T, j.nz_cells);
         L.max_nzl = std::max(L.max_nzl, j.ax[2].hi[z1 - 1] - j.ax[2].lo[z0] + 1);
     }
-    L.strip = strip ? std::min(strip, L.nby) : L.nby;
-    L.nstrips = (L.nby + std::max(L.strip, 1u) - 1u) / std::max(L.strip, 1u);
-    const size_t rows = std::min(L.strip + 1u, L.nby);  // of the words and values
+    L.px = std::max(px ? std::min(px, L.nbx) : L.nbx, 1u);
+    L.py = std::max(py ? std::min(py, L.nby) : L.nby, 1u);
+    L.nparts = ((L.nbx + L.px - 1u) / L.px) * ((L.nby + L.py - 1u) / L.py);
+    const size_t held = (size_t)std::min(L.px + 1u, L.nbx) * std::min(L.py + 1u, L.nby);  // per layer
     const size_t nbricks = bricks ? (size_t)L.nbx * L.nby * ((L.max_nzl + 3u) / 4u) : 0;
     L.max_blocks = (uint32_t)((plane * T + kCellsPerBlock - 1) / kCellsPerBlock);
     L.stage_cap = bricks ? (size_t)(stage_cap ? std::min<uint64_t>(stage_cap, plane * T) : plane * T) : 0;
     L.piped = piped;
     L.tables = tables_bytes(j);
-    L.words = bricks ? L.nbx * rows * ((L.max_nzl + 3u) / 4u) * sizeof(uint64_t) : 0;
-    L.vals = vals ? L.nbx * rows * 16 * L.max_nzl * sizeof(float) : 0;  // brick_vals
+    L.words = bricks ? held * ((L.max_nzl + 3u) / 4u) * sizeof(uint64_t) : 0;
+    L.vals = vals ? held * 16 * L.max_nzl * sizeof(float) : 0;  // brick_vals
     L.recs = nbricks * sizeof(BrickRec);
     L.stage = L.stage_cap * 3 * sizeof(float);
     L.stage_sign = L.stage_cap;
@@ -1518,7 +1519,7 @@ DenseLayout dense_layout(const Job& j, uint32_t T, bool bricks, bool piped, uint
     L.wpre = (size_t)L.max_blocks * (kCellsPerBlock / 64) * sizeof(uint16_t);
     L.tblocks = (size_t)((plane * T + kBlock - 1) / kBlock) * sizeof(uint32_t);
     L.chunks = kRankChunks * sizeof(uint32_t);
-    L.counters = (kNumCounters + (L.nstrips > 1 ? L.nstrips : 0)) * sizeof(uint64_t);  // and the strips' kBrickAlloc
+    L.counters = (kNumCounters + (L.nparts > 1 ? L.nparts : 0)) * sizeof(uint64_t);  // and the parts' kBrickAlloc
     return L;
 }
 
@@ -1568,14 +1569,15 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
     // until the slab two before has contoured its bricks (the last reader of its words and
     // kept values), and the first evaluation waits for the tables queued before it.
     const bool piped = !fx && !h_corners && slab < j.nz_cells;
-    // the values a compiled program's vertices are placed from; a tape's are evaluated where
-    // they are not kept
-    const bool keep_vals = prog && !h_corners && (prog->module || (!fx && !sign_early(prog->ops.data(), prog->n)));
+    // the Mandelbulb's signs decided early, else the values of the sign pass kept
+    const s2m_op* const early = prog && sign_early(prog->ops.data(), prog->n) ? prog->d_ops : nullptr;
+    const bool keep_vals = prog && !h_corners && !early;
     DenseLayout L = dense_layout(j, slab, !h_corners, piped, want_s, keep_vals);
     if (fx) {  // the largest slab (at most the usual one) whose buffers fit the scratch
         while (L.T > 1 && L.carved() > fx->scratch_bytes) L = dense_layout(j, L.T - 1, true, false, 0, keep_vals);
-        while (keep_vals && L.strip > 1 && L.carved() > fx->scratch_bytes)  // one cell plane in strips
-            L = dense_layout(j, 1, true, false, 0, true, (L.strip + 1) / 2);
+        while (keep_vals && L.px > 1 && L.carved() > fx->scratch_bytes)  // one cell plane in parts
+            L = L.py > 1 ? dense_layout(j, 1, true, false, 0, true, L.px, (L.py + 1) / 2)
+                         : dense_layout(j, 1, true, false, 0, true, (L.px + 1) / 2, 1);
         if (L.carved() > fx->scratch_bytes)
             return fail(S2M_E_ARG, "a %u x %u grid needs %llu bytes of working memory per cell plane; "
                                    "the no-allocation scratch holds %llu",
@@ -1739,8 +1741,8 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
             A.ny = L.ny;
             A.nzl = nzl;
             A.lz0 = lz0;
-            A.nbx = L.nbx;
-            A.nby = A.own = L.nby;
+            A.nbx = A.ownx = L.nbx;
+            A.nby = A.owny = L.nby;
             A.nbz = (nzl + 3u) / 4u;
             A.rx = a.rx;
             A.ry = a.ry;
@@ -1764,18 +1766,25 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
             A.eps = p->eps;
             A.normals = normals ? 1u : 0u;
             A.run = sign_run((uint64_t)A.nbx * A.nby * A.nbz);
-            auto strip = [&](uint32_t k) {  // brick rows k * L.strip ..: its own records and staging space
+            auto part = [&](uint32_t k) {  // its own records and staging space
                 BrickArgs B = A;
-                if (L.nstrips == 1) return B;
-                B.by0 = k * L.strip;
-                B.own = std::min(L.strip, L.nby - B.by0);
-                B.nby = std::min(B.own + 1u, L.nby - B.by0);
+                if (L.nparts == 1) return B;
+                const uint32_t npx = (L.nbx + L.px - 1u) / L.px;
+                B.bx0 = k % npx * L.px;
+                B.by0 = k / npx * L.py;
+                B.ownx = std::min(L.px, L.nbx - B.bx0);
+                B.owny = std::min(L.py, L.nby - B.by0);
+                B.nbx = std::min(B.ownx + 1u, L.nbx - B.bx0);
+                B.nby = std::min(B.owny + 1u, L.nby - B.by0);
                 B.run = sign_run((uint64_t)B.nbx * B.nby * B.nbz);
-                B.recs = recs + (size_t)B.by0 * B.nbx * B.nbz;
+                B.recs = recs + ((size_t)B.by0 * L.nbx + (size_t)B.bx0 * B.owny) * B.nbz;
                 B.alloc = b.counters + kNumCounters + k;
-                const std::vector<uint32_t>& lo = j.ax[1].lo;  // ascending
-                const size_t rows = std::lower_bound(lo.begin(), lo.end(), 4u * B.by0) - lo.begin();
-                B.stage0 = (uint32_t)(rows * a.rx * nzc);
+                auto cells = [&](int axis, uint32_t brick) {  // cells of the axis in the bricks before it
+                    const std::vector<uint32_t>& lo = j.ax[axis].lo;  // ascending
+                    return (size_t)(std::lower_bound(lo.begin(), lo.end(), 4u * brick) - lo.begin());
+                };
+                const size_t y0 = cells(1, B.by0), ny = cells(1, B.by0 + B.owny) - y0;
+                B.stage0 = (uint32_t)((y0 * a.rx + cells(0, B.bx0) * ny) * nzc);
                 return B;
             };
 
@@ -1785,7 +1794,7 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
             if (piped && words_free[cur]) HIP_TRY(hipStreamWaitEvent(es, words_free[cur], 0));
             if (m[0]) HIP_TRY(hipEventRecord(m[0], es));
             if (!h_corners) {
-                HIP_TRY(signs_prog(es, prog, strip(0)));
+                HIP_TRY(signs_prog(es, prog, part(0)));
                 lattice_points += (uint64_t)L.nx * L.ny * nzl;
             }
             if (m[1]) HIP_TRY(hipEventRecord(m[1], es));
@@ -1796,15 +1805,13 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
             }
             if (m[5]) HIP_TRY(hipEventRecord(m[5], ctx->stream));
             const float* src = h_corners ? ctx->corners.as<float>() + (size_t)z0 * plane * 8 : nullptr;
-            const uint32_t tape_ops = prog && !prog->module ? prog->n : 0u;
-            const s2m_op* host_ops = tape_ops ? prog->ops.data() : nullptr;
             if (h_corners) {
                 HIP_TRY(launch_cells_from_corners(ctx->stream, a, src, bs, 0));
             } else {
-                for (uint32_t k = 0; k < L.nstrips; ++k) {
-                    if (k) HIP_TRY(signs_prog(ctx->stream, prog, strip(k)));
-                    HIP_TRY(launch_find_bricks(ctx->stream, strip(k)));
-                    HIP_TRY(launch_contour(ctx->stream, strip(k), host_ops, prog->d_ops, tape_ops));
+                for (uint32_t k = 0; k < L.nparts; ++k) {
+                    if (k) HIP_TRY(signs_prog(ctx->stream, prog, part(k)));
+                    HIP_TRY(launch_find_bricks(ctx->stream, part(k)));
+                    HIP_TRY(launch_contour(ctx->stream, part(k), early));
                 }
                 if (piped) {
                     words_free[cur] = mark(ctx->stream);
@@ -1814,9 +1821,8 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
             HIP_TRY(launch_ranks(ctx->stream, bs, a.ncells));
             if (m[2]) HIP_TRY(hipEventRecord(m[2], ctx->stream));
             if (h_corners) HIP_TRY(launch_cells_from_corners(ctx->stream, a, src, bs, 1));
-            for (uint32_t k = 0; !h_corners && k < L.nstrips; ++k)
-                HIP_TRY(launch_emit(ctx->stream, strip(k), host_ops, prog->d_ops, tape_ops));
-            if (!h_corners && normals) HIP_TRY(normals_prog(ctx->stream, prog, p->eps, b));
+            for (uint32_t k = 0; !h_corners && k < L.nparts; ++k) HIP_TRY(launch_emit(ctx->stream, part(k), early));
+            if (keep_vals && normals) HIP_TRY(normals_prog(ctx->stream, prog, p->eps, b));
             if (m[3]) HIP_TRY(hipEventRecord(m[3], ctx->stream));
             HIP_TRY(launch_quads(ctx->stream, a, bs, prev, snap_dev ? snap_dev + kSnapWords * slabs : nullptr,
                                  z1 == j.nz_cells ? static_cast<uint64_t*>(back_dev) : nullptr));

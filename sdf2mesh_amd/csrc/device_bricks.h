@@ -94,11 +94,10 @@ struct KeptValues {};  // in place of an SDF: its values are in `vals`
 
 // The listed bricks, four at a time per block of 256 (one wave each).  The SDF at the
 // corners of the cells with a sign change (at most 5 x 5 x 5 points per brick) goes into
-// LDS: kept values are read, the four bricks' other points listed together so that the
-// evaluating waves are full (with KeptValues as the SDF every point is kept); then one lane
-// per cell, the vertex rule.  Vertices are staged (position, sign bits) at the record's base
-// in cell order, the record's mask becomes the cells with a vertex and their bits are set in
-// `actbits` (zero on entry).
+// LDS: with KeptValues from `vals`, else evaluated, the four bricks' points listed together
+// so that the evaluating waves are full; then one lane per cell, the vertex rule.  Vertices
+// are staged (position, sign bits) at the record's base in cell order, the record's mask
+// becomes the cells with a vertex and their bits are set in `actbits` (zero on entry).
 template <class F>
 __device__ __forceinline__ void contour_bricks(const F& sdf, const BrickArgs& a)
 {
@@ -114,18 +113,14 @@ __device__ __forceinline__ void contour_bricks(const F& sdf, const BrickArgs& a)
         const uint32_t ix0 = R->bx * 4u, iy0 = R->by * 4u, iz0 = a.lz0 + R->bz * 4u;
         // points p = (z * 5 + y) * 5 + x used by a cell of the mask: of the cells x - 1, x (and
         // so on), as a 64-bit product of the three axes' pairs
-        uint32_t kept = 0;  // bit dz * 4 + dy * 2 + dx: the brick there has its values kept
-        size_t brick = 0;   // the values of the lane's brick of the eight
-        if (kKept || a.vals) {
-            const uint32_t d = l & 7u, bx = R->bx + (d & 1u), by = R->by - a.by0 + ((d >> 1) & 1u), bz = R->bz + (d >> 2);
-            const bool in = l < 8u && bx < a.nbx && by < a.nby && bz < a.nbz;
-            uint64_t word = 0;
-            if (!kKept && in) word = a.words[((size_t)bz * a.nby + by) * a.nbx + bx];
-            if (in) brick = brick_vals(a, bx, by, bz);
-            kept = kKept ? 0xffu : (uint32_t)__ballot(word != 0ull && word != ~0ull);
+        size_t brick = 0;  // the values of the lane's brick of the eight
+        if constexpr (kKept) {
+            const uint32_t d = l & 7u, bx = R->bx - a.bx0 + (d & 1u), by = R->by - a.by0 + ((d >> 1) & 1u);
+            const uint32_t bz = R->bz + (d >> 2);
+            if (l < 8u && bx < a.nbx && by < a.nby && bz < a.nbz) brick = brick_vals(a, bx, by, bz);
         }
-        uint64_t need[2];
-        uint32_t n = 0;
+        [[maybe_unused]] uint64_t need[2];
+        [[maybe_unused]] uint32_t n = 0;
 #pragma unroll
         for (uint32_t h = 0; h < 2; ++h) {
             const uint32_t p = h * 64u + l, pz = p / 25u, py = (p / 5u) % 5u, px = p % 5u;
@@ -133,14 +128,12 @@ __device__ __forceinline__ void contour_bricks(const F& sdf, const BrickArgs& a)
             const uint32_t rows = ((ym & 1u) | (ym & 2u) << 3 | (ym & 4u) << 6 | (ym & 8u) << 9) * xm;
             const uint64_t cells = (zm & 1u ? (uint64_t)rows : 0ull) | (zm & 2u ? (uint64_t)rows << 16 : 0ull) |
                                    (zm & 4u ? (uint64_t)rows << 32 : 0ull) | (zm & 8u ? (uint64_t)rows << 48 : 0ull);
-            bool used = p < 125u && (mask & cells) != 0ull;
-            const uint32_t d = (px >> 2) | (py >> 2) << 1 | (pz >> 2) << 2;
-            const size_t at = (size_t)__shfl((long long)brick, (int)(d & 7u), 64);
-            if (used && ((kept >> d) & 1u)) {
-                val[w * 125u + p] = a.vals[at + (pz & 3u) * 16u + (py & 3u) * 4u + (px & 3u)];
-                used = false;
-            }
-            if constexpr (!kKept) {
+            const bool used = p < 125u && (mask & cells) != 0ull;
+            if constexpr (kKept) {
+                const uint32_t d = (px >> 2) | (py >> 2) << 1 | (pz >> 2) << 2;
+                const size_t at = (size_t)__shfl((long long)brick, (int)(d & 7u), 64);
+                if (used) val[w * 125u + p] = a.vals[at + (pz & 3u) * 16u + (py & 3u) * 4u + (px & 3u)];
+            } else {
                 need[h] = __ballot(used);
                 n += (uint32_t)__popcll(need[h]);
             }

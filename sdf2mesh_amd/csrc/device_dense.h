@@ -8,9 +8,9 @@
 // A slab's corner lattice is handled in bricks of 4 x 4 x 4 points.  sign_words evaluates
 // every point and keeps `value > 0`, one 64-bit word per brick; bricks whose cells change
 // sign are listed (k_find_bricks), and contour_bricks needs the values at just the corners
-// of those cells.  A compiled program's values are all kept (4 bytes a point beside a whole
-// program each).  Of a tape's, those inside bricks with both signs are kept (a 256-byte line
-// per brick), the others evaluated again: well under 1 % of the points at 512^3.
+// of those cells.  sign_words keeps the values it takes (4 bytes a point beside a whole
+// program each), brick by brick, so that a brick's lie in few lines; where the sign is
+// decided without the value (the Mandelbulb's early signs) they are evaluated then.
 #pragma once
 #ifndef __HIPCC_RTC__
 #include <hip/hip_runtime.h>
@@ -56,7 +56,7 @@ __device__ __forceinline__ void write_unit(float* o, float gx, float gy, float g
 
 __device__ __forceinline__ uint32_t clamp_to(uint32_t i, uint32_t n) { return i < n ? i : n - 1u; }
 
-// Where the values of brick (bx, by, bz), by counted from by0, start: 16 per lattice plane of
+// Where the values of brick (bx, by, bz), counted from (bx0, by0), start: 16 per lattice plane of
 // the slab in it, bricks of one layer after each other.
 __device__ __forceinline__ size_t brick_vals(const BrickArgs& a, uint32_t bx, uint32_t by, uint32_t bz)
 {
@@ -65,12 +65,11 @@ __device__ __forceinline__ size_t brick_vals(const BrickArgs& a, uint32_t bx, ui
 }
 
 // Sign of an SDF at a point as that of its value, without a test on whole bricks.
-template <class F, bool KEEP_ALL>
+template <class F>
 struct PointSign {
     F sdf;
     static constexpr bool kBricks = false;   // brick() decides whole bricks
-    static constexpr bool kValue = true;     // operator() returns the value itself
-    static constexpr bool kAll = KEEP_ALL;   // every brick's values are kept
+    static constexpr bool kValue = true;     // operator() returns the value itself, which is kept
     __device__ float operator()(float x, float y, float z) const { return sdf(x, y, z); }
     __device__ int brick(float, float, float, float, float, float) const { return -1; }
 };
@@ -87,13 +86,13 @@ __device__ __forceinline__ void sign_words(const S& sign, const BrickArgs& a)
     const uint32_t l = threadIdx.x & 63u, w = threadIdx.x >> 6;
     const uint32_t b0 = blockIdx.x * a.run, by = blockIdx.y * 4u + w, bz = blockIdx.z;
     if (by >= a.nby) return;
-    const float xr = a.cx[clamp_to(b0 * 4u + l, a.nx)];
+    const float xr = a.cx[clamp_to((a.bx0 + b0) * 4u + l, a.nx)];
     const float y = a.cy[clamp_to((a.by0 + by) * 4u + ((l >> 2) & 3u), a.ny)];
     const float z = a.cz[a.lz0 + clamp_to(bz * 4u + (l >> 4), a.nzl)];
     const uint32_t nb = min(a.run, a.nbx - b0);
     const size_t row = ((size_t)bz * a.nby + by) * a.nbx + b0;
     const uint32_t planes16 = 16u * min(a.nzl - 4u * bz, 4u);  // values of a brick
-    float* const vals = a.vals ? a.vals + brick_vals(a, b0, by, bz) : nullptr;
+    float* const vals = S::kValue ? a.vals + brick_vals(a, b0, by, bz) : nullptr;
     uint64_t word = 0;  // lane b: brick b's
     uint32_t todo = (1u << nb) - 1u;
     if constexpr (S::kBricks) {
@@ -117,7 +116,7 @@ __device__ __forceinline__ void sign_words(const S& sign, const BrickArgs& a)
         const uint64_t m = __ballot(v > 0.0f);
         if (l == b) word = m;
         if constexpr (S::kValue) {
-            if ((S::kAll || (a.vals && m != 0ull && m != ~0ull)) && l < planes16) vals[b * planes16 + l] = v;
+            if (l < planes16) vals[b * planes16 + l] = v;
         }
     }
     if (l < nb) a.words[row + l] = word;
@@ -144,7 +143,7 @@ __device__ __forceinline__ void tap_normal(const F& sdf, float px, float py, flo
     write_unit(o, ((d1 + (-d2)) + (-d3)) + d4, (((-d1) + (-d2)) + d3) + d4, (((-d1) + d2) + (-d3)) + d4);
 }
 
-// A compiled program's normals: the vertices the slab has written, [counters[kDenseVtxPrev],
+// Normals of the vertices the slab has written, [counters[kDenseVtxPrev],
 // counters[kDenseVtxTotal]) below vcap, their positions in place.  LIB: the library's
 // normal of the SDF F, else F(px, py, pz, eps, o) writes o[3..5].
 constexpr uint32_t kDenseVtxTotal = 0, kDenseVtxPrev = 1;  // Counter (internal.h)

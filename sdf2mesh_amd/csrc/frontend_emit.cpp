@@ -813,7 +813,7 @@ bool emit_hip(const Module& m, Lang lang, const std::string& entry, std::string&
          "    uint32_t nzl, uint32_t pitch, float* __restrict__ lat)\n{\n"
          "    s2m::eval_lattice_point(s2m_shared_fn{}, cx, cy, cz, nx, ny, lz0, nzl, pitch, lat);\n}\n"
          "extern \"C\" __global__ __launch_bounds__(256) void s2m_c_signs(s2m::BrickArgs a)\n{\n"
-         "    s2m::sign_words(s2m::PointSign<s2m_user_fn, true>{}, a);\n}\n";
+         "    s2m::sign_words(s2m::PointSign<s2m_user_fn>{}, a);\n}\n";
     if (user_normal)
         o << "struct s2m_user_normal {\n"
              "    __device__ void operator()(float px, float py, float pz, float eps, float* o) const\n    {\n"

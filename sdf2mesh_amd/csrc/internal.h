@@ -18,6 +18,7 @@ constexpr uint32_t kRankChunks = kMaxScanBlocks / 1024;  // chunks of 1024 block
 static_assert(kRankChunks <= 256, "one block's threads set up the chunk bases");
 constexpr uint32_t kBrickBlocks = 2048;      // blocks of 4 waves of the per-brick kernels: 8 waves per
                                              // SIMD of 256 CUs
+constexpr uint32_t kNormalBlocks = 4096;     // blocks of 64 vertices of the normal kernels
 constexpr uint32_t kNone = 0xffffffffu;      // "no vertex" (u32::MAX, mesh.rs:330)
 
 // Unsigned division by a runtime constant d >= 1 (round-up multiplier method):
@@ -231,7 +232,8 @@ hipError_t launch_eval_lattice(hipStream_t s, const s2m_op* ops, uint32_t nops, 
                                const float* cy, const float* cz, uint32_t nx, uint32_t ny,
                                uint32_t lz0, uint32_t nzl, uint32_t pitch, float* lat);
 // The dense slab's kernels (kernels.hip, bodies in device_dense.h and device_bricks.h).  host_ops: the host copy
-// of the tape (it selects the kernel); nops = 0: a compiled program, whose values are kept.
+// of the tape (it selects the kernel); op: the Mandelbulb op whose signs were decided early
+// (sign_early), NULL where the sign pass has kept the values.
 struct BrickArgs;
 bool mandel_power8(const s2m_op* ops, uint32_t n);  // the tape is one power-8 Mandelbulb op
 bool sign_early(const s2m_op* ops, uint32_t n);     // its signs are decided early (no values to keep)
@@ -239,8 +241,10 @@ dim3 sign_grid(const BrickArgs& a);                 // blocks of 256
 uint32_t sign_run(uint64_t bricks);                 // BrickArgs::run for a slab of so many bricks
 hipError_t launch_signs(hipStream_t s, const BrickArgs& a, const s2m_op* host_ops, const s2m_op* ops, uint32_t nops);
 hipError_t launch_find_bricks(hipStream_t s, const BrickArgs& a);
-hipError_t launch_contour(hipStream_t s, const BrickArgs& a, const s2m_op* host_ops, const s2m_op* ops, uint32_t nops);
-hipError_t launch_emit(hipStream_t s, const BrickArgs& a, const s2m_op* host_ops, const s2m_op* ops, uint32_t nops);
+hipError_t launch_contour(hipStream_t s, const BrickArgs& a, const s2m_op* op);
+hipError_t launch_emit(hipStream_t s, const BrickArgs& a, const s2m_op* op);
+hipError_t launch_normals(hipStream_t s, const s2m_op* host_ops, const s2m_op* ops, uint32_t nops, float eps,
+                          const MeshBufs& b);
 hipError_t launch_ranks(hipStream_t s, const MeshBufs& b, uint32_t ncells);
 hipError_t launch_dense_begin(hipStream_t s, uint64_t* counters, uint32_t ncounters, uint64_t* words, uint32_t ncells,
                               const void* host_tables, void* tables, size_t bytes, uint32_t* cbase);

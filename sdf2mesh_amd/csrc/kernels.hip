@@ -6,11 +6,13 @@
 // s2m_c_normals are in its own module):
 //   k_signs            sign of the SDF at every corner-lattice point, one bit each  (VALU bound)
 //   k_find_bricks      the 4x4x4 bricks whose cells change sign
-//   k_contour          their cells' corner values (kept by the sign pass or taken again), the
-//                      vertex rule, staged vertices, one activity bit per cell
+//   k_contour          their cells' corner values (kept by the sign pass, or taken where the signs
+//                      were decided early), the vertex rule, staged vertices, one activity bit
+//                      per cell
 //   k_ranks            vertices before each word of 64 cells, block of 1024 cells and chunk
-//   k_emit             staged vertices at their ordered index, with 4-tap normals (a compiled
-//                      program's: s2m_c_normals after it)
+//   k_emit             staged vertices at their ordered index (after early signs with their 4-tap
+//                      normals)
+//   k_normals          4-tap normals
 //   k_quads<0>, k_tri_offsets, k_quads<1>   triangles per 256 vertices, their offsets, triangles
 //   k_slab_end         between slabs: the other slab's bits cleared
 // (with several slabs the signs are evaluated one slab ahead on a second stream; per-cell
@@ -141,28 +143,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
                                                                                          uint32_t nops)
 {
     if constexpr (MANDEL == 2) sign_words(MandelSign(ops), a);
-    else if constexpr (MANDEL == 1) sign_words(PointSign<MandelSdf, false>{MandelSdf(ops)}, a);
-    else sign_words(PointSign<TapeSdf, false>{TapeSdf{ops, nops}}, a);
+    else if constexpr (MANDEL == 1) sign_words(PointSign<MandelSdf>{MandelSdf(ops)}, a);
+    else sign_words(PointSign<TapeSdf>{TapeSdf{ops, nops}}, a);
 }
 
-// What the kernels of the listed bricks evaluate: a tape, one power-8 Mandelbulb op, or nothing
-// (a compiled program's kept values).
-enum BrickSdf : int { kTapeSdf = 0, kMandelSdf = 1, kNoSdf = 2 };
-
-template <int SDF>
-__global__ __launch_bounds__(256) void k_contour(BrickArgs a, const s2m_op* __restrict__ ops, uint32_t nops)
+// KEPT: from the values the sign pass has kept (normals from k_normals or s2m_c_normals), else
+// with the power-8 Mandelbulb op `op`, whose signs were decided early.
+template <bool KEPT>
+__global__ __launch_bounds__(256) void k_contour(BrickArgs a, const s2m_op* __restrict__ op)
 {
-    if constexpr (SDF == kMandelSdf) contour_bricks(MandelSdf(ops), a);
-    else if constexpr (SDF == kTapeSdf) contour_bricks(TapeSdf{ops, nops}, a);
-    else contour_bricks(KeptValues{}, a);
+    if constexpr (KEPT) contour_bricks(KeptValues{}, a);
+    else contour_bricks(MandelSdf(op), a);
 }
 
-template <int SDF>
-__global__ __launch_bounds__(256) void k_emit(BrickArgs a, const s2m_op* __restrict__ ops, uint32_t nops)
+template <bool KEPT>
+__global__ __launch_bounds__(256) void k_emit(BrickArgs a, const s2m_op* __restrict__ op)
 {
-    if constexpr (SDF == kMandelSdf) emit_bricks(MandelSdf(ops), a);
-    else if constexpr (SDF == kTapeSdf) emit_bricks(TapeSdf{ops, nops}, a);
-    else emit_bricks(KeptValues{}, a);
+    if constexpr (KEPT) emit_bricks(KeptValues{}, a);
+    else emit_bricks(MandelSdf(op), a);
+}
+
+// Normals of a tape's vertices, four full lanes each: a tap costs a whole program, where k_emit's
+// rounds over the vertices of four bricks leave a third of the lanes idle (252 us for 136 in
+// CSG-64 at 256^3).
+template <bool MANDEL>
+__global__ __launch_bounds__(256) void k_normals(const s2m_op* __restrict__ ops, uint32_t nops, float eps, float* vtx,
+                                                 const uint64_t* counters, uint64_t vcap)
+{
+    if constexpr (MANDEL) vertex_normals<true>(MandelSdf(ops), eps, vtx, counters, vcap);
+    else vertex_normals<true>(TapeSdf{ops, nops}, eps, vtx, counters, vcap);
 }
 
 // ---------------------------------------------------------------------------------
@@ -180,10 +189,10 @@ constexpr uint32_t kFindBricks = 4;
 
 __device__ __forceinline__ uint64_t mixed_cells(const BrickArgs& a, uint32_t i, uint32_t& bx, uint32_t& by, uint32_t& bz)
 {
-    const uint32_t row = i / a.nbx;
-    bx = i - row * a.nbx;
-    bz = row / a.own;
-    by = row - bz * a.own;
+    const uint32_t row = i / a.ownx;
+    bx = i - row * a.ownx;
+    bz = row / a.owny;
+    by = row - bz * a.owny;
     const uint32_t dx = bx + 1 < a.nbx ? 1u : 0u;  // past the end: cells that are masked off
     const size_t dy = by + 1 < a.nby ? a.nbx : 0u, dz = bz + 1 < a.nbz ? (size_t)a.nbx * a.nby : 0u;
     const uint64_t* w = a.words + ((size_t)bz * a.nby + by) * a.nbx + bx;
@@ -206,7 +215,7 @@ __device__ __forceinline__ uint64_t mixed_cells(const BrickArgs& a, uint32_t i, 
     uint32_t vx = 0, vy = 0, vz = 0;  // the axes' cells
 #pragma unroll
     for (uint32_t k = 0; k < 4; ++k) {
-        const uint32_t ix = bx * 4u + k, iy = (a.by0 + by) * 4u + k, iz = bz * 4u + k;
+        const uint32_t ix = (a.bx0 + bx) * 4u + k, iy = (a.by0 + by) * 4u + k, iz = bz * 4u + k;
         if (ix < a.nx && a.cox[ix] != kNoCell) vx |= 1u << k;
         if (iy < a.ny && a.coy[iy] != kNoCell) vy |= 1u << (4u * k);
         if (iz + 1u < a.nzl) {
@@ -223,7 +232,7 @@ __global__ __launch_bounds__(256) void k_find_bricks(BrickArgs a)
 {
     __shared__ uint32_t wrecs[kBlock / 64], wcells[kBlock / 64];
     __shared__ uint64_t base;
-    const uint32_t n = a.nbx * a.own * a.nbz;
+    const uint32_t n = a.ownx * a.owny * a.nbz;
     uint64_t mask[kFindBricks];
     BrickRec rec[kFindBricks];
     uint32_t recs = 0, cells = 0;  // of this thread
@@ -232,7 +241,7 @@ __global__ __launch_bounds__(256) void k_find_bricks(BrickArgs a)
         const uint32_t i = (blockIdx.x * kFindBricks + k) * kBlock + threadIdx.x;
         uint32_t bx = 0, by = 0, bz = 0;
         mask[k] = i < n ? mixed_cells(a, i, bx, by, bz) : 0ull;
-        rec[k] = BrickRec{mask[k], 0u, (uint16_t)bx, (uint16_t)(a.by0 + by), (uint16_t)bz, 0};
+        rec[k] = BrickRec{mask[k], 0u, (uint16_t)(a.bx0 + bx), (uint16_t)(a.by0 + by), (uint16_t)bz, 0};
         recs += mask[k] != 0ull ? 1u : 0u;
         cells += (uint32_t)__popcll(mask[k]);
     }
@@ -676,29 +685,34 @@ hipError_t launch_signs(hipStream_t s, const BrickArgs& a, const s2m_op* host_op
     return hipGetLastError();
 }
 
-template <class K0, class K1, class K2>
-static hipError_t launch_bricks(hipStream_t s, K0 tape, K1 mandel, K2 kept, const BrickArgs& a, const s2m_op* host_ops,
-                                const s2m_op* ops, uint32_t nops)
+hipError_t launch_contour(hipStream_t s, const BrickArgs& a, const s2m_op* op)
 {
-    if (nops == 0) hipLaunchKernelGGL(kept, dim3(kBrickBlocks), dim3(256), 0, s, a, ops, nops);
-    else if (mandel_power8(host_ops, nops)) hipLaunchKernelGGL(mandel, dim3(kBrickBlocks), dim3(256), 0, s, a, ops, nops);
-    else hipLaunchKernelGGL(tape, dim3(kBrickBlocks), dim3(256), 0, s, a, ops, nops);
+    if (op) hipLaunchKernelGGL(k_contour<false>, dim3(kBrickBlocks), dim3(256), 0, s, a, op);
+    else hipLaunchKernelGGL(k_contour<true>, dim3(kBrickBlocks), dim3(256), 0, s, a, op);
     return hipGetLastError();
 }
 
-hipError_t launch_contour(hipStream_t s, const BrickArgs& a, const s2m_op* host_ops, const s2m_op* ops, uint32_t nops)
+hipError_t launch_emit(hipStream_t s, const BrickArgs& a, const s2m_op* op)
 {
-    return launch_bricks(s, k_contour<kTapeSdf>, k_contour<kMandelSdf>, k_contour<kNoSdf>, a, host_ops, ops, nops);
+    if (op) hipLaunchKernelGGL(k_emit<false>, dim3(kBrickBlocks), dim3(256), 0, s, a, op);
+    else hipLaunchKernelGGL(k_emit<true>, dim3(kBrickBlocks), dim3(256), 0, s, a, op);
+    return hipGetLastError();
 }
 
-hipError_t launch_emit(hipStream_t s, const BrickArgs& a, const s2m_op* host_ops, const s2m_op* ops, uint32_t nops)
+hipError_t launch_normals(hipStream_t s, const s2m_op* host_ops, const s2m_op* ops, uint32_t nops, float eps,
+                          const MeshBufs& b)
 {
-    return launch_bricks(s, k_emit<kTapeSdf>, k_emit<kMandelSdf>, k_emit<kNoSdf>, a, host_ops, ops, nops);
+    const dim3 grid(kNormalBlocks);
+    if (mandel_power8(host_ops, nops))
+        hipLaunchKernelGGL(k_normals<true>, grid, dim3(256), 0, s, ops, nops, eps, b.vtx, b.counters, b.vcap);
+    else
+        hipLaunchKernelGGL(k_normals<false>, grid, dim3(256), 0, s, ops, nops, eps, b.vtx, b.counters, b.vcap);
+    return hipGetLastError();
 }
 
 hipError_t launch_find_bricks(hipStream_t s, const BrickArgs& a)
 {
-    const uint64_t n = (uint64_t)a.nbx * a.own * a.nbz;
+    const uint64_t n = (uint64_t)a.ownx * a.owny * a.nbz;
     if (n > 0x7fffffffull) return hipErrorInvalidValue;
     const uint64_t per = kFindBricks * kBlock;
     hipLaunchKernelGGL(k_find_bricks, dim3((uint32_t)((n + per - 1u) / per)), dim3(kBlock), 0, s, a);
@@ -767,7 +781,7 @@ __global__ __launch_bounds__(256) void k_dense_begin(uint64_t* __restrict__ coun
     for (uint32_t i = t; i < nwords; i += stride) words[i] = 0ull;
 }
 
-// After the quad pass of a slab that is not the last: the allocation counter (of strips:
+// After the quad pass of a slab that is not the last: the allocation counter (of parts:
 // counters) reset, and the other activity words and chunk bases (the previous slab's, read for
 // the last time by this slab's quads) set up for the next slab.
 __global__ __launch_bounds__(256) void k_slab_end(uint64_t* __restrict__ counters, uint32_t ncounters,

@@ -179,18 +179,24 @@ def test_compiled_bricks(ctx, res, flags):
         same_mesh(ctx.mesh(c, p), ctx.mesh(t, p))
 
 
-@pytest.mark.parametrize("res", [(130, 70, 40), (1750, 1740, 3), (330, 9000, 3)])
-def test_compiled_noalloc(ctx, res):
+# (long planes: parts of one row of bricks, and parts of such rows)
+NOALLOC_GRIDS = [(130, 70, 40), (1750, 1740, 3), (330, 9000, 3), (46000, 64, 3), (52000, 77, 3), (65535, 65, 3)]
+
+
+@pytest.mark.parametrize("res", NOALLOC_GRIDS)
+@pytest.mark.parametrize("compiled", [False, True])
+def test_kept_values_noalloc(ctx, res, compiled):
     # without allocation: a few slabs; one cell plane per slab whose values do not fit the
-    # scratch at once (strips of brick rows), on square and on long planes
+    # scratch at once (parts of it in turn), on square and on long planes
     from test_zz_no_alloc import DeviceBuffers, check_same
 
-    c = ctx.program_from_source(GOLDEN / "random_csg1.sdf3d", path=True, force_compiled=True)
+    prog = ctx.program_from_source(GOLDEN / "random_csg1.sdf3d", path=True, force_compiled=compiled)
     bufs = DeviceBuffers(6_000_000, 12_000_000)
     try:
-        print(f"compiled noalloc {res}", flush=True)
-        for flags in (0, s2m.NO_NORMALS):
+        print(f"noalloc {res} compiled={compiled}", flush=True)
+        exact = s2m.CORNERS_EXACT if res[0] < 40000 else 0  # (more points per cell plane)
+        for flags in (0, s2m.NO_NORMALS | exact):
             p = s2m.Params((-1.0, -1.1, -0.9), (1.05, 1.0, 1.1), res, 1e-4, flags)
-            check_same(ctx, c, p, bufs)
+            check_same(ctx, prog, p, bufs)
     finally:
         bufs.free()
