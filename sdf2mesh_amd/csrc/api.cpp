@@ -1765,7 +1765,7 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
             A.vcap = b.vcap;
             A.eps = p->eps;
             A.normals = normals ? 1u : 0u;
-            A.run = sign_run((uint64_t)A.nbx * A.nby * A.nbz);
+            A.run = sign_run((uint64_t)A.nbx * A.nby * A.nbz, prog ? prog->n : 0u);
             auto part = [&](uint32_t k) {  // its own records and staging space
                 BrickArgs B = A;
                 if (L.nparts == 1) return B;
@@ -1776,7 +1776,7 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
                 B.owny = std::min(L.py, L.nby - B.by0);
                 B.nbx = std::min(B.ownx + 1u, L.nbx - B.bx0);
                 B.nby = std::min(B.owny + 1u, L.nby - B.by0);
-                B.run = sign_run((uint64_t)B.nbx * B.nby * B.nbz);
+                B.run = sign_run((uint64_t)B.nbx * B.nby * B.nbz, prog->n);
                 B.recs = recs + ((size_t)B.by0 * L.nbx + (size_t)B.bx0 * B.owny) * B.nbz;
                 B.alloc = b.counters + kNumCounters + k;
                 auto cells = [&](int axis, uint32_t brick) {  // cells of the axis in the bricks before it

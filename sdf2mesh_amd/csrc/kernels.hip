@@ -669,9 +669,12 @@ dim3 sign_grid(const BrickArgs& a) { return dim3((a.nbx + a.run - 1u) / a.run, (
 // over whole jobs, run 1 / 4 / 16: Mandelbulb 1024^3 in slabs of 680 K bricks 8.7 / 6.5 /
 // 6.1 ms, 128^3 (43 K bricks) 136 / 134 / 151 us, the compiled estimator at 200^3 (157 K
 // bricks) 1258 / 1249 / 1313 us.
-uint32_t sign_run(uint64_t bricks)
+// Long tapes take single bricks: their points cost so much that only the last round counts
+// (CSG-64 at 256^3 2.14 -> 2.00 ms, without allocation at 512^3 50.0 -> 48.8; a 9-op tree at
+// 256^3, 300 us, loses 15).
+uint32_t sign_run(uint64_t bricks, uint32_t nops)
 {
-    uint32_t run = 16;
+    uint32_t run = nops >= 100u ? 1u : 16u;
     while (run > 1u && bricks / run < 4u * 8192u) run /= 2u;
     return run;
 }
