@@ -263,4 +263,32 @@ __device__ __forceinline__ void run_general(const TT& T, uint32_t n, const float
     }
 }
 
+// tape_eval over a pruned tape too long to be staged: `list` holds the indices of the ops to run,
+// in order (a valid postfix program whose value equals the full tape's on its box); an operator
+// marked kSwapped takes its operands swapped.  The list is the same for all lanes of the wave,
+// which the opcodes' scalar dispatch relies on.
+__device__ __forceinline__ float tape_eval_list(const s2m_op* __restrict__ ops,
+                                                const uint16_t* __restrict__ list, uint32_t n,
+                                                float px, float py, float pz)
+{
+    float st[S2M_MAX_STACK];
+    float acc = 0.0f;
+    uint32_t sp = 0;
+    for (uint32_t k = 0; k < n; ++k) {
+        const uint32_t e = __builtin_amdgcn_readfirstlane(list[k]);
+        const s2m_op* o = ops + (e & (kSwapped - 1u));
+        const uint32_t code = __builtin_amdgcn_readfirstlane(o->code);
+        if (code < S2M_OP_UNION) {
+            const float d = eval_primitive(code, o->iarg, o->f, px, py, pz);
+            if (k != 0) st[sp++] = acc;
+            acc = d;
+        } else {
+            const float d1 = st[--sp];
+            const bool swapped = (e & kSwapped) != 0;
+            acc = apply_op(code, swapped ? acc : d1, swapped ? d1 : acc, o->f[0]);
+        }
+    }
+    return acc;
+}
+
 }  // namespace s2m
