@@ -1218,8 +1218,9 @@ int run_sparse(s2m_ctx* ctx, uint32_t n, const s2m_program* const* progs, const 
         HIP_TRY(ctx->sp_cellbits.ensure(want_s * 16 * sizeof(uint32_t)));
         HIP_TRY(ctx->sp_slot_rows.ensure(want_s * 4 * 64 * sizeof(uint32_t)));
         // staged cells are reserved 8 per live brick of a slot, in per-block chunks: about
-        // 2 x vertices + blocks x chunk (two launches); the device count is checked below
-        stage_cap = std::max(stage_cap, 2 * want_v + 2 * tile_blocks * kStageChunkHost);
+        // 2 x vertices + blocks x chunk (two launches, three with long programs); the device count
+        // is checked below
+        stage_cap = std::max(stage_cap, 2 * want_v + (lists_by_tile ? 3 : 2) * tile_blocks * kStageChunkHost);
         HIP_TRY(ctx->sp_stage.ensure(stage_cap * sizeof(float4)));
         ctx->stage_cap = stage_cap;
         HIP_TRY(ctx->sp_slot_stage.ensure(want_s * 2 * sizeof(uint32_t)));

@@ -104,7 +104,7 @@ constexpr uint32_t kTileBlocksPerCU = 8;    // most k_sp_tiles blocks per comput
 constexpr uint32_t kTileRecBytes = 2720;    // per slot: k_sp_tiles' staged record (sparse.hip)
 constexpr uint32_t kRowChunk = 4096;        // rows per chunk of the row offset scan (sparse.hip)
 constexpr uint32_t kChunkSumStride = 32;    // words between chunk sums (one 128-byte line each)
-constexpr uint32_t kQueues = 4;        // work queues of a pass (k_sp_tiles<1/0>, k_sp_emit<1/0>)
+constexpr uint32_t kQueues = 5;        // work queues of a pass (k_sp_tiles<1/0>, k_sp_emit<1/0>, k_sp_tiles<3>)
 constexpr uint32_t kQueueGroups = 64;  // counters per queue, 32 u32 (128 bytes) apart
 // Profiling marks of one sparse pass: prune (tiles, bricks) | eval+contour | quad count |
 // scan | emission
@@ -181,6 +181,7 @@ struct SpPass {
     uint16_t* lists;           // [slot][list_stride] pruned op indices ([tile] with lists_by_tile: programs
                                // longer than kStageOps are listed before their tile has a slot)
     uint32_t lists_by_tile;
+    uint32_t long_apart;       // k_sp_tiles<3> runs the slots whose program is not staged
     uint4* slot_info;          // [slot] tile, job, pruned length (| kLinearFlag), its flops per point
     uint32_t* gen_slots;       // the slots whose program is no fold (kGenUsed of them)
     uint32_t slot_cap;
@@ -263,7 +264,7 @@ hipError_t launch_tape_prepare(hipStream_t s, s2m_op* ops, uint32_t n);
 // cus: compute units of the device; tile_blocks: most blocks of a k_sp_tiles launch (each
 // holds a staging chunk); general_tiles: some tile's pruned program may not be a left fold
 // (false when every job's whole program is one: its pruned programs are then left folds).
-hipError_t launch_sparse_pass(hipStream_t s, const SpPass& P, const MeshBufs& b, int cus,
+hipError_t launch_sparse_pass(hipStream_t s, SpPass P, const MeshBufs& b, int cus,
                               uint32_t tile_blocks, bool general_tiles, int boundary_plane, hipEvent_t* marks);
 // Contour corner values given per cell (test hook): cells of the slab read their 8
 // corners from `corners` (8 floats per cell, cells in (z,y,x) order from plane z0).

@@ -838,6 +838,10 @@ struct TileGen {  // k_sp_tiles<0>: the same parts, staged per slot
     float pc[3][16];
     uint32_t mandel;  // the program holds a Mandelbulb
 };
+struct TileLong {  // k_sp_tiles<3>
+    TileAxes A;
+    float pc[3][16];
+};
 
 // ---------------------------------------------------------------------------------
 // n / d for n < 2^16 and d <= 256, r = recip(d): (n + 0.5) / d is at least 1 / (2 d) from an
@@ -1130,36 +1134,52 @@ constexpr uint32_t kBoxAxis = 16;  // most lattice indices of a tile box per axi
 static_assert(kList >= 8 * 8 * 8, "the point list doubles as the contour's candidate cells");
 static_assert(kTileThreads >= kBoxAxis * kBoxAxis, "one box row per thread");
 
+// Kinds of slots a launch runs: those that are no folds, folds, or both, each by a share of the
+// blocks.  Two launches leave most of the device idle while a small pass's few slots of the
+// one kind run, each some 15 to 30 us of latency; in one launch the folds are held to the
+// registers of the other kind (four waves per SIMD instead of seven), which costs more than it
+// saves from some 130 k tiles on.  Three trees, one launch against two, us: 160^3 182 / 222,
+// 256^3 168 / 195, 352^3 249 / 273, 384^3 279 / 287, 448^3 297 / 298, 640^3 478 / 441.
+// Slots whose program is too long to be staged have a launch of their own from some 2 k tiles on,
+// without the operand stacks in LDS (32 KB and more beside the box: three blocks per compute
+// unit instead of seven), and no other kinds share a launch then.  One launch for all against one
+// for each, us: a 599-op fold at 64^3 3120 / 3360, 128^3 2800 / 2720, 256^3 2810 / 2150, 512^3
+// 13,700 / 5600; a 511-op tree 3830 / 3900, 4700 / 4300, 3980 / 3920, 33,400 / 22,100.
+enum Kind : int { kGeneralKind = 0, kFoldKind = 1, kBothKinds = 2, kLongKind = 3 };
+constexpr uint64_t kBothTiles = 128u << 10, kBothTilesLong = 2u << 10;
+
 // k_sp_tiles: per slot (persistent, slots drawn from a work queue), the tile's pruned
 // program, staged in
 // LDS, at the lattice points of its closed box that the tile's cells need (all points for
 // programs that are not left folds), into an LDS box; then the tile's cells are contoured
-// from it (contour_tile).  LINEAR = 1 runs the slots whose program is a left fold and skips
-// the others, LINEAR = 0 the others (gen_slots).
+// from it (contour_tile).  KIND (below) selects the slots: left folds (the others are skipped),
+// the others (gen_slots) whose program is staged, or those whose program is longer and read
+// from memory.
 // Bound by instruction issue (three quarters of the issue slots at CSG-64 1024^3: 69.5 k slots,
 // 258 points and 57 vertices each): of 277 us there, 60 evaluate, 42 place vertices, 28 look for
 // sign changes, the rest is the fixed work of a tile.  355 us with the points dealt to all
 // lanes, half of them twice, and a 64-bit division per row; 300 with every block's first
 // staging chunk counted (512^3: 166, 151, now 136).
-template <int LINEAR>
+template <int KIND>
 __device__ __forceinline__ void tiles_body(const SpPass& P, uint32_t block, uint32_t blocks)
 {
-    extern __shared__ float box[];  // P.box_stride floats; LINEAR = 0: then the operand stacks
+    constexpr bool LINEAR = KIND == kFoldKind, LONG = KIND == kLongKind;
+    extern __shared__ float box[];  // P.box_stride floats; kGeneralKind: then the operand stacks
                                     // (P.prune_depth entries per thread and point)
     // left folds: the slot's record (k_sp_bricks); other programs: staged here
-    __shared__ std::conditional_t<LINEAR != 0, TileRec, TileGen> R;
+    __shared__ std::conditional_t<LINEAR, TileRec, std::conditional_t<LONG, TileLong, TileGen>> R;
     // points to evaluate; then the contour's candidate cells (contour_tile's `cand`)
     __shared__ uint16_t list[LINEAR ? kList : 8 * 8 * 8];
     __shared__ uint32_t nlist;
     __shared__ ContourLds L;
     __shared__ uint32_t sh_slot, sh_next;
     __shared__ uint8_t lb[64];  // the live bricks of the slot (contour_tile)
-    // LINEAR = 0: indices into the list of the slots that are no folds
+    // other programs: indices into the list of the slots that are no folds
     const uint32_t nslots = active_slots(P, LINEAR ? kSlotsUsed : kGenUsed);
-    constexpr uint32_t kQueue = LINEAR ? 0u : 1u;
+    constexpr uint32_t kQueue = LINEAR ? 0u : LONG ? 4u : 1u;
     if (thread_id() == 0) {  // the block's first staging chunk; published by the first slot's barriers
         L.base = (block + (LINEAR ? 0u : P.tile_blocks)) * kStageChunk;
-        L.left = kStageChunk;
+        L.left = LONG ? 0u : kStageChunk;  // (long programs' first chunks are counted)
     }
     uint64_t tiles_done = 0, points_done = 0, flops_done = 0;  // thread 0: this block's share
     const Turns Q(P, kQueue, block, blocks);
@@ -1171,7 +1191,7 @@ __device__ __forceinline__ void tiles_body(const SpPass& P, uint32_t block, uint
         const uint32_t s = sh_next;
         if (thread_id() < kRecPre && s < nslots) pre = P.slot_rec[(size_t)s * kRecVec + thread_id()];
     };
-    if constexpr (LINEAR != 0) {
+    if constexpr (LINEAR) {
         if (thread_id() == 0) nlist = 0;
         if (thread_id() == 0) sh_next = next;
         __syncthreads();
@@ -1186,7 +1206,7 @@ __device__ __forceinline__ void tiles_body(const SpPass& P, uint32_t block, uint
         const uint32_t slot = LINEAR ? sh_slot : P.gen_slots[sh_slot];
         if (thread_id() == 0) next = Q.drawn(Q.draw());  // prefetched
         const SlotHdr& H = [&]() -> const SlotHdr& {
-            if constexpr (LINEAR != 0) return R.H;
+            if constexpr (LINEAR) return R.H;
             else return P.slot_hdr[__builtin_amdgcn_readfirstlane(slot)];
         }();
         const uint32_t lens = __builtin_amdgcn_readfirstlane(H.lens);
@@ -1197,7 +1217,7 @@ __device__ __forceinline__ void tiles_body(const SpPass& P, uint32_t block, uint
                 prefetch();
             }
         };
-        if (((lens & kLinearFlag) != 0) != (LINEAR != 0)) {  // same for the whole block
+        if (((lens & kLinearFlag) != 0) != LINEAR || (!LINEAR && P.long_apart && (lens > kStageOps) != LONG)) {  // same for the block
             skip();
             continue;
         }
@@ -1218,7 +1238,7 @@ __device__ __forceinline__ void tiles_body(const SpPass& P, uint32_t block, uint
         uint64_t lv = ~0ull;
         uint32_t evaluated = 0;
         contour_reset(L);
-        if constexpr (LINEAR != 0) {
+        if constexpr (LINEAR) {
             lv = R.live;
             if (lv == 0) {  // no brick can hold an active cell: empty rows, no cell bits
                 if (thread_id() < 64) slot_row(P, kRowVtx, slot)[thread_id()] = 0;
@@ -1330,20 +1350,22 @@ __device__ __forceinline__ void tiles_body(const SpPass& P, uint32_t block, uint
             const uint32_t x0 = bxh & 0xffffffu, y0 = byh & 0xffffffu, z0 = bzh & 0xffffffu;
             const uint32_t nxy = nx * ny, npts = nxy * nz;
             const float rx = recip(nx), rxy = recip(nxy);
-            const bool staged = n <= kStageOps;
             if (thread_id() == 0) contour_reserve(P, L, 8u * 8u * 8u);
-            if (staged) stage_tape(R.T, J.ops, Lst, n);
+            const bool staged = !LONG && n <= kStageOps;
+            if constexpr (!LONG)
+                if (staged) stage_tape(R.T, J.ops, Lst, n);
             if (thread_id() < 24) load_tile_axes(R.A, J, tx, ty, J.tz0 + tzl, thread_id());
             if (thread_id() < 48) {
                 const uint32_t a = thread_id() >> 4, i = thread_id() & 15u;
                 const float* c = a == 0 ? J.cx + x0 : a == 1 ? J.cy + y0 : J.cz + z0;
                 if (i < (a == 0 ? nx : a == 1 ? ny : nz)) R.pc[a][i] = c[i];
             }
-            if (thread_id() == 0) R.mandel = 0;
-            __syncthreads();
-            if (staged)
-                for (uint32_t q = thread_id(); q < n; q += kTileThreads)
+            if constexpr (!LONG) {
+                if (thread_id() == 0) R.mandel = 0;
+                __syncthreads();
+                for (uint32_t q = thread_id(); staged && q < n; q += kTileThreads)
                     if (R.T.code[q] == S2M_OP_MANDELBULB) R.mandel = 1;
+            }
             __syncthreads();
             auto point = [&](uint32_t q, float& x, float& y, float& z) {  // its entry in the box
                 const uint32_t iz = div_by(q, rxy), r = q - iz * nxy;
@@ -1353,28 +1375,36 @@ __device__ __forceinline__ void tiles_body(const SpPass& P, uint32_t block, uint
                 z = R.pc[2][iz];
                 return (iz * by + iy) * bx + ix;
             };
-            float* stack = box + P.box_stride + thread_id();
-            if (staged && !R.mandel && P.prune_depth <= kWideDepth) {
-                for (uint32_t q0 = thread_id(); q0 < npts; q0 += kGeneralPoints * kTileThreads) {
-                    float x[kGeneralPoints], y[kGeneralPoints], z[kGeneralPoints], v[kGeneralPoints];
-                    uint32_t at[kGeneralPoints];
-#pragma unroll
-                    for (int p = 0; p < kGeneralPoints; ++p) {
-                        const uint32_t q = q0 + p * kTileThreads;
-                        at[p] = point(q < npts ? q : q0, x[p], y[p], z[p]);
-                    }
-                    run_general<kGeneralPoints, false>(R.T, n, x, y, z, v, stack, kTileThreads);
-#pragma unroll
-                    for (int p = 0; p < kGeneralPoints; ++p)
-                        if (q0 + p * kTileThreads < npts) box[at[p]] = v[p];
-                }
-            } else {
+            if (!staged) {
                 for (uint32_t q = thread_id(); q < npts; q += kTileThreads) {
-                    float x[1], y[1], z[1], v[1];
-                    const uint32_t at = point(q, x[0], y[0], z[0]);
-                    if (staged) run_general<1, true>(R.T, n, x, y, z, v, stack, kTileThreads);
-                    else v[0] = tape_eval_list(J.ops, Lst, n, x[0], y[0], z[0]);
-                    box[at] = v[0];
+                    float x, y, z;
+                    const uint32_t at = point(q, x, y, z);
+                    box[at] = tape_eval_list(J.ops, Lst, n, x, y, z);
+                }
+            }
+            if constexpr (!LONG) {
+                float* stack = box + P.box_stride + thread_id();
+                if (staged && !R.mandel && P.prune_depth <= kWideDepth) {
+                    for (uint32_t q0 = thread_id(); q0 < npts; q0 += kGeneralPoints * kTileThreads) {
+                        float x[kGeneralPoints], y[kGeneralPoints], z[kGeneralPoints], v[kGeneralPoints];
+                        uint32_t at[kGeneralPoints];
+#pragma unroll
+                        for (int p = 0; p < kGeneralPoints; ++p) {
+                            const uint32_t q = q0 + p * kTileThreads;
+                            at[p] = point(q < npts ? q : q0, x[p], y[p], z[p]);
+                        }
+                        run_general<kGeneralPoints, false>(R.T, n, x, y, z, v, stack, kTileThreads);
+#pragma unroll
+                        for (int p = 0; p < kGeneralPoints; ++p)
+                            if (q0 + p * kTileThreads < npts) box[at[p]] = v[p];
+                    }
+                } else if (staged) {
+                    for (uint32_t q = thread_id(); q < npts; q += kTileThreads) {
+                        float x[1], y[1], z[1], v[1];
+                        const uint32_t at = point(q, x[0], y[0], z[0]);
+                        run_general<1, true>(R.T, n, x, y, z, v, stack, kTileThreads);
+                        box[at] = v[0];
+                    }
                 }
             }
             evaluated = npts;
@@ -1401,33 +1431,29 @@ __device__ __forceinline__ void tiles_body(const SpPass& P, uint32_t block, uint
     }
 }
 
-// Kinds of slots a launch runs: those that are no folds, folds, or both, each by a share of the
-// blocks.  Two launches leave most of the device idle while a small pass's few slots of the
-// one kind run, each some 15 to 30 us of latency; in one launch the folds are held to the
-// registers of the other kind (four waves per SIMD instead of seven), which costs more than it
-// saves from some 130 k tiles on.  Three trees, one launch against two, us: 160^3 182 / 222,
-// 256^3 168 / 195, 352^3 249 / 273, 384^3 279 / 287, 448^3 297 / 298, 640^3 478 / 441.
-enum Kind : int { kGeneralKind = 0, kFoldKind = 1, kBothKinds = 2 };
-constexpr uint64_t kBothTiles = 128u << 10;
-
 template <int KIND>
 __global__ void k_sp_tiles(SpPass P);
 template <>
 __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_sp_tiles<kFoldKind>(SpPass P)
 {
-    tiles_body<1>(P, blockIdx.x, gridDim.x);
+    tiles_body<kFoldKind>(P, blockIdx.x, gridDim.x);
 }
 template <>
 __global__ __launch_bounds__(kTileThreads) void k_sp_tiles<kGeneralKind>(SpPass P)
 {
-    tiles_body<0>(P, blockIdx.x, gridDim.x);
+    tiles_body<kGeneralKind>(P, blockIdx.x, gridDim.x);
+}
+template <>
+__global__ __launch_bounds__(kTileThreads) void k_sp_tiles<kLongKind>(SpPass P)
+{
+    tiles_body<kLongKind>(P, blockIdx.x, gridDim.x);
 }
 template <>
 __global__ __launch_bounds__(kTileThreads) void k_sp_tiles<kBothKinds>(SpPass P)
 {
     const uint32_t general = general_blocks(active_slots(P, kGenUsed), active_slots(P, kSlotsUsed));
-    if (blockIdx.x >= general) tiles_body<1>(P, blockIdx.x - general, gridDim.x - general);
-    else tiles_body<0>(P, blockIdx.x, general);
+    if (blockIdx.x >= general) tiles_body<kFoldKind>(P, blockIdx.x - general, gridDim.x - general);
+    else tiles_body<kGeneralKind>(P, blockIdx.x, general);
 }
 
 // ---------------------------------------------------------------------------------
@@ -1986,7 +2012,7 @@ static uint32_t resident_blocks(K kernel, int threads, size_t smem, int cus, uin
     return std::min<uint32_t>(cap, (uint32_t)cus * (uint32_t)per_cu);
 }
 
-hipError_t launch_sparse_pass(hipStream_t s, const SpPass& P, const MeshBufs& b, int cus,
+hipError_t launch_sparse_pass(hipStream_t s, SpPass P, const MeshBufs& b, int cus,
                               uint32_t tile_blocks, bool general_tiles, int boundary_plane, hipEvent_t* marks)
 {
     if (P.ntiles == 0) return hipSuccess;
@@ -2007,7 +2033,8 @@ hipError_t launch_sparse_pass(hipStream_t s, const SpPass& P, const MeshBufs& b,
     const size_t gsmem = smem + (size_t)P.prune_depth * (P.prune_depth <= kWideDepth ? kGeneralPoints : 1) *
                                     kTileThreads * sizeof(float);
     const size_t esmem = (size_t)P.prune_depth * 4u * 64u * sizeof(float);
-    const bool both = general_tiles && P.ntiles <= kBothTiles;
+    const bool both = general_tiles && P.ntiles <= (P.lists_by_tile ? kBothTilesLong : kBothTiles);
+    P.long_apart = P.lists_by_tile && !both ? 1u : 0u;
     auto tiles = [&](auto kernel, size_t lds) {
         hipLaunchKernelGGL(kernel, dim3(resident_blocks(kernel, kTileThreads, lds, cus, tile_blocks)), dim3(kTileThreads),
                            lds, s, P);
@@ -2020,6 +2047,7 @@ hipError_t launch_sparse_pass(hipStream_t s, const SpPass& P, const MeshBufs& b,
     } else {
         tiles(k_sp_tiles<kFoldKind>, smem);
         if (general_tiles) tiles(k_sp_tiles<kGeneralKind>, gsmem);
+        if (P.long_apart) tiles(k_sp_tiles<kLongKind>, smem);
     }
     mark(2);
     hipLaunchKernelGGL(k_sp_quadcount, dim3(resident_blocks(k_sp_quadcount, 64, 0, cus, big)), dim3(64), 0, s,
