@@ -1432,9 +1432,9 @@ hipError_t lattice_prog(hipStream_t s, const s2m_program* prog, const float* cx,
                                  args, nullptr);
 }
 
-hipError_t signs_prog(hipStream_t s, const s2m_program* prog, BrickArgs a)
+hipError_t signs_prog(hipStream_t s, const s2m_program* prog, BrickArgs a, bool early)
 {
-    if (!prog->module) return launch_signs(s, a, prog->ops.data(), prog->d_ops, prog->n);
+    if (!prog->module) return launch_signs(s, a, prog->ops.data(), prog->d_ops, prog->n, early);
     void* args[] = {&a};
     const dim3 g = sign_grid(a);
     return hipModuleLaunchKernel(prog->k_signs, g.x, g.y, g.z, 256, 1, 1, 0, s, args, nullptr);
@@ -1571,7 +1571,8 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
     // kept values), and the first evaluation waits for the tables queued before it.
     const bool piped = !fx && !h_corners && slab < j.nz_cells;
     // the Mandelbulb's signs decided early, else the values of the sign pass kept
-    const s2m_op* const early = prog && sign_early(prog->ops.data(), prog->n) ? prog->d_ops : nullptr;
+    const uint64_t points = (uint64_t)j.ax[0].coord.size() * j.ax[1].coord.size() * j.ax[2].coord.size();
+    const s2m_op* const early = prog && sign_early(prog->ops.data(), prog->n, points) ? prog->d_ops : nullptr;
     const bool keep_vals = prog && !h_corners && !early;
     DenseLayout L = dense_layout(j, slab, !h_corners, piped, want_s, keep_vals);
     if (fx) {  // the largest slab (at most the usual one) whose buffers fit the scratch
@@ -1766,7 +1767,7 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
             A.vcap = b.vcap;
             A.eps = p->eps;
             A.normals = normals ? 1u : 0u;
-            A.run = sign_run((uint64_t)A.nbx * A.nby * A.nbz, prog ? prog->n : 0u);
+            A.run = prog ? sign_run((uint64_t)A.nbx * A.nby * A.nbz, prog->ops.data(), prog->n) : 1u;
             auto part = [&](uint32_t k) {  // its own records and staging space
                 BrickArgs B = A;
                 if (L.nparts == 1) return B;
@@ -1777,7 +1778,7 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
                 B.owny = std::min(L.py, L.nby - B.by0);
                 B.nbx = std::min(B.ownx + 1u, L.nbx - B.bx0);
                 B.nby = std::min(B.owny + 1u, L.nby - B.by0);
-                B.run = sign_run((uint64_t)B.nbx * B.nby * B.nbz, prog->n);
+                B.run = sign_run((uint64_t)B.nbx * B.nby * B.nbz, prog->ops.data(), prog->n);
                 B.recs = recs + ((size_t)B.by0 * L.nbx + (size_t)B.bx0 * B.owny) * B.nbz;
                 B.alloc = b.counters + kNumCounters + k;
                 auto cells = [&](int axis, uint32_t brick) {  // cells of the axis in the bricks before it
@@ -1795,7 +1796,7 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
             if (piped && words_free[cur]) HIP_TRY(hipStreamWaitEvent(es, words_free[cur], 0));
             if (m[0]) HIP_TRY(hipEventRecord(m[0], es));
             if (!h_corners) {
-                HIP_TRY(signs_prog(es, prog, part(0)));
+                HIP_TRY(signs_prog(es, prog, part(0), early != nullptr));
                 lattice_points += (uint64_t)L.nx * L.ny * nzl;
             }
             if (m[1]) HIP_TRY(hipEventRecord(m[1], es));
@@ -1810,7 +1811,7 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
                 HIP_TRY(launch_cells_from_corners(ctx->stream, a, src, bs, 0));
             } else {
                 for (uint32_t k = 0; k < L.nparts; ++k) {
-                    if (k) HIP_TRY(signs_prog(ctx->stream, prog, part(k)));
+                    if (k) HIP_TRY(signs_prog(ctx->stream, prog, part(k), early != nullptr));
                     HIP_TRY(launch_find_bricks(ctx->stream, part(k)));
                     HIP_TRY(launch_contour(ctx->stream, part(k), early));
                 }

@@ -237,10 +237,11 @@ hipError_t launch_eval_lattice(hipStream_t s, const s2m_op* ops, uint32_t nops, 
 // (sign_early), NULL where the sign pass has kept the values.
 struct BrickArgs;
 bool mandel_power8(const s2m_op* ops, uint32_t n);  // the tape is one power-8 Mandelbulb op
-bool sign_early(const s2m_op* ops, uint32_t n);     // its signs are decided early (no values to keep)
+bool sign_early(const s2m_op* ops, uint32_t n, uint64_t points);  // its signs are decided early (no values to keep)
 dim3 sign_grid(const BrickArgs& a);                 // blocks of 256
-uint32_t sign_run(uint64_t bricks, uint32_t nops);  // BrickArgs::run for a slab of so many bricks and a tape
-hipError_t launch_signs(hipStream_t s, const BrickArgs& a, const s2m_op* host_ops, const s2m_op* ops, uint32_t nops);
+uint32_t sign_run(uint64_t bricks, const s2m_op* ops, uint32_t nops);  // BrickArgs::run
+hipError_t launch_signs(hipStream_t s, const BrickArgs& a, const s2m_op* host_ops, const s2m_op* ops, uint32_t nops,
+                        bool early);
 hipError_t launch_find_bricks(hipStream_t s, const BrickArgs& a);
 hipError_t launch_contour(hipStream_t s, const BrickArgs& a, const s2m_op* op);
 hipError_t launch_emit(hipStream_t s, const BrickArgs& a, const s2m_op* op);

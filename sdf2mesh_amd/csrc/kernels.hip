@@ -659,7 +659,16 @@ static bool mandel_sign_ok(const s2m_op& o)
     return o.f[1] >= 1.5f && o.f[1] <= 16.0f && o.f[2] >= 0.0f && o.f[2] <= 1000.0f && (o.iarg & 0xffffu) >= 1u;
 }
 
-bool sign_early(const s2m_op* ops, uint32_t n) { return mandel_power8(ops, n) && mandel_sign_ok(*ops); }
+// Whether a Mandelbulb's signs are decided early.  That saves part of every orbit, but the surface's
+// corners and taps are evaluated afterwards, in waves that are not full and for orbits that take
+// every iteration; else values are kept.  So it pays with many points to an iteration.  Early / kept,
+// us, on the cube of edge 2.5: 8 iterations 128^3 90 / 85, 256^3 190 / 184, 640^3 1350 / 1450,
+// 16 iterations 128^3 104 / 92, 256^3 250 / 229, 640^3 1710 / 1840, 60 iterations 128^3 180 / 134,
+// 400^3 1228 / 1129, 640^3 3790 / 4090, 128 iterations 256^3 963 / 628.
+bool sign_early(const s2m_op* ops, uint32_t n, uint64_t points)
+{
+    return mandel_power8(ops, n) && mandel_sign_ok(*ops) && points >= (uint64_t)(ops->iarg & 0xffffu) << 20;
+}
 
 dim3 sign_grid(const BrickArgs& a) { return dim3((a.nbx + a.run - 1u) / a.run, (a.nby + 3u) / 4u, a.nbz); }
 
@@ -672,19 +681,24 @@ dim3 sign_grid(const BrickArgs& a) { return dim3((a.nbx + a.run - 1u) / a.run, (
 // Long tapes take single bricks: their points cost so much that only the last round counts
 // (CSG-64 at 256^3 2.14 -> 2.00 ms, without allocation at 512^3 50.0 -> 48.8; a 9-op tree at
 // 256^3, 300 us, loses 15).
-uint32_t sign_run(uint64_t bricks, uint32_t nops)
+// Likewise the more iterations a Mandelbulb takes, the shorter its runs (60 iterations, exact corners:
+// 256^3 1.68 ms with runs of 1, 2.14 of 16; 512^3 7.2, 6.3).
+uint32_t sign_run(uint64_t bricks, const s2m_op* ops, uint32_t nops)
 {
-    uint32_t run = nops >= 100u ? 1u : 16u;
-    while (run > 1u && bricks / run < 4u * 8192u) run /= 2u;
+    if (nops >= 100u) return 1;
+    const uint32_t iters = mandel_power8(ops, nops) ? ops->iarg & 0xffffu : 0u;
+    uint32_t run = 16;
+    while (run > 1u && bricks / run < 4u * 8192u * std::max(1u, iters / 8u)) run /= 2u;
     return run;
 }
 
-hipError_t launch_signs(hipStream_t s, const BrickArgs& a, const s2m_op* host_ops, const s2m_op* ops, uint32_t nops)
+hipError_t launch_signs(hipStream_t s, const BrickArgs& a, const s2m_op* host_ops, const s2m_op* ops, uint32_t nops,
+                        bool early)
 {
     const dim3 grid = sign_grid(a);
-    if (!mandel_power8(host_ops, nops)) hipLaunchKernelGGL(k_signs<0>, grid, dim3(256), 0, s, a, ops, nops);
-    else if (!mandel_sign_ok(*host_ops)) hipLaunchKernelGGL(k_signs<1>, grid, dim3(256), 0, s, a, ops, nops);
-    else hipLaunchKernelGGL(k_signs<2>, grid, dim3(256), 0, s, a, ops, nops);
+    if (early) hipLaunchKernelGGL(k_signs<2>, grid, dim3(256), 0, s, a, ops, nops);
+    else if (mandel_power8(host_ops, nops)) hipLaunchKernelGGL(k_signs<1>, grid, dim3(256), 0, s, a, ops, nops);
+    else hipLaunchKernelGGL(k_signs<0>, grid, dim3(256), 0, s, a, ops, nops);
     return hipGetLastError();
 }
 

@@ -65,6 +65,21 @@ def test_mandelbulb_signs_of_deep_orbits(ctx, iterations, swap):
     same(ctx.mesh(a, p), ctx.mesh(b, p))
 
 
+# Signs are decided early from 2^20 lattice points per iteration on: grids around that line and past
+# it, with bailouts and offsets at their limits, and one whose orbits take 256 iterations.
+@pytest.mark.parametrize("iterations,bailout,offset,swap,res", [
+    (1, 2.0, 0.003, True, 100), (1, 2.0, 0.003, True, 101), (2, 4.0, 0.0, True, 131), (8, 2.0, 0.003, True, 202),
+    (8, 2.0, 0.003, False, 203), (8, 1.5, 0.003, True, 206), (8, 16.0, 0.003, False, 206), (8, 2.0, 1.0, True, 206),
+    (256, 2.0, 0.0, True, 646)])
+def test_mandelbulb_early_signs(ctx, iterations, bailout, offset, swap, res):
+    m = tape.mandelbulb(iterations, bailout=bailout, offset=offset, swap_yz=swap)
+    a, b = ctx.program(m), ctx.program(tape.union(m, m))
+    for flags in (0, s2m.CORNERS_EXACT) if res < 300 else (0,):
+        print(f"early signs {iterations} {bailout} {offset} {swap} {res} {flags}", flush=True)
+        p = s2m.Params((-1.25,) * 3, (1.25, 1.25, 1.2), (res, res, res), 1e-4, flags)
+        same(ctx.mesh(a, p), ctx.mesh(b, s2m.Params(p.bb_min, p.bb_max, p.res, p.eps, flags | s2m.DENSE_EVAL)))
+
+
 OPS = [tape.union, tape.intersection, tape.subtraction] + [
     (lambda f: lambda a, b: f(a, b, 0.08))(f)
     for f in (tape.smooth_union, tape.smooth_intersection, tape.smooth_subtraction)]
