@@ -568,12 +568,9 @@ struct Readback {
     }
 };
 
-// Before an attempt of the job: host arrays of at least vcap vertices and tcap triangles
-// (kept from an earlier call when large enough), no copy queued, no earlier attempt's copy
-// still reading the device buffers the attempt will write.
-int readback_begin(s2m_ctx* ctx, Readback& rb, uint64_t vcap, uint64_t tcap)
+// Host arrays of at least vcap vertices and tcap triangles (kept when large enough).
+int readback_arrays(Readback& rb, uint64_t vcap, uint64_t tcap)
 {
-    HIP_TRY(hipStreamSynchronize(ctx->copy_stream));
     if (rb.vcap < vcap || !rb.vtx) {
         host_release(rb.vtx);
         host_release(rb.keys);
@@ -595,6 +592,16 @@ int readback_begin(s2m_ctx* ctx, Readback& rb, uint64_t vcap, uint64_t tcap)
     if (!rb.vtx || !rb.tri || (rb.want_keys && (!rb.keys || !rb.signs)))
         return fail(S2M_E_OOM, "host allocation of %llu vertices / %llu triangles failed",
                     (unsigned long long)vcap, (unsigned long long)tcap);
+    return S2M_OK;
+}
+
+// Before an attempt of the job: host arrays of at least vcap vertices and tcap triangles, no
+// copy queued, no earlier attempt's copy still reading the device buffers the attempt will write.
+int readback_begin(s2m_ctx* ctx, Readback& rb, uint64_t vcap, uint64_t tcap)
+{
+    HIP_TRY(hipStreamSynchronize(ctx->copy_stream));
+    const int rc = readback_arrays(rb, vcap, tcap);
+    if (rc) return rc;
     rb.v_done = rb.t_done = 0;
     rb.passes_done = 0;
     rb.stopped = false;
@@ -738,8 +745,11 @@ int readback_copy(s2m_ctx* ctx, Readback& rb, uint64_t nv, uint64_t nt)
 
 // Pass rb.passes_done is queued and followed by readback_mark: once its totals are known,
 // queue the copies of its vertices and triangles behind its event.  A pass whose totals or capacity use exceed
-// the attempt's capacities stops the copies (the attempt will repeat).
-int readback_pass(s2m_ctx* ctx, Readback& rb, uint64_t vcap, uint64_t tcap, uint64_t slot_cap, uint64_t stage_cap)
+// the attempt's capacities stops the copies (the attempt will repeat).  npass: slabs of a dense job,
+// whose host arrays grow, before anything is copied, to what its first vertices foretell (else
+// a mesh above the estimate is copied when the job has ended), 0: as they are.
+int readback_pass(s2m_ctx* ctx, Readback& rb, uint64_t vcap, uint64_t tcap, uint64_t slot_cap, uint64_t stage_cap,
+                  uint32_t npass = 0)
 {
     const uint32_t k = rb.passes_done++;
     if (rb.stopped) return S2M_OK;
@@ -747,6 +757,12 @@ int readback_pass(s2m_ctx* ctx, Readback& rb, uint64_t vcap, uint64_t tcap, uint
     const int wrc = snapshot_wait(ctx, k, snap);
     if (wrc) return wrc;
     const uint64_t nv = snap[0], nt = snap[1], slots = snap[2], staged = snap[3];
+    if (npass && rb.v_done == 0 && rb.t_done == 0 && nv <= vcap && nt <= tcap) {
+        auto foretold = [&](uint64_t n) { return n * npass / (k + 1) + n * npass / (k + 1) / 8; };
+        const int grc = readback_arrays(rb, std::max(rb.vcap, std::min(vcap, foretold(nv))),
+                                        std::max(rb.tcap, std::min(tcap, foretold(nt))));
+        if (grc) return grc;
+    }
     if (nv > vcap || nt > tcap || nv > rb.vcap || nt > rb.tcap || slots > slot_cap || staged > stage_cap ||
         nv < rb.v_done || nt < rb.t_done) {
         rb.stopped = true;
@@ -758,10 +774,10 @@ int readback_pass(s2m_ctx* ctx, Readback& rb, uint64_t vcap, uint64_t tcap, uint
 
 // Every pass up to npass-1 whose copies are not queued yet, in order.
 int readback_passes(s2m_ctx* ctx, Readback& rb, uint32_t npass, uint64_t vcap, uint64_t tcap, uint64_t slot_cap,
-                    uint64_t stage_cap)
+                    uint64_t stage_cap, bool dense = false)
 {
     while (rb.passes_done < npass) {
-        const int rc = readback_pass(ctx, rb, vcap, tcap, slot_cap, stage_cap);
+        const int rc = readback_pass(ctx, rb, vcap, tcap, slot_cap, stage_cap, dense ? npass : 0);
         if (rc) return rc;
     }
     return S2M_OK;
@@ -1835,7 +1851,7 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
             if (rb) {  // the slab's vertices and triangles are final; the copies of the slab two
                        // before (waiting for it leaves this slab and the next evaluation queued)
                 int rrc = readback_mark(ctx, (uint32_t)slabs);
-                if (!rrc && slabs > 1) rrc = readback_pass(ctx, *rb, want_v, want_t, ~0ull, L.stage_cap);
+                if (!rrc && slabs > 1) rrc = readback_pass(ctx, *rb, want_v, want_t, ~0ull, L.stage_cap, nslabs);
                 if (rrc) return rrc;
             }
             if (prof) ev.insert(ev.end(), m, m + 6);
@@ -1846,7 +1862,7 @@ int run_job(s2m_ctx* ctx, const s2m_program* prog, const s2m_params* p, const Jo
             HIP_TRY(hipEventRecord(ev_end, ctx->stream));
         }
         if (rb) {  // copies of each slab's mesh while the later slabs run
-            const int rrc = readback_passes(ctx, *rb, (uint32_t)slabs, want_v, want_t, ~0ull, L.stage_cap);
+            const int rrc = readback_passes(ctx, *rb, (uint32_t)slabs, want_v, want_t, ~0ull, L.stage_cap, true);
             if (rrc) return rrc;
         }
         if (land) {  // a small mesh's copy behind its last kernel

@@ -55,6 +55,25 @@ def test_streamed_equals_device_resident(ctx, node, res, bounds):
     same(streamed, device_mesh_copied(ctx, prog, p))
 
 
+@pytest.mark.parametrize("where", ["everywhere", "below", "above"])
+def test_streamed_mesh_above_its_estimate(where):
+    # dense slabs whose first vertices foretell more than the estimate of 12 per cell of a plane
+    # (rightly, or too much), or less than the mesh has: the host arrays grow before the first
+    # copy, keep their size, or are replaced at the end
+    z = {"everywhere": np.arange(-0.9, 0.9, 0.06), "below": np.arange(-0.95, -0.4, 0.03),
+         "above": np.arange(0.1, 0.95, 0.04)}[where]
+    node = tape.fold([tape.box((0.0, 0.0, float(c)), (1.4, 1.4, 0.018)) for c in z], op=tape.union)
+    p = s2m.Params((-0.75,) * 2 + (-1.0,), (0.75,) * 2 + (1.0,), (208, 208, 256), 1e-4, s2m.DENSE_EVAL)
+    with s2m.Context(0) as fresh:
+        prog = fresh.program(node)
+        for _ in range(2):
+            streamed = fresh.mesh(prog, p)
+            assert fresh.last_timing()["slabs"] > 1
+            print(f"{where}: {len(streamed.vertices)} vertices", flush=True)
+            assert len(streamed.vertices) > 12 * 208 * 208
+            same(streamed, device_mesh_copied(fresh, prog, p))
+
+
 def test_pool_steady_state(ctx):
     prog = ctx.program(tape.csg64())
     big = s2m.Params.reference(512, 2.0)
