@@ -279,12 +279,13 @@ void s2m_mesh_free(s2m_mesh_out* out);
 /* No counterpart in the reference.  For callers that cannot allocate device memory
  * (serving loops that must not call hipMalloc, harnesses that forbid it): the mesh of
  * s2m_mesh_device, computed by the dense-path kernels, written into the caller's device
- * buffers.  Every working buffer (coordinate tables, the slab's sign words, bricks and staged
- * vertices, block counts, activity bits, counters) is carved from one static device array of
- * S2M_NOALLOC_SCRATCH_BYTES that each GPU the library runs on holds until the process
- * ends; slabs shrink until they fit it.  The call performs no hipMalloc, hipFree or
- * other allocating HIP call.  Errors: S2M_E_ARG when one cell plane per slab does not fit
- * the scratch; S2M_E_OOM when the mesh exceeds vcap / tcap, with out->nvtx / out->ntri set
+ * buffers.  Every working buffer (coordinate tables, the slab's sign words, kept values,
+ * bricks and staged vertices, block counts, activity bits, counters) is carved from one static
+ * device array of S2M_NOALLOC_SCRATCH_BYTES that each GPU the library runs on holds until the
+ * process ends; slabs shrink until they fit it, and a single cell plane's signs and values are
+ * taken in parts where they do not fit at once.  The call performs no hipMalloc, hipFree or
+ * other allocating HIP call.  Errors: S2M_E_ARG when what is left of one cell plane (records and
+ * staged vertices of every cell, some 15 bytes a cell) does not fit the scratch; S2M_E_OOM when the mesh exceeds vcap / tcap, with out->nvtx / out->ntri set
  * to the sizes it needs (the triangle count is a lower bound when the vertices
  * overflowed).  All calls on one GPU share the array: calls that overlapped would race,
  * so the library runs them one at a time per device (a lock held until the call has

@@ -167,10 +167,10 @@ struct s2m_ctx {
     // copy_stream while later passes compute on `stream`
     hipStream_t copy_stream = nullptr;
     // dense slabs: the signs of slab k + 1 are evaluated on eval_stream while slab k is
-    // contoured on `stream`
-    // created by the first such job: the device runs a process's streams on four hardware
-    // queues, and a stream nobody uses can still put two busy ones on the same queue (a server's
-    // three contexts: 24 requests in 4.5 - 4.9 ms, 5.3 - 7.1 with a third stream for each)
+    // contoured on `stream`.  Created by the first such job: the device runs a process's
+    // streams on four hardware queues, and a stream nobody uses can still put two busy ones on
+    // the same queue (a server's three contexts: 24 requests in 5.0 - 5.2 ms; when that was
+    // 4.5 - 4.9, it took 5.3 - 7.1 with a third stream for each)
     hipStream_t eval_stream = nullptr;
     PinnedBuf host_snap;                 // per pass: its totals and capacity use (kSnapWords)
     PinnedBuf host_land;                 // land_mesh's staging of arrays too small to page-lock
@@ -814,8 +814,10 @@ int readback_finish(s2m_ctx* ctx, Readback& rb, uint64_t nv, uint64_t nt)
 
 // Passes of a single sparse job whose mesh is streamed to host memory: the copy of one pass
 // overlaps the next pass's work, but a pass costs about 110 us beside its tiles and its copies
-// some 30.  One per 256 cell planes, 2 to 4 from 256 planes on (at 256^3 one would do, but a
-// job of that size is expected to be streamed); us in 1 / 2 / 3 / 4 passes:
+// some 30.  One per 256 cell planes, 2 to 4 from 256 planes on.  That is the right side of the
+// line from 512 planes on; at 256 one pass would be quicker (the table) and at 384 is as quick
+// for two of three programs, but that a job of 256 planes is streamed is a behaviour the tests
+// hold (test_gpu_readback.py), and s2m_tune takes one pass where that is quicker.  us in 1 / 2 / 3 / 4 passes:
 //             CSG-64 (much to copy)          a tree                      a torus
 //   256^3     453 / 477 / 528 / 601     199 / 248 / 316 / 359     204 / 223 / 261 / 303
 //   384^3     810 / 729 / 803 / 840     300 / 327 / 380 / 428     349 / 352 / 377 / 409
@@ -832,9 +834,6 @@ uint32_t stream_passes(uint32_t tile_layers)
 // one.  2.3 GB of 288 there; the next power of two is split in four.
 constexpr uint64_t kSparsePassBytes = 4ull << 30;
 
-// Is the program a left fold of library primitives (P0 P1 op1 P2 op2 ...) short enough to
-// be staged (sparse.hip, kStageOps = 128)?  Every pruned sub-program of one is one too:
-// pruning keeps either the accumulated value or the right operand, a single primitive.
 // Is the program a left fold of unions and smooth unions (k > 0) of library primitives
 // other than the Mandelbulb (prune_fold)?
 bool union_fold_program(const std::vector<s2m_op>& ops)
@@ -852,6 +851,9 @@ bool union_fold_program(const std::vector<s2m_op>& ops)
     return true;
 }
 
+// Is the program a left fold of library primitives (P0 P1 op1 P2 op2 ...) short enough to
+// be staged (sparse.hip, kStageOps = 128)?  Every pruned sub-program of one is one too:
+// pruning keeps either the accumulated value or the right operand, a single primitive.
 bool left_fold_program(const std::vector<s2m_op>& ops)
 {
     const size_t n = ops.size();

@@ -877,8 +877,8 @@ hipError_t launch_quads(hipStream_t s, const SlabArgs& a, const MeshBufs& b, con
 // ---------------------------------------------------------------------------------
 // Scratch of the no-allocation entry point (s2m_mesh_device_noalloc): one static device
 // array per GPU that holds every working buffer of a dense job (coordinate tables, the
-// slab lattice, cell -> vertex planes, block counts and offsets, activity bits,
-// counters).  Host code never passes the array's name to a kernel or a copy (on the
+// slab's sign words, kept values, brick records and staged vertices, activity bits with
+// their prefix tables, block counts and offsets, counters).  Host code never passes the array's name to a kernel or a copy (on the
 // host it names a stand-in, not the device memory): it uses the address
 // hipGetSymbolAddress returns for the device, taken once per device by noalloc_scratch.
 // ---------------------------------------------------------------------------------

@@ -18,9 +18,11 @@
 //   k_sp_tiles      per slot (one block): the pruned program in LDS (left folds: from the
 //                   record, read while the block contours the slot before), at the
 //                   lattice points the tile's live bricks use (left folds) or at all
-//                   points of its box (other programs), into an LDS box; then the tile's
-//                   cells: vertex and sign bits of each active cell, staged compactly, the
-//                   slot's cell bits and each row segment's vertex count
+//                   points of its box (other programs; those too long to be staged in
+//                   a large pass: a launch without operand stacks in LDS), into an LDS
+//                   box; then the tile's cells: vertex and sign bits of each active cell,
+//                   staged compactly, the slot's cell bits and each row segment's vertex
+//                   count
 //   k_sp_quadcount  per slot: valid quads of the staged cells (neighbour cells' bits),
 //                   two triangles each, per row segment; invalid quads counted
 //   k_sp_rowsum / k_sp_rowdown   offsets of the row segments in the reference's
