@@ -759,9 +759,12 @@ int readback_pass(s2m_ctx* ctx, Readback& rb, uint64_t vcap, uint64_t tcap, uint
     const uint64_t nv = snap[0], nt = snap[1], slots = snap[2], staged = snap[3];
     if (npass && rb.v_done == 0 && rb.t_done == 0 && nv <= vcap && nt <= tcap) {
         auto foretold = [&](uint64_t n) { return n * npass / (k + 1) + n * npass / (k + 1) / 8; };
-        const int grc = readback_arrays(rb, std::max(rb.vcap, std::min(vcap, foretold(nv))),
-                                        std::max(rb.tcap, std::min(tcap, foretold(nt))));
-        if (grc) return grc;
+        if (readback_arrays(rb, std::max(rb.vcap, std::min(vcap, foretold(nv))),
+                            std::max(rb.tcap, std::min(tcap, foretold(nt)))) != S2M_OK) {
+            rb.release();  // more than it may need: copied into arrays of its size at the end
+            rb.stopped = true;
+            return S2M_OK;
+        }
     }
     if (nv > vcap || nt > tcap || nv > rb.vcap || nt > rb.tcap || slots > slot_cap || staged > stage_cap ||
         nv < rb.v_done || nt < rb.t_done) {
